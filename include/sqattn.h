@@ -120,6 +120,15 @@ typedef struct sq_prefill_params {
 size_t sq_prefill_workspace_bytes(int64_t batch, int64_t num_kv_heads, int64_t kv_len, int64_t head_dim);
 
 /*
+ * The workspace with which sq_prefill_fwd / sq_prefill_int8qk_fwd also split the key ranges of a launch whose query blocks
+ * do not fill the chip (short sequences, few heads, chunks behind a long context) over more workgroups: the size above plus
+ * the parts' fp32 partial results, where this call would be split, else the size above.  `params` is the call's.  With a
+ * smaller workspace the call runs unsplit.
+ */
+size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t qo_len, int64_t kv_len,
+                                        const sq_prefill_params* params);
+
+/*
  * out = softmax2(q~ k^T) v per the reference's blockwise algorithm, q~ = q * log2e/sqrt(D) rounded to q's
  * dtype.  q, k, v: bf16 or fp16 (same type), D == 128 (the host zero-pads smaller heads).  q4/k4 (may be NULL = alias of q/k) are the
  * operands used inside the 4-bit window range.  out: bf16/fp16/fp32, same shape as q.

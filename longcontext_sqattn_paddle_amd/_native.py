@@ -86,6 +86,7 @@ SYMBOLS = {
     "sq_abi_version": (ctypes.c_int, []),
     "sq_last_error": (ctypes.c_char_p, []),
     "sq_prefill_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 4),
+    "sq_prefill_workspace_bytes_split": (ctypes.c_size_t, [ctypes.c_int64] * 5 + [ctypes.POINTER(PrefillParams)]),
     "sq_prefill_fwd": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, ctypes.POINTER(PrefillParams), ctypes.c_void_p]),
     "sq_decode_num_splits": (ctypes.c_int32, [ctypes.c_int64] * 3),
     "sq_decode_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]),

@@ -20,6 +20,7 @@
 //   * the tile step is laid out by hand in slots of one MFMA plus the vector and LDS work that runs beside it;
 //   * blockIdx -> (kv head, q head, q block) mapping keeps the q-heads of one KV head on the same XCD(s) so
 //     their K/V tiles are shared in that XCD's L2, and issues the longest (last) query blocks first.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -39,6 +40,14 @@ constexpr int kKTileBytes = kBN * kKStride;
 constexpr int kVTileBytes = kD * kVStride;
 constexpr int kStageBytes = kKTileBytes + kVTileBytes;
 constexpr int kMaxHeads = 128;
+constexpr int kMaxSplitWork = 512;       // workgroups per (batch, q head) of a launch with split key ranges
+
+// One workgroup of a split launch: part `part` of `parts` of query block `qb`; `slot` is the first of the block's `parts`
+// places in the partial results (parts > 1)
+struct SplitWork {
+  uint16_t qb, slot;
+  uint8_t part, parts;
+};
 
 struct PrefillArgs {
   const void* q;
@@ -56,11 +65,16 @@ struct PrefillArgs {
   int32_t B, Hq, Hkv, group, Nq, Nk, nT, nQB;
   int32_t q_offset, p_quant, window_mode, block_m, sink, out_dtype;
   int32_t sched_mode, sched_xpp, sched_items, sched_pairs;
+  // launches with split key ranges (plan_split): `work` lists the workgroups of a q head in place of its nQB query blocks
+  int32_t n_slots;   // places for parts per q head
+  float* part_o;       // [B * Hq, n_slots, 8 waves, 16, 64] float4: a part's accumulators as its lanes hold them
+  float2* part_lm;     // [B * Hq, n_slots, 8 waves, 64]: denominator and reference point of the lane's row
   const float* k_scale;   // MODE 6: per-token scales of the int8 key codes in `k`, fp32 [B, Hkv, nT * 64]
   int32_t q_quant;   // 8: the rows of q (not of q4) are fake-quantised to 8 bits per token as they are loaded
   float sm;
   int32_t w8[kMaxHeads];
   int32_t w4[kMaxHeads];
+  SplitWork work[kMaxSplitWork];
 };
 
 struct PrepArgs {
@@ -391,13 +405,32 @@ __device__ __forceinline__ void quant_pack4(float p0, float p1, float p2, float 
   }
 }
 
+// Four neighbouring channels of an output row, `ch` their index in the per-channel scale table, `off` in the output
+template <bool PV8>
+__device__ __forceinline__ void store_out4(const PrefillArgs& a, int64_t ch, int64_t off, float v0, float v1, float v2, float v3) {
+  if constexpr (PV8) {  // undo the per-channel V scale
+    const float4 isc = *(const float4*)(a.v_inv_scale + ch);
+    v0 *= isc.x;
+    v1 *= isc.y;
+    v2 *= isc.z;
+    v3 *= isc.w;
+  }
+  if (a.out_dtype == 0) {
+    *(uint2*)((uint16_t*)a.out + off) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+  } else if (a.out_dtype == 1) {
+    *(uint2*)((uint16_t*)a.out + off) = make_uint2(pack_f16(v0, v1), pack_f16(v2, v3));
+  } else {
+    *(float4*)((float*)a.out + off) = make_float4(v0, v1, v2, v3);
+  }
+}
+
 // One workgroup = WAVES waves x 32 query rows of one q-head (2 waves per SIMD when WAVES == 8, so that one
 // wave's MFMA phase overlaps the other's softmax phase).  MODE as in quant_pack8.
 // DUAL (WAVES == 8, absolute windows with their own 4-bit operands, block_m == 128): the workgroup holds two query blocks,
 // A = waves 0..3 and B = waves 4..7, whose 4-bit ranges end 128 keys apart.  On the up to two tiles in between -- 8-bit
 // for A, 4-bit for B -- the blocks want different K tiles, so those tiles are walked twice: once as they are (B skips
 // them), once as 4-bit copies right behind (A skips those).  Everywhere else the blocks agree, or only one of them visits.
-template <bool BF16, int WAVES, int MODE, bool DUAL = false>
+template <bool BF16, int WAVES, int MODE, bool DUAL = false, bool SPLIT = false>
 __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   constexpr int NT = WAVES * 64;
   constexpr int CH = (kBN * kD * 2 / 16) / NT;  // 16-byte chunks per thread and tile operand
@@ -409,6 +442,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   constexpr bool kQK8 = MODE == 6;
   constexpr bool kPlain = MODE == 2 || MODE == 6;   // tile step left to the compiler's scheduling
   constexpr bool kPV8 = MODE == 4 || MODE == 5;     // e4m3 V tiles, fp8 P.V
+  constexpr bool kOwn4 = WAVES == 2 || DUAL;        // the launches that can have their own 4-bit operands
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // MODE 2: tile maxima of the two waves of a 64-row group, behind the tile rings (which start at LDS address 0)
   float (*s_amax)[WAVES] = (float (*)[WAVES])(smem + 4 * kStageBytes);
@@ -433,7 +467,8 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   }
   const int b = pair / a.Hkv, kvh = pair % a.Hkv;
   const int hg = item % a.group;
-  const int qb = a.nQB - 1 - item / a.group;
+  const SplitWork sw = SPLIT ? a.work[item / a.group] : SplitWork{0, 0, 0, 1};
+  const int qb = SPLIT ? (int)sw.qb : a.nQB - 1 - item / a.group;
   const int head = kvh * a.group + hg;
 
   const int tid = threadIdx.x;
@@ -465,7 +500,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     segB_lo = 0;
   }
   // separate 4-bit operands run with WAVES*32 == block_m (all waves agree on a tile's operand set), or as DUAL
-  const bool distinct4 = (WAVES < 8 || DUAL) && a.q4 != nullptr;
+  const bool distinct4 = kOwn4 && a.q4 != nullptr;
   // The tiles that are copied from the 4-bit key, [t4_lo, t4_hi): the 4-bit range of the workgroup's first query block.
   // DUAL: tiles [c_lo, c_lo + n_dup), from where block A's 4-bit range ends to where block B's ends (128 keys later, unless
   // the sink cuts both), are walked twice -- first as 4-bit copies for B, then as they are for A.
@@ -484,6 +519,12 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
         t4_hi = c_lo;                        // (where A has one, it ends at c_lo anyway)
       }
     }
+  }
+  // this workgroup's share of the item's steps
+  int nTot = max(segA_hi + segB_hi - segB_lo, 0) + n_dup, t_off = 0;
+  if constexpr (SPLIT) {
+    t_off = nTot * sw.part / sw.parts;
+    nTot = nTot * (sw.part + 1) / sw.parts - t_off;
   }
   // ---- Q~ fragments (B operand of S^T = K.Q~^T): lane (column = query row c32, k-group g)
   uint4 qf[8];
@@ -622,14 +663,18 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   auto stage_v = [&](int j, int stage) {
     char* vbuf = vbase_lds + stage * kVTileBytes;
     if constexpr (kPV8) {
-      // e4m3 tile: 128 rows x 64 bytes = 8 KB, one wave instruction per wave; 16-byte chunk c of row d -> slot
+      // e4m3 tile: 128 rows x 64 bytes = 8 KB, eight wave instructions; 16-byte chunk c of row d -> slot
       // c ^ ((d >> 2) & 3), which spreads the 16 rows a quarter-wave reads over all 16 bank groups
       const uint8_t* vsrc8 = a.vt8 + (((int64_t)b * a.Hkv + kvh) * a.nT + j) * (int64_t)(kD * kBN);
-      const int vr = 16 * wave + (lane >> 2);
-      const int vc = (lane & 3) ^ ((vr >> 2) & 3);
-      uint32_t off = (uint32_t)(vr * kBN + 16 * vc);
-      asm volatile("" : "+v"(off));   // 32-bit per-lane offset next to the uniform 64-bit tile base
-      __builtin_amdgcn_global_load_lds((const void*)(vsrc8 + off), (lds_ptr_t)(vbuf + wave * 1024), 16, 0, 0);
+#pragma unroll
+      for (int c = 0; c < 8 / WAVES; ++c) {
+        const int q = wave * (8 / WAVES) + c;
+        const int vr = 16 * q + (lane >> 2);
+        const int vc = (lane & 3) ^ ((vr >> 2) & 3);
+        uint32_t off = (uint32_t)(vr * kBN + 16 * vc);
+        asm volatile("" : "+v"(off));   // 32-bit per-lane offset next to the uniform 64-bit tile base
+        __builtin_amdgcn_global_load_lds((const void*)(vsrc8 + off), (lds_ptr_t)(vbuf + q * 1024), 16, 0, 0);
+      }
       return;
     }
     const _Float16* vsrc = vt_base + (int64_t)j * (kD * kBN);
@@ -783,7 +828,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     asm volatile("; tile from memory" : "+v"(ln));
     // (with separate 4-bit operands the fragments in qf may already belong to the next step's operand set)
     bool other_q = false;
-    if constexpr (WAVES < 8 || DUAL) {
+    if constexpr (kOwn4) {
       other_q = distinct4 && use4 != q_is4;
       if (other_q) reload_q(use4 ? a.q4 : a.q);
     }
@@ -799,7 +844,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if constexpr (WAVES < 8 || DUAL) {
+    if constexpr (kOwn4) {
       if (other_q) reload_q(q_is4 ? a.q4 : a.q);
     }
     if (masked) {
@@ -1280,11 +1325,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   // DUAL: the 4-bit copies of tiles [c_lo, c_lo + n_dup) sit at steps [d1 - n_dup, d1), where those tiles would sit
   // anyway; the tiles themselves and everything behind them move up by n_dup steps.  The steps whose K tile comes from
   // the 4-bit key then form one interval [u4_lo, u4_hi): block A's 4-bit range and, right behind it, the copies.
-  const int nA = segA_hi, shiftB = segB_lo - segA_hi;
+  // (t counts from the first step of this workgroup's part, t_off)
+  const int nA = segA_hi - t_off, shiftB = segB_lo - segA_hi + t_off;
   const int d1 = (DUAL && n_dup > 0) ? c_lo - shiftB + n_dup : (1 << 30);
-  const int nTot = max(nA + segB_hi - segB_lo, 0) + n_dup;
   auto tile_of = [&](int t) {
-    if (t < nA) return t;
+    if (t < nA) return t + t_off;
     if constexpr (DUAL) return t + shiftB - (t >= d1 ? n_dup : 0);
     return t + shiftB;
   };
@@ -1299,9 +1344,9 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   // waves the tiles below c_lo + n_dup are the copies, and they skip the originals.
   const int thr = wave < 4 ? c_lo : c_lo + n_dup;
   auto step_of = [&](int j) { return j - shiftB + ((DUAL && j >= thr) ? n_dup : 0); };   // a tile of segment B
-  const int fa = wave_active ? wr.sink_hi : 0;
+  const int fa = wave_active ? min(wr.sink_hi - t_off, nTot) : 0;
   const int fb = wave_active ? step_of(wr.win_lo) : (1 << 30);
-  const int fe = step_of(wr.diag_hi), fm = step_of(wr.diag_lo);
+  const int fe = min(step_of(wr.diag_hi), nTot - 1), fm = step_of(wr.diag_lo);
   const int sk_lo = (DUAL && n_dup > 0) ? (wave < 4 ? d1 - n_dup : d1) : 0;
   auto visits_step = [&](int t) {
     const bool in = t < fa || (t >= fb && t <= fe);
@@ -1368,7 +1413,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   auto switch_q = [&](int t) __attribute__((always_inline)) {   // t: a step this wave visits
-    if constexpr (WAVES < 8 || DUAL) {
+    if constexpr (kOwn4) {
       if (distinct4) {  // switch the Q~ operand set when entering/leaving the 4-bit window range
         const bool want4 = step_uses4(t);
         if (want4 != q_is4) {
@@ -1394,7 +1439,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     if ((t & 1) == 0) {   // start of a pair: refill the four buffers the previous pair released
       if (t + 4 < nFull) {
         const int j2 = tile_of(t + 2), j3 = tile_of(t + 3), j4 = tile_of(t + 4);
-        if constexpr (WAVES == 8 && !kQK8) {
+        if constexpr (WAVES >= 4 && !kQK8) {
           stage_k_full(j3, (t + 3) & 3, DUAL && step_uses4(t + 3));
           stage_k_full(j4, t & 3, DUAL && step_uses4(t + 4));
         } else {
@@ -1422,7 +1467,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     }
     const bool vis_nxt = visits_step(t + 1);
     const char* knext = kbase_lds + ((t + 1) & 3) * kKTileBytes;
-    if constexpr (WAVES < 8 || DUAL) {
+    if constexpr (kOwn4) {
       if (vis_nxt) switch_q(t + 1);
     }
     if (vis_cur) {
@@ -1468,6 +1513,17 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   // (kDefer: nothing is pending here -- the step after a wave's last visited step is never visited, so that step flushed)
   const float l = xor32_sum(l_run);
   const int row = row_w0 + c32;
+  if (SPLIT && sw.parts > 1) {   // accumulators, denominator and reference as they are; prefill_merge_kernel does the rest
+    const int64_t wslot = (((int64_t)b * a.Hq + head) * a.n_slots + sw.slot + sw.part) * WAVES + wave;
+    float4* po = (float4*)a.part_o + wslot * 1024 + lane;
+#pragma unroll
+    for (int bd = 0; bd < 4; ++bd)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4)
+        po[(4 * bd + i4) * 64] = make_float4(O[bd][4 * i4], O[bd][4 * i4 + 1], O[bd][4 * i4 + 2], O[bd][4 * i4 + 3]);
+    a.part_lm[wslot * 64 + lane] = make_float2(l, m_run);
+    return;
+  }
   if (row >= a.Nq) return;
   const int64_t obase = (int64_t)b * a.o_sb + (int64_t)head * a.o_sh + (int64_t)row * a.o_sn;
   const float inv_l = 1.0f / l;   // one division per row instead of 64 per lane: within 1 ulp of acc / l, before the rounding to the output type
@@ -1476,31 +1532,150 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       const int d = 32 * bd + 8 * i4 + 4 * g;
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = O[bd][4 * i4 + e] * inv_l;
-      if constexpr (kPV8) {  // undo the per-channel V scale
-        const float4 isc = *(const float4*)(a.v_inv_scale + ((int64_t)b * a.Hkv + kvh) * kD + d);
-        v[0] *= isc.x;
-        v[1] *= isc.y;
-        v[2] *= isc.z;
-        v[3] *= isc.w;
-      }
-      if (a.out_dtype == 0) {
-        uint2 w = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-        *(uint2*)((uint16_t*)a.out + obase + d) = w;
-      } else if (a.out_dtype == 1) {
-        uint2 w = make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3]));
-        *(uint2*)((uint16_t*)a.out + obase + d) = w;
-      } else {
-        *(float4*)((float*)a.out + obase + d) = make_float4(v[0], v[1], v[2], v[3]);
-      }
+      store_out4<kPV8>(a, ((int64_t)b * a.Hkv + kvh) * kD + d, obase + d, O[bd][4 * i4] * inv_l, O[bd][4 * i4 + 1] * inv_l, O[bd][4 * i4 + 2] * inv_l,
+                       O[bd][4 * i4 + 3] * inv_l);
     }
   if (a.lse && g == 0) {
     const float lt = (MODE >= 3 && MODE <= 5) ? l * (1.0f / 448.0f) : l;
     a.lse[((int64_t)b * a.Hq + head) * a.Nq + row] = log2f(lt) + m_run;
   }
 }
+
+// Memory-bound: 130 KB per part and workgroup read, 64 KB of output per block (bf16) written; 7 us for 196 parts.
+// Merges the parts of split key ranges: o = sum_p 2^(m_p - m) o_p, l likewise, out = o / l.  One workgroup per (block of the
+// work list that is split, wave of its workgroups, q head); lanes and accumulator elements keep the places they had there,
+// and wave bd of this workgroup takes output channels 32 bd .. +31.
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  constexpr int WAVES = 8;
+  const SplitWork sw = a.work[blockIdx.x];
+  if (sw.part != 0 || sw.parts == 1) return;
+  const int wave = blockIdx.y, bd = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t bh = blockIdx.z;
+  const int row = (sw.qb * WAVES + wave) * 32 + (lane & 31);
+  if (row >= a.Nq) return;
+  const int64_t wslot = (bh * a.n_slots + sw.slot) * WAVES + wave;
+  const float2* lm = a.part_lm + wslot * 64 + lane;
+  const float4* po = (const float4*)a.part_o + (wslot * 16 + 4 * bd) * 64 + lane;
+  float m = -INFINITY, l = 0.f;
+  float4 o[4] = {};
+  // one pass: the sums are rescaled when a part raises the reference point
+  for (int p = 0; p < sw.parts; ++p) {
+    const float2 x = lm[p * WAVES * 64];
+    float4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = po[((int64_t)p * WAVES * 16 + i) * 64];
+    if (x.x > 0.f) {   // a part in which the row has no key has no denominator
+      const float m_new = fmaxf(m, x.y);
+      const float w_old = __builtin_amdgcn_exp2f(m - m_new), w = __builtin_amdgcn_exp2f(x.y - m_new);
+      l = l * w_old + x.x * w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o[i].x = o[i].x * w_old + v[i].x * w;
+        o[i].y = o[i].y * w_old + v[i].y * w;
+        o[i].z = o[i].z * w_old + v[i].z * w;
+        o[i].w = o[i].w * w_old + v[i].w * w;
+      }
+      m = m_new;
+    }
+  }
+  const float inv_l = 1.0f / l;
+  const int head = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
+  const int64_t obase = (int64_t)b * a.o_sb + (int64_t)head * a.o_sh + (int64_t)row * a.o_sn;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int d = 32 * bd + 8 * i + 4 * (lane >> 5);
+    store_out4<false>(a, 0, obase + d, o[i].x * inv_l, o[i].y * inv_l, o[i].z * inv_l, o[i].w * inv_l);
+  }
+  if (a.lse && bd == 0 && lane < 32) a.lse[bh * a.Nq + row] = log2f(l) + m;
+}
+
+// ---- which launches split their key ranges, and how.
+struct SplitPlan {
+  int n_work = 0, n_slots = 0;   // n_work == 0: one workgroup per query block
+  SplitWork work[kMaxSplitWork];
+};
+
+// Tiles the workgroup of query rows [r0, r1) walks: everything up to its diagonal, or sink and windows (of the widest head)
+int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, int w_max) {
+  const int64_t hi = (p->q_offset + r1 + kBN - 1) / kBN;
+  if (p->window_mode == SQ_WINDOW_NONE) return (int)hi;
+  const int64_t lo = std::max<int64_t>(0, (p->q_offset + r0) / p->block_m * p->block_m + p->block_m - w_max) / kBN;
+  return (int)std::min(hi, hi - std::min(lo, hi) + p->sink / kBN);
+}
+
+// A launch is as long as its longest chain of tiles when its query blocks do not fill the chip: 64 workgroups of up to 64
+// tiles (4096 tokens, 4 heads) left three quarters of the CUs idle.  Such a launch gets several workgroups per query block,
+// each with a contiguous share of the block's steps, and a second kernel merges their accumulators.  Worth it when the
+// shares shorten the launch by more than the merge costs; in units of one tile of an 8-wave workgroup (1.35 us) a workgroup
+// costs its tiles plus kFix (8 us: launch, first loads, epilogue) and the merge kMerge (12 us with the parts' stores), both
+// sides measured: 4096 tokens, 4 / 1 heads 88 -> 42 us, 8192 tokens 163 -> 89 us, a chunk of 512 rows behind 16384 tokens
+// at 28 / 4 heads 325 -> 132 us; 777 tokens at 28 / 4 heads would go 31 -> 34 us and stay whole.  Shares below 4 tiles
+// never paid.  A launch that keeps all CUs busy gains nothing (the chip then runs at a lower clock: 8192 rows behind 24576
+// tokens, 3.5 workgroups per CU, 2685 us either way), hence the limit of 4 per CU.
+// Split is the mode whose probabilities are plain floating-point numbers relative to the row's reference point (0, and 6 with
+// it): the parts of a row start from reference points of their own, which moves a probability by its rounding at most.  The
+// e4m3 grids of the other modes are tied to the row's running maximum or to its first tile.
+void plan_split(const sq_prefill_params* p, int64_t B, int64_t Hq, int64_t Nq, int rows_wg, SplitPlan& plan) {
+  constexpr int kCUs = 256, kMaxRounds = 4, kMinTiles = 4;
+  plan.n_work = plan.n_slots = 0;
+  constexpr int kFix = 6, kMerge = 9;
+  if (rows_wg != 256 || p->p_quant != SQ_P_NONE) return;
+  const int64_t nQB = (Nq + rows_wg - 1) / rows_wg, mult = B * Hq;
+  if (mult * nQB > kMaxRounds * kCUs) return;
+  int w_max = 0;
+  if (p->window_mode == SQ_WINDOW_SIZES)
+    for (int h = 0; h < Hq; ++h) w_max = std::max(w_max, std::max(p->w8[h], p->w4[h]));
+  int len[kMaxRounds * kCUs], longest = 0;
+  for (int qb = 0; qb < nQB; ++qb) {
+    len[qb] = tiles_of_block(p, (int64_t)qb * rows_wg, std::min<int64_t>(Nq, (int64_t)(qb + 1) * rows_wg), w_max);
+    longest = std::max(longest, len[qb]);
+  }
+  if (longest <= kMinTiles + kMerge) return;
+  // Unsplit: the blocks of one head, longest first, on kCUs / mult CUs (each stands for the same block of every head)
+  int load[kCUs] = {0}, best = 0;
+  const int cus = (int)std::max<int64_t>(1, kCUs / mult), rounds = (int)((mult + kCUs - 1) / kCUs);
+  for (int64_t qb = nQB - 1; qb >= 0; --qb) {
+    int* least = std::min_element(load, load + cus);
+    *least += (len[qb] + kFix) * rounds;
+    best = std::max(best, *least);
+  }
+  // Split: for each number of workgroups per CU the smallest share that keeps to it
+  auto workgroups = [&](int cap) {
+    int64_t n = 0;
+    for (int qb = 0; qb < nQB; ++qb) n += (len[qb] + cap - 1) / cap;
+    return n;
+  };
+  int cap = 0;
+  for (int m = 1; m <= kMaxRounds; ++m) {
+    int lo = kMinTiles, hi = longest;
+    while (lo < hi) {
+      const int c = (lo + hi) / 2;
+      if (workgroups(c) * mult <= m * kCUs) hi = c;
+      else lo = c + 1;
+    }
+    const int est = m * (lo + kFix) + kMerge;
+    if (lo < longest && est * 20 < best * 19 && workgroups(lo) <= kMaxSplitWork) {
+      best = est;
+      cap = lo;
+    }
+  }
+  if (cap == 0) return;
+  for (int64_t qb = nQB - 1; qb >= 0; --qb) {
+    const int parts = std::min((len[qb] + cap - 1) / cap, 255);
+    for (int i = 0; i < parts; ++i) plan.work[plan.n_work++] = SplitWork{(uint16_t)qb, (uint16_t)plan.n_slots, (uint8_t)i, (uint8_t)parts};
+    if (parts > 1) plan.n_slots += parts;
+  }
+  // longest shares first
+  std::stable_sort(plan.work, plan.work + plan.n_work, [&](const SplitWork& x, const SplitWork& y) { return len[x.qb] * y.parts > len[y.qb] * x.parts; });
+}
+
+constexpr size_t kPartRowBytes = 64 * 16 * 16 + 64 * 8;   // per wave of a part: accumulators, denominator and reference point
+
+size_t part_bytes(const SplitPlan& plan, int64_t B, int64_t Hq) { return (size_t)(B * Hq) * plan.n_slots * 8 * kPartRowBytes; }
+
+// waves per workgroup: separate 4-bit operands with 64-row blocks take a workgroup of one block (two waves); 128-row blocks
+// one of two blocks that walk the few tiles on which they disagree twice (DUAL)
+int waves_of(const sq_prefill_params* p, bool own4) { return p->window_mode == SQ_WINDOW_SIZES && own4 && p->block_m == 64 ? 2 : 8; }
 
 }  // namespace
 }  // namespace sq
@@ -1512,6 +1687,16 @@ extern "C" size_t sq_prefill_workspace_bytes(int64_t batch, int64_t num_kv_heads
   if (batch <= 0 || num_kv_heads <= 0 || kv_len <= 0) return 0;
   const int64_t nT = (kv_len + kBN - 1) / kBN;
   return (size_t)(batch * num_kv_heads * nT) * (size_t)(kD * kBN) * sizeof(_Float16);
+}
+
+extern "C" size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t qo_len, int64_t kv_len,
+                                                   const sq_prefill_params* p) {
+  const size_t need = sq_prefill_workspace_bytes(batch, num_kv_heads, kv_len, kD);
+  if (!p || need == 0 || num_q_heads <= 0 || num_q_heads > kMaxHeads || qo_len <= 0) return need;
+  if (p->window_mode == SQ_WINDOW_SIZES && (!p->w8 || !p->w4 || p->num_heads_w != num_q_heads || p->block_m <= 0 || p->sink < 0)) return need;
+  SplitPlan plan;
+  plan_split(p, batch, num_q_heads, qo_len, 256, plan);
+  return need + part_bytes(plan, batch, num_q_heads);
 }
 
 namespace {
@@ -1595,7 +1780,6 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
     SQ_REQUIRE(dtype_of(lse) == DType::F32 && numel_of(lse) == B * Hq * Nq && is_compact(lse), SQ_ESHAPE,
                "sq_prefill_fwd: lse must be a compact fp32 [B,Hq,Nq]");
   }
-  int waves = 8;
   if (p->window_mode == SQ_WINDOW_SIZES) {
     SQ_REQUIRE(p->block_m == 64 || p->block_m == 128, SQ_EINVAL, "sq_prefill_fwd: block_m must be 64 or 128");
     SQ_REQUIRE(p->sink >= 0, SQ_EINVAL, "sink_size must be a non-negative integer, got %d", p->sink);
@@ -1611,9 +1795,6 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
                  "sq_prefill_fwd: head %d: a 4-bit window wider than an 8-bit window smaller than block_m reads future keys "
                  "in the reference and is not supported", h);
     }
-    // separate 4-bit operands: a workgroup of one 64-row query block (two waves), or, for 128-row blocks, of two blocks
-    // that walk the few tiles on which they disagree twice (DUAL)
-    if (q4 && p->block_m == 64) waves = 2;
   } else {
     SQ_REQUIRE(p->window_mode == SQ_WINDOW_NONE, SQ_EINVAL, "sq_prefill_fwd: window_mode %d not supported", p->window_mode);
     SQ_REQUIRE(!q4, SQ_EINVAL, "sq_prefill_fwd: q4/k4 only apply to window mode");
@@ -1700,7 +1881,7 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   local.Nq = (int)Nq;
   local.Nk = (int)Nk;
   local.nT = nT;
-  const int rows_wg = waves * 32;
+  const int waves = waves_of(p, q4 != nullptr), rows_wg = waves * 32;
   local.nQB = (int)((Nq + rows_wg - 1) / rows_wg);
   SQ_REQUIRE(p->q_quant == 0 || p->q_quant == 8, SQ_EINVAL, "sq_prefill_fwd: q_quant must be 0 or 8 (got %d)", (int)p->q_quant);
   SQ_REQUIRE(!(p->q_quant && q4), SQ_EINVAL, "sq_prefill_fwd: q_quant applies to launches without a separate 4-bit operand set");
@@ -1720,7 +1901,17 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
       local.w4[h] = p->w4[h];
     }
   const int pairs = (int)(B * Hkv);
-  const int items = local.group * local.nQB;
+  int items = local.group * local.nQB;
+  SplitPlan plan;
+  plan_split(p, B, Hq, Nq, rows_wg, plan);
+  const bool split = plan.n_work > 0 && (size_t)numel_of(workspace) * (workspace->dtype.bits / 8) >= need + part_bytes(plan, B, Hq);
+  if (split) {
+    local.n_slots = plan.n_slots;
+    local.part_o = (float*)(wsp + need);
+    local.part_lm = (float2*)(wsp + need + (size_t)(B * Hq) * plan.n_slots * 8 * (64 * 16 * 16));
+    memcpy(local.work, plan.work, plan.n_work * sizeof(SplitWork));
+    items = local.group * plan.n_work;
+  }
   local.sched_pairs = pairs;
   local.sched_items = items;
   unsigned blocks;
@@ -1760,6 +1951,18 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
       default: SQ_LAUNCH_PREFILL_DUAL(BF, 3); break;                 \
     }                                                               \
   } while (0)
+#define SQ_LAUNCH_SPLIT(BF, M, DU)                                                                                           \
+  do {                                                                                                                     \
+    SQ_HIP(hipFuncSetAttribute((const void*)prefill_kernel<BF, 8, M, DU, true>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                               (int)smem));                                                                                \
+    hipLaunchKernelGGL((prefill_kernel<BF, 8, M, DU, true>), dim3(blocks), dim3(8 * 64), smem, st, local);                 \
+  } while (0)
+#define SQ_LAUNCH_SPLITS(BF)                                                                                  \
+  do {                                                                                                        \
+    if (k_scale) SQ_LAUNCH_SPLIT(BF, 6, false);                                                               \
+    else if (q4) SQ_LAUNCH_SPLIT(BF, 0, true);                                                                \
+    else SQ_LAUNCH_SPLIT(BF, 0, false);                                                                       \
+  } while (0)
 #define SQ_LAUNCH_MODE(BF, W)                                   \
   do {                                                          \
     if (k_scale) {                                              \
@@ -1775,13 +1978,16 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
       default: SQ_LAUNCH_PREFILL(BF, W, 3); break;               \
     }                                                           \
   } while (0)
-  if (waves == 8 && q4) {
+  if (split) {
+    if (bf) SQ_LAUNCH_SPLITS(true); else SQ_LAUNCH_SPLITS(false);
+  } else if (waves == 8 && q4) {
     if (bf) SQ_LAUNCH_DUAL(true); else SQ_LAUNCH_DUAL(false);
   } else if (waves == 8) {
     if (bf) SQ_LAUNCH_MODE(true, 8); else SQ_LAUNCH_MODE(false, 8);
   } else {
     if (bf) SQ_LAUNCH_MODE(true, 2); else SQ_LAUNCH_MODE(false, 2);
   }
+  if (split) hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)plan.n_work, 8, (unsigned)(B * Hq)), dim3(256), 0, st, local);
 #undef SQ_LAUNCH_DUAL
 #undef SQ_LAUNCH_PREFILL_DUAL
 #undef SQ_LAUNCH_MODE

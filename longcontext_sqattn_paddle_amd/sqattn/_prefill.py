@@ -40,8 +40,6 @@ def run_prefill(q, k, v, *, tensor_layout="HND", output_dtype=torch.float16, ret
     B, Hq, Nq = q.size(0), q.size(hdim), q.size(ndim)
     Hkv, Nk = k.size(hdim), k.size(ndim)
     lib = N.lib()
-    if workspace is None:
-        workspace = prefill_workspace(B, Hkv, Nk, q.device)
     o = out if out is not None else torch.empty(q.shape, dtype=output_dtype, device=q.device)
     lse = torch.empty([B, Hq, Nq], dtype=torch.float32, device=q.device) if return_lse else None
     params = N.PrefillParams()
@@ -64,6 +62,9 @@ def run_prefill(q, k, v, *, tensor_layout="HND", output_dtype=torch.float16, ret
         params.num_heads_w = Hq
         params.w8 = ctypes.cast(w8, ctypes.POINTER(ctypes.c_int32))
         params.w4 = ctypes.cast(w4, ctypes.POINTER(ctypes.c_int32))
+    if workspace is None:
+        # room for the parts of split key ranges where this launch is split
+        workspace = torch.empty(lib.sq_prefill_workspace_bytes_split(B, Hq, Hkv, Nq, Nk, ctypes.byref(params)), dtype=torch.uint8, device=q.device)
     if k_scale is not None:
         b = [N.dl(t) for t in (q, k, k_scale, v, o, lse, workspace)]
         N.check(lib.sq_prefill_int8qk_fwd(*[N.ptr(x) for x in b], ctypes.byref(params), N.current_stream(q.device)))

@@ -257,6 +257,57 @@ def test_chunked_prefill_offset():
     assert torch.allclose(lse.cpu(), lse_ref[:, :, 512:], atol=2e-4)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,N,offset,window", [
+    (1, 4, 1, 4096, 0, None),            # shares of unequal blocks
+    (1, 2, 2, 1217, 0, None),            # ragged: last block of 193 rows, last tile of one key
+    (1, 2, 1, 1025, 0, None),            # last block of a single row: seven of its waves have none
+    (3, 2, 1, 300, 2048, None),          # a chunk behind a context, several sequences
+    (1, 2, 1, 64, 4096, None),           # one 64-row block over 65 tiles
+    (1, 4, 2, 2500, 0, (256, 0.125, 0.5)),   # sink and windows: a share may begin inside the sink or at the jump behind it
+    (1, 2, 1, 2304, 0, (64, 512, 1024)),     # absolute windows with their own 4-bit operands (tiles walked twice)
+])
+def test_split_key_ranges_match_unsplit_launch_and_oracle(B, Hq, Hkv, N, offset, window):
+    """Launches too small to fill the chip split the key range of a query block over several workgroups (given the workspace
+    for it).  A row's parts start from reference points of their own, so p differs by its fp16 rounding: the unquantised
+    criterion of this file, against the oracle and against the unsplit launch (twice that criterion: both sides round)."""
+    from longcontext_sqattn_paddle_amd import _native as NV
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton_mix_bad import attn_hierarchical_window
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton_mix_relative import attn_hierarchical_relative_window
+    from oracle import fake_quant as FQ
+
+    print(f"case prefill split B={B} Hq={Hq} Hkv={Hkv} N={N} offset={offset} window={window}", flush=True)
+    _, k, v = _rand(B, Hq, Hkv, offset + N, 128, 300 + N)
+    q = _rand(B, Hq, Hkv, N, 128, 301 + N)[0]
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    small = prefill_workspace(B, Hkv, offset + N, qd.device)     # no room for parts: the unsplit launch
+    if window is None:
+        ref, lse_ref = A.exact_attention(A.fold_scale(q, 128), k, v, causal=True, q_offset=offset, score_scale=math.log(2.0))
+        call = lambda **kw: attn_causal(qd, kd, vd, "HND", torch.float32, return_lse=True, q_offset=offset, **kw)
+        assert NV.lib().sq_prefill_workspace_bytes_split(B, Hq, Hkv, N, offset + N, NV.PrefillParams(q_offset=offset)) > small.numel() * 2
+    elif isinstance(window[1], float):
+        w8, w4 = ([A.window_size_relative(r, N)] * Hq for r in window[1:])
+        ref, lse_ref = A.prefill_blockwise(q, k, v, block_m=64, sink=window[0], w8=w8, w4=w4, out_dtype=torch.float32)
+        call = lambda **kw: attn_hierarchical_relative_window(qd, kd, qd, kd, vd, window[1], window[2], window[0], "HND", torch.float32,
+                                                              return_lse=True, **kw)
+    else:
+        q4, k4 = FQ.int_fake_quant(q, 4, True, "per_token"), FQ.int_fake_quant(k, 4, True, "per_token")
+        ref, lse_ref = A.prefill_blockwise(q, k, v, block_m=128, sink=window[0], w8=[window[1]] * Hq, w4=[window[2]] * Hq, q4=q4, k4=k4,
+                                           out_dtype=torch.float32)
+        q4d, k4d = q4.to(DEV), k4.to(DEV)
+        call = lambda **kw: attn_hierarchical_window(qd, kd, q4d, k4d, vd, window[1], window[2], window[0], "HND", torch.float32,
+                                                     return_lse=True, **kw)
+    out, lse = call()
+    whole, lse_whole = call(workspace=small)
+    torch.cuda.synchronize()
+    _check(out, ref.reshape(out.shape), False)
+    _check(whole, ref.reshape(out.shape), False)
+    assert torch.allclose(lse.cpu(), lse_ref.reshape(lse.shape).float(), atol=2e-4)
+    assert torch.allclose(lse, lse_whole, atol=2e-4)
+    assert not torch.equal(out, whole)     # the workspace the wrapper takes by itself does split these launches
+
+
 @pytest.mark.parametrize("sink,r8,r4", [(128, 0.25, 0.25), (256, [0.125, 0.5], [0.5, 0.5]), (0, 0.0, 0.0), (64, 2.0, 2.0)])
 def test_relative_window_matches_oracle(sink, r8, r4):
     from longcontext_sqattn_paddle_amd.sqattn.attn_triton_mix_relative import attn_hierarchical_relative_window
