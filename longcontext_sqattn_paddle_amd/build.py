@@ -24,7 +24,8 @@ HIPCC_FLAGS = [
 
 # Per-source flags.  The k-means assign kernel reads its MFMA results with the vector ALU right away (arg-max): the MFMAs
 # are kept in their VGPR form there, otherwise every score passes through a v_accvgpr_read first.
-SOURCE_FLAGS = {"kmeans_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# The 4-wave prefill workgroups may use 512 registers per lane; in the other form their score accumulators move to AGPRs and back.
+SOURCE_FLAGS = {"kmeans_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "prefill_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def build(verbose: bool = True, extra_flags=()) -> str:

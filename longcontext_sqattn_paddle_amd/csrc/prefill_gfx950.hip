@@ -8,7 +8,7 @@
 // round trip of p, acc += fp16(p).fp16(v)); they differ only in which 64-key blocks a query block visits.
 //
 // Design (CDNA4, 64-wide waves, 2 waves per SIMD, at most 256 registers per lane):
-//   * workgroup = WAVES (8) waves x 32 query rows of one q-head; K and V^T tiles of 64 keys are copied once per
+//   * workgroup = WAVES (8; 4 for short prompts) waves x 32 query rows of one q-head; K and V^T tiles of 64 keys are copied once per
 //     workgroup into rings of 4 LDS buffers by global_load_lds (unpadded, XOR-swizzled) and shared by all its rows;
 //     one workgroup barrier per two tiles;
 //   * S^T = K . Q~^T on v_mfma_f32_32x32x16 (bf16 or f16): K rows are the A operand straight out of LDS, Q~
@@ -65,9 +65,10 @@ struct PrefillArgs {
   int32_t B, Hq, Hkv, group, Nq, Nk, nT, nQB;
   int32_t q_offset, p_quant, window_mode, block_m, sink, out_dtype;
   int32_t sched_mode, sched_xpp, sched_items, sched_pairs;
-  // launches with split key ranges (plan_split): `work` lists the workgroups of a q head in place of its nQB query blocks
+  // launches with split key ranges (plan_launch): `work` lists the workgroups of a q head in place of its nQB query blocks
   int32_t n_slots;   // places for parts per q head
   float* part_o;       // [B * Hq, n_slots, 8 waves, 16, 64] float4: a part's accumulators as its lanes hold them
+  float* part_ref;     // [B * Hq, n_slots, 8 waves, 32]: a part's row maxima (MODE 7)
   float2* part_lm;     // [B * Hq, n_slots, 8 waves, 64]: denominator and reference point of the lane's row
   const float* k_scale;   // MODE 6: per-token scales of the int8 key codes in `k`, fp32 [B, Hkv, nT * 64]
   int32_t q_quant;   // 8: the rows of q (not of q4) are fake-quantised to 8 bits per token as they are loaded
@@ -440,7 +441,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   // are sum(code products) x scale_k x (scale_q log2e / sqrt(D)); from there on the step is MODE 0's (fp16 P, fp16 V), on
   // the plain schedule MODE 2 also uses (no hand-placed slots).
   constexpr bool kQK8 = MODE == 6;
-  constexpr bool kPlain = MODE == 2 || MODE == 6;   // tile step left to the compiler's scheduling
+  // MODE 7: no output, only the row maxima of a part's scores, from which the later parts of the row take the reference
+  // point the running maximum would have there (the modes whose e4m3 grid is tied to it).
+  constexpr bool kRefPass = MODE == 7;
+  constexpr bool kPlain = MODE == 2 || MODE == 6 || kRefPass;   // tile step left to the compiler's scheduling
   constexpr bool kPV8 = MODE == 4 || MODE == 5;     // e4m3 V tiles, fp8 P.V
   constexpr bool kOwn4 = WAVES == 2 || DUAL;        // the launches that can have their own 4-bit operands
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -525,6 +529,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   if constexpr (SPLIT) {
     t_off = nTot * sw.part / sw.parts;
     nTot = nTot * (sw.part + 1) / sw.parts - t_off;
+    if (kRefPass && sw.part + 1 == sw.parts) return;   // nobody comes after the last part
   }
   // ---- Q~ fragments (B operand of S^T = K.Q~^T): lane (column = query row c32, k-group g)
   uint4 qf[8];
@@ -661,6 +666,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     else stage_k16(j, stage, use4);
   };
   auto stage_v = [&](int j, int stage) {
+    if constexpr (kRefPass) return;
     char* vbuf = vbase_lds + stage * kVTileBytes;
     if constexpr (kPV8) {
       // e4m3 tile: 128 rows x 64 bytes = 8 KB, eight wave instructions; 16-byte chunk c of row d -> slot
@@ -1301,7 +1307,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) P[bn][t] = quant_pack8<(kPV8 ? 3 : (kQK8 ? 0 : MODE))>(S[bn], t, sc, inv);
+      for (int t = 0; t < 2; ++t) P[bn][t] = quant_pack8<(kPV8 ? 3 : (kQK8 || kRefPass ? 0 : MODE))>(S[bn], t, sc, inv);
     // O^T[d, row] += V^T[d, key] . P^T[key, row]
 #pragma unroll
     for (int bd = 0; bd < 4; ++bd)
@@ -1410,6 +1416,20 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   } else {
     load_q(a.q);
   }
+  // a later part of a row in the modes whose P is tied to the reference point: the reference it would have here unsplit
+  if constexpr (SPLIT && (MODE >= 1 && MODE <= 4)) {
+    if (sw.part > 0) {
+      const float* pr = a.part_ref + ((((int64_t)b * a.Hq + head) * a.n_slots + sw.slot) * WAVES + wave) * 32 + c32;
+      float m0 = pr[0];
+      for (int p = 1; p < sw.part; ++p) m0 = fmaxf(m0, pr[p * WAVES * 32]);
+      if (__any(m0 > -INFINITY)) {
+        m_run = m0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Cinit[i] = kC - m0;
+        first = false;
+      }
+    }
+  }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   auto switch_q = [&](int t) __attribute__((always_inline)) {   // t: a step this wave visits
@@ -1423,6 +1443,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
       }
     }
   };
+  float ref_max = -INFINITY;   // MODE 7
   f32x16_t Sa[2], Sb[2];
   bool vis_cur = nTot > 0 && visits_step(0);
   if (vis_cur) {
@@ -1473,6 +1494,19 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     if (vis_cur) {
       // Q.K^T of the next tile is computed even if this wave will not use it (the buffer then holds an older
       // tile or nothing meaningful; the result is dropped): the common path stays free of branches
+      if constexpr (kRefPass) {
+        if (t >= fm) {
+          const int rel = pos0 + c32 - tile_of(t) * kBN - 4 * g;
+#pragma unroll
+          for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              if (32 * bn + 8 * (i >> 2) + (i & 3) > rel) Scur[bn][i] = -INFINITY;
+        }
+        mfma_settle(Scur[0], Scur[1]);
+        ref_max = fmaxf(ref_max, lane_max(Scur));
+        qk_tile(knext, Snxt);
+      } else
       softmax_pv(rg, tile_of(t), t, step_uses4(t), vbase_lds + (t & 3) * kVTileBytes, t >= fm, Scur, knext, Snxt);
     } else {
       if (vis_nxt) {
@@ -1511,6 +1545,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   // ---- epilogue: out = acc / l (attn_triton.py:208-209), lse2 = log2(l) + m (:210-213)
   if (!wave_active) return;
   // (kDefer: nothing is pending here -- the step after a wave's last visited step is never visited, so that step flushed)
+  if constexpr (kRefPass) {
+    const float m = xor32_max(ref_max);
+    if (g == 0) a.part_ref[((((int64_t)b * a.Hq + head) * a.n_slots + sw.slot + sw.part) * WAVES + wave) * 32 + c32] = m;
+    return;
+  }
   const float l = xor32_sum(l_run);
   const int row = row_w0 + c32;
   if (SPLIT && sw.parts > 1) {   // accumulators, denominator and reference as they are; prefill_merge_kernel does the rest
@@ -1545,6 +1584,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
 // Merges the parts of split key ranges: o = sum_p 2^(m_p - m) o_p, l likewise, out = o / l.  One workgroup per (block of the
 // work list that is split, wave of its workgroups, q head); lanes and accumulator elements keep the places they had there,
 // and wave bd of this workgroup takes output channels 32 bd .. +31.
+template <bool PV8>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   constexpr int WAVES = 8;
   const SplitWork sw = a.work[blockIdx.x];
@@ -1584,13 +1624,14 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int d = 32 * bd + 8 * i + 4 * (lane >> 5);
-    store_out4<false>(a, 0, obase + d, o[i].x * inv_l, o[i].y * inv_l, o[i].z * inv_l, o[i].w * inv_l);
+    store_out4<PV8>(a, ((int64_t)b * a.Hkv + head / a.group) * kD + d, obase + d, o[i].x * inv_l, o[i].y * inv_l, o[i].z * inv_l, o[i].w * inv_l);
   }
-  if (a.lse && bd == 0 && lane < 32) a.lse[bh * a.Nq + row] = log2f(l) + m;
+  if (a.lse && bd == 0 && lane < 32) a.lse[bh * a.Nq + row] = log2f(a.p_quant >= SQ_P_E4M3_STATIC_FAST ? l * (1.0f / 448.0f) : l) + m;
 }
 
-// ---- which launches split their key ranges, and how.
-struct SplitPlan {
+// ---- how a launch is cut into workgroups.
+struct LaunchPlan {
+  int waves = 8;                 // per workgroup
   int n_work = 0, n_slots = 0;   // n_work == 0: one workgroup per query block
   SplitWork work[kMaxSplitWork];
 };
@@ -1603,63 +1644,104 @@ int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, int w_max
   return (int)std::min(hi, hi - std::min(lo, hi) + p->sink / kBN);
 }
 
-// A launch is as long as its longest chain of tiles when its query blocks do not fill the chip: 64 workgroups of up to 64
-// tiles (4096 tokens, 4 heads) left three quarters of the CUs idle.  Such a launch gets several workgroups per query block,
-// each with a contiguous share of the block's steps, and a second kernel merges their accumulators.  Worth it when the
-// shares shorten the launch by more than the merge costs; in units of one tile of an 8-wave workgroup (1.35 us) a workgroup
-// costs its tiles plus kFix (8 us: launch, first loads, epilogue) and the merge kMerge (12 us with the parts' stores), both
-// sides measured: 4096 tokens, 4 / 1 heads 88 -> 42 us, 8192 tokens 163 -> 89 us, a chunk of 512 rows behind 16384 tokens
-// at 28 / 4 heads 325 -> 132 us; 777 tokens at 28 / 4 heads would go 31 -> 34 us and stay whole.  Shares below 4 tiles
-// never paid.  A launch that keeps all CUs busy gains nothing (the chip then runs at a lower clock: 8192 rows behind 24576
-// tokens, 3.5 workgroups per CU, 2685 us either way), hence the limit of 4 per CU.
-// Split is the mode whose probabilities are plain floating-point numbers relative to the row's reference point (0, and 6 with
-// it): the parts of a row start from reference points of their own, which moves a probability by its rounding at most.  The
-// e4m3 grids of the other modes are tied to the row's running maximum or to its first tile.
-void plan_split(const sq_prefill_params* p, int64_t B, int64_t Hq, int64_t Nq, int rows_wg, SplitPlan& plan) {
+// A launch whose query blocks do not fill the chip is as long as its longest chain of tiles: 64 workgroups of up to 64 tiles
+// (4096 tokens, 4 heads) left three quarters of the CUs idle.  Two remedies, chosen by an estimate of the launch's
+// length; all constants are measured times.
+//  * Split key ranges: several workgroups per query block, each with a contiguous share of the block's steps, and a second
+//    kernel that merges their accumulators.  The e4m3 modes with a static or absmax grid (1 .. 4), whose P depends on the
+//    row's running maximum, first run a pass that only forms the parts' row maxima (MODE 7), so that every part starts from
+//    the reference point it would have had.  4096 tokens, 4 / 1 heads: mode 0 88 -> 42 us, mode 1 132 -> 66, mode 2 186 ->
+//    75; a chunk of 512 rows behind 16384 tokens at 28 / 4 heads 325 -> 132 us in mode 0.  Mode 5 stays whole: where its reference
+//    point stands depends on every tile sum before (a jump of 2^100 puts it on that tile's maximum), not on a maximum.
+//  * Workgroups of 128 rows (4 waves): one wave per SIMD walks a tile in 0.7 to 0.82 of the time two take for theirs.  Short
+//    prompts, where a merge costs more than it saves: 777 tokens, 28 / 4 heads, mode 0 30.5 -> 24.1 us (split: 34), mode 1
+//    38.2 -> 28.4, mode 5 38.0 -> 30.2; 2048 tokens (448 workgroups) 57 -> 52, at 3000 the 8-wave launch is ahead (82
+//    against 95).
+// A tile of an 8-wave workgroup takes kStepUs on an otherwise idle chip and about 30 % more on a full one, which lowers its
+// clock: 8192 rows behind 24576 tokens, 3.5 workgroups per CU, take 2685 us split evenly or not.
+void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_t Hq, int64_t Nq, LaunchPlan& plan) {
   constexpr int kCUs = 256, kMaxRounds = 4, kMinTiles = 4;
+  static const float kStepUs[6] = {1.35f, 1.75f, 2.6f, 1.4f, 1.15f, 1.15f};   // by P mode
+  constexpr float kFixUs = 8.f;      // a workgroup's launch, first loads and epilogue
+  static const float kFourWaves[6] = {0.76f, 0.7f, 0.82f, 1.f, 1.f, 0.76f};
+  constexpr float kFullChip = 0.3f;
+  constexpr float kMergeUs = 6.f, kPartUs = 0.07f;   // the merge; a part's 130 KB written and read again
+  constexpr float kRefUs = 8.f, kRefTileUs = 0.6f;   // MODE 7: launch and fixed part, per tile
+  plan.waves = 8;
   plan.n_work = plan.n_slots = 0;
-  constexpr int kFix = 6, kMerge = 9;
-  if (rows_wg != 256 || p->p_quant != SQ_P_NONE) return;
-  const int64_t nQB = (Nq + rows_wg - 1) / rows_wg, mult = B * Hq;
+  if (own4 && p->window_mode == SQ_WINDOW_SIZES && p->block_m == 64) {
+    plan.waves = 2;   // separate 4-bit operands with 64-row blocks: a workgroup of one block (with 128-row blocks: DUAL)
+    return;
+  }
+  const int64_t nQB = (Nq + 255) / 256, mult = B * Hq;
   if (mult * nQB > kMaxRounds * kCUs) return;
+  const float step = kStepUs[p->p_quant];
   int w_max = 0;
   if (p->window_mode == SQ_WINDOW_SIZES)
     for (int h = 0; h < Hq; ++h) w_max = std::max(w_max, std::max(p->w8[h], p->w4[h]));
+  // one workgroup per block of `rows` rows: the blocks of a head, longest first, on kCUs / mult CUs (each of them stands
+  // for the same block of every head)
   int len[kMaxRounds * kCUs], longest = 0;
-  for (int qb = 0; qb < nQB; ++qb) {
-    len[qb] = tiles_of_block(p, (int64_t)qb * rows_wg, std::min<int64_t>(Nq, (int64_t)(qb + 1) * rows_wg), w_max);
-    longest = std::max(longest, len[qb]);
+  auto unsplit_us = [&](int rows, float tile_us) {
+    const int n = (int)((Nq + rows - 1) / rows), cus = (int)std::max<int64_t>(1, kCUs / mult), rounds = (int)((mult + kCUs - 1) / kCUs);
+    struct Cu { float load, tiles; } cu[kCUs] = {};
+    const auto later = [](const Cu& x, const Cu& y) { return x.load > y.load; };   // a heap with the least loaded CU in front
+    float total = 0, last = 0, last_tiles = 0;
+    for (int qb = n - 1; qb >= 0; --qb) {
+      const int t = tiles_of_block(p, (int64_t)qb * rows, std::min<int64_t>(Nq, (int64_t)(qb + 1) * rows), w_max);
+      if (rows == 256) {
+        len[qb] = t;
+        longest = std::max(longest, t);
+      }
+      std::pop_heap(cu, cu + cus, later);
+      Cu& c = cu[cus - 1];
+      c.load += (t * tile_us + kFixUs) * rounds;
+      c.tiles += (float)t * rounds;
+      total += (float)t * mult;
+      if (c.load > last) {
+        last = c.load;
+        last_tiles = c.tiles;
+      }
+      std::push_heap(cu, cu + cus, later);
+    }
+    return last + kFullChip * std::min(1.f, total / (kCUs * last_tiles)) * last_tiles * tile_us;
+  };
+  float best = unsplit_us(256, step);
+  const bool four_waves = !own4 && (p->p_quant <= SQ_P_E4M3_BLOCK || p->p_quant == SQ_P_E4M3_MX_FP8_PV);
+  if (four_waves && mult * ((Nq + 127) / 128) <= 2 * kCUs) {
+    const float us = unsplit_us(128, step * kFourWaves[p->p_quant]);
+    if (us < best) {
+      best = us;
+      plan.waves = 4;
+    }
   }
-  if (longest <= kMinTiles + kMerge) return;
-  // Unsplit: the blocks of one head, longest first, on kCUs / mult CUs (each stands for the same block of every head)
-  int load[kCUs] = {0}, best = 0;
-  const int cus = (int)std::max<int64_t>(1, kCUs / mult), rounds = (int)((mult + kCUs - 1) / kCUs);
-  for (int64_t qb = nQB - 1; qb >= 0; --qb) {
-    int* least = std::min_element(load, load + cus);
-    *least += (len[qb] + kFix) * rounds;
-    best = std::max(best, *least);
-  }
-  // Split: for each number of workgroups per CU the smallest share that keeps to it
+  if (longest <= kMinTiles || (own4 && p->p_quant != SQ_P_NONE) || p->p_quant == SQ_P_E4M3_MX_FP8_PV) return;
+  const bool ref_pass = p->p_quant >= SQ_P_E4M3_STATIC && p->p_quant <= SQ_P_E4M3_FP8_PV;
   auto workgroups = [&](int cap) {
     int64_t n = 0;
     for (int qb = 0; qb < nQB; ++qb) n += (len[qb] + cap - 1) / cap;
     return n;
   };
+  float total = 0;
+  for (int qb = 0; qb < nQB; ++qb) total += (float)len[qb] * mult;
   int cap = 0;
   for (int m = 1; m <= kMaxRounds; ++m) {
-    int lo = kMinTiles, hi = longest;
+    int lo = kMinTiles, hi = longest;   // the smallest share that keeps to m workgroups per CU
     while (lo < hi) {
       const int c = (lo + hi) / 2;
       if (workgroups(c) * mult <= m * kCUs) hi = c;
       else lo = c + 1;
     }
-    const int est = m * (lo + kFix) + kMerge;
-    if (lo < longest && est * 20 < best * 19 && workgroups(lo) <= kMaxSplitWork) {
-      best = est;
+    if (lo >= longest || workgroups(lo) > kMaxSplitWork) continue;
+    float us = m * (lo * step * (1.f + kFullChip * std::min(1.f, total / (kCUs * m * lo))) + kFixUs) + kMergeUs + kPartUs * mult * workgroups(lo);
+    if (ref_pass) us += m * lo * kRefTileUs + kRefUs;
+    if (us < 0.97f * best) {
+      best = us;
       cap = lo;
     }
   }
   if (cap == 0) return;
+  plan.waves = 8;
   for (int64_t qb = nQB - 1; qb >= 0; --qb) {
     const int parts = std::min((len[qb] + cap - 1) / cap, 255);
     for (int i = 0; i < parts; ++i) plan.work[plan.n_work++] = SplitWork{(uint16_t)qb, (uint16_t)plan.n_slots, (uint8_t)i, (uint8_t)parts};
@@ -1669,13 +1751,9 @@ void plan_split(const sq_prefill_params* p, int64_t B, int64_t Hq, int64_t Nq, i
   std::stable_sort(plan.work, plan.work + plan.n_work, [&](const SplitWork& x, const SplitWork& y) { return len[x.qb] * y.parts > len[y.qb] * x.parts; });
 }
 
-constexpr size_t kPartRowBytes = 64 * 16 * 16 + 64 * 8;   // per wave of a part: accumulators, denominator and reference point
+constexpr size_t kPartRowBytes = 64 * 16 * 16 + 64 * 8 + 32 * 4;   // per wave of a part: accumulators, denominator and reference point
 
-size_t part_bytes(const SplitPlan& plan, int64_t B, int64_t Hq) { return (size_t)(B * Hq) * plan.n_slots * 8 * kPartRowBytes; }
-
-// waves per workgroup: separate 4-bit operands with 64-row blocks take a workgroup of one block (two waves); 128-row blocks
-// one of two blocks that walk the few tiles on which they disagree twice (DUAL)
-int waves_of(const sq_prefill_params* p, bool own4) { return p->window_mode == SQ_WINDOW_SIZES && own4 && p->block_m == 64 ? 2 : 8; }
+size_t part_bytes(const LaunchPlan& plan, int64_t B, int64_t Hq) { return (size_t)(B * Hq) * plan.n_slots * 8 * kPartRowBytes; }
 
 }  // namespace
 }  // namespace sq
@@ -1692,10 +1770,11 @@ extern "C" size_t sq_prefill_workspace_bytes(int64_t batch, int64_t num_kv_heads
 extern "C" size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t qo_len, int64_t kv_len,
                                                    const sq_prefill_params* p) {
   const size_t need = sq_prefill_workspace_bytes(batch, num_kv_heads, kv_len, kD);
-  if (!p || need == 0 || num_q_heads <= 0 || num_q_heads > kMaxHeads || qo_len <= 0) return need;
+  if (!p || need == 0 || p->p_quant < SQ_P_NONE || p->p_quant > SQ_P_E4M3_MX_FP8_PV || num_q_heads <= 0 || num_q_heads > kMaxHeads || qo_len <= 0) return need;
   if (p->window_mode == SQ_WINDOW_SIZES && (!p->w8 || !p->w4 || p->num_heads_w != num_q_heads || p->block_m <= 0 || p->sink < 0)) return need;
-  SplitPlan plan;
-  plan_split(p, batch, num_q_heads, qo_len, 256, plan);
+  LaunchPlan plan;
+  // (operands of their own for the 4-bit range are what the launches with 128-row query blocks come with)
+  plan_launch(p, p->window_mode == SQ_WINDOW_SIZES && p->block_m == 128, batch, num_q_heads, qo_len, plan);
   return need + part_bytes(plan, batch, num_q_heads);
 }
 
@@ -1881,7 +1960,10 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   local.Nq = (int)Nq;
   local.Nk = (int)Nk;
   local.nT = nT;
-  const int waves = waves_of(p, q4 != nullptr), rows_wg = waves * 32;
+  LaunchPlan plan;
+  plan_launch(p, q4 != nullptr, B, Hq, Nq, plan);
+  const bool split = plan.n_work > 0 && (size_t)numel_of(workspace) * (workspace->dtype.bits / 8) >= need + part_bytes(plan, B, Hq);
+  const int waves = plan.waves, rows_wg = waves * 32;
   local.nQB = (int)((Nq + rows_wg - 1) / rows_wg);
   SQ_REQUIRE(p->q_quant == 0 || p->q_quant == 8, SQ_EINVAL, "sq_prefill_fwd: q_quant must be 0 or 8 (got %d)", (int)p->q_quant);
   SQ_REQUIRE(!(p->q_quant && q4), SQ_EINVAL, "sq_prefill_fwd: q_quant applies to launches without a separate 4-bit operand set");
@@ -1902,13 +1984,11 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
     }
   const int pairs = (int)(B * Hkv);
   int items = local.group * local.nQB;
-  SplitPlan plan;
-  plan_split(p, B, Hq, Nq, rows_wg, plan);
-  const bool split = plan.n_work > 0 && (size_t)numel_of(workspace) * (workspace->dtype.bits / 8) >= need + part_bytes(plan, B, Hq);
   if (split) {
     local.n_slots = plan.n_slots;
     local.part_o = (float*)(wsp + need);
     local.part_lm = (float2*)(wsp + need + (size_t)(B * Hq) * plan.n_slots * 8 * (64 * 16 * 16));
+    local.part_ref = (float*)(wsp + need + (size_t)(B * Hq) * plan.n_slots * 8 * (64 * 16 * 16 + 64 * 8));
     memcpy(local.work, plan.work, plan.n_work * sizeof(SplitWork));
     items = local.group * plan.n_work;
   }
@@ -1951,17 +2031,35 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
       default: SQ_LAUNCH_PREFILL_DUAL(BF, 3); break;                 \
     }                                                               \
   } while (0)
+#define SQ_LAUNCH_FOUR(BF)                                             \
+  do {                                                                 \
+    switch (k_scale ? 6 : p->p_quant) {                                \
+      case SQ_P_NONE: SQ_LAUNCH_PREFILL(BF, 4, 0); break;              \
+      case SQ_P_E4M3_STATIC: SQ_LAUNCH_PREFILL(BF, 4, 1); break;       \
+      case SQ_P_E4M3_BLOCK: SQ_LAUNCH_PREFILL(BF, 4, 2); break;        \
+      case SQ_P_E4M3_MX_FP8_PV: SQ_LAUNCH_PREFILL(BF, 4, 5); break;    \
+      default: SQ_LAUNCH_PREFILL(BF, 4, 6); break;                     \
+    }                                                                  \
+  } while (0)
 #define SQ_LAUNCH_SPLIT(BF, M, DU)                                                                                           \
   do {                                                                                                                     \
     SQ_HIP(hipFuncSetAttribute((const void*)prefill_kernel<BF, 8, M, DU, true>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                (int)smem));                                                                                \
     hipLaunchKernelGGL((prefill_kernel<BF, 8, M, DU, true>), dim3(blocks), dim3(8 * 64), smem, st, local);                 \
   } while (0)
-#define SQ_LAUNCH_SPLITS(BF)                                                                                  \
-  do {                                                                                                        \
-    if (k_scale) SQ_LAUNCH_SPLIT(BF, 6, false);                                                               \
-    else if (q4) SQ_LAUNCH_SPLIT(BF, 0, true);                                                                \
-    else SQ_LAUNCH_SPLIT(BF, 0, false);                                                                       \
+#define SQ_LAUNCH_SPLITS(BF)                                                     \
+  do {                                                                           \
+    if (ref_pass) SQ_LAUNCH_SPLIT(BF, 7, false);                                 \
+    switch (k_scale ? 6 : p->p_quant) {                                          \
+      case SQ_P_NONE:                                                            \
+        if (q4) SQ_LAUNCH_SPLIT(BF, 0, true); else SQ_LAUNCH_SPLIT(BF, 0, false); \
+        break;                                                                   \
+      case SQ_P_E4M3_STATIC: SQ_LAUNCH_SPLIT(BF, 1, false); break;               \
+      case SQ_P_E4M3_BLOCK: SQ_LAUNCH_SPLIT(BF, 2, false); break;                \
+      case SQ_P_E4M3_STATIC_FAST: SQ_LAUNCH_SPLIT(BF, 3, false); break;          \
+      case SQ_P_E4M3_FP8_PV: SQ_LAUNCH_SPLIT(BF, 4, false); break;               \
+      default: SQ_LAUNCH_SPLIT(BF, 6, false); break;                             \
+    }                                                                            \
   } while (0)
 #define SQ_LAUNCH_MODE(BF, W)                                   \
   do {                                                          \
@@ -1978,16 +2076,23 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
       default: SQ_LAUNCH_PREFILL(BF, W, 3); break;               \
     }                                                           \
   } while (0)
+  const bool ref_pass = p->p_quant >= SQ_P_E4M3_STATIC && p->p_quant <= SQ_P_E4M3_FP8_PV;   // as in plan_launch
   if (split) {
     if (bf) SQ_LAUNCH_SPLITS(true); else SQ_LAUNCH_SPLITS(false);
   } else if (waves == 8 && q4) {
     if (bf) SQ_LAUNCH_DUAL(true); else SQ_LAUNCH_DUAL(false);
   } else if (waves == 8) {
     if (bf) SQ_LAUNCH_MODE(true, 8); else SQ_LAUNCH_MODE(false, 8);
+  } else if (waves == 4) {
+    if (bf) SQ_LAUNCH_FOUR(true); else SQ_LAUNCH_FOUR(false);
   } else {
     if (bf) SQ_LAUNCH_MODE(true, 2); else SQ_LAUNCH_MODE(false, 2);
   }
-  if (split) hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)plan.n_work, 8, (unsigned)(B * Hq)), dim3(256), 0, st, local);
+  if (split) {
+    const dim3 mgrid((unsigned)plan.n_work, 8, (unsigned)(B * Hq));
+    if (pv8) hipLaunchKernelGGL((prefill_merge_kernel<true>), mgrid, dim3(256), 0, st, local);
+    else hipLaunchKernelGGL((prefill_merge_kernel<false>), mgrid, dim3(256), 0, st, local);
+  }
 #undef SQ_LAUNCH_DUAL
 #undef SQ_LAUNCH_PREFILL_DUAL
 #undef SQ_LAUNCH_MODE

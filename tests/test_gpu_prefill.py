@@ -263,8 +263,8 @@ def test_chunked_prefill_offset():
     (1, 2, 1, 1025, 0, None),            # last block of a single row: seven of its waves have none
     (3, 2, 1, 300, 2048, None),          # a chunk behind a context, several sequences
     (1, 2, 1, 64, 4096, None),           # one 64-row block over 65 tiles
-    (1, 4, 2, 2500, 0, (256, 0.125, 0.5)),   # sink and windows: a share may begin inside the sink or at the jump behind it
-    (1, 2, 1, 2304, 0, (64, 512, 1024)),     # absolute windows with their own 4-bit operands (tiles walked twice)
+    (1, 4, 2, 4000, 0, (256, 0.125, 0.75)),   # sink and windows: a share may begin inside the sink or at the jump behind it
+    (1, 2, 1, 3008, 0, (64, 512, 2048)),     # absolute windows with their own 4-bit operands (tiles walked twice)
 ])
 def test_split_key_ranges_match_unsplit_launch_and_oracle(B, Hq, Hkv, N, offset, window):
     """Launches too small to fill the chip split the key range of a query block over several workgroups (given the workspace
@@ -306,6 +306,50 @@ def test_split_key_ranges_match_unsplit_launch_and_oracle(B, Hq, Hkv, N, offset,
     assert torch.allclose(lse.cpu(), lse_ref.reshape(lse.shape).float(), atol=2e-4)
     assert torch.allclose(lse, lse_whole, atol=2e-4)
     assert not torch.equal(out, whole)     # the workspace the wrapper takes by itself does split these launches
+
+
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,offset", [(3010, 0), (200, 3072)])
+def test_split_key_ranges_keep_the_e4m3_grid(mode, N, offset):
+    """The parts of a split row start from the reference point the whole row would have had there (a pass that forms the
+    parts' row maxima), so the e4m3 grid is the unsplit launch's: what differs is a score's last bit, which moves the few
+    probabilities that sit on a rounding boundary by one step of the grid (up to 2^-3 of themselves).  With scores of unit
+    variance a row of n keys averages about n / e of them, so one such step moves an output element by about
+    2^-3 / sqrt(n / e) of its rms: 4e-3 at n = 3000.  Against the unsplit launch: cosine, 99.9 % of the elements within two
+    such steps (8e-3 rms), all within 0.25 rms."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
+
+    print(f"case prefill split grid mode={mode} N={N} offset={offset}", flush=True)
+    _, k, v = _rand(1, 3, 1, offset + N, 128, 41)
+    q = _rand(1, 3, 1, N, 128, 42)[0]
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    out, lse = attn_causal(qd, kd, vd, "HND", torch.float32, return_lse=True, p_quant=mode, q_offset=offset)
+    whole, lse_whole = attn_causal(qd, kd, vd, "HND", torch.float32, return_lse=True, p_quant=mode, q_offset=offset,
+                                   workspace=prefill_workspace(1, 1, offset + N, qd.device))
+    torch.cuda.synchronize()
+    assert not torch.equal(out, whole)
+    _check(out, whole.cpu(), True, q_tol=8e-3)
+    assert torch.allclose(lse, lse_whole, atol=2e-4)
+    exact, _ = A.exact_attention(A.fold_scale(q, 128), k, v, causal=True, q_offset=offset, score_scale=math.log(2.0))
+    assert _cos(out.cpu(), exact) >= 0.999
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 5])
+@pytest.mark.parametrize("N,window", [(257, None), (640, (64, 128, 256))])
+def test_rows_do_not_depend_on_the_workgroup_size(mode, N, window):
+    """Short launches run in workgroups of 128 rows, launches that fill the chip in workgroups of 256; a row's arithmetic is the same in
+    both (mode 2: the same 64-row groups), so a sequence alone gives the bits it gives in a batch of 130."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace, run_prefill
+
+    print(f"case prefill workgroup size mode={mode} N={N} window={window}", flush=True)
+    q, k, v = (t.to(DEV) for t in _rand(1, 4, 2, N, 128, 77))
+    w = None if window is None else {"block_m": 64, "sink": window[0], "w8": [window[1]] * 4, "w4": [window[2]] * 4}
+    one = run_prefill(q, k, v, output_dtype=torch.float32, p_quant=mode, window=w, workspace=prefill_workspace(1, 2, N, q.device))
+    many = run_prefill(*(t.repeat(130, 1, 1, 1) for t in (q, k, v)), output_dtype=torch.float32, p_quant=mode, window=w,
+                       workspace=prefill_workspace(130, 2, N, q.device))
+    torch.cuda.synchronize()
+    assert torch.equal(one[0], many[0]) and torch.equal(one[0], many[129])
 
 
 @pytest.mark.parametrize("sink,r8,r4", [(128, 0.25, 0.25), (256, [0.125, 0.5], [0.5, 0.5]), (0, 0.0, 0.0), (64, 2.0, 2.0)])
