@@ -79,7 +79,9 @@ class HistogramParams(ctypes.Structure):
 
 HIST_ABSOLUTE, HIST_RELATIVE, HIST_RELATIVE_SINK = 0, 1, 2
 
-_P = ctypes.POINTER(DLTensor)
+# tensor arguments are DLTensor*, handed over as the plain addresses the capsules hold (`Borrowed.ptr`): a typed
+# ctypes pointer per argument cost three times as much to make as the capsule itself
+_P = ctypes.c_void_p
 
 # every symbol include/sqattn.h declares: name -> (restype, argtypes)
 SYMBOLS = {
@@ -171,20 +173,22 @@ def probe_lib() -> ctypes.CDLL:
 _capsule_ptr = ctypes.pythonapi.PyCapsule_GetPointer
 _capsule_ptr.restype = ctypes.c_void_p
 _capsule_ptr.argtypes = [ctypes.py_object, ctypes.c_char_p]
+_to_dlpack = torch.utils.dlpack.to_dlpack
 
 
 class Borrowed:
     """A DLTensor borrowed from a torch tensor through its DLPack capsule.
 
     The capsule is kept alive (and never consumed) for the lifetime of this object; dropping it runs
-    the producer's deleter, so the library only ever sees borrowed memory.
+    the producer's deleter, so the library only ever sees borrowed memory.  `ptr` is the DLTensor's address.
     """
+
+    __slots__ = ("tensor", "capsule", "ptr")
 
     def __init__(self, t: torch.Tensor):
         self.tensor = t
-        self.capsule = torch.utils.dlpack.to_dlpack(t)
-        addr = _capsule_ptr(self.capsule, b"dltensor")
-        self.ptr = ctypes.cast(addr, _P)  # DLManagedTensor starts with its DLTensor
+        self.capsule = _to_dlpack(t)
+        self.ptr = _capsule_ptr(self.capsule, b"dltensor")  # DLManagedTensor starts with its DLTensor
 
 
 def dl(t: Optional[torch.Tensor]):
@@ -193,6 +197,16 @@ def dl(t: Optional[torch.Tensor]):
 
 def ptr(b: Optional[Borrowed]):
     return None if b is None else b.ptr
+
+
+def borrow(*tensors: Optional[torch.Tensor]):
+    """(addresses, capsules) of several tensors for one library call, None for None.  The second list has to outlive the call:
+    it holds the capsules the addresses point into.
+
+    For the calls whose kernels are shorter than their host side: a `dl` / `ptr` pair with a typed pointer took 1.8 us per
+    tensor, this takes 0.6 us (decode over 1531 tokens 22.0 -> 15.4 us a call, selection + decode over it 38.7 -> 26.3 us)."""
+    capsules = [None if t is None else _to_dlpack(t) for t in tensors]
+    return [None if c is None else _capsule_ptr(c, b"dltensor") for c in capsules], capsules
 
 
 def check(code: int, library: Optional[ctypes.CDLL] = None) -> None:
@@ -207,5 +221,11 @@ def check(code: int, library: Optional[ctypes.CDLL] = None) -> None:
     raise RuntimeError(f"libsqattn_hip error {code}: {msg}")
 
 
-def current_stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def current_stream(device) -> int:
+    """Handle of the calling thread's current stream on `device`."""
+    if isinstance(device, torch.device) and device.index is not None:   # a GPU tensor's device
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream

@@ -126,8 +126,8 @@ def topk_select(query, centroids, clusters, cluster_size, k: int, num_kv_groups:
     if out is None:
         out = torch.empty((G, k), dtype=torch.int32, device=query.device)
     ws = workspace if workspace is not None else _workspace(G, 1, C, query.device)
-    b = [N.dl(t) for t in (query, centroids, clusters, cluster_size, out, ws)]
-    N.check(N.lib().sq_topk_select(*[N.ptr(x) for x in b], num_kv_groups, N.current_stream(query.device)))
+    ptrs, held = N.borrow(query, centroids, clusters, cluster_size, out, ws)
+    N.check(N.lib().sq_topk_select(*ptrs, num_kv_groups, N.current_stream(query.device)))
     return out
 
 

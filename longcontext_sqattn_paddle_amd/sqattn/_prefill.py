@@ -7,7 +7,7 @@ from typing import Optional, Sequence
 import torch
 
 from .. import _native as N
-from ._common import pad_head_dim, require_gpu
+from ._common import KERNEL_HEAD_DIM, pad_head_dim, require_gpu
 
 
 def prefill_workspace(B: int, Hkv: int, kv_len: int, device) -> torch.Tensor:
@@ -53,8 +53,8 @@ def run_prefill(q, k, v, *, tensor_layout="HND", output_dtype=torch.float16, ret
         params.window_mode = N.WINDOW_NONE
         params.block_m = 128
     else:
-        w8 = (ctypes.c_int32 * Hq)(*[int(x) for x in window["w8"]])
-        w4 = (ctypes.c_int32 * Hq)(*[int(x) for x in window["w4"]])
+        w8 = (ctypes.c_int32 * Hq)(*map(int, window["w8"]))
+        w4 = (ctypes.c_int32 * Hq)(*map(int, window["w4"]))
         keep += [w8, w4]
         params.window_mode = N.WINDOW_SIZES
         params.block_m = int(window["block_m"])
@@ -66,12 +66,13 @@ def run_prefill(q, k, v, *, tensor_layout="HND", output_dtype=torch.float16, ret
         # room for the parts of split key ranges where this launch is split
         workspace = torch.empty(lib.sq_prefill_workspace_bytes_split(B, Hq, Hkv, Nq, Nk, ctypes.byref(params)), dtype=torch.uint8, device=q.device)
     if k_scale is not None:
-        b = [N.dl(t) for t in (q, k, k_scale, v, o, lse, workspace)]
-        N.check(lib.sq_prefill_int8qk_fwd(*[N.ptr(x) for x in b], ctypes.byref(params), N.current_stream(q.device)))
+        ptrs, held = N.borrow(q, k, k_scale, v, o, lse, workspace)
+        N.check(lib.sq_prefill_int8qk_fwd(*ptrs, ctypes.byref(params), N.current_stream(q.device)))
     else:
-        b = [N.dl(t) for t in (q, k, v, q4, k4, o, lse, workspace)]
-        N.check(lib.sq_prefill_fwd(*[N.ptr(x) for x in b], ctypes.byref(params), N.current_stream(q.device)))
-    o = o[..., :head_dim_og]
+        ptrs, held = N.borrow(q, k, v, q4, k4, o, lse, workspace)
+        N.check(lib.sq_prefill_fwd(*ptrs, ctypes.byref(params), N.current_stream(q.device)))
+    if head_dim_og != KERNEL_HEAD_DIM:
+        o = o[..., :head_dim_og]
     return (o, lse) if return_lse else o
 
 
@@ -102,7 +103,12 @@ def align_windows(w8, w4, sink: int, block_m: int):
     window is raised to the query block in that case: the 4-bit range then ends where the block starts, and the
     block's own keys are visited once, masked, as 8-bit operands."""
     up = lambda x, m: (int(x) + m - 1) // m * m
-    w8 = [up(x, 64) for x in w8]
-    w4 = [up(x, 64) for x in w4]
-    w8 = [max(a, block_m) if b > a and a < block_m else a for a, b in zip(w8, w4)]
-    return w8, w4, up(sink, 64)
+
+    def aligned(a, b):
+        a, b = up(a, 64), up(b, 64)
+        return (max(a, block_m) if b > a and a < block_m else a), b
+
+    # heads mostly share their sizes: each pair once (28 heads: 11 us of host otherwise, as much as a short launch)
+    pairs = list(zip(w8, w4))
+    sizes = {p: aligned(*p) for p in set(pairs)}
+    return [sizes[p][0] for p in pairs], [sizes[p][1] for p in pairs], up(sink, 64)

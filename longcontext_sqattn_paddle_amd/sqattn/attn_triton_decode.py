@@ -11,7 +11,7 @@ from typing import Optional
 import torch
 
 from .. import _native as N
-from ._common import pad_head_dim, require_gpu
+from ._common import KERNEL_HEAD_DIM, pad_head_dim, require_gpu
 
 
 def attn_decode(q, k, v, tensor_layout="HND", output_dtype=torch.float16, return_lse=False, is_P_fp8_quant=False,
@@ -41,10 +41,10 @@ def attn_decode(q, k, v, tensor_layout="HND", output_dtype=torch.float16, return
     o = out if out is not None else torch.empty(q.shape, dtype=output_dtype, device=q.device)
     lse = torch.empty([B, Hq, 1], dtype=torch.float32, device=q.device) if return_lse else None
     params = N.DecodeParams(N.LAYOUT[tensor_layout], N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE, max(num_splits, 0), head_dim_og)
-    bq, bk, bv, bs, bo, bl, bw = (N.dl(t) for t in (q, k, v, seqlens, o, lse, workspace))
-    N.check(lib.sq_decode_fwd(N.ptr(bq), N.ptr(bk), N.ptr(bv), N.ptr(bs), N.ptr(bo), N.ptr(bl), N.ptr(bw),
-                              params, N.current_stream(q.device)))
-    o = o[..., :head_dim_og]
+    ptrs, held = N.borrow(q, k, v, seqlens, o, lse, workspace)
+    N.check(lib.sq_decode_fwd(*ptrs, params, N.current_stream(q.device)))
+    if head_dim_og != KERNEL_HEAD_DIM:
+        o = o[..., :head_dim_og]
     return (o, lse) if return_lse else o
 
 
@@ -86,9 +86,10 @@ def attn_decode_selected(q, k, v, token_ids, tensor_layout="NHD", output_dtype=t
     o = out if out is not None else torch.empty(q.shape, dtype=output_dtype, device=q.device)
     lse = torch.empty([B, Hq, 1], dtype=torch.float32, device=q.device) if return_lse else None
     params = N.DecodeParams(N.LAYOUT[tensor_layout], N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE, max(num_splits, 0), head_dim_og)
-    b = [N.dl(t) for t in (q, k, v, token_ids, seqlens, o, lse, workspace)]
-    N.check(lib.sq_decode_selected_fwd(*[N.ptr(x) for x in b], params, N.current_stream(q.device)))
-    o = o[..., :head_dim_og]
+    ptrs, held = N.borrow(q, k, v, token_ids, seqlens, o, lse, workspace)
+    N.check(lib.sq_decode_selected_fwd(*ptrs, params, N.current_stream(q.device)))
+    if head_dim_og != KERNEL_HEAD_DIM:
+        o = o[..., :head_dim_og]
     return (o, lse) if return_lse else o
 
 

@@ -171,11 +171,11 @@ def fused_int_prepass(query, key, value, want_4bit=True, tensor_layout="NHD", qk
     k4 = torch.empty_like(key) if want_4bit else None
     need = lib.sq_fake_quant_prepass_workspace_bytes(B, Hkv, Nk)
     ws = torch.empty((need + 7) // 8, dtype=torch.float64, device=query.device)
-    b = [N.dl(t) for t in (query, key, value, q8, q4, k8, k4, v8, ws)]
+    ptrs, held = N.borrow(query, key, value, q8, q4, k8, k4, v8, ws)
     for name in (qk_qtype, v_qtype):
         if name not in N.QTYPE:
             raise ValueError(f"Invalid quantization type: {name}")
-    N.check(lib.sq_fake_quant_prepass_typed(*[N.ptr(x) for x in b], N.LAYOUT[tensor_layout], N.QTYPE[qk_qtype], N.QTYPE[v_qtype],
+    N.check(lib.sq_fake_quant_prepass_typed(*ptrs, N.LAYOUT[tensor_layout], N.QTYPE[qk_qtype], N.QTYPE[v_qtype],
                                             N.current_stream(query.device)))
     return q8, q4, k8, k4, v8
 
