@@ -139,6 +139,13 @@ int sq_prefill_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v, cons
                    const sq_prefill_params* params, void* stream);
 
 /*
+ * sq_prefill_fwd for a value that sq_fake_quant_prepass_vtiles has left as tiles (p_quant 0 - 3; the fp8 P.V modes make tiles
+ * of their own from v).  The value's token and head counts are the key's.  Other arguments as sq_prefill_fwd.
+ */
+int sq_prefill_vtiles_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v_tiles, const DLTensor* q4, const DLTensor* k4,
+                          DLTensor* out, DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream);
+
+/*
  * The same attention with Q.K^T as a real integer product (the second half of what sqattn/attn_replacer.py:334-365 and
  * the launch sqattn/attn_triton_mix_relative.py:439-475 only simulate: they fake-quantise query and key to 8 bits and
  * then multiply them as bf16).  k_codes: int8, laid out like k above, the per-token symmetric 8-bit codes of the
@@ -286,6 +293,15 @@ int sq_fake_quant_prepass(const DLTensor* query, const DLTensor* key, const DLTe
  * library's fp32 log2 rounds a value just below a power of two up to the integer.
  */
 enum { SQ_QTYPE_INT = 0, SQ_QTYPE_E4M3 = 1, SQ_QTYPE_E5M2 = 2 };
+/*
+ * sq_fake_quant_prepass_typed with the value written as the prefill kernel's fp16 V^T tiles instead of as rows: `v_tiles` is
+ * a compact, 16-byte aligned buffer of at least batch * Hkv * ceil(N / 64) * 16384 bytes for sq_prefill_vtiles_fwd.
+ * The tiles are the ones sq_prefill_fwd makes of v8.  bf16 tensors only.
+ */
+int sq_fake_quant_prepass_vtiles(const DLTensor* query, const DLTensor* key, const DLTensor* value, DLTensor* q8, DLTensor* q4,
+                                 DLTensor* k8, DLTensor* k4, DLTensor* v_tiles, DLTensor* workspace, int32_t layout, int32_t qk_qtype,
+                                 int32_t v_qtype, void* stream);
+
 /*
  * The pre-pass for a real integer Q.K^T (sq_prefill_int8qk_fwd): key centring as above, then instead of the fake-
  * quantised key its two factors -- k_codes int8 [like key] = clamp(round(key_c / scale), -128, 127), the codes

@@ -106,6 +106,8 @@ SYMBOLS = {
     "sq_fake_quant_prepass_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 3),
     "sq_fake_quant_prepass": (ctypes.c_int, [_P] * 9 + [ctypes.c_int32, ctypes.c_void_p]),
     "sq_fake_quant_prepass_typed": (ctypes.c_int, [_P] * 9 + [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]),
+    "sq_fake_quant_prepass_vtiles": (ctypes.c_int, [_P] * 9 + [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]),
+    "sq_prefill_vtiles_fwd": (ctypes.c_int, [_P] * 8 + [ctypes.POINTER(PrefillParams), ctypes.c_void_p]),
     "sq_rmsnorm": (ctypes.c_int, [_P, _P, _P, ctypes.c_float, ctypes.c_void_p]),
     "sq_silu_and_mul": (ctypes.c_int, [_P, _P, ctypes.c_void_p]),
     "sq_rope": (ctypes.c_int, [_P] * 6 + [ctypes.c_int32, ctypes.c_void_p]),

@@ -108,6 +108,11 @@ __device__ __forceinline__ float e4m3_roundtrip(float x) {
   return __builtin_amdgcn_cvt_f32_fp8(pk, 0);
 }
 
+// V^T tiles of the prefill kernel: 64 keys per tile; position of key u (0..15) inside its group of 16: bits 2 and 3 swapped,
+// so that the 8 keys a lane owns in one half of the S^T accumulator are 8 consecutive halfs.
+constexpr int kVTileKeys = 64;
+__device__ __forceinline__ int perm16(int u) { return (u & 3) | ((u & 4) << 1) | ((u & 8) >> 1); }
+
 __device__ __forceinline__ float wave_xor_max(float v, int mask) { return fmaxf(v, __shfl_xor(v, mask)); }
 
 // ---- division by a divisor that many dividends share.  A correctly rounded fp32 division is, on this hardware, a

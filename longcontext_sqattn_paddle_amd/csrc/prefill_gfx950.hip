@@ -29,7 +29,7 @@ namespace sq {
 namespace {
 
 constexpr int kD = 128;
-constexpr int kBN = 64;                  // keys per tile (BLOCK_N of every reference kernel)
+constexpr int kBN = kVTileKeys;          // keys per tile (BLOCK_N of every reference kernel)
 // LDS tiles are unpadded and XOR-swizzled at 16-byte granularity (they are filled by global_load_lds, which
 // writes 64 consecutive 16-byte slots per wave instruction): chunk c of K row n sits in slot c ^ (n & 15),
 // chunk c of V^T row d in slot c ^ ((d >> 1) & 7).  The 16 rows a quarter-wave reads at one chunk index then
@@ -87,10 +87,6 @@ struct PrepArgs {
   int64_t v_sb, v_sh, v_sn;
   int32_t Nk, nT, Hkv, is_bf16;
 };
-
-// position of key u (0..15) inside its group of 16 in the V^T tile: bits 2 and 3 swapped, so that the 8
-// keys a lane owns in one half of the S^T accumulator are 8 consecutive halfs.
-__device__ __forceinline__ int perm16(int u) { return (u & 3) | ((u & 4) << 1) | ((u & 8) >> 1); }
 
 __global__ __launch_bounds__(256) void prefill_prep_v_kernel(PrepArgs a) {
   const int j = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
@@ -1780,33 +1776,40 @@ extern "C" size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_
 
 namespace {
 int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const DLTensor* q4, const DLTensor* k4, DLTensor* out,
-                 DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream, const DLTensor* k_scale);
+                 DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream, const DLTensor* k_scale, const DLTensor* v_tiles);
 }
 
 extern "C" int sq_prefill_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v, const DLTensor* q4,
                               const DLTensor* k4, DLTensor* out, DLTensor* lse, DLTensor* workspace,
                               const sq_prefill_params* p, void* stream) {
-  return prefill_impl(q, k, v, q4, k4, out, lse, workspace, p, stream, nullptr);
+  return prefill_impl(q, k, v, q4, k4, out, lse, workspace, p, stream, nullptr, nullptr);
+}
+
+extern "C" int sq_prefill_vtiles_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v_tiles, const DLTensor* q4, const DLTensor* k4,
+                                     DLTensor* out, DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream) {
+  SQ_REQUIRE(v_tiles, SQ_EINVAL, "sq_prefill_vtiles_fwd: v_tiles is null");
+  return prefill_impl(q, k, nullptr, q4, k4, out, lse, workspace, p, stream, nullptr, v_tiles);
 }
 
 extern "C" int sq_prefill_int8qk_fwd(const DLTensor* q, const DLTensor* k_codes, const DLTensor* k_scale, const DLTensor* v,
                                      DLTensor* out, DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream) {
   SQ_REQUIRE(k_scale, SQ_EINVAL, "sq_prefill_int8qk_fwd: k_scale is null");
-  return prefill_impl(q, k_codes, v, nullptr, nullptr, out, lse, workspace, p, stream, k_scale);
+  return prefill_impl(q, k_codes, v, nullptr, nullptr, out, lse, workspace, p, stream, k_scale, nullptr);
 }
 
 namespace {
 // k_scale != null: `k` holds int8 codes and the scores come from the int8 matrix instruction (sq_prefill_int8qk_fwd)
+// v_tiles != null: v is null, the fp16 V^T tiles are there already (sq_prefill_vtiles_fwd)
 int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const DLTensor* q4, const DLTensor* k4, DLTensor* out,
-                 DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream, const DLTensor* k_scale) {
+                 DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream, const DLTensor* k_scale, const DLTensor* v_tiles) {
   SQ_REQUIRE(p, SQ_EINVAL, "sq_prefill_fwd: params is null");
-  SQ_REQUIRE(q && k && v && out, SQ_EINVAL, "sq_prefill_fwd: q, k, v and out must be non-null");
+  SQ_REQUIRE(q && k && (v || v_tiles) && out, SQ_EINVAL, "sq_prefill_fwd: q, k, v and out must be non-null");
   SQ_REQUIRE(p->layout == SQ_LAYOUT_HND || p->layout == SQ_LAYOUT_NHD, SQ_EINVAL, "tensor_layout %d not supported", p->layout);
   SQ_REQUIRE(p->p_quant >= SQ_P_NONE && p->p_quant <= SQ_P_E4M3_MX_FP8_PV, SQ_EINVAL, "sq_prefill_fwd: p_quant %d not supported", p->p_quant);
   SQ_REQUIRE((q4 == nullptr) == (k4 == nullptr), SQ_EINVAL, "sq_prefill_fwd: q4 and k4 must be given together");
   int rc;
   const int dev = q->device.device_id;
-  if ((rc = check_tensor(q, "q", 4, dev)) || (rc = check_tensor(k, "k", 4, dev)) || (rc = check_tensor(v, "v", 4, dev)) ||
+  if ((rc = check_tensor(q, "q", 4, dev)) || (rc = check_tensor(k, "k", 4, dev)) || (v && (rc = check_tensor(v, "v", 4, dev))) ||
       (rc = check_tensor(out, "out", 4, dev)))
     return rc;
   if (q4 && ((rc = check_tensor(q4, "q4", 4, dev)) || (rc = check_tensor(k4, "k4", 4, dev)))) return rc;
@@ -1818,7 +1821,7 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
     SQ_REQUIRE(p->p_quant == SQ_P_NONE && p->q_quant == 0, SQ_EINVAL,
                "sq_prefill_int8qk_fwd: p_quant and q_quant must be 0 (the query's codes are formed by the kernel, P stays fp16)");
   } else {
-    SQ_REQUIRE(dtype_of(k) == dt && dtype_of(v) == dt, SQ_EDTYPE, "sq_prefill_fwd: q, k, v dtypes differ");
+    SQ_REQUIRE(dtype_of(k) == dt && (!v || dtype_of(v) == dt), SQ_EDTYPE, "sq_prefill_fwd: q, k, v dtypes differ");
   }
   if (q4) SQ_REQUIRE(dtype_of(q4) == dt && dtype_of(k4) == dt, SQ_EDTYPE, "sq_prefill_fwd: q4/k4 dtype differs from q");
   const DType odt = dtype_of(out);
@@ -1833,7 +1836,7 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   SQ_REQUIRE(Hq <= kMaxHeads, SQ_EUNSUPPORTED, "sq_prefill_fwd: more than %d q heads", kMaxHeads);
   SQ_REQUIRE(k->shape[0] == B && k->shape[3] == D, SQ_ESHAPE, "sq_prefill_fwd: k shape mismatch");
   for (int i = 0; i < 4; ++i) {
-    SQ_REQUIRE(v->shape[i] == k->shape[i], SQ_ESHAPE, "sq_prefill_fwd: v shape differs from k");
+    SQ_REQUIRE(!v || v->shape[i] == k->shape[i], SQ_ESHAPE, "sq_prefill_fwd: v shape differs from k");
     SQ_REQUIRE(out->shape[i] == q->shape[i], SQ_ESHAPE, "sq_prefill_fwd: out shape differs from q");
     if (q4) {
       SQ_REQUIRE(q4->shape[i] == q->shape[i] && k4->shape[i] == k->shape[i], SQ_ESHAPE, "sq_prefill_fwd: q4/k4 shapes differ from q/k");
@@ -1847,12 +1850,12 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
              (long long)(p->q_offset + Nq), (long long)Nk);
   SQ_REQUIRE(Nk < (1ll << 31) - 65536, SQ_EUNSUPPORTED, "sq_prefill_fwd: more than 2^31 keys");
   // a 64-key tile is copied with one 64-bit tile base and 32-bit per-lane byte offsets: a tile must span less than 4 GiB
-  SQ_REQUIRE(stride_of(k, ndim) > 0 && stride_of(k, ndim) < (1ll << 24) && stride_of(v, ndim) > 0 && stride_of(v, ndim) < (1ll << 31), SQ_EUNSUPPORTED,
+  SQ_REQUIRE(stride_of(k, ndim) > 0 && stride_of(k, ndim) < (1ll << 24) && (!v || (stride_of(v, ndim) > 0 && stride_of(v, ndim) < (1ll << 31))), SQ_EUNSUPPORTED,
              "sq_prefill_fwd: token stride of k must be below 2^24 elements (got %lld)", (long long)stride_of(k, ndim));
   const DLTensor* ts[5] = {q, k, v, out, nullptr};
   for (int t = 0; t < 4; ++t)
     for (int i = 0; i < 3; ++i)
-      SQ_REQUIRE(stride_of(ts[t], i) % (t == 3 && odt == DType::F32 ? 4 : 8) == 0 || ts[t]->shape[i] == 1, SQ_ESHAPE,
+      SQ_REQUIRE(!ts[t] || stride_of(ts[t], i) % (t == 3 && odt == DType::F32 ? 4 : 8) == 0 || ts[t]->shape[i] == 1, SQ_ESHAPE,
                  "sq_prefill_fwd: strides must keep rows 16-byte aligned");
   if (lse) {
     SQ_REQUIRE(on_gpu(lse) && lse->device.device_id == dev, SQ_EDEVICE, "sq_prefill_fwd: lse not on the same device");
@@ -1898,20 +1901,27 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   // workspace: fp16 tiles (modes 0-3), or e4m3 tiles (half the size) followed by the per-channel scale tables
   const size_t tiles8 = ((size_t)B * Hkv * nT * (kD * kBN) + 255) / 256 * 256;
   PrepArgs pa;
-  pa.v = data_of(v);
+  pa.v = v ? data_of(v) : nullptr;
   pa.vt = (_Float16*)wsp;
   pa.vt8 = (uint8_t*)wsp;
   pa.vmax_bits = (uint32_t*)(wsp + tiles8);
   pa.v_inv_scale = (float*)(wsp + tiles8 + (size_t)B * Hkv * kD * 4);
-  pa.v_sb = stride_of(v, 0);
-  pa.v_sh = stride_of(v, hdim);
-  pa.v_sn = stride_of(v, ndim);
+  pa.v_sb = v ? stride_of(v, 0) : 0;
+  pa.v_sh = v ? stride_of(v, hdim) : 0;
+  pa.v_sn = v ? stride_of(v, ndim) : 0;
   pa.Nk = (int)Nk;
   pa.nT = nT;
   pa.Hkv = (int)Hkv;
   pa.is_bf16 = dt == DType::BF16;
   const dim3 pgrid(nT, (unsigned)Hkv, (unsigned)B);
-  if (pv8) {
+  if (v_tiles) {
+    SQ_REQUIRE(!pv8, SQ_EUNSUPPORTED, "sq_prefill_vtiles_fwd: the fp8 P.V modes form their own tiles from v");
+    SQ_REQUIRE(on_gpu(v_tiles) && v_tiles->device.device_id == dev, SQ_EDEVICE, "sq_prefill_vtiles_fwd: v_tiles not on the device of q");
+    SQ_REQUIRE((size_t)numel_of(v_tiles) * (v_tiles->dtype.bits / 8) >= (size_t)B * Hkv * nT * (kD * kBN) * 2 && is_compact(v_tiles) &&
+                   ((uintptr_t)data_of(v_tiles) & 15) == 0,
+               SQ_EWORKSPACE, "sq_prefill_vtiles_fwd: v_tiles must be compact, 16-byte aligned and hold every tile of the key range");
+    pa.vt = (_Float16*)data_of(v_tiles);
+  } else if (pv8) {
     SQ_REQUIRE(tiles8 + (size_t)B * Hkv * kD * 8 <= need, SQ_EWORKSPACE, "sq_prefill_fwd: workspace too small for the fp8 tiles");
     hipLaunchKernelGGL(prefill_fill_u32_kernel, dim3(1), dim3(256), 0, st, pa.vmax_bits, (int)(B * Hkv * kD));
     hipLaunchKernelGGL(prefill_vabsmax_kernel, pgrid, dim3(256), 0, st, pa);

@@ -43,6 +43,11 @@ struct PrepassArgs {
   View kcodes;
   float* kscale;
   int64_t scale_stride;
+  // value as V^T tiles of the attention kernel (null: v8 is written)
+  _Float16* vt;
+  int32_t vt_tiles;   // tiles per (batch, head)
+  int32_t mean_blk;   // workgroups of the key mean
+  uint32_t key_blk;   // workgroups of the key rows
 };
 
 
@@ -130,10 +135,10 @@ __device__ __forceinline__ float scale_of(float amax) {
 // With few columns (Qwen2.5-7B: 4 kv heads x 16 groups of 8 channels = 64) the 256 threads split the tokens of the
 // workgroup between them and combine through LDS in a fixed order.
 template <bool BF16>
-__global__ __launch_bounds__(256) void prepass_ksum_kernel(PrepassArgs a) {
+__device__ __forceinline__ void key_sums(const PrepassArgs& a, int blk) {
   __shared__ double red[256][8];
   const int ncol8 = a.B * a.Hkv * (kPD / 8);   // column groups of 8 channels
-  const int n0 = blockIdx.x * a.tok_per_blk, n1 = min(n0 + a.tok_per_blk, a.N);
+  const int n0 = blk * a.tok_per_blk, n1 = min(n0 + a.tok_per_blk, a.N);
   const int TL = ncol8 < 256 ? 256 / ncol8 : 1;   // token lanes per column group
   for (int cg0 = 0; cg0 < ncol8; cg0 += 256) {
     const int cg = cg0 + (TL > 1 ? (int)threadIdx.x % ncol8 : (int)threadIdx.x);
@@ -177,7 +182,7 @@ __global__ __launch_bounds__(256) void prepass_ksum_kernel(PrepassArgs a) {
       __syncthreads();
     }
     if (live && tl == 0) {
-      double* dst = a.part + (int64_t)blockIdx.x * (ncol8 * 8) + cg * 8;
+      double* dst = a.part + (int64_t)blk * (ncol8 * 8) + cg * 8;
 #pragma unroll
       for (int e = 0; e < 8; ++e) dst[e] = s[e];
     }
@@ -187,9 +192,9 @@ __global__ __launch_bounds__(256) void prepass_ksum_kernel(PrepassArgs a) {
 // ---- key mean, stage 2: 16 lanes per column add the partial sums l, l+16, ... and combine in a fixed tree;
 // mean = dtype(float(sum / N))
 template <bool BF16>
-__global__ __launch_bounds__(256) void prepass_kmean_kernel(PrepassArgs a) {
+__device__ __forceinline__ void key_mean(const PrepassArgs& a, int blk) {
   const int ncol = a.B * a.Hkv * kPD;
-  const int c = (blockIdx.x * blockDim.x + threadIdx.x) >> 4, l = threadIdx.x & 15;
+  const int c = (blk * 256 + (int)threadIdx.x) >> 4, l = threadIdx.x & 15;
   double s = 0;
   if (c < ncol) {   // four partial sums requested at a time (one after the other they were 32 dependent round trips)
     double s4[4] = {0, 0, 0, 0};
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(256) void prepass_kmean_kernel(PrepassArgs a) {
 
 // ---- per-token 8-bit (and 4-bit) fake quantisation of the rows of q (CENTRE = false) or of k minus its mean
 template <bool BF16, bool CENTRE, int QT>
-__global__ __launch_bounds__(256) void prepass_rows_kernel(PrepassArgs a) {
+__device__ __forceinline__ void quantise_rows(const PrepassArgs& a, unsigned blk) {
   const View& src = CENTRE ? a.k : a.q;
   const View& d8 = CENTRE ? a.k8 : a.q8;
   const View& d4 = CENTRE ? a.k4 : a.q4;
@@ -225,7 +230,7 @@ __global__ __launch_bounds__(256) void prepass_rows_kernel(PrepassArgs a) {
   const int l16 = threadIdx.x & 15;
   // two consecutive rows per 16-lane group, both loads issued before any arithmetic
   constexpr int R = 2;
-  const int64_t row0 = ((int64_t)blockIdx.x * (blockDim.x / 16) + (threadIdx.x >> 4)) * R;
+  const int64_t row0 = ((int64_t)blk * 16 + (threadIdx.x >> 4)) * R;
   if (row0 >= rows) return;   // whole 16-lane groups leave together; the shuffles below stay inside a group
   uint4 raw[R], mraw[R];
   int64_t off8[R], off4[R], nn[R], bbv[R];
@@ -313,8 +318,8 @@ __global__ __launch_bounds__(256) void prepass_rows_kernel(PrepassArgs a) {
 
 // ---- value: one 8-bit scale per (token, channel) over batch and heads
 template <bool BF16, int QT>
-__global__ __launch_bounds__(256) void prepass_v_kernel(PrepassArgs a) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;   // (token, group of 8 channels)
+__device__ __forceinline__ void quantise_values(const PrepassArgs& a, unsigned blk) {
+  const int64_t t = (int64_t)blk * 256 + threadIdx.x;   // (token, group of 8 channels)
   if (t >= (int64_t)a.N * (kPD / 8)) return;
   const int c8 = (int)(t % (kPD / 8));
   const int64_t n = t / (kPD / 8);
@@ -383,6 +388,125 @@ __global__ __launch_bounds__(256) void prepass_v_kernel(PrepassArgs a) {
     }
 }
 
+// Bound by HBM latency and the divisions, not by bandwidth (30011 tokens: 62 MB in 21.6 us with the key mean beside it; the two
+// passes over rows it replaces and the mean took 40 us).
+// The same values as the attention kernel's V^T tiles instead of rows (vt: fp16 [B, Hkv, nT, 128 channels, 64 keys], keys past
+// N zero): what prefill_prep_v_kernel makes of v8, without v8's way through memory and back.  Workgroup = the 64 keys of a
+// tile for all (batch, head) rows; thread = 8 channels x 4 keys.  NR rows per key stay in registers (all their loads travel
+// at once); NR = 0: any number of rows, read twice.  bf16 only: with fp16 the compiler contracts the last product and its
+// rounding (v_fma_mixlo_f16) or not, depending on the code around it, and the tiles would not be v8's to the bit.
+template <bool BF16, int QT, int NR>
+__device__ __forceinline__ void value_tiles(const PrepassArgs& a, unsigned blk) {
+  const int o = threadIdx.x & 15, tq = threadIdx.x >> 4;
+  const int nrow = a.B * a.Hkv;
+  const int n0 = (int)blk * kVTileKeys + 4 * tq;
+  const uint16_t* base = (const uint16_t*)a.v.p + (int64_t)n0 * a.v.sn + 8 * o;
+  const int pos = (4 * tq & ~15) | perm16(4 * tq & 15);
+  auto load4 = [&](uint4 (&raw)[4], int64_t row_off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      raw[i] = make_uint4(0, 0, 0, 0);
+      if (n0 + i < a.N) raw[i] = *(const uint4*)(base + row_off + (int64_t)i * a.v.sn);
+    }
+  };
+  auto element = [](const uint4& r, int e) __attribute__((always_inline)) {
+    const uint32_t w = e < 2 ? r.x : (e < 4 ? r.y : (e < 6 ? r.z : r.w));
+    return ld<BF16>((e & 1) ? (w >> 16) : (w & 0xffffu));
+  };
+  // quantised, rounded to the tensor dtype (v8's bits), then to the fp16 of the tile
+  auto value = [](float x, const Divisor& s) __attribute__((always_inline)) { return (_Float16)ld<BF16>(st<BF16>(qdq8<QT>(x, s))); };
+  auto store = [&](int r, int e, const f16x4_t& val) __attribute__((always_inline)) {
+    *(f16x4_t*)(a.vt + ((int64_t)r * a.vt_tiles + blk) * (kPD * kVTileKeys) + (8 * o + e) * kVTileKeys + pos) = val;
+  };
+  if constexpr (NR > 0) {
+    uint4 raw[NR][4];
+    int b = 0, h = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r < nrow) {
+        load4(raw[r], b * a.v.sb + h * a.v.sh);
+        if (++h == a.Hkv) {
+          h = 0;
+          ++b;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) raw[r][i] = make_uint4(0, 0, 0, 0);   // no effect on the maximum
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f16x4_t val[NR];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float amax = 1e-5f;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) amax = fmaxf(amax, fabsf(element(raw[r][i], e)));
+        const Divisor sc = make_divisor(scale_of<QT>(amax));
+#pragma unroll
+        for (int r = 0; r < NR; ++r) val[r][i] = value(element(raw[r][i], e), sc);
+      }
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        if (r < nrow) store(r, e, val[r]);
+    }
+  } else {
+    float amax[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) amax[i][e] = 1e-5f;
+    for (int b = 0; b < a.B; ++b)
+      for (int h = 0; h < a.Hkv; ++h) {
+        uint4 raw[4];
+        load4(raw, b * a.v.sb + h * a.v.sh);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) amax[i][e] = fmaxf(amax[i][e], fabsf(element(raw[i], e)));
+      }
+    for (int b = 0; b < a.B; ++b)
+      for (int h = 0; h < a.Hkv; ++h) {
+        uint4 raw[4];
+        load4(raw, b * a.v.sb + h * a.v.sh);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          f16x4_t val;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) val[i] = value(element(raw[i], e), make_divisor(scale_of<QT>(amax[i][e])));
+          store(b * a.Hkv + h, e, val);
+        }
+      }
+  }
+}
+
+// The three launches of a call: key sums, key mean with the value, key rows with the query's.  The value has nothing to do
+// with the key's mean and the query's rows nothing with the key's; as kernels of their own they ran one behind the other, each
+// with the 5 us or so a dependent launch of any size takes.  Workgroups of the shorter part come first.  (The query's rows
+// share a launch with the key's, which need the same registers and no LDS: next to the key sums, with their 16 KB of LDS and
+// half as many registers again, they took 48 us at 8192 tokens x 28 heads instead of 32.)  Whole closure calls, six / seven
+// launches before and four with tiles: 30011 tokens, relative windows 1278 -> 1261 us; 8192 tokens, absolute windows 436 -> 419 us.
+template <bool BF16>
+__global__ __launch_bounds__(256) void prepass_ksum_kernel(PrepassArgs a) {
+  key_sums<BF16>(a, (int)blockIdx.x);
+}
+// key mean | value.  NR < 0: value rows (v8), else tiles.
+template <bool BF16, int QT, int NR>
+__global__ __launch_bounds__(256) void prepass_mean_value_kernel(PrepassArgs a) {
+  if (blockIdx.x < (unsigned)a.mean_blk) {
+    key_mean<BF16>(a, (int)blockIdx.x);
+    return;
+  }
+  if constexpr (NR < 0) quantise_values<BF16, QT>(a, blockIdx.x - (unsigned)a.mean_blk);
+  else value_tiles<BF16, QT, NR>(a, blockIdx.x - (unsigned)a.mean_blk);
+}
+// key rows | query rows
+template <bool BF16, int QT>
+__global__ __launch_bounds__(256) void prepass_rows_kernel(PrepassArgs a) {
+  if (blockIdx.x < a.key_blk) quantise_rows<BF16, true, QT>(a, blockIdx.x);
+  else quantise_rows<BF16, false, QT>(a, blockIdx.x - a.key_blk);
+}
+
 int make_view(const DLTensor* t, const char* name, int layout, int dev, DType dt, int64_t B, int64_t N, int64_t H, View* out) {
   int rc;
   if ((rc = check_tensor(t, name, 4, dev))) return rc;
@@ -417,29 +541,36 @@ extern "C" size_t sq_fake_quant_prepass_workspace_bytes(int64_t batch, int64_t n
 namespace {
 int prepass_impl(const DLTensor* query, const DLTensor* key, const DLTensor* value, DLTensor* q8, DLTensor* q4, DLTensor* k8, DLTensor* k4,
                  DLTensor* v8, DLTensor* workspace, int32_t layout, int32_t qk_qtype, int32_t v_qtype, void* stream, DLTensor* k_codes,
-                 DLTensor* k_scale);
+                 DLTensor* k_scale, DLTensor* v_tiles);
 }
 
 extern "C" int sq_fake_quant_prepass_typed(const DLTensor* query, const DLTensor* key, const DLTensor* value, DLTensor* q8,
                                            DLTensor* q4, DLTensor* k8, DLTensor* k4, DLTensor* v8, DLTensor* workspace,
                                            int32_t layout, int32_t qk_qtype, int32_t v_qtype, void* stream) {
-  return prepass_impl(query, key, value, q8, q4, k8, k4, v8, workspace, layout, qk_qtype, v_qtype, stream, nullptr, nullptr);
+  return prepass_impl(query, key, value, q8, q4, k8, k4, v8, workspace, layout, qk_qtype, v_qtype, stream, nullptr, nullptr, nullptr);
+}
+
+extern "C" int sq_fake_quant_prepass_vtiles(const DLTensor* query, const DLTensor* key, const DLTensor* value, DLTensor* q8,
+                                            DLTensor* q4, DLTensor* k8, DLTensor* k4, DLTensor* v_tiles, DLTensor* workspace,
+                                            int32_t layout, int32_t qk_qtype, int32_t v_qtype, void* stream) {
+  SQ_REQUIRE(v_tiles, SQ_EINVAL, "sq_fake_quant_prepass_vtiles: null tensor argument");
+  return prepass_impl(query, key, value, q8, q4, k8, k4, nullptr, workspace, layout, qk_qtype, v_qtype, stream, nullptr, nullptr, v_tiles);
 }
 
 extern "C" int sq_fake_quant_prepass_int8qk(const DLTensor* query, const DLTensor* key, const DLTensor* value, DLTensor* k_codes,
                                             DLTensor* k_scale, DLTensor* v8, DLTensor* workspace, int32_t layout, void* stream) {
   SQ_REQUIRE(k_codes && k_scale, SQ_EINVAL, "sq_fake_quant_prepass_int8qk: null tensor argument");
   return prepass_impl(query, key, value, nullptr, nullptr, nullptr, nullptr, v8, workspace, layout, SQ_QTYPE_INT, SQ_QTYPE_INT, stream, k_codes,
-                      k_scale);
+                      k_scale, nullptr);
 }
 
 namespace {
 int prepass_impl(const DLTensor* query, const DLTensor* key, const DLTensor* value, DLTensor* q8, DLTensor* q4, DLTensor* k8, DLTensor* k4,
                  DLTensor* v8, DLTensor* workspace, int32_t layout, int32_t qk_qtype, int32_t v_qtype, void* stream, DLTensor* k_codes,
-                 DLTensor* k_scale) {
+                 DLTensor* k_scale, DLTensor* v_tiles) {
   SQ_REQUIRE(qk_qtype >= SQ_QTYPE_INT && qk_qtype <= SQ_QTYPE_E5M2 && v_qtype >= SQ_QTYPE_INT && v_qtype <= SQ_QTYPE_E5M2, SQ_EINVAL,
              "Invalid quantization type: %d / %d", (int)qk_qtype, (int)v_qtype);
-  SQ_REQUIRE(query && key && value && (k8 || k_codes) && v8, SQ_EINVAL, "sq_fake_quant_prepass: null tensor argument");
+  SQ_REQUIRE(query && key && value && (k8 || k_codes) && (v8 || v_tiles), SQ_EINVAL, "sq_fake_quant_prepass: null tensor argument");
   SQ_REQUIRE((q4 == nullptr) == (k4 == nullptr), SQ_EINVAL, "sq_fake_quant_prepass: q4 and k4 must be given together");
   // q8 == NULL: the query rows are left alone (the attention kernel can quantise them as it loads them, q_quant = 8)
   SQ_REQUIRE(q8 || !q4, SQ_EINVAL, "sq_fake_quant_prepass: without q8 there are no 4-bit operands either");
@@ -463,8 +594,17 @@ int prepass_impl(const DLTensor* query, const DLTensor* key, const DLTensor* val
   memset(&a, 0, sizeof(a));
   if ((rc = make_view(query, "query", layout, dev, dt, B, N, Hq, &a.q)) || (rc = make_view(key, "key", layout, dev, dt, B, N, Hkv, &a.k)) ||
       (rc = make_view(value, "value", layout, dev, dt, B, N, Hkv, &a.v)) || (!skip_q && (rc = make_view(q8, "q8", layout, dev, dt, B, N, Hq, &a.q8))) ||
-      (k8 && (rc = make_view(k8, "k8", layout, dev, dt, B, N, Hkv, &a.k8))) || (rc = make_view(v8, "v8", layout, dev, dt, B, N, Hkv, &a.v8)))
+      (k8 && (rc = make_view(k8, "k8", layout, dev, dt, B, N, Hkv, &a.k8))) || (v8 && (rc = make_view(v8, "v8", layout, dev, dt, B, N, Hkv, &a.v8))))
     return rc;
+  if (v_tiles) {
+    SQ_REQUIRE(dt == DType::BF16, SQ_EDTYPE, "sq_fake_quant_prepass_vtiles: bf16 tensors only");
+    a.vt_tiles = (int)((N + kVTileKeys - 1) / kVTileKeys);
+    const size_t tile_bytes = (size_t)(B * Hkv) * a.vt_tiles * (kPD * kVTileKeys) * 2;
+    SQ_REQUIRE(on_gpu(v_tiles) && v_tiles->device.device_id == dev, SQ_EDEVICE, "sq_fake_quant_prepass_vtiles: v_tiles not on the device of query");
+    SQ_REQUIRE((size_t)numel_of(v_tiles) * (v_tiles->dtype.bits / 8) >= tile_bytes && is_compact(v_tiles) && ((uintptr_t)data_of(v_tiles) & 15) == 0,
+               SQ_EWORKSPACE, "sq_fake_quant_prepass_vtiles: v_tiles must be compact, 16-byte aligned and hold %zu bytes", tile_bytes);
+    a.vt = (_Float16*)data_of(v_tiles);
+  }
   if (k_codes) {
     // int8 [like key]; rows of 128 bytes on 16-byte boundaries.  k_scale: fp32 [B, Hkv, >= N], contiguous
     if ((rc = check_tensor(k_codes, "k_codes", 4, dev)) || (rc = check_tensor(k_scale, "k_scale", 3, dev))) return rc;
@@ -512,27 +652,37 @@ int prepass_impl(const DLTensor* query, const DLTensor* key, const DLTensor* val
   a.mean = (uint16_t*)(data_of(workspace) + (size_t)a.nblk * cols * sizeof(double));
   hipStream_t s = (hipStream_t)stream;
   const int64_t qrows = B * N * Hq, krows = B * N * Hkv, vthreads = N * (kPD / 8);
-#define SQ_PREPASS_ROWS(BF, QT)                                                                                        \
-  do {                                                                                                                 \
-    if (!skip_q)                                                                                                       \
-      hipLaunchKernelGGL((prepass_rows_kernel<BF, false, QT>), dim3((unsigned)((qrows + 31) / 32)), dim3(256), 0, s, a); \
-    hipLaunchKernelGGL((prepass_rows_kernel<BF, true, QT>), dim3((unsigned)((krows + 31) / 32)), dim3(256), 0, s, a);  \
+  a.mean_blk = (int)((cols * 16 + 255) / 256);
+  const int64_t kblk = (krows + 31) / 32, qblk = skip_q ? 0 : (qrows + 31) / 32, vblk = v_tiles ? a.vt_tiles : (vthreads + 255) / 256;
+  const int64_t vrows = B * Hkv;
+  a.key_blk = (uint32_t)kblk;
+  SQ_REQUIRE(kblk + qblk < ((int64_t)1 << 31) && a.mean_blk + vblk < ((int64_t)1 << 31), SQ_EUNSUPPORTED, "sq_fake_quant_prepass: tensor too large");
+#define SQ_PREPASS_ROWS(BF, QT)                                                                                                      \
+  do {                                                                                                                               \
+    hipLaunchKernelGGL((prepass_ksum_kernel<BF>), dim3((unsigned)a.nblk), dim3(256), 0, s, a);                                        \
+    if (v_qtype == SQ_QTYPE_E4M3) SQ_PREPASS_VALUE(BF, 1);                                                                           \
+    else if (v_qtype == SQ_QTYPE_E5M2) SQ_PREPASS_VALUE(BF, 2);                                                                      \
+    else SQ_PREPASS_VALUE(BF, 0);                                                                                                    \
+    hipLaunchKernelGGL((prepass_rows_kernel<BF, QT>), dim3((unsigned)(kblk + qblk)), dim3(256), 0, s, a);                             \
   } while (0)
-#define SQ_PREPASS_LAUNCH(BF)                                                                                       \
-  do {                                                                                                              \
-    hipLaunchKernelGGL(prepass_ksum_kernel<BF>, dim3(a.nblk), dim3(256), 0, s, a);                                  \
-    hipLaunchKernelGGL(prepass_kmean_kernel<BF>, dim3((unsigned)((cols * 16 + 255) / 256)), dim3(256), 0, s, a);    \
-    if (qk_qtype == SQ_QTYPE_E4M3) SQ_PREPASS_ROWS(BF, 1);                                                          \
-    else if (qk_qtype == SQ_QTYPE_E5M2) SQ_PREPASS_ROWS(BF, 2);                                                     \
-    else SQ_PREPASS_ROWS(BF, 0);                                                                                    \
-    const dim3 vgrid((unsigned)((vthreads + 255) / 256));                                                           \
-    if (v_qtype == SQ_QTYPE_E4M3) hipLaunchKernelGGL((prepass_v_kernel<BF, 1>), vgrid, dim3(256), 0, s, a);         \
-    else if (v_qtype == SQ_QTYPE_E5M2) hipLaunchKernelGGL((prepass_v_kernel<BF, 2>), vgrid, dim3(256), 0, s, a);    \
-    else hipLaunchKernelGGL((prepass_v_kernel<BF, 0>), vgrid, dim3(256), 0, s, a);                                  \
+#define SQ_PREPASS_VALUE(BF, VT)                                                                                                     \
+  do {                                                                                                                               \
+    const dim3 mv((unsigned)(a.mean_blk + vblk));                                                                                    \
+    if (!v_tiles) hipLaunchKernelGGL((prepass_mean_value_kernel<BF, VT, -1>), mv, dim3(256), 0, s, a);                                \
+    else if (vrows <= 4) hipLaunchKernelGGL((prepass_mean_value_kernel<true, VT, 4>), mv, dim3(256), 0, s, a);                        \
+    else if (vrows <= 8) hipLaunchKernelGGL((prepass_mean_value_kernel<true, VT, 8>), mv, dim3(256), 0, s, a);                        \
+    else hipLaunchKernelGGL((prepass_mean_value_kernel<true, VT, 0>), mv, dim3(256), 0, s, a);                                       \
+  } while (0)
+#define SQ_PREPASS_LAUNCH(BF)                                \
+  do {                                                       \
+    if (qk_qtype == SQ_QTYPE_E4M3) SQ_PREPASS_ROWS(BF, 1);   \
+    else if (qk_qtype == SQ_QTYPE_E5M2) SQ_PREPASS_ROWS(BF, 2); \
+    else SQ_PREPASS_ROWS(BF, 0);                             \
   } while (0)
   if (a.is_bf16) SQ_PREPASS_LAUNCH(true);
   else SQ_PREPASS_LAUNCH(false);
 #undef SQ_PREPASS_LAUNCH
+#undef SQ_PREPASS_VALUE
 #undef SQ_PREPASS_ROWS
   SQ_HIP(hipGetLastError());
   return SQ_OK;

@@ -18,6 +18,7 @@ import types
 
 import torch
 
+from .. import _native as N
 from .attn_triton_decode import attn_decode
 from .attn_triton_mix_bad import attn_hierarchical_window
 from .attn_triton_mix_relative import attn_hierarchical_relative_window
@@ -142,12 +143,15 @@ def mp_triton_wrapper(layer_idx, bit8_window_sizes=0, bit4_window_sizes=0, sink_
                     attn_output = attn_output.transpose(1, 2).contiguous()
                 bs, seq_len, head, head_dim = attn_output.shape
                 return attn_output.reshape(bs, seq_len, head * head_dim)
+            # bf16: the value goes straight into the tiles the attention kernel reads (the fp8 P.V modes make their own from rows)
+            tiled = query.dtype == torch.bfloat16 and (p_quant is None or p_quant < N.P_E4M3_FP8_PV)
             q_bit8, q_bit4, k_bit8, k_bit4, v_bit8 = fused_int_prepass(query, key, value, want_4bit=not relative, tensor_layout=layout,
-                                                                       qk_qtype=args.qk_qtype, v_qtype=args.v_qtype, skip_query=q_in_kernel)
+                                                                       qk_qtype=args.qk_qtype, v_qtype=args.v_qtype, skip_query=q_in_kernel,
+                                                                       value_tiles=tiled)
             if q_in_kernel:
                 q_bit8 = query
         else:
-            q_in_kernel = False
+            q_in_kernel = tiled = False
             bit8_qk, bit4_qk, bit8_v = _quantizers(args)
             if nhd:   # the quantisers' "per_channel" range is over dims (0, 1) of [B,H,N,D]: quantise HND views
                 query, key, value = (t.permute(0, 2, 1, 3) for t in (query, key, value))
@@ -161,16 +165,17 @@ def mp_triton_wrapper(layer_idx, bit8_window_sizes=0, bit4_window_sizes=0, sink_
                 k_bit4 = bit4_qk.fake_quant_tensor(key)
             layout = "HND"
         del query, key, value
+        v_bit8, v_tiles = (None, v_bit8) if tiled else (v_bit8, None)
         if relative:
             attn_output = attn_hierarchical_relative_window(
                 q_bit8, k_bit8, q_bit8, k_bit8, v_bit8, int8_window_ratios=bit8_window_sizes,
                 int4_window_ratios=bit4_window_sizes, sink_size=sink_window_size, tensor_layout=layout,
-                output_dtype=torch.bfloat16, p_quant=p_quant, q_quant=8 if q_in_kernel else 0)
+                output_dtype=torch.bfloat16, p_quant=p_quant, q_quant=8 if q_in_kernel else 0, v_tiles=v_tiles)
         else:
             attn_output = attn_hierarchical_window(
                 q_bit8, k_bit8, q_bit4, k_bit4, v_bit8, int8_window_sizes=bit8_window_sizes,
                 int4_window_sizes=bit4_window_sizes, sink_size=sink_window_size, tensor_layout=layout,
-                output_dtype=torch.bfloat16, p_quant=p_quant)
+                output_dtype=torch.bfloat16, p_quant=p_quant, v_tiles=v_tiles)
         if layout == "HND":
             attn_output = attn_output.transpose(1, 2).contiguous()
         bs, seq_len, head, head_dim = attn_output.shape

@@ -15,7 +15,7 @@ from ._prefill import align_windows, per_head, run_prefill
 
 def attn_hierarchical_window(q_int8, k_int8, q_int4, k_int4, v, int8_window_sizes, int4_window_sizes, sink_size,
                              tensor_layout="HND", output_dtype=torch.float16, return_lse=False,
-                             is_P_fp8_quant=False, *, p_quant=None, workspace=None, out=None):
+                             is_P_fp8_quant=False, *, p_quant=None, workspace=None, out=None, v_tiles=None):
     if tensor_layout not in N.LAYOUT:
         raise ValueError(f"tensor_layout {tensor_layout} not supported")
     H = q_int8.size(1) if tensor_layout == "HND" else q_int8.size(2)
@@ -31,4 +31,4 @@ def attn_hierarchical_window(q_int8, k_int8, q_int4, k_int4, v, int8_window_size
     mode = p_quant if p_quant is not None else (N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE)
     return run_prefill(q_int8, k_int8, v, q4=None if same else q_int4, k4=None if same else k_int4,
                        tensor_layout=tensor_layout, output_dtype=output_dtype, return_lse=return_lse, p_quant=mode,
-                       window=window, workspace=workspace, out=out)
+                       window=window, workspace=workspace, out=out, v_tiles=v_tiles)

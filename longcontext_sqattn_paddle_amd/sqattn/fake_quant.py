@@ -140,7 +140,8 @@ class FloatQuantizer(BaseQuantizer):
         return float_quantize(scaled.float(), self.e_bits, self.m_bits, rounding="nearest")
 
 
-def fused_int_prepass(query, key, value, want_4bit=True, tensor_layout="NHD", qk_qtype="int", v_qtype="int", skip_query=False):
+def fused_int_prepass(query, key, value, want_4bit=True, tensor_layout="NHD", qk_qtype="int", v_qtype="int", skip_query=False,
+                      value_tiles=False):
     """The operand pre-pass of `mp_triton_wrapper`'s closure (attn_replacer.py:334-365) as one call into the HIP
     library: key centring, per-token 8-bit (and integer 4-bit) fake quantisation of query and centred key, per-channel
     8-bit fake quantisation of value -- without expanding the kv heads.  `qk_qtype` / `v_qtype` pick the 8-bit
@@ -149,7 +150,9 @@ def fused_int_prepass(query, key, value, want_4bit=True, tensor_layout="NHD", qk
     query [B,N,Hq,D], key/value [B,N,Hkv,D] for "NHD" ([B,H,N,D] for "HND"), bf16 or fp16, D == 128.
     Returns (q8, q4, k8, k4, v8) in the layout of the inputs; q4 and k4 are None unless `want_4bit`.  With `skip_query`
     the query is left alone and q8 is None (the attention kernel applies the 8-bit integer quantiser while it loads the
-    rows, `q_quant=8`); not together with `want_4bit`.
+    rows, `q_quant=8`); not together with `want_4bit`.  With `value_tiles` the last output is the value as the attention
+    kernel's V^T tiles (fp16 [B, Hkv, ceil(N / 64), 128, 64], `run_prefill(v_tiles=...)`; the bits that kernel's own pass
+    would make of v8; bf16 only).
     """
     from .. import _native as N
     from ._common import require_gpu
@@ -166,7 +169,8 @@ def fused_int_prepass(query, key, value, want_4bit=True, tensor_layout="NHD", qk
     if skip_query and want_4bit:
         raise ValueError("skip_query leaves no query to derive the 4-bit operands from")
     q8 = None if skip_query else torch.empty_like(query)
-    k8, v8 = torch.empty_like(key), torch.empty_like(value)
+    k8 = torch.empty_like(key)
+    v8 = torch.empty(B, Hkv, (Nk + 63) // 64, 128, 64, dtype=torch.float16, device=key.device) if value_tiles else torch.empty_like(value)
     q4 = torch.empty_like(query) if want_4bit else None
     k4 = torch.empty_like(key) if want_4bit else None
     need = lib.sq_fake_quant_prepass_workspace_bytes(B, Hkv, Nk)
@@ -175,8 +179,8 @@ def fused_int_prepass(query, key, value, want_4bit=True, tensor_layout="NHD", qk
     for name in (qk_qtype, v_qtype):
         if name not in N.QTYPE:
             raise ValueError(f"Invalid quantization type: {name}")
-    N.check(lib.sq_fake_quant_prepass_typed(*ptrs, N.LAYOUT[tensor_layout], N.QTYPE[qk_qtype], N.QTYPE[v_qtype],
-                                            N.current_stream(query.device)))
+    prepass = lib.sq_fake_quant_prepass_vtiles if value_tiles else lib.sq_fake_quant_prepass_typed
+    N.check(prepass(*ptrs, N.LAYOUT[tensor_layout], N.QTYPE[qk_qtype], N.QTYPE[v_qtype], N.current_stream(query.device)))
     return q8, q4, k8, k4, v8
 
 

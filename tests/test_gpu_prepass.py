@@ -158,3 +158,35 @@ def test_int8qk_prepass_codes_and_scales_are_the_quantisers_factors(layout, dtyp
     deq = (got_codes.float() * k_scale.cpu()[:, :, :N, None]).to(dtype)
     k8h = k8.cpu() if layout == "HND" else k8.cpu().permute(0, 2, 1, 3)
     assert torch.equal(deq.view(torch.int16), k8h.contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("B,Hkv", [(1, 1), (1, 4), (2, 3), (1, 8), (3, 3)])      # 1, 4 | 6, 8 in registers | 9 rows read twice
+@pytest.mark.parametrize("N,layout,vq", [(1, "NHD", "int"), (64, "HND", "int"), (131, "NHD", "e4m3"), (190, "HND", "int"), (257, "NHD", "e5m2")])
+def test_value_tiles_are_the_tiles_of_v8(B, Hkv, N, layout, vq):
+    """The value as V^T tiles: v8's rounded values as fp16, transposed, keys 4 i .. 4 i + 3 of a group of 16 at 4 perm(i) with
+    perm = 0 2 1 3, zeros past N -- bit for bit, since every step after v8's rounding is exact or the same rounding.  The other
+    outputs of the call and an attention call over the tiles have the bits of the call with rows."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import run_prefill
+    from longcontext_sqattn_paddle_amd.sqattn.fake_quant import fused_int_prepass
+
+    print(f"case value tiles B={B} Hkv={Hkv} N={N} {layout} {vq}", flush=True)
+    q, k, v = (t.to(DEV) for t in _inputs(B, N, 2 * Hkv, Hkv, seed=N + B, dtype=torch.bfloat16))
+    if layout == "HND":
+        q, k, v = (t.permute(0, 2, 1, 3).contiguous() for t in (q, k, v))
+    rows = fused_int_prepass(q, k, v, tensor_layout=layout, v_qtype=vq)
+    tiled = fused_int_prepass(q, k, v, tensor_layout=layout, v_qtype=vq, value_tiles=True)
+    torch.cuda.synchronize()
+    for a, b in zip(rows[:4], tiled[:4]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    v8 = rows[4] if layout == "HND" else rows[4].permute(0, 2, 1, 3)
+    nT = (N + 63) // 64
+    pad = torch.zeros(B, Hkv, nT * 64, 128, dtype=torch.float16)
+    pad[:, :, :N] = v8.cpu().half()
+    want = pad.view(B, Hkv, nT, 4, 4, 4, 128)[:, :, :, :, [0, 2, 1, 3]].reshape(B, Hkv, nT, 64, 128).transpose(3, 4).contiguous()
+    assert torch.equal(tiled[4].cpu().view(torch.int16), want.view(torch.int16))
+    a, b = (run_prefill(rows[0], rows[2], rows[4] if t is None else None, tensor_layout=layout, output_dtype=torch.float32, v_tiles=t)
+            for t in (None, tiled[4]))
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    with pytest.raises(ValueError, match="bf16"):
+        fused_int_prepass(q.half(), k.half(), v.half(), tensor_layout=layout, v_qtype=vq, value_tiles=True)
