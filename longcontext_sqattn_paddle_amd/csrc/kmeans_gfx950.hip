@@ -50,17 +50,26 @@ constexpr int kAssignWaves = 4;   // x 64 tokens; two workgroups per CU put two 
 // order, by fp64 atomics that round nothing -- the result is the sum a full re-sum would give, bit for bit.  The
 // workgroup lists its movers in LDS and applies them itself at the end (one channel per thread, the first 128 threads
 // adding, the others subtracting); kmeans_update_kernel then turns sums and sizes into centroids.
-template <bool TRACK>
+// PARTS: launches that leave CUs idle.  A workgroup's length is its chain of centroid blocks, whatever the number of
+// tokens (4096 tokens x 1024 centroids: 16 workgroups, 16 us).  With PARTS = 2 or 4 a workgroup takes 256 / PARTS tokens
+// and its waves share the centroids: wave w walks part w % PARTS of the blocks, each part streaming through buffers of its
+// own, and the parts' (score, index) pairs meet in LDS at the end.  A score is the same chain of MFMAs in any part and the
+// lowest index wins ties inside a part and across them, so the assignment is the same to the bit.
+template <bool TRACK, int PARTS>
 __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(AssignArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[2 * kCB * 256];
+  static_assert(PARTS == 1 || PARTS == 2 || PARTS == kAssignWaves, "waves per part");
+  __shared__ __attribute__((aligned(16))) char smem[PARTS * 2 * kCB * 256];
   __shared__ int32_t s_chg_n;
-  __shared__ uint2 s_chg[TRACK ? kTileTok : 1];   // (token, old cluster << 16 | new cluster)
+  __shared__ uint2 s_chg[TRACK ? kTileTok / PARTS : 1];   // (token, old cluster << 16 | new cluster)
+  __shared__ float s_best[PARTS > 1 ? kAssignWaves * 64 : 1];
+  __shared__ int32_t s_bidx[PARTS > 1 ? kAssignWaves * 64 : 1];
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   const int g_id = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c32 = lane & 31, g = lane >> 5;
-  const int tok0 = blockIdx.x * kTileTok + wave * 64;
+  const int part = wave % PARTS, sub = wave / PARTS;   // share of the centroids, 64 tokens of the tile
+  const int tok0 = blockIdx.x * (kTileTok / PARTS) + sub * 64;
 
   // token fragments (B operand of S^T = Cent . Data^T): lane (column = token 32 tb + c32, k-group g)
   const uint16_t* db = a.data + (int64_t)g_id * a.d_sg;
@@ -82,25 +91,28 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
     }
   }
   const uint16_t* cb = a.cent + (int64_t)g_id * a.c_sg;
-  // per-lane source of the wave's four 1 KB copies of a block (4 centroid rows each), as a byte offset from the block's
-  // first row; rows past C are clamped to the last centroid, which only a block that runs past C has to do
+  // per-lane source of the wave's 1 KB copies of a block (4 centroid rows each, four copies per wave and part), as a byte
+  // offset from the block's first row (the swizzle repeats every four copies); rows past C are clamped to the last
+  // centroid, which only a block that runs past C has to do
+  constexpr int kCopies = 4 * PARTS;
   int64_t src_off[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    const int row = 4 * (wave * 4 + c) + (lane >> 4);
+    const int row = 4 * (sub * kCopies + c) + (lane >> 4);
     src_off[c] = ((int64_t)row * a.c_sc + 8 * ((lane & 15) ^ (row & 15))) * 2;
   }
   auto stage = [&](int chunk, int st) {
-    char* buf = smem + st * (kCB * 256);
+    char* buf = smem + (2 * part + st) * (kCB * 256);
     const char* blk = (const char*)cb + (int64_t)chunk * kCB * a.c_sc * 2;
     if ((chunk + 1) * kCB <= a.C) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-        __builtin_amdgcn_global_load_lds((const void*)(blk + src_off[c]), (lds_ptr_t)(buf + (wave * 4 + c) * 1024), 16, 0, 0);
+      for (int c = 0; c < kCopies; ++c)
+        __builtin_amdgcn_global_load_lds((const void*)(blk + src_off[c & 3] + (int64_t)(c >> 2) * 32 * a.c_sc),
+                                         (lds_ptr_t)(buf + (sub * kCopies + c) * 1024), 16, 0, 0);
     } else {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int q = wave * 4 + c;
+      for (int c = 0; c < kCopies; ++c) {
+        const int q = sub * kCopies + c;
         const int row = 4 * q + (lane >> 4);
         const int ch = (lane & 15) ^ (row & 15);
         const int crow = min(chunk * kCB + row, a.C - 1);
@@ -112,7 +124,7 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
   // reads go through lds_read128 / lds_wait (explicit lgkmcnt counts): left to the compiler, every wait was a full
   // lgkmcnt(0), i.e. also for the fragments requested a moment ago.
   const int ksw = c32 & 15;
-  const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+  const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem + part * (2 * kCB * 256);
   uint32_t fa[8];
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) fa[kk] = smem_addr + c32 * 256 + (((2 * kk + g) ^ ksw) << 4);
@@ -195,15 +207,21 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
     bhalf[1] = (best[1] > before1) ? half_id - 1 : bhalf[1];
   };
   const int nchunks = (a.C + kCB - 1) / kCB;
-  stage(0, 0);
-  for (int chunk = 0; chunk < nchunks; ++chunk) {
+  // this part's blocks c0 .. c1 - 1; every part passes the barrier of every step, also one whose blocks have run out
+  const int steps = (nchunks + PARTS - 1) / PARTS;
+  const int c0 = PARTS > 1 ? min(part * steps, nchunks) : 0;
+  const int c1 = PARTS > 1 ? min(c0 + steps, nchunks) : nchunks;
+  if (PARTS == 1 || c0 < c1) stage(c0, 0);
+  for (int step = 0; step < steps; ++step) {
+    const int chunk = c0 + step;
     __builtin_amdgcn_s_waitcnt(0);
     // block `chunk` has landed for every wave, and every wave has finished reading block chunk - 1, whose buffer the
     // next block may now overwrite; it has this block's 32 MFMAs per wave to arrive
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    if (chunk + 1 < nchunks) stage(chunk + 1, (chunk + 1) & 1);
-    const uint32_t boff = (chunk & 1) * (kCB * 256);
+    if (PARTS > 1 && chunk >= c1) continue;   // wave-uniform
+    if (chunk + 1 < c1) stage(chunk + 1, (step + 1) & 1);
+    const uint32_t boff = (step & 1) * (kCB * 256);
     u32x4_t fr[16];
     static_for<0, kFragAhead>([&](auto I) { fr[decltype(I)::value] = frag(boff, I); });
     __builtin_amdgcn_sched_barrier(0);
@@ -215,9 +233,11 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
     static_for<0, 2>([&](auto TB) {
       static_for<0, 4>([&](auto Q) { group_step(S[decltype(TB)::value][1], decltype(TB)::value, Q); });
     });
-    bhalf[0] = (best[0] > before0) ? 2 * nchunks - 1 : bhalf[0];
-    bhalf[1] = (best[1] > before1) ? 2 * nchunks - 1 : bhalf[1];
+    bhalf[0] = (best[0] > before0) ? 2 * c1 - 1 : bhalf[0];
+    bhalf[1] = (best[1] > before1) ? 2 * c1 - 1 : bhalf[1];
   }
+  float bv2[2];
+  int bidx2[2];
 #pragma unroll
   for (int tb = 0; tb < 2; ++tb) {
     const int in_group = (keep0[tb] == best[tb]) ? 0 : (keep1[tb] == best[tb]) ? 1 : (keep2[tb] == best[tb]) ? 2 : 3;
@@ -229,11 +249,38 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
       bv = ob;
       bidx = oi;
     }
+    bv2[tb] = bv;
+    bidx2[tb] = bidx;
+    if constexpr (PARTS > 1) {
+      if (g == 0) {
+        s_best[wave * 64 + 32 * tb + c32] = bv;
+        s_bidx[wave * 64 + 32 * tb + c32] = bidx;
+      }
+    }
+  }
+  if constexpr (PARTS > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int p = 1; p < PARTS; ++p) {
+        const float ob = s_best[(sub * PARTS + p) * 64 + 32 * tb + c32];
+        const int oi = s_bidx[(sub * PARTS + p) * 64 + 32 * tb + c32];
+        if (ob > bv2[tb] || (ob == bv2[tb] && oi < bidx2[tb])) {
+          bv2[tb] = ob;
+          bidx2[tb] = oi;
+        }
+      }
+  }
+  const bool writes = g == 0 && part == 0;
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb) {
+    const int bidx = bidx2[tb];
     const int n = tok0 + 32 * tb + c32;
     // cluster sizes come out of the counting sort that follows (per-tile histograms), not out of global atomics
-    if (g == 0 && n < a.N) a.idx[(int64_t)g_id * a.i_sg + n] = bidx;
+    if (writes && n < a.N) a.idx[(int64_t)g_id * a.i_sg + n] = bidx;
     if constexpr (TRACK) {
-      const bool changed = g == 0 && n < a.N && old_idx[tb] != bidx;
+      const bool changed = writes && n < a.N && old_idx[tb] != bidx;
       const unsigned long long m = __ballot(changed);
       if (m != 0) {   // wave-uniform
         int base = 0;
@@ -1188,6 +1235,24 @@ extern "C" size_t sq_kmeans_workspace_bytes(int64_t groups, int64_t num_tokens, 
 }
 
 namespace {
+// Four parts while the launch's 64-token workgroups fit the CUs one each, two while its 128-token ones do: the waves that
+// share the centroids then run on CUs that would idle.  Beyond that a split workgroup only takes another's CU (an unsplit
+// launch with one workgroup per CU holds its 16 KB blocks twice, a launch of four parts its CU's whole LDS).
+// segment_k_means, ten steps, 1024 centroids: 4096 tokens 335 -> 267 us, 16384 tokens 342 -> 277, 20000 (two parts) 350 -> 292.
+template <bool TRACK>
+void launch_assign(const AssignArgs& a, int64_t G, hipStream_t st) {
+  constexpr int64_t kCUs = 256;
+  const int64_t N = a.N;
+  auto grid = [&](int tokens) { return dim3((unsigned)((N + tokens - 1) / tokens), (unsigned)G); };
+  const dim3 block(kAssignWaves * 64);
+  if (G * ((N + 63) / 64) <= kCUs && a.C > kCB)
+    hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 4>), grid(kTileTok / 4), block, 0, st, a);
+  else if (G * ((N + 127) / 128) <= kCUs && a.C > kCB)
+    hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 2>), grid(kTileTok / 2), block, 0, st, a);
+  else
+    hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 1>), grid(kTileTok), block, 0, st, a);
+}
+
 int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, DLTensor* cnt, DLTensor* workspace,
                       int32_t normalize, int32_t state, void* stream, const char* who) {
   SQ_REQUIRE(data && centroids && idx && cnt, SQ_EINVAL, "%s: data, centroids, idx and cnt must be non-null", who);
@@ -1222,10 +1287,9 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
   a.C = (int)C;
   a.keep_sum = (double*)(wsp + w.sum_offset());
   a.keep_cnt = (int32_t*)(wsp + w.cnt_offset());
-  const dim3 agrid((unsigned)((N + kTileTok - 1) / kTileTok), (unsigned)G);
   const int mode = normalize ? 2 : 1;
   if (state == SQ_KMEANS_APPLY_CHANGES) {
-    hipLaunchKernelGGL(kmeans_assign_kernel<true>, agrid, dim3(kAssignWaves * 64), 0, st, a);
+    launch_assign<true>(a, G, st);
     UpdateArgs u;
     u.sum = a.keep_sum;
     u.cnt = a.keep_cnt;
@@ -1239,7 +1303,7 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
     SQ_HIP(hipGetLastError());
     return SQ_OK;
   }
-  hipLaunchKernelGGL(kmeans_assign_kernel<false>, agrid, dim3(kAssignWaves * 64), 0, st, a);
+  launch_assign<false>(a, G, st);
   SQ_HIP(hipGetLastError());
   if ((rc = run_group(idx, data, wsp, w, st))) return rc;
   return run_cluster_sum(data, wsp, w, centroids, (int32_t*)data_of(cnt), mode, st, state == SQ_KMEANS_KEEP_SUMS);   // cnt = cluster sizes

@@ -374,3 +374,36 @@ def test_segment_k_means_with_carried_sums_equals_stateless_steps():
         torch.cuda.synchronize()
         for a, b in zip(got, want):
             assert a.shape == b.shape and torch.equal(a.view(torch.int16) if a.dtype == torch.bfloat16 else a, b.view(torch.int16) if b.dtype == torch.bfloat16 else b), segments
+
+
+# 64-token workgroups with four shares of the centroids up to 256 of them (G * ceil(N / 64)), 128-token ones with two shares
+# up to 256 of those, 256-token ones beyond; more than 64 centroids each
+@pytest.mark.parametrize("G,N,C", [(1, 1, 96), (1, 63, 128), (1, 65, 160), (3, 257, 1024), (1, 4097, 320), (1, 16384, 96), (1, 16385, 160),
+                                   (2, 16384, 1024), (2, 16385, 96)])
+def test_split_centroids_give_the_bits_of_the_unsplit_launch(G, N, C):
+    """The same groups alone and among so many copies that the launch is not split: assignments, centroids and sizes are equal
+    to the bit, in the step that re-sums every row and in the two that carry the sums."""
+    from longcontext_sqattn_paddle_amd import _native as NAT
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _triton_k_means_train, _workspace
+
+    print(f"case kmeans split G={G} N={N} C={C}", flush=True)
+    g = torch.Generator().manual_seed(90 + C)
+    key = torch.randn(G, N, 128, generator=g).bfloat16()
+    key[:, N // 2] = 0                                             # every score equal: index 0
+    cent = torch.randn(G, C, 128, generator=g).bfloat16()
+    cent[:, C - 1] = cent[:, C // 2] = cent[:, 1]                  # the same centroid in several shares: the lowest index wins
+    copies = 1
+    while copies * G * ((N + 127) // 128) <= 256:
+        copies *= 2
+    small, large = [], []
+    for reps, out in ((1, small), (copies, large)):
+        kd, cd = key.repeat(reps, 1, 1).to(DEV), cent.repeat(reps, 1, 1).to(DEV)
+        idx = torch.full((kd.shape[0], N), -1, dtype=torch.int32, device=DEV)
+        ws = _workspace(kd.shape[0], N, C, DEV)
+        for state in (NAT.KMEANS_STATELESS, NAT.KMEANS_KEEP_SUMS, NAT.KMEANS_APPLY_CHANGES, NAT.KMEANS_APPLY_CHANGES):
+            _triton_k_means_train(kd, cd, max_idx=idx, workspace=ws, state=state)
+            out += [idx[:G].cpu(), cd[:G].cpu().view(torch.int16)]
+    assert int(small[0][:, N // 2].max()) == 0
+    assert not bool(((small[0] == C - 1) | (small[0] == C // 2)).any())
+    for a, b in zip(small, large):
+        assert torch.equal(a, b)
