@@ -1600,19 +1600,21 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     float4 v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = po[((int64_t)p * WAVES * 16 + i) * 64];
-    if (x.x > 0.f) {   // a part in which the row has no key has no denominator
-      const float m_new = fmaxf(m, x.y);
-      const float w_old = __builtin_amdgcn_exp2f(m - m_new), w = __builtin_amdgcn_exp2f(x.y - m_new);
-      l = l * w_old + x.x * w;
+    // A part without denominator (its keys vanish against the reference point it was given) does not move the reference and
+    // has weight 0.  It is added all the same: NaN and infinite keys, scores and values have to come out of the parts as they
+    // come out of the unsplit launch -- a NaN denominator weighs in as NaN, and 0 * NaN (a value no key of the part reaches) is NaN.
+    const bool none = x.x == 0.f;
+    const float m_new = none ? m : fmaxf(m, x.y);
+    const float w_old = none ? 1.f : __builtin_amdgcn_exp2f(m - m_new), w = none ? 0.f : __builtin_amdgcn_exp2f(x.y - m_new);
+    l = l * w_old + x.x * w;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o[i].x = o[i].x * w_old + v[i].x * w;
-        o[i].y = o[i].y * w_old + v[i].y * w;
-        o[i].z = o[i].z * w_old + v[i].z * w;
-        o[i].w = o[i].w * w_old + v[i].w * w;
-      }
-      m = m_new;
+    for (int i = 0; i < 4; ++i) {
+      o[i].x = o[i].x * w_old + v[i].x * w;
+      o[i].y = o[i].y * w_old + v[i].y * w;
+      o[i].z = o[i].z * w_old + v[i].z * w;
+      o[i].w = o[i].w * w_old + v[i].w * w;
     }
+    m = m_new;
   }
   const float inv_l = 1.0f / l;
   const int head = (int)(bh % a.Hq), b = (int)(bh / a.Hq);

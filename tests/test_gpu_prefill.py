@@ -335,6 +335,40 @@ def test_split_key_ranges_keep_the_e4m3_grid(mode, N, offset):
     assert _cos(out.cpu(), exact) >= 0.999
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("window", [None, (64, 0.125, 0.75)])
+@pytest.mark.parametrize("tensor,value", [("k", math.nan), ("k", math.inf), ("v", math.nan), ("v", math.inf)])
+def test_split_key_ranges_keep_nan_and_infinity(mode, window, tensor, value):
+    """One poisoned element of a key or value row: the outputs and log-sum-exps that are not finite are the unsplit launch's,
+    wherever the row lies among the parts (first, middle, last)."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton_mix_relative import attn_hierarchical_relative_window
+
+    print(f"case prefill split poison mode={mode} window={window} {tensor}={value}", flush=True)
+    N = 3010
+    q, k, v = (t.to(DEV) for t in _rand(1, 3, 1, N, 128, 43))
+
+    def call(k, v, **kw):
+        if window is None:
+            return attn_causal(q, k, v, "HND", torch.float32, return_lse=True, p_quant=mode, **kw)
+        return attn_hierarchical_relative_window(q, k, q, k, v, window[1], window[2], window[0], "HND", torch.float32, return_lse=True,
+                                                 p_quant=mode, **kw)
+
+    small = prefill_workspace(1, 1, N, q.device)
+    clean, clean_whole = call(k, v)[0], call(k, v, workspace=small)[0]
+    assert not torch.equal(clean, clean_whole)                       # the first call is split
+    for at in (20, 1500, 2000, 2990):
+        kp, vp = k.clone(), v.clone()
+        (kp if tensor == "k" else vp)[0, 0, at, 5] = value
+        parts, whole = call(kp, vp), call(kp, vp, workspace=small)
+        torch.cuda.synchronize()
+        for a, b in zip(parts, whole):
+            assert torch.equal(a.isfinite(), b.isfinite()), (at, int(a.isfinite().sum()), int(b.isfinite().sum()))
+        assert tensor == "v" and mode == 4 or not bool(whole[0].isfinite().all())   # (mode 4 clamps the value to its e4m3 range)
+        assert bool(whole[0].isfinite().any())
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2, 5])
 @pytest.mark.parametrize("N,window", [(257, None), (640, (64, 128, 256))])
 def test_rows_do_not_depend_on_the_workgroup_size(mode, N, window):
