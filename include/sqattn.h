@@ -140,7 +140,8 @@ int sq_prefill_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v, cons
 
 /*
  * sq_prefill_fwd for a value that sq_fake_quant_prepass_vtiles has left as tiles (p_quant 0 - 3; the fp8 P.V modes make tiles
- * of their own from v).  The value's token and head counts are the key's.  Other arguments as sq_prefill_fwd.
+ * of their own from v): v_tiles is a compact, 16-byte aligned fp16 [batch, Hkv, ceil(Nk / 64), 128, 64], counts as the key's.
+ * Other arguments as sq_prefill_fwd.
  */
 int sq_prefill_vtiles_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v_tiles, const DLTensor* q4, const DLTensor* k4,
                           DLTensor* out, DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream);

@@ -1859,6 +1859,18 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
     for (int i = 0; i < 3; ++i)
       SQ_REQUIRE(!ts[t] || stride_of(ts[t], i) % (t == 3 && odt == DType::F32 ? 4 : 8) == 0 || ts[t]->shape[i] == 1, SQ_ESHAPE,
                  "sq_prefill_fwd: strides must keep rows 16-byte aligned");
+  if (v_tiles) {
+    SQ_REQUIRE(p->p_quant < SQ_P_E4M3_FP8_PV, SQ_EUNSUPPORTED, "sq_prefill_vtiles_fwd: the fp8 P.V modes form their own tiles from v");
+    SQ_REQUIRE(on_gpu(v_tiles) && v_tiles->device.device_id == dev, SQ_EDEVICE, "sq_prefill_vtiles_fwd: v_tiles not on the device of q");
+    // the kernel finds a tile by this call's tile count: tiles of another length would be read at the wrong places
+    const int64_t tiles[5] = {B, Hkv, (Nk + kBN - 1) / kBN, kD, kBN};
+    SQ_REQUIRE(dtype_of(v_tiles) == DType::F16, SQ_EDTYPE, "sq_prefill_vtiles_fwd: v_tiles must be fp16");
+    bool same = v_tiles->ndim == 5;
+    for (int i = 0; same && i < 5; ++i) same = v_tiles->shape[i] == tiles[i];
+    SQ_REQUIRE(same && is_compact(v_tiles) && ((uintptr_t)data_of(v_tiles) & 15) == 0, SQ_ESHAPE,
+               "sq_prefill_vtiles_fwd: v_tiles must be a compact, 16-byte aligned [%lld, %lld, %lld, %d, %d]", (long long)B, (long long)Hkv,
+               (long long)tiles[2], kD, kBN);
+  }
   if (lse) {
     SQ_REQUIRE(on_gpu(lse) && lse->device.device_id == dev, SQ_EDEVICE, "sq_prefill_fwd: lse not on the same device");
     SQ_REQUIRE(dtype_of(lse) == DType::F32 && numel_of(lse) == B * Hq * Nq && is_compact(lse), SQ_ESHAPE,
@@ -1917,11 +1929,6 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   pa.is_bf16 = dt == DType::BF16;
   const dim3 pgrid(nT, (unsigned)Hkv, (unsigned)B);
   if (v_tiles) {
-    SQ_REQUIRE(!pv8, SQ_EUNSUPPORTED, "sq_prefill_vtiles_fwd: the fp8 P.V modes form their own tiles from v");
-    SQ_REQUIRE(on_gpu(v_tiles) && v_tiles->device.device_id == dev, SQ_EDEVICE, "sq_prefill_vtiles_fwd: v_tiles not on the device of q");
-    SQ_REQUIRE((size_t)numel_of(v_tiles) * (v_tiles->dtype.bits / 8) >= (size_t)B * Hkv * nT * (kD * kBN) * 2 && is_compact(v_tiles) &&
-                   ((uintptr_t)data_of(v_tiles) & 15) == 0,
-               SQ_EWORKSPACE, "sq_prefill_vtiles_fwd: v_tiles must be compact, 16-byte aligned and hold every tile of the key range");
     pa.vt = (_Float16*)data_of(v_tiles);
   } else if (pv8) {
     SQ_REQUIRE(tiles8 + (size_t)B * Hkv * kD * 8 <= need, SQ_EWORKSPACE, "sq_prefill_fwd: workspace too small for the fp8 tiles");

@@ -34,6 +34,8 @@ def run_prefill(q, k, v, *, tensor_layout="HND", output_dtype=torch.float16, ret
             raise ValueError("the integer Q.K^T path takes head_dim 128, no 4-bit operands and no P or q quantisation mode")
         if k.dtype != torch.int8:
             raise ValueError(f"k must hold int8 codes when k_scale is given (got {k.dtype})")
+        if v_tiles is not None:
+            raise ValueError("the integer Q.K^T path takes v, not v_tiles")
     elif v_tiles is not None:
         if head_dim_og != KERNEL_HEAD_DIM or v is not None:
             raise ValueError("v_tiles stands in for v and takes head_dim 128")

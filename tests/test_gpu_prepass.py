@@ -190,3 +190,23 @@ def test_value_tiles_are_the_tiles_of_v8(B, Hkv, N, layout, vq):
     assert torch.equal(a, b)
     with pytest.raises(ValueError, match="bf16"):
         fused_int_prepass(q.half(), k.half(), v.half(), tensor_layout=layout, v_qtype=vq, value_tiles=True)
+
+
+def test_value_tiles_of_another_shape_or_type_are_refused():
+    """The kernel finds a tile by the call's own tile count, so tiles made for a longer prompt (more bytes than needed, other
+    strides), of another type or as a flat buffer are an error, not another answer."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import run_prefill
+
+    q, k, v = (t.to(DEV) for t in _inputs(1, 200, 4, 2, seed=5, dtype=torch.bfloat16))
+    tiles = lambda *shape, dtype=torch.float16: torch.zeros(*shape, dtype=dtype, device=DEV)
+    run_prefill(q, k, None, tensor_layout="NHD", v_tiles=tiles(1, 2, 4, 128, 64))
+    for bad in (tiles(1, 2, 5, 128, 64), tiles(1, 2, 3, 128, 64), tiles(1, 3, 4, 128, 64), tiles(2, 2, 4, 128, 64), tiles(1, 2, 4, 64, 128),
+                tiles(1, 2, 4 * 64 * 128), tiles(1, 2, 4, 64, 128).transpose(3, 4)):
+        with pytest.raises(AssertionError, match="v_tiles must be"):
+            run_prefill(q, k, None, tensor_layout="NHD", v_tiles=bad)
+    for dtype in (torch.bfloat16, torch.float32):
+        with pytest.raises(ValueError, match="v_tiles must be fp16"):
+            run_prefill(q, k, None, tensor_layout="NHD", v_tiles=tiles(1, 2, 4, 128, 64, dtype=dtype))
+    with pytest.raises(ValueError, match="not v_tiles"):
+        run_prefill(q, k.to(torch.int8), v, tensor_layout="NHD", k_scale=torch.zeros(1, 2, 256, device=DEV), v_tiles=tiles(1, 2, 4, 128, 64))
+    torch.cuda.synchronize()
