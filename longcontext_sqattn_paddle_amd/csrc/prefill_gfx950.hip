@@ -1768,8 +1768,14 @@ extern "C" size_t sq_prefill_workspace_bytes(int64_t batch, int64_t num_kv_heads
 extern "C" size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t qo_len, int64_t kv_len,
                                                    const sq_prefill_params* p) {
   const size_t need = sq_prefill_workspace_bytes(batch, num_kv_heads, kv_len, kD);
+  // only a call that sq_prefill_fwd would accept is planned: the plan divides by block_m and counts tiles in 32 bits
   if (!p || need == 0 || p->p_quant < SQ_P_NONE || p->p_quant > SQ_P_E4M3_MX_FP8_PV || num_q_heads <= 0 || num_q_heads > kMaxHeads || qo_len <= 0) return need;
-  if (p->window_mode == SQ_WINDOW_SIZES && (!p->w8 || !p->w4 || p->num_heads_w != num_q_heads || p->block_m <= 0 || p->sink < 0)) return need;
+  if (p->q_offset < 0 || p->q_offset > kv_len || qo_len != kv_len - p->q_offset || kv_len >= (1ll << 31) - 65536 || batch > (1 << 20)) return need;
+  if (p->window_mode == SQ_WINDOW_SIZES) {
+    if (!p->w8 || !p->w4 || p->num_heads_w != num_q_heads || (p->block_m != 64 && p->block_m != 128) || p->sink < 0) return need;
+  } else if (p->window_mode != SQ_WINDOW_NONE) {
+    return need;
+  }
   LaunchPlan plan;
   // (operands of their own for the 4-bit range are what the launches with 128-row query blocks come with)
   plan_launch(p, p->window_mode == SQ_WINDOW_SIZES && p->block_m == 128, batch, num_q_heads, qo_len, plan);

@@ -39,6 +39,35 @@ def test_sizes_and_split_heuristic():
     assert lib.sq_decode_num_splits(1, 4, 10) == 1
 
 
+def test_split_workspace_size_of_calls_that_are_refused():
+    """The size of a call that sq_prefill_fwd refuses is the plain one, whatever its arguments: an unknown window mode with a
+    block of 0 rows, offsets and lengths that do not fit each other or 32-bit tile counts."""
+    lib = N.lib()
+    w = (ctypes.c_int32 * 4)(128, 128, 128, 128)
+    wp = ctypes.cast(w, ctypes.POINTER(ctypes.c_int32))
+
+    def size(batch=1, Hq=4, Hkv=1, Nq=4096, Nk=4096, **fields):
+        p = N.PrefillParams(**fields)
+        return lib.sq_prefill_workspace_bytes_split(batch, Hq, Hkv, Nq, Nk, ctypes.byref(p))
+
+    plain = lambda batch=1, Nk=4096: lib.sq_prefill_workspace_bytes(batch, 1, Nk, 128)
+    assert size() > plain()                                            # this call is split
+    for mode in (2, 7, -1):
+        for block_m in (0, 64):
+            assert size(window_mode=mode, block_m=block_m) == plain()
+    sizes = dict(window_mode=N.WINDOW_SIZES, num_heads_w=4, w8=wp, w4=wp)
+    for block_m in (0, -64, 1, 32, 256):
+        assert size(**sizes, block_m=block_m) == plain()
+    assert size(window_mode=N.WINDOW_SIZES, block_m=64) == plain()     # no windows
+    for offset in (-64, 64, 1 << 40, (1 << 63) - 1):
+        assert size(q_offset=offset) == plain()
+    assert size(Nq=1 << 40) == plain()
+    assert size(Nq=4096, Nk=1 << 40, q_offset=(1 << 40) - 4096) == plain(Nk=1 << 40)
+    assert size(batch=1 << 40) == plain(batch=1 << 40)
+    assert size(p_quant=9) == plain() and size(p_quant=-1) == plain()
+    assert lib.sq_prefill_workspace_bytes_split(0, 4, 1, 4096, 4096, ctypes.byref(N.PrefillParams())) == 0
+
+
 def _dec(q, k, v, out, ws, layout=0, p_quant=0):
     lib = N.lib()
     b = [N.dl(t) for t in (q, k, v, None, out, None, ws)]
