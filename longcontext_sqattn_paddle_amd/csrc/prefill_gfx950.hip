@@ -24,12 +24,14 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "prefill_plan.hpp"
 
 namespace sq {
 namespace {
 
 constexpr int kD = 128;
 constexpr int kBN = kVTileKeys;          // keys per tile (BLOCK_N of every reference kernel)
+static_assert(kBN == kPlanTile, "the plan counts the kernel's tiles");
 // LDS tiles are unpadded and XOR-swizzled at 16-byte granularity (they are filled by global_load_lds, which
 // writes 64 consecutive 16-byte slots per wave instruction): chunk c of K row n sits in slot c ^ (n & 15),
 // chunk c of V^T row d in slot c ^ ((d >> 1) & 7).  The 16 rows a quarter-wave reads at one chunk index then
@@ -40,15 +42,6 @@ constexpr int kKTileBytes = kBN * kKStride;
 constexpr int kVTileBytes = kD * kVStride;
 constexpr int kStageBytes = kKTileBytes + kVTileBytes;
 constexpr int kMaxHeads = 128;
-constexpr int kMaxSplitWork = 512;       // workgroups per (batch, q head) of a launch with split key ranges
-
-// One workgroup of a split launch: part `part` of `parts` of query block `qb`; `slot` is the first of the block's `parts`
-// places in the partial results (parts > 1)
-struct SplitWork {
-  uint16_t qb, slot;
-  uint8_t part, parts;
-};
-
 struct PrefillArgs {
   const void* q;
   const void* k;
@@ -1627,128 +1620,6 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   if (a.lse && bd == 0 && lane < 32) a.lse[bh * a.Nq + row] = log2f(a.p_quant >= SQ_P_E4M3_STATIC_FAST ? l * (1.0f / 448.0f) : l) + m;
 }
 
-// ---- how a launch is cut into workgroups.
-struct LaunchPlan {
-  int waves = 8;                 // per workgroup
-  int n_work = 0, n_slots = 0;   // n_work == 0: one workgroup per query block
-  SplitWork work[kMaxSplitWork];
-};
-
-// Tiles the workgroup of query rows [r0, r1) walks: everything up to its diagonal, or sink and windows (of the widest head)
-int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, int w_max) {
-  const int64_t hi = (p->q_offset + r1 + kBN - 1) / kBN;
-  if (p->window_mode == SQ_WINDOW_NONE) return (int)hi;
-  const int64_t lo = std::max<int64_t>(0, (p->q_offset + r0) / p->block_m * p->block_m + p->block_m - w_max) / kBN;
-  return (int)std::min(hi, hi - std::min(lo, hi) + p->sink / kBN);
-}
-
-// A launch whose query blocks do not fill the chip is as long as its longest chain of tiles: 64 workgroups of up to 64 tiles
-// (4096 tokens, 4 heads) left three quarters of the CUs idle.  Two remedies, chosen by an estimate of the launch's
-// length; all constants are measured times.
-//  * Split key ranges: several workgroups per query block, each with a contiguous share of the block's steps, and a second
-//    kernel that merges their accumulators.  The e4m3 modes with a static or absmax grid (1 .. 4), whose P depends on the
-//    row's running maximum, first run a pass that only forms the parts' row maxima (MODE 7), so that every part starts from
-//    the reference point it would have had.  4096 tokens, 4 / 1 heads: mode 0 88 -> 42 us, mode 1 132 -> 66, mode 2 186 ->
-//    75; a chunk of 512 rows behind 16384 tokens at 28 / 4 heads 325 -> 132 us in mode 0.  Mode 5 stays whole: where its reference
-//    point stands depends on every tile sum before (a jump of 2^100 puts it on that tile's maximum), not on a maximum.
-//  * Workgroups of 128 rows (4 waves): one wave per SIMD walks a tile in 0.7 to 0.82 of the time two take for theirs.  Short
-//    prompts, where a merge costs more than it saves: 777 tokens, 28 / 4 heads, mode 0 30.5 -> 24.1 us (split: 34), mode 1
-//    38.2 -> 28.4, mode 5 38.0 -> 30.2; 2048 tokens (448 workgroups) 57 -> 52, at 3000 the 8-wave launch is ahead (82
-//    against 95).
-// A tile of an 8-wave workgroup takes kStepUs on an otherwise idle chip and about 30 % more on a full one, which lowers its
-// clock: 8192 rows behind 24576 tokens, 3.5 workgroups per CU, take 2685 us split evenly or not.
-void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_t Hq, int64_t Nq, LaunchPlan& plan) {
-  constexpr int kCUs = 256, kMaxRounds = 4, kMinTiles = 4;
-  static const float kStepUs[6] = {1.35f, 1.75f, 2.6f, 1.4f, 1.15f, 1.15f};   // by P mode
-  constexpr float kFixUs = 8.f;      // a workgroup's launch, first loads and epilogue
-  static const float kFourWaves[6] = {0.76f, 0.7f, 0.82f, 1.f, 1.f, 0.76f};
-  constexpr float kFullChip = 0.3f;
-  constexpr float kMergeUs = 6.f, kPartUs = 0.07f;   // the merge; a part's 130 KB written and read again
-  constexpr float kRefUs = 8.f, kRefTileUs = 0.6f;   // MODE 7: launch and fixed part, per tile
-  plan.waves = 8;
-  plan.n_work = plan.n_slots = 0;
-  if (own4 && p->window_mode == SQ_WINDOW_SIZES && p->block_m == 64) {
-    plan.waves = 2;   // separate 4-bit operands with 64-row blocks: a workgroup of one block (with 128-row blocks: DUAL)
-    return;
-  }
-  const int64_t nQB = (Nq + 255) / 256, mult = B * Hq;
-  if (mult * nQB > kMaxRounds * kCUs) return;
-  const float step = kStepUs[p->p_quant];
-  int w_max = 0;
-  if (p->window_mode == SQ_WINDOW_SIZES)
-    for (int h = 0; h < Hq; ++h) w_max = std::max(w_max, std::max(p->w8[h], p->w4[h]));
-  // one workgroup per block of `rows` rows: the blocks of a head, longest first, on kCUs / mult CUs (each of them stands
-  // for the same block of every head)
-  int len[kMaxRounds * kCUs], longest = 0;
-  auto unsplit_us = [&](int rows, float tile_us) {
-    const int n = (int)((Nq + rows - 1) / rows), cus = (int)std::max<int64_t>(1, kCUs / mult), rounds = (int)((mult + kCUs - 1) / kCUs);
-    struct Cu { float load, tiles; } cu[kCUs] = {};
-    const auto later = [](const Cu& x, const Cu& y) { return x.load > y.load; };   // a heap with the least loaded CU in front
-    float total = 0, last = 0, last_tiles = 0;
-    for (int qb = n - 1; qb >= 0; --qb) {
-      const int t = tiles_of_block(p, (int64_t)qb * rows, std::min<int64_t>(Nq, (int64_t)(qb + 1) * rows), w_max);
-      if (rows == 256) {
-        len[qb] = t;
-        longest = std::max(longest, t);
-      }
-      std::pop_heap(cu, cu + cus, later);
-      Cu& c = cu[cus - 1];
-      c.load += (t * tile_us + kFixUs) * rounds;
-      c.tiles += (float)t * rounds;
-      total += (float)t * mult;
-      if (c.load > last) {
-        last = c.load;
-        last_tiles = c.tiles;
-      }
-      std::push_heap(cu, cu + cus, later);
-    }
-    return last + kFullChip * std::min(1.f, total / (kCUs * last_tiles)) * last_tiles * tile_us;
-  };
-  float best = unsplit_us(256, step);
-  const bool four_waves = !own4 && (p->p_quant <= SQ_P_E4M3_BLOCK || p->p_quant == SQ_P_E4M3_MX_FP8_PV);
-  if (four_waves && mult * ((Nq + 127) / 128) <= 2 * kCUs) {
-    const float us = unsplit_us(128, step * kFourWaves[p->p_quant]);
-    if (us < best) {
-      best = us;
-      plan.waves = 4;
-    }
-  }
-  if (longest <= kMinTiles || (own4 && p->p_quant != SQ_P_NONE) || p->p_quant == SQ_P_E4M3_MX_FP8_PV) return;
-  const bool ref_pass = p->p_quant >= SQ_P_E4M3_STATIC && p->p_quant <= SQ_P_E4M3_FP8_PV;
-  auto workgroups = [&](int cap) {
-    int64_t n = 0;
-    for (int qb = 0; qb < nQB; ++qb) n += (len[qb] + cap - 1) / cap;
-    return n;
-  };
-  float total = 0;
-  for (int qb = 0; qb < nQB; ++qb) total += (float)len[qb] * mult;
-  int cap = 0;
-  for (int m = 1; m <= kMaxRounds; ++m) {
-    int lo = kMinTiles, hi = longest;   // the smallest share that keeps to m workgroups per CU
-    while (lo < hi) {
-      const int c = (lo + hi) / 2;
-      if (workgroups(c) * mult <= m * kCUs) hi = c;
-      else lo = c + 1;
-    }
-    if (lo >= longest || workgroups(lo) > kMaxSplitWork) continue;
-    float us = m * (lo * step * (1.f + kFullChip * std::min(1.f, total / (kCUs * m * lo))) + kFixUs) + kMergeUs + kPartUs * mult * workgroups(lo);
-    if (ref_pass) us += m * lo * kRefTileUs + kRefUs;
-    if (us < 0.97f * best) {
-      best = us;
-      cap = lo;
-    }
-  }
-  if (cap == 0) return;
-  plan.waves = 8;
-  for (int64_t qb = nQB - 1; qb >= 0; --qb) {
-    const int parts = std::min((len[qb] + cap - 1) / cap, 255);
-    for (int i = 0; i < parts; ++i) plan.work[plan.n_work++] = SplitWork{(uint16_t)qb, (uint16_t)plan.n_slots, (uint8_t)i, (uint8_t)parts};
-    if (parts > 1) plan.n_slots += parts;
-  }
-  // longest shares first
-  std::stable_sort(plan.work, plan.work + plan.n_work, [&](const SplitWork& x, const SplitWork& y) { return len[x.qb] * y.parts > len[y.qb] * x.parts; });
-}
-
 constexpr size_t kPartRowBytes = 64 * 16 * 16 + 64 * 8 + 32 * 4;   // per wave of a part: accumulators, denominator and reference point
 
 size_t part_bytes(const LaunchPlan& plan, int64_t B, int64_t Hq) { return (size_t)(B * Hq) * plan.n_slots * 8 * kPartRowBytes; }
@@ -1776,10 +1647,15 @@ extern "C" size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_
   } else if (p->window_mode != SQ_WINDOW_NONE) {
     return need;
   }
+  // (operands of their own for the 4-bit range, which windows can come with, are planned differently: room for either)
   LaunchPlan plan;
-  // (operands of their own for the 4-bit range are what the launches with 128-row query blocks come with)
-  plan_launch(p, p->window_mode == SQ_WINDOW_SIZES && p->block_m == 128, batch, num_q_heads, qo_len, plan);
-  return need + part_bytes(plan, batch, num_q_heads);
+  plan_launch(p, false, batch, num_q_heads, qo_len, plan);
+  size_t parts = part_bytes(plan, batch, num_q_heads);
+  if (p->window_mode == SQ_WINDOW_SIZES) {
+    plan_launch(p, true, batch, num_q_heads, qo_len, plan);
+    parts = std::max(parts, part_bytes(plan, batch, num_q_heads));
+  }
+  return need + parts;
 }
 
 namespace {
@@ -1988,7 +1864,7 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   LaunchPlan plan;
   plan_launch(p, q4 != nullptr, B, Hq, Nq, plan);
   const bool split = plan.n_work > 0 && (size_t)numel_of(workspace) * (workspace->dtype.bits / 8) >= need + part_bytes(plan, B, Hq);
-  const int waves = plan.waves, rows_wg = waves * 32;
+  const int waves = split ? 8 : plan.waves, rows_wg = waves * 32;
   local.nQB = (int)((Nq + rows_wg - 1) / rows_wg);
   SQ_REQUIRE(p->q_quant == 0 || p->q_quant == 8, SQ_EINVAL, "sq_prefill_fwd: q_quant must be 0 or 8 (got %d)", (int)p->q_quant);
   SQ_REQUIRE(!(p->q_quant && q4), SQ_EINVAL, "sq_prefill_fwd: q_quant applies to launches without a separate 4-bit operand set");
