@@ -46,7 +46,8 @@ inline int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, in
 //  * Workgroups of 128 rows (4 waves): one wave per SIMD walks a tile in 0.7 to 0.82 of the time two take for theirs.  Short
 //    prompts, where a merge costs more than it saves: 777 tokens, 28 / 4 heads, mode 0 30.5 -> 24.1 us (split: 34), mode 1
 //    38.2 -> 28.4, mode 5 38.0 -> 30.2; 2048 tokens (448 workgroups) 57 -> 52, at 3000 the 8-wave launch is ahead (82
-//    against 95).
+//    against 95).  Not up to 128 rows: four waves of the 8-wave workgroup have no rows, the others have a SIMD each there too,
+//    and all eight copy the tiles (64 rows behind 131008 keys, 4 / 1 heads, mode 5: 1376 us, with 4 waves 1560).
 // A tile of an 8-wave workgroup takes kStepUs on an otherwise idle chip and about 30 % more on a full one, which lowers its
 // clock: 8192 rows behind 24576 tokens, 3.5 workgroups per CU, take 2685 us split evenly or not.
 inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_t Hq, int64_t Nq, LaunchPlan& plan) {
@@ -98,7 +99,7 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
   };
   float best = unsplit_us(256, step);
   const bool four_waves = !own4 && (p->p_quant <= SQ_P_E4M3_BLOCK || p->p_quant == SQ_P_E4M3_MX_FP8_PV);
-  if (four_waves && mult * ((Nq + 127) / 128) <= 2 * kCUs) {
+  if (four_waves && Nq > 128 && mult * ((Nq + 127) / 128) <= 2 * kCUs) {
     const float us = unsplit_us(128, step * kFourWaves[p->p_quant]);
     if (us < best) {
       best = us;

@@ -128,3 +128,11 @@ def test_unsplit_choice_stands_beside_the_split(plan):
         for n in (300, 500, 777):
             plans = plan([{"p_quant": 0, "Hq": h, "Nq": n, "offset": o} for o in (0, 256, 1024, 4096, 16384)])
             assert plans[-1][2] and all(waves == 4 for waves, _, _, _ in plans), (h, n, [waves for waves, _, _, _ in plans])
+
+
+def test_a_single_half_filled_workgroup_keeps_its_waves(plan):
+    """Up to 128 rows a 256-row workgroup has at most four waves with rows anyway, and eight that copy the tiles."""
+    for mode in (0, 1, 2, 5):
+        calls = [{"p_quant": mode, "Hq": h, "Nq": n, "offset": o} for h in (1, 4, 28) for n in (1, 64, 100, 128) for o in (0, 4096, 131072)]
+        assert all(waves == 8 for waves, _, _, _ in plan(calls)), mode
+        assert all(waves == 4 for waves, _, _, _ in plan([dict(c, Nq=129) for c in calls])), mode
