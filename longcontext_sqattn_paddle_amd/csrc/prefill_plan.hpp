@@ -67,12 +67,18 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
   const int64_t nQB = (Nq + 255) / 256, mult = B * Hq;
   if (mult * nQB > kMaxRounds * kCUs) return;
   const float step = kStepUs[p->p_quant];
+  // Mode 4's step is the shortest beside the same row-maximum pass, so a split in two that fills the chip loses: chains of like
+  // length on up to half the CUs run at the idle chip's rate (1.00 us a tile, 1.02 on 128 CUs), the pass slows down on a full
+  // chip.  8192 rows behind 57344 keys, 4 / 1 heads (128 chains): 1057 us whole, 1163 split; 4096 behind 32768: 637 whole, 393
+  // split; without a context, where the chains are unlike, 3000 rows of 8 / 8 heads 80 whole, 70 split.
+  const bool fp8_pv = p->p_quant == SQ_P_E4M3_FP8_PV;
   int w_max = 0;
   if (p->window_mode == SQ_WINDOW_SIZES)
     for (int h = 0; h < Hq; ++h) w_max = std::max(w_max, std::max(p->w8[h], p->w4[h]));
   // one workgroup per block of `rows` rows: the blocks of a head, longest first, on kCUs / mult CUs (each of them stands
   // for the same block of every head)
   int len[kMaxRounds * kCUs], longest = 0;
+  bool even_fp8 = false;
   auto unsplit_us = [&](int rows, float tile_us) {
     const int n = (int)((Nq + rows - 1) / rows), cus = (int)std::max<int64_t>(1, kCUs / mult), rounds = (int)((mult + kCUs - 1) / kCUs);
     struct Cu { float load, tiles; } cu[kCUs] = {};
@@ -95,7 +101,8 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
       }
       std::push_heap(cu, cu + cus, later);
     }
-    return last + kFullChip * std::min(1.f, total / (kCUs * last_tiles)) * last_tiles * tile_us;
+    if (rows == 256) even_fp8 = fp8_pv && n * mult <= kCUs / 2 && total > 0.75f * n * mult * longest;
+    return last + (even_fp8 ? 0.f : kFullChip) * std::min(1.f, total / (kCUs * last_tiles)) * last_tiles * tile_us;
   };
   float best = unsplit_us(256, step);
   const bool four_waves = !own4 && (p->p_quant <= SQ_P_E4M3_BLOCK || p->p_quant == SQ_P_E4M3_MX_FP8_PV);
@@ -125,7 +132,7 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
     }
     if (lo >= longest || workgroups(lo) > kMaxSplitWork) continue;
     float us = m * (lo * step * (1.f + kFullChip * std::min(1.f, total / (kCUs * m * lo))) + kFixUs) + kMergeUs + kPartUs * mult * workgroups(lo);
-    if (ref_pass) us += m * lo * kRefTileUs + kRefUs;
+    if (ref_pass) us += m * lo * kRefTileUs * (even_fp8 ? 1.f + kFullChip * std::min(1.f, total / (kCUs * m * lo)) : 1.f) + kRefUs;
     if (us < 0.97f * best) {
       best = us;
       cap = lo;

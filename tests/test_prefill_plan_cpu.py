@@ -136,3 +136,12 @@ def test_a_single_half_filled_workgroup_keeps_its_waves(plan):
         calls = [{"p_quant": mode, "Hq": h, "Nq": n, "offset": o} for h in (1, 4, 28) for n in (1, 64, 100, 128) for o in (0, 4096, 131072)]
         assert all(waves == 8 for waves, _, _, _ in plan(calls)), mode
         assert all(waves == 4 for waves, _, _, _ in plan([dict(c, Nq=129) for c in calls])), mode
+
+
+def test_mode_4_is_not_split_where_that_only_fills_the_chip(plan):
+    """Half the chip's CUs with chains of like length: split in two they run beside each other at the full chip's rate and need
+    the row-maximum pass on top.  Half as many chains, or chains of unlike length, are split."""
+    whole = [(4, 8192, 57344), (8, 4096, 32768), (4, 8192, 8192), (8, 4096, 131072)]
+    assert not any(work for _, _, work, _ in plan([{"p_quant": 4, "Hq": h, "Nq": n, "offset": o} for h, n, o in whole]))
+    split = [(4, 4096, 57344), (8, 2048, 32768), (4, 4096, 131072), (8, 4096, 0), (4, 2048, 0)]
+    assert all(work for _, _, work, _ in plan([{"p_quant": 4, "Hq": h, "Nq": n, "offset": o} for h, n, o in split]))
