@@ -1862,7 +1862,7 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   local.Nk = (int)Nk;
   local.nT = nT;
   LaunchPlan plan;
-  plan_launch(p, q4 != nullptr, B, Hq, Nq, plan);
+  plan_launch(p, q4 != nullptr, B, Hq, Nq, plan, k_scale != nullptr);
   const bool split = plan.n_work > 0 && (size_t)numel_of(workspace) * (workspace->dtype.bits / 8) >= need + part_bytes(plan, B, Hq);
   const int waves = split ? 8 : plan.waves, rows_wg = waves * 32;
   local.nQB = (int)((Nq + rows_wg - 1) / rows_wg);

@@ -46,15 +46,19 @@ inline int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, in
 //  * Workgroups of 128 rows (4 waves): one wave per SIMD walks a tile in 0.7 to 0.82 of the time two take for theirs.  Short
 //    prompts, where a merge costs more than it saves: 777 tokens, 28 / 4 heads, mode 0 30.5 -> 24.1 us (split: 34), mode 1
 //    38.2 -> 28.4, mode 5 38.0 -> 30.2; 2048 tokens (448 workgroups) 57 -> 52, at 3000 the 8-wave launch is ahead (82
-//    against 95).  Not up to 128 rows: four waves of the 8-wave workgroup have no rows, the others have a SIMD each there too,
-//    and all eight copy the tiles (64 rows behind 131008 keys, 4 / 1 heads, mode 5: 1376 us, with 4 waves 1560).
+//    against 95).  Up to 128 rows four waves of the 8-wave workgroup have no rows, so the others have a SIMD each there too
+//    and all eight copy the tiles: 0.07 to 0.1 us less per tile, against a smaller launch's 0.1 (mode 0) to 1.5 us.  The
+//    sides meet at kFewRowsTiles: 64 rows, 28 / 4 heads, mode 5: 1 tile 21.1 us with 4 waves, 22.4 with 8; 17 tiles 33.2 / 33.4; 65
+//    tiles 69.8 / 65.8 (2049 tiles 1560 / 1376); int8 Q.K^T: 1 tile 13.3 / 15.0, 17 tiles 33.8 / 33.7, 65 tiles 95.6 / 90.7.
 // A tile of an 8-wave workgroup takes kStepUs on an otherwise idle chip and about 30 % more on a full one, which lowers its
 // clock: 8192 rows behind 24576 tokens, 3.5 workgroups per CU, take 2685 us split evenly or not.
-inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_t Hq, int64_t Nq, LaunchPlan& plan) {
+inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_t Hq, int64_t Nq, LaunchPlan& plan, bool int8qk = false) {
+  const int mode = int8qk ? 6 : p->p_quant;
   constexpr int kCUs = kPlanCUs, kMaxRounds = kPlanMaxRounds, kMinTiles = 4;
-  static const float kStepUs[6] = {1.35f, 1.75f, 2.6f, 1.4f, 1.15f, 1.15f};   // by P mode
+  static const float kStepUs[7] = {1.35f, 1.75f, 2.6f, 1.4f, 1.15f, 1.15f, 1.35f};   // by P mode; 6: int8 Q.K^T
   constexpr float kFixUs = 8.f;      // a workgroup's launch, first loads and epilogue
-  static const float kFourWaves[6] = {0.76f, 0.7f, 0.82f, 1.f, 1.f, 0.76f};
+  static const float kFourWaves[7] = {0.76f, 0.7f, 0.82f, 1.f, 1.f, 0.76f, 0.76f};
+  static const int kFewRowsTiles[7] = {2, 2, 5, 0, 0, 16, 11};
   constexpr float kFullChip = 0.3f;
   constexpr float kMergeUs = 6.f, kPartUs = 0.07f;   // the merge; a part's 130 KB written and read again
   constexpr float kRefUs = 8.f, kRefTileUs = 0.6f;   // MODE 7: launch and fixed part, per tile
@@ -66,7 +70,7 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
   }
   const int64_t nQB = (Nq + 255) / 256, mult = B * Hq;
   if (mult * nQB > kMaxRounds * kCUs) return;
-  const float step = kStepUs[p->p_quant];
+  const float step = kStepUs[mode];
   // Mode 4's step is the shortest beside the same row-maximum pass, so a split in two that fills the chip loses: chains of like
   // length on up to half the CUs run at the idle chip's rate (1.00 us a tile, 1.02 on 128 CUs), the pass slows down on a full
   // chip.  8192 rows behind 57344 keys, 4 / 1 heads (128 chains): 1057 us whole, 1163 split; 4096 behind 32768: 637 whole, 393
@@ -106,8 +110,8 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
   };
   float best = unsplit_us(256, step);
   const bool four_waves = !own4 && (p->p_quant <= SQ_P_E4M3_BLOCK || p->p_quant == SQ_P_E4M3_MX_FP8_PV);
-  if (four_waves && Nq > 128 && mult * ((Nq + 127) / 128) <= 2 * kCUs) {
-    const float us = unsplit_us(128, step * kFourWaves[p->p_quant]);
+  if (four_waves && (Nq > 128 || longest <= kFewRowsTiles[mode]) && mult * ((Nq + 127) / 128) <= 2 * kCUs) {
+    const float us = unsplit_us(128, step * kFourWaves[mode]);
     if (us < best) {
       best = us;
       plan.waves = 4;

@@ -19,9 +19,9 @@ int main() {
   while (scanf("%d %d %d %d %d %d %d %lld %lld %lld %lld", &pq, &wm, &bm, &sink, &w8, &w4, &own4, &off, &B, &Hq, &Nq) == 11) {
     std::vector<int32_t> a(Hq, w8), b(Hq, w4);
     sq_prefill_params p = {};
-    p.p_quant = pq; p.q_offset = off; p.window_mode = wm; p.block_m = bm; p.sink = sink; p.num_heads_w = (int)Hq; p.w8 = a.data(); p.w4 = b.data();
+    p.p_quant = pq == 6 ? 0 : pq; p.q_offset = off; p.window_mode = wm; p.block_m = bm; p.sink = sink; p.num_heads_w = (int)Hq; p.w8 = a.data(); p.w4 = b.data();
     sq::LaunchPlan plan;
-    sq::plan_launch(&p, own4 != 0, B, Hq, Nq, plan);
+    sq::plan_launch(&p, own4 != 0, B, Hq, Nq, plan, pq == 6);   // 6: the int8 Q.K^T form of mode 0
     int w_max = w8 > w4 ? w8 : w4;
     printf("%d %d %d |", plan.waves, plan.n_work, plan.n_slots);
     for (int i = 0; i < plan.n_work; ++i) printf(" %d %d %d %d", plan.work[i].qb, plan.work[i].slot, plan.work[i].part, plan.work[i].parts);
@@ -130,12 +130,16 @@ def test_unsplit_choice_stands_beside_the_split(plan):
             assert plans[-1][2] and all(waves == 4 for waves, _, _, _ in plans), (h, n, [waves for waves, _, _, _ in plans])
 
 
-def test_a_single_half_filled_workgroup_keeps_its_waves(plan):
-    """Up to 128 rows a 256-row workgroup has at most four waves with rows anyway, and eight that copy the tiles."""
-    for mode in (0, 1, 2, 5):
-        calls = [{"p_quant": mode, "Hq": h, "Nq": n, "offset": o} for h in (1, 4, 28) for n in (1, 64, 100, 128) for o in (0, 4096, 131072)]
-        assert all(waves == 8 for waves, _, _, _ in plan(calls)), mode
-        assert all(waves == 4 for waves, _, _, _ in plan([dict(c, Nq=129) for c in calls])), mode
+def test_a_single_half_filled_workgroup(plan):
+    """Up to 128 rows a 256-row workgroup has at most four waves with rows anyway, and eight that copy the tiles: the smaller
+    workgroup only where the chain of tiles is short."""
+    for mode, tiles in ((0, 2), (1, 2), (2, 5), (5, 16), (6, 11)):
+        for h in (1, 4, 28):
+            for n in (1, 64, 100, 128):
+                room = tiles - (n + 63) // 64
+                got = [w for w, _, _, _ in plan([{"p_quant": mode, "Hq": h, "Nq": n, "offset": 64 * o} for o in (0, room, room + 1, 64, 2048)])]
+                assert got == [4, 4, 8, 8, 8], (mode, h, n, got)
+            assert all(w == 4 for w, _, _, _ in plan([{"p_quant": mode, "Hq": h, "Nq": 129, "offset": 64 * o} for o in (0, 16, 64, 2048)]))
 
 
 def test_mode_4_is_not_split_where_that_only_fills_the_chip(plan):
