@@ -1822,7 +1822,9 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
   }
   SQ_HIP(hipGetLastError());
 
-  PrefillArgs local;  // passed to the kernel by value (about 1.2 KB with the per-head windows)
+  // passed to the kernel by value: 1.3 KB with the per-head windows and 3 KB of a split launch's work list (handing the list to
+  // split launches only measured the same: 172 small calls, 0.2 % in the mean, within the spread)
+  PrefillArgs local;
   memset(&local, 0, sizeof(local));
   local.q = data_of(q);
   local.k = data_of(k);
