@@ -12,7 +12,11 @@ all deliberate:
   * the decode update never leaves the device (no host copy of the lengths), and it also maintains
     `attend_length = valid_length + 1` during a step, the per-sequence length the decode attention kernel takes,
     where the reference attends over the whole buffer;
-  * `sync` really waits for the copy (the reference's wait is commented out, :234-238).
+  * `prefill_update_kv_cache` copies on the caller's stream.  The reference has a copy stream beside it; here the waits that
+    tie such a stream to the caller's sat at the head of a second hardware queue as soon as the host ran ahead, and slowed
+    down every launch on the first one (512-token prompt and 8 decode steps through 4 layers: 6700 us with a copy stream,
+    6450 on one stream), while the copy is 5 us of a short prompt's layer and 0.09 of the 148 ms of a 131072-token one's;
+  * `sync` makes another stream wait for the copy (the reference's wait is commented out, :234-238).
 """
 from __future__ import annotations
 
@@ -56,9 +60,7 @@ class flash_attn_cache(KV_Cache):
         self.valid_length = torch.zeros(self.batch_size, dtype=torch.int32, device=self.device)
         self.attend_length = torch.zeros(self.batch_size, dtype=torch.int32, device=self.device)
         self._host_valid = [0] * self.batch_size     # host mirror of valid_length: bounds checks without a sync
-        self.copystream = torch.cuda.Stream(device=self.device)
-        self.copyevents = {str(self.device): torch.cuda.Event()}
-        self.KVreadyevents = {str(self.device): torch.cuda.Event()}
+        self._store_stream = None                    # stream of the last prefill copy
         self._lib = N.lib()
 
     def _kv_gib(self) -> float:
@@ -75,8 +77,8 @@ class flash_attn_cache(KV_Cache):
         """Store one sequence's keys and values from `valid_start` on (flash_attn_cache.py:153-232).
 
         key_states/value_states [1, seq_len, kv_heads, head_dim].  Returns the stored slices
-        `key_states[:, valid_start:]`, `value_states[:, valid_start:]` like the reference.  The copy runs on the
-        cache's copy stream behind the work already queued on the current stream; `sync` joins it.
+        `key_states[:, valid_start:]`, `value_states[:, valid_start:]` like the reference.  The copy runs on the current
+        stream; `sync` joins it from another one.
         """
         bsz, seq_len, _, _ = key_states.shape
         assert bsz == 1, "Multi-batch prefilling only support prefill single batch one by one."
@@ -85,26 +87,21 @@ class flash_attn_cache(KV_Cache):
             raise IndexError(f"batch index {start_bdx} outside the cache's {self.batch_size} sequences")
         _valid_start = self.valid_start[start_bdx]
         _valid_length = seq_len - _valid_start
-        dev = str(self.device)
-        self.KVreadyevents[dev].record()
-        with torch.cuda.stream(self.copystream):
-            self.copystream.wait_event(self.KVreadyevents[dev])
-            b = [N.dl(t) for t in (key_states, value_states, self.key_cache[layer_idx], self.value_cache[layer_idx])]
-            N.check(self._lib.sq_kv_cache_store(*[N.ptr(x) for x in b], int(start_bdx), int(_valid_start),
-                                                N.current_stream(self.device)))
-            key_states.record_stream(self.copystream)
-            value_states.record_stream(self.copystream)
-            if self._host_valid[start_bdx] != _valid_length:
-                self.valid_length[start_bdx:start_bdx + 1].fill_(_valid_length)
-                self._host_valid[start_bdx] = _valid_length
-            self.copyevents[dev].record()
+        b = [N.dl(t) for t in (key_states, value_states, self.key_cache[layer_idx], self.value_cache[layer_idx])]
+        N.check(self._lib.sq_kv_cache_store(*[N.ptr(x) for x in b], int(start_bdx), int(_valid_start), N.current_stream(self.device)))
+        if self._host_valid[start_bdx] != _valid_length:
+            self.valid_length[start_bdx:start_bdx + 1].fill_(_valid_length)
+            self._host_valid[start_bdx] = _valid_length
+        self._store_stream = torch.cuda.current_stream(self.device)
         if layer_idx == self.layer_num - 1 and start_bdx + bsz == self.batch_size:
             self.context += seq_len
         return key_states[:, _valid_start:, :, :], value_states[:, _valid_start:, :, :]
 
     def sync(self, layer_idx, start_bdx) -> None:
         """The current stream waits for the last prefill copy (flash_attn_cache.py:234-238)."""
-        torch.cuda.current_stream(self.device).wait_event(self.copyevents[str(self.device)])
+        current = torch.cuda.current_stream(self.device)
+        if self._store_stream is not None and current != self._store_stream:
+            current.wait_stream(self._store_stream)
 
     def decode_append_targets(self, layer_idx):
         """(key_cache, value_cache, valid_length, attend_length) of a layer, for a projection kernel that writes the

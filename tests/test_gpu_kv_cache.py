@@ -102,6 +102,39 @@ def test_decode_attention_over_the_cache_uses_the_valid_prefix_only():
         assert err < 2e-3, f"sequence {b}: max abs err {err}"   # bf16 inputs, fp32 accumulation (decode tests use 2e-4 * rms)
 
 
+def test_store_runs_on_the_callers_stream_and_sync_joins_another_one():
+    """One hardware queue per request: the copy is queued where the caller's work is, and a reader on a second stream sees the
+    rows after `sync`, without a device-wide wait."""
+    print("case kv-cache store stream", flush=True)
+    T, H, D = 4096, 4, 128
+    ks, vs = _rand((1, T, H, D), 61).to(DEV), _rand((1, T, H, D), 62).to(DEV)
+    cache = _cache(0, layers=1, batch=1, max_length=T, kv_heads=H)
+    cache.sync(0, 0)                                                  # nothing to wait for yet
+    queued = []
+
+    class Spy:
+        def __getattr__(self, name, lib=cache._lib):
+            def call(*args):
+                queued.append((name, args[-1]))
+                return getattr(lib, name)(*args)
+            return call
+
+    cache._lib = Spy()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        x = torch.randn(4096, 4096, device=DEV)
+        for _ in range(20):
+            x = x @ x * 1e-3                                          # keeps the first stream busy while the second one reads
+        cache.prefill_update_kv_cache(None, ks, vs, 0, 0)
+    with torch.cuda.stream(second):
+        cache.sync(0, 0)
+        k, v, n = cache.key_cache[0].clone(), cache.value_cache[0].clone(), cache.valid_length.clone()
+    torch.cuda.synchronize()
+    assert queued == [("sq_kv_cache_store", first.cuda_stream)]
+    assert torch.equal(k, ks) and torch.equal(v, vs) and int(n) == T
+
+
 def test_full_size_store_128k():
     """BASELINE's 128K prompt with 4 kv heads: 268 MB into the cache, checked on the device."""
     print("case kv-cache store 128K", flush=True)
