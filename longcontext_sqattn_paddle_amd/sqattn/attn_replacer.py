@@ -143,8 +143,11 @@ def mp_triton_wrapper(layer_idx, bit8_window_sizes=0, bit4_window_sizes=0, sink_
                     attn_output = attn_output.transpose(1, 2).contiguous()
                 bs, seq_len, head, head_dim = attn_output.shape
                 return attn_output.reshape(bs, seq_len, head * head_dim)
-            # bf16: the value goes straight into the tiles the attention kernel reads (the fp8 P.V modes make their own from rows)
-            tiled = query.dtype == torch.bfloat16 and (p_quant is None or p_quant < N.P_E4M3_FP8_PV)
+            # bf16: the value goes straight into the tiles the attention kernel reads (the fp8 P.V modes make their own from
+            # rows).  Up to 8 (batch, kv head) rows, which the tile pass holds in registers; with more it reads them twice, one
+            # workgroup per 64 keys: 700 tokens of 32 rows 128 - 160 us a call against 95 - 115 with the value as rows, level at 8192
+            tiled = (query.dtype == torch.bfloat16 and (p_quant is None or p_quant < N.P_E4M3_FP8_PV)
+                     and value.size(0) * value.size(2 if nhd else 1) <= 8)
             q_bit8, q_bit4, k_bit8, k_bit4, v_bit8 = fused_int_prepass(query, key, value, want_4bit=not relative, tensor_layout=layout,
                                                                        qk_qtype=args.qk_qtype, v_qtype=args.v_qtype, skip_query=q_in_kernel,
                                                                        value_tiles=tiled)

@@ -140,6 +140,40 @@ def test_config1_full_causal_with_block_fp8_p():
     assert _cos(o, e) >= 0.999   # int8 Q/K/V + e4m3 P against exact attention: the benchmark's stated bar
 
 
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+def test_closure_takes_value_tiles_up_to_eight_rows(layout, monkeypatch):
+    """Up to 8 (batch, kv head) rows of a bf16 value become tiles in the pre-pass, more go as rows (as do fp16 values and the
+    fp8 P.V modes); the output has the same bits either way."""
+    from longcontext_sqattn_paddle_amd.sqattn import attn_replacer as R
+
+    tiles = []
+    inner = R.fused_int_prepass
+
+    def spy(*a, value_tiles=False, **kw):
+        tiles.append(value_tiles)
+        return inner(*a, value_tiles=value_tiles, **kw)
+
+    for B, Hkv, dtype, p_quant, want in ((1, 8, torch.bfloat16, None, True), (2, 4, torch.bfloat16, None, True), (3, 3, torch.bfloat16, None, False),
+                                         (1, 9, torch.bfloat16, None, False), (1, 2, torch.float16, None, False), (1, 2, torch.bfloat16, 5, False)):
+        print(f"case closure tiles {layout} B={B} Hkv={Hkv} {dtype} p_quant={p_quant}", flush=True)
+        g = torch.Generator().manual_seed(70 + B)
+        q, k, v = (torch.randn(B, 200, h, 128, generator=g).to(dtype).to(DEV) for h in (2 * Hkv, Hkv, Hkv))
+        layer = types.SimpleNamespace(num_key_value_groups=2) if layout == "NHD" else types.SimpleNamespace()
+        if layout == "HND":
+            q, k, v = (t.transpose(1, 2).contiguous() for t in (q, k, v))
+        fn = R.mp_triton_wrapper(1, 0.25, 0.5, 64, types.SimpleNamespace(qk_qtype="int", v_qtype="int", use_relative_distance=True))
+        monkeypatch.setattr(R, "fused_int_prepass", spy)
+        out = fn(layer, q, k, v, None, p_quant=p_quant)
+        assert tiles.pop() is want and not tiles
+        monkeypatch.setattr(R, "fused_int_prepass", inner)
+        if want:   # the other route, by hand
+            _, _, k8, _, v8 = inner(q, k, v, want_4bit=False, tensor_layout=layout, skip_query=True)
+            rows = R.attn_hierarchical_relative_window(q, k8, q, k8, v8, 0.25, 0.5, 64, tensor_layout=layout, output_dtype=torch.bfloat16, q_quant=8)
+            rows = (rows if layout == "NHD" else rows.transpose(1, 2)).reshape(out.shape)
+            assert torch.equal(out, rows)
+    torch.cuda.synchronize()
+
+
 def test_decode_slot():
     from longcontext_sqattn_paddle_amd.sqattn.attn_replacer import decode_attention_fn
 
