@@ -1239,15 +1239,23 @@ namespace {
 // share the centroids then run on CUs that would idle.  Beyond that a split workgroup only takes another's CU (an unsplit
 // launch with one workgroup per CU holds its 16 KB blocks twice, a launch of four parts its CU's whole LDS).
 // segment_k_means, ten steps, 1024 centroids: 4096 tokens 335 -> 267 us, 16384 tokens 342 -> 277, 20000 (two parts) 350 -> 292.
+// Unsplit all the same
+//  * up to 128 tokens with up to three blocks of centroids, where the chain is short and the shares' meeting is not (64 tokens x 96
+//    centroids: 6.7 us a step, 7.9 with four parts; 256 centroids 8.0 / 8.0, 512: 10.8 / 9.1);
+//  * from 32 groups on, where every group has centroids of its own and a full chip reads them all at once, a launch over half
+//    the CUs, unless its chain is long: 32 groups x 500 tokens, 256 workgroups of four parts against 64 whole ones, 256
+//    centroids 12.1 us whole, 14.1 split, 1024: 27.4 / 26.2; 1000 tokens in two parts 320 centroids 14.3 / 15.7.
 template <bool TRACK>
 void launch_assign(const AssignArgs& a, int64_t G, hipStream_t st) {
   constexpr int64_t kCUs = 256;
   const int64_t N = a.N;
   auto grid = [&](int tokens) { return dim3((unsigned)((N + tokens - 1) / tokens), (unsigned)G); };
   const dim3 block(kAssignWaves * 64);
-  if (G * ((N + 63) / 64) <= kCUs && a.C > kCB)
+  const int blocks = (a.C + kCB - 1) / kCB;
+  const bool splits = blocks > 3 || (blocks > 1 && N > 128);
+  if (splits && G * ((N + 63) / 64) <= (G < 32 || blocks >= 16 ? kCUs : kCUs / 2))
     hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 4>), grid(kTileTok / 4), block, 0, st, a);
-  else if (G * ((N + 127) / 128) <= kCUs && a.C > kCB)
+  else if (splits && G * ((N + 127) / 128) <= (G < 32 || blocks >= 8 ? kCUs : kCUs / 2))
     hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 2>), grid(kTileTok / 2), block, 0, st, a);
   else
     hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 1>), grid(kTileTok), block, 0, st, a);

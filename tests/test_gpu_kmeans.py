@@ -376,25 +376,37 @@ def test_segment_k_means_with_carried_sums_equals_stateless_steps():
             assert a.shape == b.shape and torch.equal(a.view(torch.int16) if a.dtype == torch.bfloat16 else a, b.view(torch.int16) if b.dtype == torch.bfloat16 else b), segments
 
 
-# 64-token workgroups with four shares of the centroids up to 256 of them (G * ceil(N / 64)), 128-token ones with two shares
-# up to 256 of those, 256-token ones beyond; more than 64 centroids each
-@pytest.mark.parametrize("G,N,C", [(1, 1, 96), (1, 63, 128), (1, 65, 160), (3, 257, 1024), (1, 4097, 320), (1, 16384, 96), (1, 16385, 160),
-                                   (2, 16384, 1024), (2, 16385, 96)])
-def test_split_centroids_give_the_bits_of_the_unsplit_launch(G, N, C):
+def _parts(G, N, C):
+    """Shares of the centroids per workgroup (launch_assign): 64-token workgroups with four while 256 of them do, 128-token ones
+    with two while 256 do, else 256-token ones; one up to 128 tokens of up to three blocks of 64 centroids; from 32 groups on
+    half as many workgroups, unless the chain of blocks is long."""
+    blocks = -(-C // 64)
+    if blocks == 1 or (blocks <= 3 and N <= 128):
+        return 1
+    if G * -(-N // 64) <= (256 if G < 32 or blocks >= 16 else 128):
+        return 4
+    return 2 if G * -(-N // 128) <= (256 if G < 32 or blocks >= 8 else 128) else 1
+
+
+@pytest.mark.parametrize("G,N,C,parts", [(1, 1, 256, 4), (1, 63, 224, 4), (1, 65, 320, 4), (1, 129, 96, 4), (1, 200, 160, 4), (3, 257, 1024, 4), (1, 4097, 320, 4),
+                                         (1, 16384, 96, 4), (1, 16385, 160, 2), (2, 16384, 1024, 2), (32, 256, 256, 4), (32, 257, 160, 2), (32, 512, 1024, 4),
+                                         (32, 1000, 512, 2)])
+def test_split_centroids_give_the_bits_of_the_unsplit_launch(G, N, C, parts):
     """The same groups alone and among so many copies that the launch is not split: assignments, centroids and sizes are equal
     to the bit, in the step that re-sums every row and in the two that carry the sums."""
     from longcontext_sqattn_paddle_amd import _native as NAT
     from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _triton_k_means_train, _workspace
 
-    print(f"case kmeans split G={G} N={N} C={C}", flush=True)
+    print(f"case kmeans split G={G} N={N} C={C} parts={parts}", flush=True)
     g = torch.Generator().manual_seed(90 + C)
     key = torch.randn(G, N, 128, generator=g).bfloat16()
     key[:, N // 2] = 0                                             # every score equal: index 0
     cent = torch.randn(G, C, 128, generator=g).bfloat16()
     cent[:, C - 1] = cent[:, C // 2] = cent[:, 1]                  # the same centroid in several shares: the lowest index wins
     copies = 1
-    while copies * G * ((N + 127) // 128) <= 256:
+    while _parts(copies * G, N, C) > 1:
         copies *= 2
+    assert _parts(G, N, C) == parts > 1 and copies > 1
     small, large = [], []
     for reps, out in ((1, small), (copies, large)):
         kd, cd = key.repeat(reps, 1, 1).to(DEV), cent.repeat(reps, 1, 1).to(DEV)
