@@ -118,17 +118,8 @@ def test_block_scaled_p_keeps_small_probabilities_the_static_scale_flushes():
     assert errs[5] <= 0.5 * errs[4]
 
 
-@pytest.mark.parametrize("step_up,jump", [(6.0, 40.0), (0.0, 140.0), (3.0, 17.0)])
-def test_block_scaled_p_reference_moves_and_overflows(step_up, jump):
-    """Mode 5 forms a tile's probabilities against the standing reference point without looking at the scores first.
-    Scores that climb by `step_up` (log2) per 64-key tile push the row sums past 2^16 every few tiles (the reference then
-    moves up by whole binades, which rescales the tile packed just before as well); one key that leads everything before
-    it by `jump` does the same in one step, and by 140 it overflows 2^(s - reference): the tile is formed again from the
-    key rows in memory.  Against the oracle's restatement of the same rule, and against exact attention."""
-    from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
-
+def _climbing_scores(step_up, jump):
     N, D = 1536, 128
-    print(f"case prefill mode 5 reference moves step_up={step_up} jump={jump}", flush=True)
     g = torch.Generator().manual_seed(91)
     q = torch.randn(1, 4, N, D, generator=g) * 0.5
     k = torch.randn(1, 2, N, D, generator=g) * 0.5
@@ -138,7 +129,20 @@ def test_block_scaled_p_reference_moves_and_overflows(step_up, jump):
     ramp[1000:] += jump / 2
     q[..., 0] = 1.0
     k[:, :, :, 0] = (ramp * (D ** 0.5 / 1.44269504))[None, None]
-    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    return q.bfloat16(), k.bfloat16(), v.bfloat16()
+
+
+@pytest.mark.parametrize("step_up,jump", [(6.0, 40.0), (0.0, 140.0), (3.0, 17.0)])
+def test_block_scaled_p_reference_moves_and_overflows(step_up, jump):
+    """Mode 5 forms a tile's probabilities against the standing reference point without looking at the scores first.
+    Scores that climb by `step_up` (log2) per 64-key tile push the row sums past 2^16 every few tiles (the reference then
+    moves up by whole binades, which rescales the tile packed just before as well); one key that leads everything before
+    it by `jump` does the same in one step, and by 140 it overflows 2^(s - reference): the tile is formed again from the
+    key rows in memory.  Against the oracle's restatement of the same rule, and against exact attention."""
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
+
+    print(f"case prefill mode 5 reference moves step_up={step_up} jump={jump}", flush=True)
+    q, k, v = _climbing_scores(step_up, jump)
     ref, lse_ref = A.prefill_blockwise(q, k, v, p_quant=A.P_MX_ROW, v_quant="e4m3_channel", out_dtype=torch.float32)
     out, lse = attn_causal(q.to(DEV), k.to(DEV), v.to(DEV), "HND", torch.float32, return_lse=True, p_quant=5)
     torch.cuda.synchronize()
@@ -158,16 +162,7 @@ def test_block_scaled_p_reference_moves_and_overflows(step_up, jump):
     assert torch.allclose(lse.cpu(), lse_exact.float(), atol=2e-2, rtol=5e-3)
 
 
-@pytest.mark.parametrize("pattern", ["spikes", "late_giant", "alternating", "edge_spikes", "ramp_down"])
-@pytest.mark.parametrize("N,window", [(777, None), (1536, (64, 128, 256)), (2304, (0, 64, 64))])
-def test_block_scaled_p_score_patterns_with_and_without_windows(pattern, N, window):
-    """Mode 5 on score patterns chosen against its rare paths, full causal and with sink + windows (where a wave leaves
-    and re-enters its key range with a tile pending): lone keys 20 to 170 (log2) above the rest, a block of keys 150 above
-    everything before it, tiles that alternate between two levels 85 apart, spikes on the last key of a tile and the
-    first of the next, scores that fall by 7 per tile.  Same criteria as the test above."""
-    from longcontext_sqattn_paddle_amd.sqattn._prefill import run_prefill
-
-    print(f"case prefill mode 5 pattern={pattern} N={N} window={window}", flush=True)
+def _pattern_scores(pattern, N):
     D = 128
     g = torch.Generator().manual_seed(1001)
     q = torch.randn(1, 4, N, D, generator=g) * 0.5
@@ -189,7 +184,20 @@ def test_block_scaled_p_score_patterns_with_and_without_windows(pattern, N, wind
         r = -pos / 64.0 * 7.0
     q[..., 0] = 1.0
     k[:, :, :, 0] = (r * (D ** 0.5 / 1.44269504))[None, None]
-    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    return q.bfloat16(), k.bfloat16(), v.bfloat16()
+
+
+@pytest.mark.parametrize("pattern", ["spikes", "late_giant", "alternating", "edge_spikes", "ramp_down"])
+@pytest.mark.parametrize("N,window", [(777, None), (1536, (64, 128, 256)), (2304, (0, 64, 64))])
+def test_block_scaled_p_score_patterns_with_and_without_windows(pattern, N, window):
+    """Mode 5 on score patterns chosen against its rare paths, full causal and with sink + windows (where a wave leaves
+    and re-enters its key range with a tile pending): lone keys 20 to 170 (log2) above the rest, a block of keys 150 above
+    everything before it, tiles that alternate between two levels 85 apart, spikes on the last key of a tile and the
+    first of the next, scores that fall by 7 per tile.  Same criteria as the test above."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import run_prefill
+
+    print(f"case prefill mode 5 pattern={pattern} N={N} window={window}", flush=True)
+    q, k, v = _pattern_scores(pattern, N)
     kw = {} if window is None else dict(block_m=64, sink=window[0], w8=[window[1]] * 4, w4=[window[2]] * 4)
     ref, lse_ref = A.prefill_blockwise(q, k, v, p_quant=A.P_MX_ROW, v_quant="e4m3_channel", out_dtype=torch.float32, **kw)
     out, lse = run_prefill(q.to(DEV), k.to(DEV), v.to(DEV), tensor_layout="HND", output_dtype=torch.float32, return_lse=True,
@@ -386,6 +394,44 @@ def test_rows_do_not_depend_on_the_workgroup_size(mode, N, window):
     assert torch.equal(one[0], many[0]) and torch.equal(one[0], many[129])
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2, 5])
+@pytest.mark.parametrize("case", ["climb", "overflow", "step", "spikes", "late_giant", "alternating", "edge_spikes", "ramp_down", "sink", "chunk"])
+@pytest.mark.parametrize("window", [None, (64, 128, 256), (0, 64, 64)])
+def test_score_patterns_in_workgroups_of_256_rows(mode, case, window):
+    """The score patterns of the tests above run in 128-row workgroups at their sizes; launches that fill the chip, the long
+    prompts among them, run in 256-row ones, whose instantiations are others.  The same sequence in a batch too large for the small
+    workgroups (they are taken for at most 512 of them) gives the bits it gives alone."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace, run_prefill
+
+    print(f"case prefill 256 rows mode={mode} {case} window={window}", flush=True)
+    offset = 0
+    if case in ("climb", "overflow", "step"):
+        q, k, v = _climbing_scores(*{"climb": (6.0, 40.0), "overflow": (0.0, 140.0), "step": (3.0, 17.0)}[case])
+    elif case == "sink":
+        q, k, v = _rand(1, 4, 2, 777, 128, 79, scale=0.3)
+        q[..., 0] = 4.0
+        k[:, :, 0] = 0.0
+        k[:, :, 0, 0] = 33.0
+    elif case == "chunk":
+        q, k, v = _rand(1, 4, 2, 2560, 128, 31)
+        q, offset = q[:, :, 2048:].contiguous(), 2048
+    else:
+        q, k, v = _pattern_scores(case, 1536 if window else 777)
+    w = None if window is None else {"block_m": 64, "sink": window[0], "w8": [window[1]] * 4, "w4": [window[2]] * 4}
+    copies = 512 // (4 * ((q.shape[2] + 127) // 128)) + 1
+
+    def run(reps):
+        qd, kd, vd = (t.to(DEV).repeat(reps, 1, 1, 1) for t in (q, k, v))
+        return run_prefill(qd, kd, vd, output_dtype=torch.float32, p_quant=mode, window=w, return_lse=True, q_offset=offset,
+                           workspace=prefill_workspace(reps, 2, k.shape[2], qd.device))   # no room for parts
+
+    one, many = run(1), run(copies)
+    torch.cuda.synchronize()
+    for a, b in zip(one, many):
+        assert bool(a.isfinite().all())
+        assert torch.equal(a[0], b[0]) and torch.equal(a[0], b[copies - 1])
+
+
 @pytest.mark.parametrize("sink,r8,r4", [(128, 0.25, 0.25), (256, [0.125, 0.5], [0.5, 0.5]), (0, 0.0, 0.0), (64, 2.0, 2.0)])
 def test_relative_window_matches_oracle(sink, r8, r4):
     from longcontext_sqattn_paddle_amd.sqattn.attn_triton_mix_relative import attn_hierarchical_relative_window
@@ -482,8 +528,8 @@ def test_relative_window_quantised_modes(mode, sink, r8, r4, N):
 
 @pytest.mark.parametrize("mode", [0, 1, 3, 4, 5])
 def test_chunked_prefill_offset_all_modes(mode):
-    """8 waves x 32 rows against 2.5K keys with a query offset: every wave runs interior (unmasked) pairs, its own
-    diagonal tiles and idle steps."""
+    """512 rows behind 2K keys, in the workgroups the launch plan takes for them (mode 5: four waves; the others: eight, with
+    split key ranges): every wave runs interior (unmasked) pairs, its own diagonal tiles and idle steps."""
     from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
 
     print(f"case prefill chunked mode={mode}", flush=True)

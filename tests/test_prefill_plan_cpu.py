@@ -149,3 +149,13 @@ def test_mode_4_is_not_split_where_that_only_fills_the_chip(plan):
     assert not any(work for _, _, work, _ in plan([{"p_quant": 4, "Hq": h, "Nq": n, "offset": o} for h, n, o in whole]))
     split = [(4, 4096, 57344), (8, 2048, 32768), (4, 4096, 131072), (8, 4096, 0), (4, 2048, 0)]
     assert all(work for _, _, work, _ in plan([{"p_quant": 4, "Hq": h, "Nq": n, "offset": o} for h, n, o in split]))
+
+
+def test_batches_of_the_pattern_tests_take_the_large_workgroups(plan):
+    """The shapes whose two workgroup sizes the GPU tests compare: alone 4 waves, in the smallest batch past 512 small workgroups 8."""
+    for mode in (0, 1, 2, 5):
+        for n, offset in ((777, 0), (1536, 0), (512, 2048)):
+            for window in (None, (64, 64, 128, 256), (64, 0, 64, 64)):
+                copies = 512 // (4 * ((n + 127) // 128)) + 1
+                alone, many = plan([{"p_quant": mode, "Hq": 4, "Nq": n, "offset": offset, "window": window, "B": b} for b in (1, copies)])
+                assert alone[0] == 4 and many[0] == 8, (mode, n, window)
