@@ -1296,7 +1296,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) P[bn][t] = quant_pack8<(kPV8 ? 3 : (kQK8 || kRefPass ? 0 : MODE))>(S[bn], t, sc, inv);
+      for (int t = 0; t < 2; ++t) P[bn][t] = quant_pack8<(kPV8 ? 3 : (kQK8 ? 0 : MODE))>(S[bn], t, sc, inv);
     // O^T[d, row] += V^T[d, key] . P^T[key, row]
 #pragma unroll
     for (int bd = 0; bd < 4; ++bd)
