@@ -436,6 +436,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   constexpr bool kPlain = MODE == 2 || MODE == 6 || kRefPass;   // tile step left to the compiler's scheduling
   constexpr bool kPV8 = MODE == 4 || MODE == 5;     // e4m3 V tiles, fp8 P.V
   constexpr bool kOwn4 = WAVES == 2 || DUAL;        // the launches that can have their own 4-bit operands
+  constexpr bool kFirstRef = SPLIT && (MODE == 0 || MODE == 6);   // parts that take their reference point from the row's first tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // MODE 2: tile maxima of the two waves of a 64-row group, behind the tile rings (which start at LDS address 0)
   float (*s_amax)[WAVES] = (float (*)[WAVES])(smem + 4 * kStageBytes);
@@ -1361,6 +1362,9 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     if constexpr (!kDefer) stage_v(tile_of(1), 1);
   }
   if (2 < nTot) stage_k(tile_of(2), 2, step_uses4(2));
+  if constexpr (kFirstRef) {
+    if (sw.part > 0) stage_k(0, 3, false);   // buffer 3 is free until step 0 refills it
+  }
   if constexpr (kDefer) {
     // ring buffer 3 is read by step 0's P.V MFMAs, which have zeros for probabilities: it must hold finite numbers
     for (int i = tid; i < kVTileBytes / 16; i += NT) *(uint4*)(vbase_lds + 3 * kVTileBytes + 16 * i) = make_uint4(0, 0, 0, 0);
@@ -1421,6 +1425,21 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
+  // the lazy modes: a later part of a row starts from the reference point the whole row starts from, the maximum over tile 0 (every
+  // row of a split block sees all of it: the plan wants a sink or no windows, and blocks of more than four tiles).  The part's own
+  // first tile will not do: where its keys are masked out by the type's lowest value or -inf, the scores behind it would be
+  // accumulated on top of 1e37 or NaN.  16 MFMAs and a tile copy per part.
+  if constexpr (kFirstRef) {
+    if (sw.part > 0) {
+      f32x16_t S0[2];
+      qk_tile(kbase_lds + 3 * kKTileBytes, S0);
+      mfma_settle(S0[0], S0[1]);
+      m_run = xor32_max(lane_max(S0)) - kC;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) Cinit[i] = kC - m_run;
+      first = false;
+    }
+  }
   auto switch_q = [&](int t) __attribute__((always_inline)) {   // t: a step this wave visits
     if constexpr (kOwn4) {
       if (distinct4) {  // switch the Q~ operand set when entering/leaving the 4-bit window range

@@ -119,6 +119,8 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
   }
   if (longest <= kMinTiles || (own4 && p->p_quant != SQ_P_NONE) || p->p_quant == SQ_P_E4M3_MX_FP8_PV) return;
   const bool ref_pass = p->p_quant >= SQ_P_E4M3_STATIC && p->p_quant <= SQ_P_E4M3_FP8_PV;
+  // the parts of modes 0 and 6 start from the row's scores of tile 0, which windows without a sink do not reach
+  if (!ref_pass && p->window_mode == SQ_WINDOW_SIZES && p->sink < kPlanTile) return;
   auto workgroups = [&](int cap) {
     int64_t n = 0;
     for (int qb = 0; qb < nQB; ++qb) n += (len[qb] + cap - 1) / cap;

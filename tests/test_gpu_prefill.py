@@ -377,6 +377,80 @@ def test_split_key_ranges_keep_nan_and_infinity(mode, window, tensor, value):
         assert bool(whole[0].isfinite().any())
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("value", [-3.38e38, -math.inf, -3e6])
+@pytest.mark.parametrize("window", [None, (64, 0.25, 0.75)])
+def test_split_key_ranges_over_masked_keys(mode, value, window):
+    """Keys masked out through a channel of their own (query 1, masked keys the type's lowest value, -infinity or just far below
+    the others) in runs that some parts begin inside of: a part's reference point must not come from them.  The unmasked keys
+    in front set the unsplit launch's reference; exact attention over the unmasked keys is the result."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace, run_prefill
+
+    print(f"case prefill split masked keys mode={mode} value={value} window={window}", flush=True)
+    N = 3010
+    q, k, v = _rand(1, 3, 1, N, 128, 44)
+    q[..., 7] = 1.0
+    k[..., 7] = 0.0
+    k *= torch.linspace(0.5, 2.0, N)[None, None, :, None].bfloat16()      # (no two tiles with the same maximum)
+    masked = torch.zeros(N, dtype=torch.bool)
+    for lo, hi in ((300, 800), (900, 1100), (1250, 1900), (2000, 2400), (2500, 2700)):
+        masked[lo:hi] = True
+    km = k.clone()
+    km[:, :, masked, 7] = value
+    w = None if window is None else {"block_m": 64, "sink": window[0], "w8": [A.window_size_relative(window[1], N)] * 3,
+                                     "w4": [A.window_size_relative(window[2], N)] * 3}
+    qd, kd, vd = q.to(DEV), km.to(DEV), v.to(DEV)
+    parts = run_prefill(qd, kd, vd, output_dtype=torch.float32, p_quant=mode, window=w, return_lse=True)
+    whole = run_prefill(qd, kd, vd, output_dtype=torch.float32, p_quant=mode, window=w, return_lse=True, workspace=prefill_workspace(1, 1, N, qd.device))
+    torch.cuda.synchronize()
+    rows = ~masked                                            # a masked key's own row may see nothing else in its first tiles
+    assert not torch.equal(parts[0], whole[0])
+    for t in (*parts, *whole):
+        assert bool(t[:, :, rows].isfinite().all())
+    _check(parts[0][:, :, rows], whole[0][:, :, rows].cpu(), mode != 0, q_tol=8e-3)
+    assert torch.allclose(parts[1][:, :, rows], whole[1][:, :, rows], atol=2e-4)
+    if window is None:
+        qs = A.fold_scale(q, 128)
+        s = torch.matmul(qs[0].float(), k[0, 0].float().T) * math.log(2.0)
+        s = s.masked_fill(masked[None, None, :] | torch.ones(N, N, dtype=torch.bool).triu(1)[None], -math.inf)
+        exact = torch.matmul(torch.softmax(s.double(), -1), v[0, 0].double())
+        assert _cos(parts[0][0, :, rows].cpu(), exact[:, rows]) >= 0.999
+
+
+@pytest.mark.parametrize("scale", [2.6e36, 1e3])
+@pytest.mark.parametrize("window", [None, (64, 768, 2304)])
+def test_split_key_ranges_over_masked_codes(scale, window):
+    """The same for the integer Q.K^T form: masked keys are a code of -127 in a channel where the query is 1, with a scale that takes
+    the score to -4e37 or to a few thousand below the others."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace, run_prefill
+
+    print(f"case prefill split masked codes scale={scale} window={window}", flush=True)
+    N = 3010
+    q, _, v = _rand(1, 3, 1, N, 128, 45)
+    g = torch.Generator().manual_seed(46)
+    codes = torch.randint(-127, 128, (1, 1, N, 128), generator=g, dtype=torch.int8)
+    codes[..., 7] = 0
+    k_scale = torch.full((1, 1, 3072), 0.012)
+    q[..., 7] = 1.0
+    masked = torch.zeros(N, dtype=torch.bool)
+    for lo, hi in ((300, 800), (900, 1100), (1250, 1900), (2000, 2400), (2500, 2700)):
+        masked[lo:hi] = True
+    codes[:, :, masked] = 0
+    codes[:, :, masked, 7] = -127
+    k_scale[:, :, :N][:, :, masked] = scale
+    w = None if window is None else {"block_m": 64, "sink": window[0], "w8": [window[1]] * 3, "w4": [window[2]] * 3}
+    qd, kd, vd, sd = q.to(DEV), codes.to(DEV), v.to(DEV), k_scale.to(DEV)
+    kw = dict(output_dtype=torch.float32, window=w, return_lse=True, k_scale=sd)
+    parts, whole = run_prefill(qd, kd, vd, **kw), run_prefill(qd, kd, vd, workspace=prefill_workspace(1, 1, N, qd.device), **kw)
+    torch.cuda.synchronize()
+    rows = ~masked
+    assert not torch.equal(parts[0], whole[0])
+    for t in (*parts, *whole):
+        assert bool(t[:, :, rows].isfinite().all())
+    _check(parts[0][:, :, rows], whole[0][:, :, rows].cpu(), False)
+    assert torch.allclose(parts[1][:, :, rows], whole[1][:, :, rows], atol=2e-4)
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2, 5])
 @pytest.mark.parametrize("N,window", [(257, None), (640, (64, 128, 256))])
 def test_rows_do_not_depend_on_the_workgroup_size(mode, N, window):

@@ -159,3 +159,17 @@ def test_batches_of_the_pattern_tests_take_the_large_workgroups(plan):
                 copies = 512 // (4 * ((n + 127) // 128)) + 1
                 alone, many = plan([{"p_quant": mode, "Hq": 4, "Nq": n, "offset": offset, "window": window, "B": b} for b in (1, copies)])
                 assert alone[0] == 4 and many[0] == 8, (mode, n, window)
+
+
+def test_windows_without_a_sink_are_split_in_the_grid_modes_only(plan):
+    """The parts of modes 0 and 6 start from the row's scores of tile 0, which such windows do not reach."""
+    for mode, sink, split in ((0, 64, True), (6, 64, True), (0, 0, False), (6, 0, False), (1, 0, True), (2, 0, True), (4, 0, True)):
+        (_, _, work, _), = plan([{"p_quant": mode, "Hq": 2, "Nq": 4096, "window": (64, sink, 1024, 2048)}])
+        assert bool(work) is split, (mode, sink)
+
+
+def test_split_blocks_see_all_of_the_first_tile(plan):
+    """No row of a block with parts sits among the first 64 keys."""
+    calls = _calls()
+    for c, (_, _, work, _) in zip(calls, plan(calls)):
+        assert all(c["offset"] + 256 * qb >= 64 for qb, _, _, parts in work if parts > 1), c
