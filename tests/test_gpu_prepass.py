@@ -1,6 +1,8 @@
 """GPU parity of `sq_fake_quant_prepass` (through the C ABI) with the oracle's restatement of the operand pre-pass
 of sqattn/attn_replacer.py:334-365: bit-exact outputs, both layouts and dtypes, ragged sizes, error paths, and
 sampled rows at the benchmark shape."""
+import math
+
 import pytest
 import torch
 
@@ -210,3 +212,29 @@ def test_value_tiles_of_another_shape_or_type_are_refused():
     with pytest.raises(ValueError, match="not v_tiles"):
         run_prefill(q, k.to(torch.int8), v, tensor_layout="NHD", k_scale=torch.zeros(1, 2, 256, device=DEV), v_tiles=tiles(1, 2, 4, 128, 64))
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("B,Hkv", [(1, 4), (2, 4), (3, 3)])
+def test_value_tiles_of_special_values(B, Hkv):
+    """NaN, infinities, values past fp16's range, signed zeros and subnormals come out of the tile pass as out of the rows."""
+    from longcontext_sqattn_paddle_amd.sqattn.fake_quant import fused_int_prepass
+
+    print(f"case value tiles special values B={B} Hkv={Hkv}", flush=True)
+    N = 130
+    q, k, v = _inputs(B, N, Hkv, Hkv, seed=9, dtype=torch.bfloat16)
+    special = torch.tensor([math.nan, math.inf, -math.inf, 3.3e38, -3.3e38, 1e5, 7e4, -0.0, 0.0, 1e-40, -1e-39, 65504.0, 1e-5]).bfloat16()
+    g = torch.Generator().manual_seed(10)
+    at = torch.rand(v.shape, generator=g) < 0.1
+    v[at] = special[torch.randint(0, len(special), (int(at.sum()),), generator=g)]
+    v[:, :, 0] = 0                                                 # rows without a value and a whole NaN row
+    v[:, 5] = math.nan
+    q, k, v = (t.to(DEV) for t in (q, k, v))
+    for vq in ("int", "e4m3", "e5m2"):
+        rows = fused_int_prepass(q, k, v, tensor_layout="NHD", v_qtype=vq)[4].permute(0, 2, 1, 3)
+        tiles = fused_int_prepass(q, k, v, tensor_layout="NHD", v_qtype=vq, value_tiles=True)[4].cpu()
+        nT = (N + 63) // 64
+        pad = torch.zeros(B, Hkv, nT * 64, 128, dtype=torch.float16)
+        pad[:, :, :N] = rows.cpu().half()
+        want = pad.view(B, Hkv, nT, 4, 4, 4, 128)[:, :, :, :, [0, 2, 1, 3]].reshape(B, Hkv, nT, 64, 128).transpose(3, 4).contiguous()
+        assert torch.equal(tiles.isnan(), want.isnan()) and not bool(want.isfinite().all())
+        assert torch.equal(tiles.view(torch.int16)[~want.isnan()], want.view(torch.int16)[~want.isnan()])
