@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
       for (int p = 1; p < PARTS; ++p) {
         const float ob = s_best[(sub * PARTS + p) * 64 + 32 * tb + c32];
         const int oi = s_bidx[(sub * PARTS + p) * 64 + 32 * tb + c32];
-        if (ob > bv2[tb] || (ob == bv2[tb] && oi < bidx2[tb])) {
+        if (ob > bv2[tb]) {   // a tie stays with the lower part, whose indices are lower; so does a token without a score above -inf (NaN)
           bv2[tb] = ob;
           bidx2[tb] = oi;
         }

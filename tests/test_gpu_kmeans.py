@@ -6,6 +6,8 @@ Cluster sums are exact on both sides, so centroids computed from the same assign
 bit (one bf16 ulp is tolerated on at most 0.1 % of the components: the squared norm is reduced in a
 different fp64 order before it is rounded to fp32).
 """
+import math
+
 import pytest
 import torch
 
@@ -419,3 +421,33 @@ def test_split_centroids_give_the_bits_of_the_unsplit_launch(G, N, C, parts):
     assert not bool(((small[0] == C - 1) | (small[0] == C // 2)).any())
     for a, b in zip(small, large):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("G,N,C,parts", [(2, 200, 320, 4), (1, 16400, 160, 2)])
+def test_split_centroids_with_special_values(G, N, C, parts):
+    """NaN keys (no score above -inf), extreme elements of keys, infinite and extreme ones of centroids (whole shares of centroids
+    without a finite score among them): the assignments of the unsplit launch."""
+    from longcontext_sqattn_paddle_amd import _native as NAT
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _triton_k_means_train, _workspace
+
+    print(f"case kmeans split special values G={G} N={N} C={C} parts={parts}", flush=True)
+    g = torch.Generator().manual_seed(17)
+    key = torch.randn(G, N, 128, generator=g).bfloat16()
+    cent = torch.randn(G, C, 128, generator=g).bfloat16()
+    special = torch.tensor([1e37, -1e37, 1e30, -0.0, 1e-40]).bfloat16()
+    key[:, :50, 3] = special[torch.randint(0, 5, (G, 50), generator=g)]
+    key[:, 60:70] = math.nan
+    cent[:, : C // 4, 9] = -math.inf                               # half of the tokens score -inf, the other half +inf
+    cent[:, C // 2: C // 2 + 70, 11] = 3.3e38
+    copies = 1
+    while _parts(copies * G, N, C) > 1:
+        copies *= 2
+    assert _parts(G, N, C) == parts and copies > 1
+    got = []
+    for reps in (1, copies):
+        kd, cd = key.repeat(reps, 1, 1).to(DEV), cent.repeat(reps, 1, 1).to(DEV)
+        idx = torch.full((kd.shape[0], N), -1, dtype=torch.int32, device=DEV)
+        _triton_k_means_train(kd, cd, max_idx=idx, workspace=_workspace(kd.shape[0], N, C, DEV), state=NAT.KMEANS_STATELESS)
+        got.append(idx[:G].cpu())
+    assert int(got[1].min()) >= 0 and int(got[1].max()) < C
+    assert torch.equal(got[0], got[1])
