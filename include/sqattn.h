@@ -123,7 +123,10 @@ size_t sq_prefill_workspace_bytes(int64_t batch, int64_t num_kv_heads, int64_t k
  * The workspace with which sq_prefill_fwd / sq_prefill_int8qk_fwd also split the key ranges of a launch whose query blocks
  * do not fill the chip (short sequences, few heads, chunks behind a long context) over more workgroups: the size above plus
  * the parts' fp32 partial results, where this call would be split, else the size above.  `params` is the call's.  With a
- * smaller workspace the call runs unsplit.
+ * smaller workspace the call runs unsplit.  P modes 0 - 4 and the integer Q.K^T form can be split, mode 5 is not.  A part (256
+ * rows of one q head: accumulators, denominators, reference points) takes 136 KB, a call at most 1024 of them = 139 MB; a call whose
+ * windows can come with 4-bit operands of their own is sized for its plan with and without them.
+ * A call refused by sq_prefill_fwd gets the plain size here and its error there.
  */
 size_t sq_prefill_workspace_bytes_split(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t qo_len, int64_t kv_len,
                                         const sq_prefill_params* params);
@@ -141,7 +144,7 @@ int sq_prefill_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v, cons
 /*
  * sq_prefill_fwd for a value that sq_fake_quant_prepass_vtiles has left as tiles (p_quant 0 - 3; the fp8 P.V modes make tiles
  * of their own from v): v_tiles is a compact, 16-byte aligned fp16 [batch, Hkv, ceil(Nk / 64), 128, 64], counts as the key's.
- * Other arguments as sq_prefill_fwd.
+ * Other arguments as sq_prefill_fwd; the workspace is that call's too, though its tile area is left untouched.
  */
 int sq_prefill_vtiles_fwd(const DLTensor* q, const DLTensor* k, const DLTensor* v_tiles, const DLTensor* q4, const DLTensor* k4,
                           DLTensor* out, DLTensor* lse, DLTensor* workspace, const sq_prefill_params* p, void* stream);

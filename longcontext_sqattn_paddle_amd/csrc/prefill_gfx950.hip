@@ -1588,7 +1588,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   }
 }
 
-// Memory-bound: 130 KB per part and workgroup read, 64 KB of output per block (bf16) written; 7 us for 196 parts.
+// Memory-bound: 130 KB per part and workgroup read, 64 KB of output per block (bf16) written: 244 parts of 61 blocks 9 us.
 // Merges the parts of split key ranges: o = sum_p 2^(m_p - m) o_p, l likewise, out = o / l.  One workgroup per (block of the
 // work list that is split, wave of its workgroups, q head); lanes and accumulator elements keep the places they had there,
 // and wave bd of this workgroup takes output channels 32 bd .. +31.

@@ -41,7 +41,7 @@ inline int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, in
 //    kernel that merges their accumulators.  The e4m3 modes with a static or absmax grid (1 .. 4), whose P depends on the
 //    row's running maximum, first run a pass that only forms the parts' row maxima (MODE 7), so that every part starts from
 //    the reference point it would have had.  4096 tokens, 4 / 1 heads: mode 0 88 -> 42 us, mode 1 132 -> 66, mode 2 186 ->
-//    75; a chunk of 512 rows behind 16384 tokens at 28 / 4 heads 325 -> 132 us in mode 0.  Mode 5 stays whole: where its reference
+//    69; a chunk of 512 rows behind 16384 tokens at 28 / 4 heads 325 -> 132 us in mode 0.  Mode 5 stays whole: where its reference
 //    point stands depends on every tile sum before (a jump of 2^100 puts it on that tile's maximum), not on a maximum.
 //  * Workgroups of 128 rows (4 waves): one wave per SIMD walks a tile in 0.7 to 0.82 of the time two take for theirs.  Short
 //    prompts, where a merge costs more than it saves: 777 tokens, 28 / 4 heads, mode 0 30.5 -> 24.1 us (split: 34), mode 1

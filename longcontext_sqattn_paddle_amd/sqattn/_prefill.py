@@ -11,7 +11,8 @@ from ._common import KERNEL_HEAD_DIM, pad_head_dim, require_gpu
 
 
 def prefill_workspace(B: int, Hkv: int, kv_len: int, device) -> torch.Tensor:
-    """Scratch for the fp16 transposed V tiles the kernel consumes (caller may cache and reuse it)."""
+    """Scratch for the fp16 transposed V tiles the kernel consumes (caller may cache and reuse it).  It has no room for the parts
+    of split key ranges: a call given it runs unsplit (`run_prefill` sizes its own scratch with them)."""
     need = N.lib().sq_prefill_workspace_bytes(B, Hkv, kv_len, 128)
     return torch.empty(need // 2, dtype=torch.float16, device=device)
 
