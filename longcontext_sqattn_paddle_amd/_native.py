@@ -223,11 +223,11 @@ def check(code: int, library: Optional[ctypes.CDLL] = None) -> None:
     raise RuntimeError(f"libsqattn_hip error {code}: {msg}")
 
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # missing in torch builds without a GPU runtime
 
 
 def current_stream(device) -> int:
     """Handle of the calling thread's current stream on `device`."""
-    if isinstance(device, torch.device) and device.index is not None:   # a GPU tensor's device
+    if _raw_stream is not None and isinstance(device, torch.device) and device.index is not None:   # a GPU tensor's device
         return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream

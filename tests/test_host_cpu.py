@@ -1,4 +1,5 @@
 """CPU checks of the host-side mirror of the reference interface (no kernel call)."""
+import os
 import types
 
 import pytest
@@ -181,3 +182,15 @@ def test_decode_shares_by_length_add_up():
         else:
             assert (n == 1).all()
         assert (base[1:] == base[:-1] + n[:-1]).all()
+
+
+def test_package_imports_on_a_torch_without_gpu_runtime():
+    """The host modules (oracle inputs, window search, quantisers) import where torch has no device streams at all."""
+    import subprocess
+    import sys
+
+    code = ("import torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'): del torch._C._cuda_getCurrentRawStream\n"
+            "import longcontext_sqattn_paddle_amd._native, longcontext_sqattn_paddle_amd.sqattn.window_search\n"
+            "import longcontext_sqattn_paddle_amd.sqattn.attn_replacer, longcontext_sqattn_paddle_amd.model_hub.qwen\n")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
