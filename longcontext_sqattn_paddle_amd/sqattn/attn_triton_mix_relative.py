@@ -11,7 +11,7 @@ import numpy as np
 import torch
 
 from .. import _native as N
-from ._prefill import align_windows, per_head, run_prefill
+from ._prefill import align_windows, once_each, per_head, run_prefill
 
 
 def window_tokens(ratio: float, kv_len: int) -> int:
@@ -40,8 +40,8 @@ def attn_hierarchical_relative_window(q_int8, k_int8, q_int4, k_int4, v, int8_wi
         raise ValueError(f"sink_size must be a non-negative integer, got {sink_size}")
     # (ratios already give multiples of 128; the sink is rounded up to a 64-key block, and an 8-bit ratio of zero under
     # a wider 4-bit window gets the query block, see align_windows)
-    tokens = {r: window_tokens(float(r), kv_len) for r in set(r8 + r4)}   # each ratio once: 23 us of host for 2 x 28 heads otherwise
-    w8, w4, sink_size = align_windows([tokens[r] for r in r8], [tokens[r] for r in r4], sink_size, 64)
+    tokens = once_each(r8 + r4, lambda r: window_tokens(float(r), kv_len))
+    w8, w4, sink_size = align_windows(tokens[:H], tokens[H:], sink_size, 64)
     window = {"block_m": 64, "sink": sink_size, "w8": w8, "w4": w4}
     mode = p_quant if p_quant is not None else (N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE)
     return run_prefill(q_int8, k_int8, v, tensor_layout=tensor_layout, output_dtype=output_dtype,

@@ -194,3 +194,22 @@ def test_package_imports_on_a_torch_without_gpu_runtime():
             "import longcontext_sqattn_paddle_amd._native, longcontext_sqattn_paddle_amd.sqattn.window_search\n"
             "import longcontext_sqattn_paddle_amd.sqattn.attn_replacer, longcontext_sqattn_paddle_amd.model_hub.qwen\n")
     subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
+def test_window_sizes_in_any_number_type():
+    """Sizes formed once per distinct value are those formed one by one, for plain numbers, numpy scalars, 0-dimensional arrays (which
+    cannot be dictionary keys) and tensors."""
+    import numpy as np
+
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import align_windows, once_each
+
+    w8, w4 = [100, 0, 64, 100, 640], [300, 300, 64, 300, 10]
+    want = align_windows(w8, w4, 70, 128)
+    assert want == ([128, 128, 64, 128, 640], [320, 320, 64, 320, 64], 128)
+    for make in (np.int64, np.array, torch.tensor, float):
+        assert align_windows([make(x) for x in w8], [make(x) for x in w4], 70, 128) == want
+    seen = []
+    assert once_each([0.5, 0.25, 0.5, 0.25], lambda r: seen.append(r) or 4 * r) == [2.0, 1.0, 2.0, 1.0] and len(seen) == 2
+    assert once_each([np.array(0.5), np.array(0.25)], lambda r: 4 * float(r)) == [2.0, 1.0]
+    with pytest.raises(TypeError):
+        once_each([None], float)
