@@ -451,6 +451,39 @@ def test_split_key_ranges_over_masked_codes(scale, window):
     assert torch.allclose(parts[1][:, :, rows], whole[1][:, :, rows], atol=2e-4)
 
 
+@pytest.mark.parametrize("mode", [0, 2, 4])
+def test_split_key_ranges_in_a_graph_and_on_two_streams(mode):
+    """A split call (row maxima, parts and merge behind each other, scratch of its own) recorded into a graph and replayed on new
+    inputs with eager work in between, and two of them at once on different streams: the bits of the eager call."""
+    from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
+
+    print(f"case prefill split graph mode={mode}", flush=True)
+    inputs_ = [tuple(t.to(DEV) for t in _rand(1, 3, 1, 2100, 128, 50 + i)) for i in range(4)]
+    call = lambda x: attn_causal(*x, "HND", torch.float32, return_lse=True, p_quant=mode)
+    want = [call(x) for x in inputs_]
+    held = tuple(t.clone() for t in inputs_[0])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, lse = call(held)
+    for x, (o, l) in list(zip(inputs_, want)) * 2:
+        for a, b in zip(held, x):
+            a.copy_(b)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, o) and torch.equal(lse, l)
+        assert torch.equal(call(x)[0], o)                        # eager work between the replays
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    got = []
+    for i in range(8):
+        with torch.cuda.stream(streams[i & 1]):
+            got.append(call(inputs_[i & 3]))
+    torch.cuda.synchronize()
+    for i, (o, l) in enumerate(got):
+        assert torch.equal(o, want[i & 3][0]) and torch.equal(l, want[i & 3][1])
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2, 5])
 @pytest.mark.parametrize("N,window", [(257, None), (640, (64, 128, 256))])
 def test_rows_do_not_depend_on_the_workgroup_size(mode, N, window):
