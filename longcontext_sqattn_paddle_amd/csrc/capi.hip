@@ -1,6 +1,8 @@
 // Library-wide pieces of the C ABI: version, thread-local error string, argument checks.
 #include <stdarg.h>
 
+#include <atomic>
+
 #include "common.hpp"
 
 namespace sq {
@@ -12,6 +14,14 @@ void set_error(const char* fmt, ...) {
   va_start(ap, fmt);
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
   va_end(ap);
+}
+
+uint32_t call_tag() {
+  static std::atomic<uint32_t> calls{0};
+  uint32_t n;
+  do n = (calls.fetch_add(1, std::memory_order_relaxed) + 1u) * 0x9E3779B9u;   // an odd factor: 2^32 different numbers
+  while (n == 0);
+  return n;
 }
 
 int check_tensor(const DLTensor* t, const char* name, int ndim, int device_id) {

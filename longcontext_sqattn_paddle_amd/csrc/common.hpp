@@ -74,6 +74,11 @@ inline bool is_compact(const DLTensor* t) {
   return true;
 }
 
+// A number of its own for every call that hands results from workgroup to workgroup inside one launch: a word in the
+// workspace that carries it was written by this call, whatever the memory held before.  Never 0, spread over 32 bits
+// (a workspace full of one small number is not mistaken for it), repeats after 2^32 calls.  Defined in capi.hip.
+uint32_t call_tag();
+
 // Common checks of one tensor argument: non-null, on a GPU, expected rank, last dim contiguous,
 // 16-byte aligned base.  Returns SQ_OK or an error code with the message set.
 int check_tensor(const DLTensor* t, const char* name, int ndim, int device_id);

@@ -689,7 +689,9 @@ struct TopkArgs {
   int64_t out_sg;
   float* score;            // workspace [G,C]
   int32_t* start;          // workspace [G,C] start position of each cluster in rank order (two-kernel path)
-  uint32_t* arrive;        // workspace [G] arrival words of the shared score phase (one-launch path; same memory as `start`)
+  unsigned long long* scored;   // workspace [G,C] score and tag of the shared score phase (one-launch path; the memory of `score` and `start`)
+  uint32_t tag;
+  int32_t share;           // waves (64 clusters each) per workgroup of the shared score phase
   int64_t q_sb, q_sh, c_sg, c_sc, cl_sg, cl_sc;
   int32_t C, M, k, Hkv, group;
 };
@@ -823,200 +825,223 @@ __global__ __launch_bounds__(1024) void topk_emit_kernel(TopkArgs a) {
 // ---- the same selection in one launch, without ordering all clusters (at most 1024 clusters and 16 q heads per kv head;
 // other shapes take the two kernels above).  One workgroup of 1024 threads per group, one cluster per thread:
 //   1. scores of all clusters on the matrix cores (fp32 accumulation of exact bf16 products), maximum over the q heads;
-//   2. the clusters that can take part are found by a radix select on the top 16 bits of the order-preserving score key,
-//      weighted by cluster size: two rounds of a 256-bin histogram in LDS (sum of sizes per bin), each read from the top
-//      bin down by one wave until k tokens are covered.  Every cluster whose 16-bit key is at or above the pivot is a
-//      candidate: all clusters above the pivot together hold fewer than k tokens, those at the pivot complete them;
-//   3. only the candidates (a few dozen of 1024 for k = 4096) are ordered by (score descending, index ascending): a
-//      counting rank while there are at most 256 of them, the bitonic network otherwise;
-//   4. prefix of the sizes in rank order by one wave, then every output position finds its cluster by binary search.
+//   2. the clusters that can take part are found from one histogram in LDS: 512 equal bins between the largest and the
+//      smallest score, weighted by cluster size, read from the top bin down by one wave until k tokens are covered.  The
+//      bin of a score is a monotone function of it, so all clusters above the pivot bin together hold fewer than k
+//      tokens and those in it complete them: every cluster at or above the pivot bin is a candidate;
+//   3. only the candidates (a few dozen of 1024 for k = 4096) are ordered by (score descending, index ascending): rank and
+//      number of tokens ahead by comparing all pairs while there are at most 256 of them, the bitonic network otherwise;
+//   4. every output position finds its cluster by binary search.
+// Bound by latency: a chain of dependent steps of one workgroup, each run once, so that fetching its instructions counts as
+// much as running them.  4 x 1024 clusters, k = 4096, in us (clock reads in the kernel; in brackets: one workgroup in four scores
+// with a masked maximum per head column, hand-over by fences and an arrival counter, two rounds of 256 bins over the key
+// bits, ranks and prefix in separate passes): scores 2.9 (4.0), hand-over 0.8 (3.1), pivot 1.2 (1.9), order 1.0 (1.5), ids
+// 1.9 (2.0); the kernel 8.8 (14.1).
 constexpr int kSelCount = 256;   // candidates ranked by counting; more go through the bitonic network
+constexpr int kSelBins = 512;
 
-// executed by the 64 lanes of one wave: the highest bin d with (weight of bins above d) < need <= (that + weight of bin d)
-__device__ __forceinline__ void find_pivot(const int32_t* hw, int need, int lane, int& digit, int& above) {
-  int w[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = hw[4 * lane + i];
-  const int s = w[0] + w[1] + w[2] + w[3];
-  int suf = s;                                   // weight of this lane's bins and of all higher lanes'
-  for (int d = 1; d < 64; d <<= 1) {
-    const int v = __shfl_down(suf, d);
-    if (lane + d < 64) suf += v;
-  }
-  const unsigned long long m = __ballot(suf >= need);
-  int dg = -1, ab = 0;
-  if (m != 0) {
-    const int lp = 63 - __builtin_clzll(m);      // suf falls with the lane index: the highest lane that still reaches `need`
-    if (lane == lp) {
-      int cum = suf - s;
-      dg = 4 * lane;
-      ab = cum + w[3] + w[2] + w[1];
-#pragma unroll
-      for (int i = 3; i >= 1; --i) {
-        if (cum + w[i] >= need) {
-          dg = 4 * lane + i;
-          ab = cum;
-          break;
-        }
-        cum += w[i];
-      }
-    }
-    dg = __shfl(dg, lp);
-    ab = __shfl(ab, lp);
-  }
-  digit = dg;    // -1: all bins together hold fewer than `need`
-  above = ab;
+// inclusive sum over the lanes of a wave
+__device__ __forceinline__ int wave_scan_add(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr 1, 2, 4, 8: within 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast 15: into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast 31: into rows 2 and 3
+  return v;
 }
 
-// The score phase pulls a head's whole centroid matrix (256 KB at 1024 clusters) through the one CU its workgroup runs
-// on, which is most of that phase's time.  With kTopkParts workgroups per (sequence, kv head), each scores its share
-// of the clusters into the workspace, and the one that arrives last carries on alone with steps 2 - 4.  Nobody waits
-// for anybody.
+// maximum over the 16 lanes of a row by rotations within the row (DPP row_ror 1, 2, 4, 8): no LDS traffic
+__device__ __forceinline__ float row_max16(float v) {
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false)));
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false)));
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false)));
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false)));
+}
+
+// maximum over the four rows of 16 lanes: lanes 16, 32 and 48 away
+__device__ __forceinline__ float max_of_rows(float v) {
+  const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(y[0]), __uint_as_float(y[1]));
+}
+
+// One CU draws about 36 GB/s from memory: a head's whole centroid matrix (256 KB at 1024 clusters) took one workgroup 7 us.
+// So workgroups of a (sequence, kv head) score a share of its clusters each, into the workspace, and whoever then finds all
+// scores there carries on with steps 2 - 4.  Nobody waits for anybody.
 //
-// The arrival counter of a head is a word in the caller's workspace, so calls that use different workspaces never meet.
-// It needs no initialisation and no reset: the word counts as "k workgroups have arrived" only while it reads
-// kArriveTag | k with 0 < k < parts; anything else -- whatever the memory held before, or the kArriveTag | parts a
-// finished call leaves behind -- counts as zero.  (Only a call that was cut short between two arrivals could leave a
-// live count behind; a launch that dies half-way takes the process's GPU context with it.)
-//
-// Ordering of the hand-over, step by step:
-//   1. every wave that stored scores waits for its own stores to be acknowledged (s_waitcnt vmcnt(0)): they are then
-//      in this XCD's L2, not somewhere between the wave and the L2;
-//   2. the workgroup barrier puts all of that before thread 0's next instruction;
-//   3. thread 0's device-scope fence writes the L2's dirty lines back, which covers every wave's scores of step 1,
-//      and orders them before its atomic on the counter (the atomic executes at device scope);
-//   4. the workgroup that reads parts - 1 earlier arrivals has thread 0 execute a device-scope fence after the atomic
-//      (acquire: stale lines of other XCDs' data leave its L2), then the barrier, and only then the scores are read,
-//      with device-scope loads that go past the CU's vector cache.
-constexpr int kTopkParts = 4;   // divides 16: every part gets whole waves of 64 clusters
-constexpr uint32_t kArriveTag = 0x5A70CB00u;   // low byte: number of arrivals so far
+// A score travels in one 64-bit word with the call's tag (`call_tag` in common.hpp), so finding the words of the call is
+// having its scores: no counter, and no state from before the call that would have to be cleared.
+//   1. the words are stored as device-scope atomics, which write through the storing XCD's L2, and every wave waits for its
+//      own to be acknowledged (s_waitcnt vmcnt(0));
+//   2. behind the workgroup barrier every thread loads one word with a device-scope load, which neither the CU's vector
+//      cache nor its XCD's L2 answers from a line of its own.  The workgroup that passes its barrier last finds all words.
+//      So may one just before it: both then write the same ids;
+//   3. who has written the ids clears the words, so that a replay of the call from a graph, whose tag is the same, does not
+//      take them for its own.  Nobody needs them any more: all parts have stored theirs, and a part that finds some cleared
+//      leaves the ids to whoever cleared them.
+// Waves (of 64 clusters) per workgroup: two, while that makes no more workgroups than there are CUs; beyond it the second
+// workgroup on a CU and the ids written by several of them cost more than the shorter score phase saves.  us for 1024 clusters,
+// k = 4096, shares of 2 / 4 / 16 waves: 4 heads 8.8 / 9.8 / 14.5, 32 heads 9.1 / 9.9 / 14.5, 64 heads 11.7 / 10.2 / 14.6,
+// 128 heads 18.1 / 14.7 / 15.2, 256 heads 28.8 / 23.5 / 17.8; for 512 clusters 4 heads 7.8 / 8.7 / 11.1, 64 heads 8.4 / 9.1 / 11.3.
+inline int topk_share(int64_t G, int waves) {
+  int share = 2;
+  while (share < 16 && G * ((waves + share - 1) / share) > 256) share *= 2;
+  return share;
+}
 
 __global__ __launch_bounds__(1024) void topk_select_kernel(TopkArgs a) {
   __shared__ float sc[1024];
-  __shared__ unsigned long long ckey[1024];
-  __shared__ int32_t pre[1025], rank_cluster[1024], rank_size[1024], hw[256], misc[8];
+  __shared__ __align__(16) unsigned long long ckey[1024];
+  __shared__ __align__(16) int32_t hw[kSelBins];
+  __shared__ __align__(16) int32_t csize[1024];
+  __shared__ int32_t pre[1025], rank_cluster[1024], misc[4];
+  __shared__ float s_ext[2][16];
   const int g = blockIdx.x, t = threadIdx.x, lane = t & 63;
   const int parts = gridDim.y, part = blockIdx.y;
   const int b = g / a.Hkv, kvh = g % a.Hkv;
   const int nh = a.group;
-  if (t < 256) hw[t] = 0;
-  if (t == 0) misc[0] = 0;
   const bool have = t < a.C;
-  const int sz = have ? min(a.size[(int64_t)g * a.C + t], a.M) : 0;   // requested ahead of the score phase
+  unsigned long long* const word = a.scored + (int64_t)g * a.C;
+  int sz = have ? a.size[(int64_t)g * a.C + t] : 0;   // requested ahead of the score phase
   // ---- 1. scores on the matrix cores: wave w takes clusters 64 w .. 64 w + 63 in four blocks of 16; per block
-  // S[cluster, head] = centroids . queries^T on v_mfma_f32_16x16x32_bf16 (the group's q heads padded to 16 columns).
-  // Lane (r = lane % 16, q = lane / 16) feeds centroid row r, columns 32 kk + 8 q .. + 7 as the A operand and the same
-  // columns of query head r as the B operand, and receives S[cluster 4 q + i][head r], i < 4.
-  const int waves_per_part = 16 / parts;
-  if ((t >> 6) < waves_per_part) {
-    const int wave = part * waves_per_part + (t >> 6), r = lane & 15, q4 = lane >> 4;
+  // S[head, cluster] = queries . centroids^T on v_mfma_f32_16x16x32_bf16.  Lane (r = lane % 16, q = lane / 16) feeds query
+  // head r (the group's last one again in the places of rows it does not have, which leaves the maximum what it is),
+  // columns 32 kk + 8 q .. + 7, as the A operand and the same columns of centroid r as the B operand, and receives
+  // S[head 4 q + i][cluster r], i < 4: the maximum over the heads is three in the lane and two exchanges.
+  if ((t >> 6) < a.share) {
+    const int wave = part * a.share + (t >> 6), r = lane & 15, q4 = lane >> 4;
     typedef __attribute__((ext_vector_type(4))) float f32x4;
-    uint4 qf[4];
+    uint4 qf[4], cf[4][4];
     const uint16_t* qp = a.query + (int64_t)b * a.q_sb + (int64_t)(kvh * a.group + min(r, nh - 1)) * a.q_sh + 8 * q4;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) qf[kk] = (r < nh) ? *(const uint4*)(qp + 32 * kk) : make_uint4(0, 0, 0, 0);
+    for (int kk = 0; kk < 4; ++kk) qf[kk] = *(const uint4*)(qp + 32 * kk);
+    // all 20 loads are on their way before the first is used: one trip to memory instead of one per block
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
-      const int c0 = 64 * wave + 16 * blk;
-      const int row = min(c0 + r, a.C - 1);
+      const int row = min(64 * wave + 16 * blk + r, a.C - 1);
       const uint16_t* cp = a.cent + (int64_t)g * a.c_sg + (int64_t)row * a.c_sc + 8 * q4;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) cf[blk][kk] = *(const uint4*)(cp + 32 * kk);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      const int c = 64 * wave + 16 * blk + r;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const uint4 cf = *(const uint4*)(cp + 32 * kk);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, cf), __builtin_bit_cast(bf16x8_t, qf[kk]), acc, 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = (r < nh) ? acc[i] : -INFINITY;   // the padded columns take no part in the maximum over the q heads
-        // maximum over the 16 lanes of a row by rotations within the row (DPP row_ror 1, 2, 4, 8): no LDS traffic
-        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false)));
-        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false)));
-        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false)));
-        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false)));
-        if (r == 0) {
-          if (parts == 1) sc[c0 + 4 * q4 + i] = v;
-          else if (c0 + 4 * q4 + i < a.C) a.score[(int64_t)g * a.C + c0 + 4 * q4 + i] = v;
-        }
+      for (int kk = 0; kk < 4; ++kk)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, qf[kk]), __builtin_bit_cast(bf16x8_t, cf[blk][kk]), acc, 0, 0, 0);
+      const float v = max_of_rows(fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])));
+      if (q4 == 0) {
+        if (parts == 1) sc[c] = v;
+        else if (c < a.C) __hip_atomic_store(word + c, ((unsigned long long)a.tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
+  if (t < kSelBins) hw[t] = 0;
+  if (t < 2) misc[t] = 0;
+  ckey[t] = 0;
+  float s = 0.f;
   if (parts > 1) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // step 1: this wave's score stores have reached the L2
-    __syncthreads();                                    // step 2
-    if (t == 0) {
-      __threadfence();                                  // step 3
-      uint32_t* ctr = a.arrive + g;
-      uint32_t old = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), before;
-      do {
-        before = ((old & ~0xffu) == kArriveTag && (old & 0xffu) < (uint32_t)parts) ? (old & 0xffu) : 0u;
-      } while (!__hip_atomic_compare_exchange_strong(ctr, &old, kArriveTag | (before + 1u), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT));
-      if ((int)before == parts - 1) __threadfence();    // step 4
-      misc[4] = (int)before;
-    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // step 1: this wave's scores have arrived
     __syncthreads();
-    if (misc[4] != parts - 1) return;    // uniform: somebody else finishes the job
-    if (have) sc[t] = __hip_atomic_load(&a.score[(int64_t)g * a.C + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long w = have ? __hip_atomic_load(word + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    if (have && (uint32_t)(w >> 32) != a.tag) misc[1] = 1;
+    __syncthreads();
+    if (misc[1] != 0) return;    // uniform: somebody else finishes the job
+    s = __uint_as_float((uint32_t)w);
+  } else {
+    __syncthreads();
+    if (have) s = sc[t];
+  }
+  sz = min(sz, a.M);
+  s += 0.0f;    // -0.0 counts as +0.0
+  const uint32_t bits = __float_as_uint(s);
+  const uint32_t key32 = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);   // ordered like the scores
+  // ---- 2. histogram between the extremes of the scores (of clusters that hold tokens), weighted by size
+  {
+    const bool in = sz > 0 && s == s;
+    const float hi = max_of_rows(row_max16(in ? s : -INFINITY)), lo = max_of_rows(row_max16(in ? -s : -INFINITY));
+    if (lane == 0) {
+      s_ext[0][t >> 6] = hi;
+      s_ext[1][t >> 6] = lo;
+    }
   }
   __syncthreads();
-  uint32_t key32 = 0;
-  if (have) {
-    const uint32_t bits = __float_as_uint(sc[t] + 0.0f);    // -0.0 counts as +0.0
-    key32 = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
+  const float top = row_max16(s_ext[0][lane & 15]), bottom = -row_max16(s_ext[1][lane & 15]);
+  // Equal steps of the score.  Where the range is not a positive finite number (equal scores, infinities, nothing to
+  // select) every cluster is in bin 0, i.e. a candidate.  A NaN goes where its key is: above everything, or below.
+  const float range = top - bottom;
+  int bin = 0;
+  if (range > 0.f && range < INFINITY) {
+    const float x = (top - s) * ((float)(kSelBins - 1) / range);   // a range too small for the quotient: infinite or NaN, bin 0 or the last
+    bin = s == s ? (int)fminf(x, (float)(kSelBins - 1)) : (key32 >> 31 ? 0 : kSelBins - 1);
   }
-  // ---- 2. radix select over the top 16 key bits, weighted by size
-  if (sz > 0) atomicAdd(&hw[key32 >> 24], sz);
+  if (sz > 0) atomicAdd(&hw[bin], sz);
   __syncthreads();
   if (t < 64) {
-    int d1, ab1;
-    find_pivot(hw, a.k, lane, d1, ab1);
-    if (t == 0) {
-      misc[1] = d1;
-      misc[2] = ab1;
+    constexpr int per = kSelBins / 64;
+    int w[per], sum = 0;
+#pragma unroll
+    for (int i = 0; i < per; ++i) {
+      w[i] = hw[per * lane + i];
+      sum += w[i];
     }
+    const int inc = wave_scan_add(sum);
+    const unsigned long long m = __ballot(inc >= a.k);
+    int pivot = kSelBins - 1;             // fewer than k tokens in all: everything
+    if (m != 0) {
+      const int lp = __ffsll((long long)m) - 1;
+      int cum = inc - sum, at = per * lane;
+#pragma unroll
+      for (int i = 0; i < per; ++i) {
+        cum += w[i];
+        at += cum < a.k ? 1 : 0;
+      }
+      pivot = __builtin_amdgcn_readlane(at, lp);
+    }
+    if (t == 0) misc[2] = pivot;
   }
   __syncthreads();
-  const int d1 = misc[1], above1 = misc[2];
-  if (t < 256) hw[t] = 0;
-  __syncthreads();
-  if (sz > 0 && d1 >= 0 && (int)(key32 >> 24) == d1) atomicAdd(&hw[(key32 >> 16) & 255], sz);
-  __syncthreads();
-  if (t < 64 && d1 >= 0) {
-    int d2, ab2;
-    find_pivot(hw, a.k - above1, lane, d2, ab2);   // bin d1 holds at least k - above1 tokens, so d2 >= 0
-    if (t == 0) misc[3] = d2;
-  }
-  __syncthreads();
-  const uint32_t pivot16 = d1 >= 0 ? (((uint32_t)d1 << 8) | (uint32_t)misc[3]) : 0u;   // fewer than k tokens in all: everything
   // ---- 3. candidates and their order
-  if (sz > 0 && (key32 >> 16) >= pivot16) {
+  if (sz > 0 && bin <= misc[2]) {
     const int pos = atomicAdd(&misc[0], 1);
     ckey[pos] = ((unsigned long long)key32 << 32) | (0xffffffffu - (uint32_t)t);
-    rank_size[pos] = sz;    // by candidate slot for now
+    csize[pos] = sz;
   }
   __syncthreads();
   const int m = misc[0];
-  int my_rank = -1, my_cluster = 0, my_size = 0;
   if (m <= kSelCount) {
     if (t < m) {
       const unsigned long long mine = ckey[t];
-      int r = 0;
-      for (int j = 0; j < m; ++j) r += ckey[j] > mine;
-      my_rank = r;
-      my_cluster = (int)(0xffffffffu - (uint32_t)mine);
-      my_size = rank_size[t];
+      int rank = 0, ahead = 0;
+      // four candidates a round, read whether they count or not (places behind the last hold key 0, which never does)
+      for (int j = 0; j < m; j += 4) {
+        unsigned long long k4[4];
+        int z4[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          k4[i] = ckey[j + i];
+          z4[i] = csize[j + i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool before = k4[i] > mine;
+          rank += before ? 1 : 0;
+          ahead += before ? z4[i] : 0;
+        }
+      }
+      rank_cluster[rank] = (int)(0xffffffffu - (uint32_t)mine);
+      pre[rank] = ahead;
+      if (rank == m - 1) pre[m] = ahead + csize[t];
     }
-    __syncthreads();
-    if (my_rank >= 0) {
-      rank_cluster[my_rank] = my_cluster;
-      rank_size[my_rank] = my_size;
-    }
+    if (m == 0 && t == 0) pre[0] = 0;
   } else {
     int P = 1;
     while (P < m) P <<= 1;
-    if (t >= m && t < P) ckey[t] = 0;            // padding sorts behind every candidate
-    __syncthreads();
+    // (the places behind the last candidate hold key 0, which sorts behind every candidate)
     for (int len = 2; len <= P; len <<= 1)
       for (int d = len >> 1; d > 0; d >>= 1) {
         if (t < P / 2) {
@@ -1033,34 +1058,31 @@ __global__ __launch_bounds__(1024) void topk_select_kernel(TopkArgs a) {
     if (t < m) {
       const int c = (int)(0xffffffffu - (uint32_t)ckey[t]);
       rank_cluster[t] = c;
-      rank_size[t] = min(a.size[(int64_t)g * a.C + c], a.M);
+      csize[t] = min(a.size[(int64_t)g * a.C + c], a.M);
     }
-  }
-  __syncthreads();
-  // ---- 4. exclusive prefix of the sizes in rank order (one wave), then the token ids
-  if (t < 64) {
-    const int per = (m + 63) / 64;
-    int run = 0;
-    for (int i = 0; i < per; ++i) {
-      const int r = lane * per + i;
-      if (r < m) run += rank_size[r];
-    }
-    int inc = run;
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(inc, d);
-      if (lane >= d) inc += v;
-    }
-    int acc = inc - run;
-    for (int i = 0; i < per; ++i) {
-      const int r = lane * per + i;
-      if (r < m) {
-        pre[r] = acc;
-        acc += rank_size[r];
+    __syncthreads();
+    // exclusive prefix of the sizes in rank order (one wave)
+    if (t < 64) {
+      const int per = (m + 63) / 64;
+      int run = 0;
+      for (int i = 0; i < per; ++i) {
+        const int r = lane * per + i;
+        if (r < m) run += csize[r];
       }
+      const int inc = wave_scan_add(run);
+      int acc = inc - run;
+      for (int i = 0; i < per; ++i) {
+        const int r = lane * per + i;
+        if (r < m) {
+          pre[r] = acc;
+          acc += csize[r];
+        }
+      }
+      if (lane == 63) pre[m] = inc;
     }
-    if (lane == 63) pre[m] = inc;
   }
   __syncthreads();
+  // ---- 4. the token ids
   const int total = pre[m];
   int32_t* out = a.out + (int64_t)g * a.out_sg;
   constexpr int U = 4;   // positions per thread and round: their table reads are independent and overlap
@@ -1087,6 +1109,7 @@ __global__ __launch_bounds__(1024) void topk_select_kernel(TopkArgs a) {
     for (int u = 0; u < U; ++u)
       if (p0 + u * 1024 < a.k) out[p0 + u * 1024] = id[u];
   }
+  if (parts > 1 && have) __hip_atomic_store(word + t, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 struct WsLayout {
@@ -1400,7 +1423,8 @@ extern "C" int sq_topk_select(const DLTensor* query, const DLTensor* centroids, 
   a.out_sg = stride_of(out, 0);
   a.score = (float*)(wsp + w.off_bytes + w.hist_bytes + w.order_bytes);
   a.start = (int32_t*)(wsp + w.off_bytes + w.hist_bytes + w.order_bytes + w.score_bytes);
-  a.arrive = (uint32_t*)a.start;   // the one-launch path does not use `start`
+  a.scored = (unsigned long long*)a.score;   // `start` follows `score`
+  a.tag = 0;
   a.q_sb = stride_of(query, 0);
   a.q_sh = stride_of(query, 1);
   a.c_sg = stride_of(centroids, 0);
@@ -1413,7 +1437,10 @@ extern "C" int sq_topk_select(const DLTensor* query, const DLTensor* centroids, 
   a.Hkv = (int)Hkv;
   a.group = num_kv_groups;
   if (C <= 1024 && num_kv_groups <= 16) {   // one launch, only the clusters that can fill k are ordered
-    const unsigned parts = (C >= 64 * 16) ? kTopkParts : 1;   // fewer clusters: not worth sharing
+    const int waves = (int)((C + 63) / 64);
+    a.share = topk_share(G, waves);
+    const unsigned parts = (unsigned)((waves + a.share - 1) / a.share);
+    if (parts > 1) a.tag = call_tag();
     hipLaunchKernelGGL(topk_select_kernel, dim3((unsigned)G, parts), dim3(1024), 0, st, a);
     SQ_HIP(hipGetLastError());
     return SQ_OK;

@@ -218,6 +218,76 @@ def test_topk_select_arrival_words_need_no_initialisation(fill):
         assert torch.equal(got.cpu(), want)
 
 
+@pytest.mark.parametrize("C", [64, 1000, 1024])
+@pytest.mark.parametrize("pattern", ["equal", "outlier", "binades", "infinite", "zeros", "falling"])
+def test_topk_select_score_patterns(pattern, C):
+    """Scores that strain the histogram between the extremes: all equal, one far above the rest, a range of 2^60, infinities
+    (no finite range), +0 beside -0, and one value per bin.  The scores are exact, so the ids are the oracle's, bit for bit."""
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import topk_select
+
+    print(f"case topk pattern {pattern} C={C}", flush=True)
+    g = torch.Generator().manual_seed(7 * C + len(pattern))
+    B, groups, Hkv = 1, 3, 2
+    G = B * Hkv
+    x = torch.randn(G, C, generator=g)
+    if pattern == "equal":
+        x.fill_(1.5)
+    elif pattern == "outlier":
+        x[:, C // 3] = 1e30
+    elif pattern == "binades":
+        x = torch.sign(x) * torch.exp2(torch.randint(-30, 31, (G, C), generator=g).float())
+    elif pattern == "infinite":
+        x[:, ::7] = float("inf")
+        x[:, 3::11] = float("-inf")
+    elif pattern == "zeros":
+        x = torch.where(x > 0.5, x, torch.where(x > 0, 0.0, -0.0))
+    else:
+        x = (C - torch.arange(C).float()).expand(G, C)
+    cent = torch.zeros(G, C, 128)
+    cent[..., 0] = x
+    q = torch.zeros(B, Hkv * groups, 128)
+    q[..., 0] = 1.0
+    cent, q = cent.bfloat16(), q.bfloat16()
+    size = torch.randint(0, 40, (G, C), generator=g, dtype=torch.int32)   # empty clusters among them
+    clusters = torch.randint(0, 100000, (G, C, 40), generator=g, dtype=torch.int32)
+    total = int(size.sum(dim=1).max())
+    for k in (1, 511, total // 2, total + 9):
+        got = topk_select(q.to(DEV), cent.to(DEV), clusters.to(DEV), size.to(DEV), k, groups)
+        assert torch.equal(got.cpu(), KM.topk_select(q, cent, clusters, size, k, groups)), k
+
+
+@pytest.mark.parametrize("B", [1, 16, 25, 80])
+def test_topk_select_replayed_from_a_graph(B):
+    """4 B heads share the score phase two, four, eight or sixteen waves a workgroup.  One captured call, replayed over another
+    query each time, with the workspace as the replay before left it and overwritten in between: the oracle's ids every time."""
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _workspace, topk_select
+
+    print(f"case topk graph B={B}", flush=True)
+    Hkv, groups, C, M, k = 4, 2, 1024, 8, 37
+    G = B * Hkv
+    g = torch.Generator().manual_seed(B)
+    size = torch.randint(0, M + 1, (G, C), generator=g, dtype=torch.int32)
+    clusters = torch.randint(0, 100000, (G, C, M), generator=g, dtype=torch.int32)
+    cent = torch.randn(G, C, 128, generator=g).bfloat16()
+    qs = [torch.randn(B, Hkv * groups, 128, generator=g).bfloat16() for _ in range(4)]
+    dq, dc, dcl, dsz = qs[0].to(DEV), cent.to(DEV), clusters.to(DEV), size.to(DEV)
+    ws = _workspace(G, 1, C, DEV)
+    out = torch.empty(G, k, dtype=torch.int32, device=DEV)
+    topk_select(dq, dc, dcl, dsz, k, groups, out=out, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        topk_select(dq, dc, dcl, dsz, k, groups, out=out, workspace=ws)
+    for i, q in enumerate(qs):
+        dq.copy_(q)
+        if i == 2:
+            ws.view(torch.int32).random_()
+        out.fill_(-7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu(), KM.topk_select(q, cent, clusters, size, k, groups)), i
+
+
 def test_topk_select_two_workspaces_on_two_streams():
     """Calls that use different workspaces share nothing: two selections with different queries run on two streams at
     the same time, 200 times, and each must equal its own oracle result."""
