@@ -412,6 +412,87 @@ constexpr int kCombineThreads = 1024;
 constexpr int kCombineChunk = 32;                       // output channels per workgroup
 constexpr int kCombineGroups = kCombineThreads / kCombineChunk;   // 32 groups of 32 threads, each sums every 32nd split
 
+__device__ __forceinline__ void store_elem(void* out, int out_dtype, int64_t off, float o) {
+  if (out_dtype == 0) {
+    ((uint16_t*)out)[off] = (uint16_t)f32_to_bf16_bits(o);
+  } else if (out_dtype == 1) {
+    ((_Float16*)out)[off] = (_Float16)o;
+  } else {
+    ((float*)out)[off] = o;
+  }
+}
+
+// The same sums by a workgroup of four waves per (q head, batch, 64 output channels).  Its additions are those of the kernel
+// below in the same order -- 32 chains, chain q over splits q, q + 32, ..., then the chains in order; the denominators by
+// the same shuffles, 64 splits at a time -- so the two give the same bits (up to kFewSplits splits, where that kernel
+// leaves its first eight rounds) and which of them runs may depend on the batch.  Wave v holds chains 8 v .. 8 v + 7, forms
+// the weights for itself, and meets the others once, for the sum over the chains.
+constexpr int kFewSplits = 256;
+__global__ __launch_bounds__(256) void decode_combine_few_kernel(CombineArgs a) {
+  __shared__ float s_chain[32][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.x >> 1, b = blockIdx.y;
+  int S = a.num_splits;
+  int64_t row0 = ((int64_t)b * a.Hq + h) * S;
+  if (a.by_length) {
+    const int W = a.B * a.num_splits;
+    int bb, base;
+    share_of(a.seqlens, a.B, a.L, W, b, 0, bb, base, S);
+    S = __builtin_amdgcn_readfirstlane(S);
+    row0 = (int64_t)h * W + __builtin_amdgcn_readfirstlane(base);
+  }
+  const int d = 64 * (blockIdx.x & 1) + lane;
+  const float* po = a.part_o + row0 * kD + d;
+  constexpr int C = kFewSplits / 64;
+  float x[2][8], w[C], acc[8] = {};
+  auto fetch = [&](int j, float (&y)[8]) __attribute__((always_inline)) {   // round j of this wave's chains
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int s = 32 * j + 8 * wave + q;
+      y[q] = s < S ? po[(int64_t)s * kD] : 0.f;
+    }
+  };
+#pragma unroll
+  for (int c = 0; c < C; ++c) w[c] = lane + 64 * c < S ? a.part_lse[row0 + lane + 64 * c] : -INFINITY;
+  fetch(0, x[0]);
+  fetch(1, x[1]);
+  float mx = -INFINITY;
+#pragma unroll
+  for (int c = 0; c < C; ++c) mx = fmaxf(mx, w[c]);
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m));
+  float tot = 0.f;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if (64 * c >= S) break;
+    w[c] = (mx > -INFINITY) ? exp2f(w[c] - mx) : 0.f;
+    float t = w[c];
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) t += __shfl_xor(t, m);
+    tot += t;
+  }
+#pragma unroll
+  for (int j = 0; j < 2 * C; j += 2) {
+    if (32 * j >= S) break;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[j >> 1]), 32 * i + 8 * wave + q)) * x[i][q];
+      fetch(j + 2 + i, x[i]);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) s_chain[8 * wave + q][lane] = acc[q];
+  __syncthreads();
+  if (wave != 0) return;
+  float o = 0.f;
+#pragma unroll
+  for (int q = 0; q < 32; ++q) o += s_chain[q][lane];
+  o = (tot > 0.f) ? o / tot : 0.f;
+  store_elem(a.out, a.out_dtype, (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + d, o);
+  if (a.lse && d == 0) a.lse[(int64_t)b * a.Hq + h] = (tot > 0.f) ? mx + log2f(tot) : -INFINITY;
+}
+
 // One workgroup per (q head, batch, 32 output channels): 32 groups of 32 threads (one thread per channel), each sums
 // every 32nd split.  A thread's first eight partial outputs are requested before anything else, so that they travel while
 // the weights of the splits are formed (maximum and sum of 2^(lse - max): one shuffle reduction per wave, the 16 wave
@@ -477,14 +558,7 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(Combine
 #pragma unroll
     for (int q = 0; q < G; ++q) o += s_part[q * kCombineChunk + dl];
     o = (tot > 0.f) ? o / tot : 0.f;
-    const int64_t off = (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + d;
-    if (a.out_dtype == 0) {
-      ((uint16_t*)a.out)[off] = (uint16_t)f32_to_bf16_bits(o);
-    } else if (a.out_dtype == 1) {
-      ((_Float16*)a.out)[off] = (_Float16)o;
-    } else {
-      ((float*)a.out)[off] = o;
-    }
+    store_elem(a.out, a.out_dtype, (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + d, o);
     if (a.lse && d == 0) a.lse[(int64_t)b * a.Hq + h] = (tot > 0.f) ? mx + log2f(tot) : -INFINITY;
   }
 }
@@ -667,8 +741,18 @@ static int decode_impl(const DLTensor* q, const DLTensor* kcache, const DLTensor
   c.L = (int32_t)L;
   c.by_length = a.by_length;
   const size_t max_slots = a.by_length ? (size_t)B * S : (size_t)S;   // a sequence may own up to all of a head's workgroups
-  hipLaunchKernelGGL(decode_combine_kernel, dim3((unsigned)Hq, (unsigned)B, kD / kCombineChunk), dim3(kCombineThreads),
-                     (max_slots + kCombineGroups * kCombineChunk) * sizeof(float), st, c);
+  // Few splits: 1024 threads a workgroup are mostly idle, and with many rows (q heads x sequences) their workgroups no longer fit
+  // the chip at once.  us per call, split and combine kernel, 1024 threads / four waves: 32 / 8 heads, batch 16, 200 tokens 19.5 / 11.5,
+  // 4096 tokens 58.3 / 47.7; 28 / 4 heads, batch 8, 96K to 128K tokens 298 / 279; batch 4, 16384 tokens (64 splits) 32.1 / 29.8; one
+  // sequence with 13 splits 8.1 / 7.9, with 96 9.2 / 9.8, with 256 11.2 / 13.1: up to 64.  Where the splits go by length one
+  // sequence may own nearly all: that costs up to 1.6 us against the wide workgroups when they all fit (64 rows, 241 slots:
+  // 11.1 / 12.7), nothing when they do not (224 rows: 18.1 / 15.3).
+  const bool few = S <= 64 && (max_slots <= 64 || (max_slots <= kFewSplits && B * Hq >= 128));
+  if (few)
+    hipLaunchKernelGGL(decode_combine_few_kernel, dim3((unsigned)(2 * Hq), (unsigned)B), dim3(256), 0, st, c);
+  else
+    hipLaunchKernelGGL(decode_combine_kernel, dim3((unsigned)Hq, (unsigned)B, kD / kCombineChunk), dim3(kCombineThreads),
+                       (max_slots + kCombineGroups * kCombineChunk) * sizeof(float), st, c);
   SQ_HIP(hipGetLastError());
   return SQ_OK;
 }

@@ -79,6 +79,28 @@ def test_decode_workgroups_dealt_by_length(lens):
         assert torch.allclose(lse[b].double(), lse_ref[b, :, 0], atol=2e-4)
 
 
+@pytest.mark.parametrize("B,lens", [(1, [2600]), (8, [2600] * 8), (8, [2600, 1, 0, 700, 2600, 33, 64, 2599]), (16, [2600] + [1] * 15)])
+@pytest.mark.parametrize("splits", [0, 1, 2, 31, 32, 33, 63, 64, 65])
+def test_decode_combine_of_few_and_of_many_splits(B, lens, splits):
+    """Both combine kernels at the edges of their rounds (32 chains, 64 weights) and of the choice between them (64 splits): closed
+    form, and for a named count the bits of a sequence do not depend on its batch mates, whichever kernel the batch takes."""
+    print(f"case decode combine B={B} splits={splits} lens={lens}", flush=True)
+    q, kc, vc, _ = inputs.decode_inputs(B, 28, 4, 2600, 128, seed=91)
+    qh, kh, vh = _to_hnd(q, kc, vc)
+    ref, lse_ref = A.exact_attention(A.fold_scale(qh, 128), kh, vh, causal=False, kv_lens=[max(n, 1) for n in lens], score_scale=math.log(2.0))
+    out, lse = (t.cpu() for t in _run(q, kc, vc, lens, "NHD", output_dtype=torch.float32, return_lse=True, num_splits=splits))
+    rms = float(ref.pow(2).mean().sqrt())
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert float(out[b].abs().max()) == 0.0 and bool(torch.isinf(lse[b]).all())
+            continue
+        assert float((out[b, 0].double() - ref[b, :, 0]).abs().max()) < 2e-4 * rms + 1e-6, b   # as test_decode_matches_closed_form
+        assert torch.allclose(lse[b, :, 0].double(), lse_ref[b, :, 0], atol=2e-4), b
+    if splits:
+        alone = _run(q[:1], kc[:1], vc[:1], lens[:1], "NHD", output_dtype=torch.float32, num_splits=splits).cpu()
+        assert torch.equal(alone[0], out[0])
+
+
 def test_decode_by_length_replayed_from_a_graph_with_changing_lengths():
     """The length-proportional dealing is computed on the device from `seqlens`, so a captured launch follows the
     lengths it finds at replay time: one graph, four sets of lengths written between the replays (with eager work in
