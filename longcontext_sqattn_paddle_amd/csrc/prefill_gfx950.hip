@@ -332,49 +332,21 @@ __device__ __forceinline__ float xor32_sum(float v) {
 
 constexpr float kLog2_448 = 8.807354922057604f;  // log2(448)
 
-// Quantise 8 probabilities (one k-step of the P.V MFMA) and pack them as fp16 B-operand registers.
+// Eight probabilities (one k-step of the P.V MFMA) as fp16 B-operand registers
+__device__ __forceinline__ uint4 pack8(const f32x16_t& s, int t) {
+  return make_uint4(pack_f16(s[8 * t], s[8 * t + 1]), pack_f16(s[8 * t + 2], s[8 * t + 3]), pack_f16(s[8 * t + 4], s[8 * t + 5]), pack_f16(s[8 * t + 6], s[8 * t + 7]));
+}
+
+// Quantise four probabilities and pack them as two fp16 B-operand words.
 //   MODE 0  p.to(fp16)
 //   MODE 1  fp16(e4m3(p*448)/448)   reference static scale (attn_triton.py:81-82): sc = 448, inv = 1/448
 //   MODE 2  fp16(e4m3(p*sc)*inv)    block absmax scale a: sc = 448/a, inv = a/448
 //   MODE 3  fp16(e4m3(p448))        p448 = 448*p, the factor folded into the exponent; the 1/448 cancels in
 //                                   acc/l because l is accumulated from p448 as well
+// MODE 2's largest product rounds to 448 (the block's maximum times 448 / maximum is within two units in the last place of it), so
+// nothing has to be clamped.
 template <int MODE>
-__device__ __forceinline__ uint4 quant_pack8(const f32x16_t& s, int t, float sc, float inv) {
-  uint32_t w[4];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const float p0 = s[8 * t + 4 * h + 0], p1 = s[8 * t + 4 * h + 1], p2 = s[8 * t + 4 * h + 2], p3 = s[8 * t + 4 * h + 3];
-    if constexpr (MODE == 0) {
-      w[2 * h] = pack_f16(p0, p1);
-      w[2 * h + 1] = pack_f16(p2, p3);
-    } else if constexpr (MODE == 3) {
-      int pk = __builtin_amdgcn_cvt_pk_fp8_f32(p0, p1, 0, false);
-      pk = __builtin_amdgcn_cvt_pk_fp8_f32(p2, p3, pk, true);
-      w[2 * h] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pk, 1.0f, false));
-      w[2 * h + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pk, 1.0f, true));
-    } else {
-      float q0 = p0 * sc, q1 = p1 * sc, q2 = p2 * sc, q3 = p3 * sc;
-      if constexpr (MODE == 2) {
-        q0 = fminf(q0, 448.f);
-        q1 = fminf(q1, 448.f);
-        q2 = fminf(q2, 448.f);
-        q3 = fminf(q3, 448.f);
-      }
-      int pk = __builtin_amdgcn_cvt_pk_fp8_f32(q0, q1, 0, false);
-      pk = __builtin_amdgcn_cvt_pk_fp8_f32(q2, q3, pk, true);
-      typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-      const f32x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(pk, 1.0f, false);
-      const f32x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(pk, 1.0f, true);
-      w[2 * h] = pack_f16(lo[0] * inv, lo[1] * inv);
-      w[2 * h + 1] = pack_f16(hi[0] * inv, hi[1] * inv);
-    }
-  }
-  return make_uint4(w[0], w[1], w[2], w[3]);
-}
-
-// Four probabilities -> two fp16 B-operand words, MODE as in quant_pack8 (0, 1 or 3)
-template <int MODE>
-__device__ __forceinline__ void quant_pack4(float p0, float p1, float p2, float p3, uint32_t& w0, uint32_t& w1) {
+__device__ __forceinline__ void quant_pack4(float p0, float p1, float p2, float p3, uint32_t& w0, uint32_t& w1, float sc = 448.f, float inv = 1.0f / 448.0f) {
   if constexpr (MODE == 0) {
     w0 = pack_f16(p0, p1);
     w1 = pack_f16(p2, p3);
@@ -384,12 +356,11 @@ __device__ __forceinline__ void quant_pack4(float p0, float p1, float p2, float 
     w0 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pk, 1.0f, false));
     w1 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(pk, 1.0f, true));
   } else {
-    int pk = __builtin_amdgcn_cvt_pk_fp8_f32(p0 * 448.f, p1 * 448.f, 0, false);
-    pk = __builtin_amdgcn_cvt_pk_fp8_f32(p2 * 448.f, p3 * 448.f, pk, true);
+    int pk = __builtin_amdgcn_cvt_pk_fp8_f32(p0 * sc, p1 * sc, 0, false);
+    pk = __builtin_amdgcn_cvt_pk_fp8_f32(p2 * sc, p3 * sc, pk, true);
     typedef __attribute__((ext_vector_type(2))) float f32x2_t;
     const f32x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(pk, 1.0f, false);
     const f32x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(pk, 1.0f, true);
-    constexpr float inv = 1.0f / 448.0f;
     w0 = pack_f16(lo[0] * inv, lo[1] * inv);
     w1 = pack_f16(hi[0] * inv, hi[1] * inv);
   }
@@ -415,7 +386,7 @@ __device__ __forceinline__ void store_out4(const PrefillArgs& a, int64_t ch, int
 }
 
 // One workgroup = WAVES waves x 32 query rows of one q-head (2 waves per SIMD when WAVES == 8, so that one
-// wave's MFMA phase overlaps the other's softmax phase).  MODE as in quant_pack8.
+// wave's MFMA phase overlaps the other's softmax phase).  MODE as in quant_pack4.
 // DUAL (WAVES == 8, absolute windows with their own 4-bit operands, block_m == 128): the workgroup holds two query blocks,
 // A = waves 0..3 and B = waves 4..7, whose 4-bit ranges end 128 keys apart.  On the up to two tiles in between -- 8-bit
 // for A, 4-bit for B -- the blocks want different K tiles, so those tiles are walked twice: once as they are (B skips
@@ -428,18 +399,19 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   // MODE 6: Q.K^T on the int8 matrix instruction -- `k` holds the 8-bit codes of the (centred) key, one byte per element,
   // `k_scale` their per-token scales; the query rows' codes and scale are formed here as the rows are loaded.  The scores
   // are sum(code products) x scale_k x (scale_q log2e / sqrt(D)); from there on the step is MODE 0's (fp16 P, fp16 V), on
-  // the plain schedule MODE 2 also uses (no hand-placed slots).
+  // the plain schedule (no hand-placed slots).
   constexpr bool kQK8 = MODE == 6;
   // MODE 7: no output, only the row maxima of a part's scores, from which the later parts of the row take the reference
   // point the running maximum would have there (the modes whose e4m3 grid is tied to it).
   constexpr bool kRefPass = MODE == 7;
-  constexpr bool kPlain = MODE == 2 || MODE == 6 || kRefPass;   // tile step left to the compiler's scheduling
+  constexpr bool kPlain = MODE == 6 || kRefPass;   // tile step left to the compiler's scheduling
   constexpr bool kPV8 = MODE == 4 || MODE == 5;     // e4m3 V tiles, fp8 P.V
   constexpr bool kOwn4 = WAVES == 2 || DUAL;        // the launches that can have their own 4-bit operands
   constexpr bool kFirstRef = SPLIT && (MODE == 0 || MODE == 6);   // parts that take their reference point from the row's first tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // MODE 2: tile maxima of the two waves of a 64-row group, behind the tile rings (which start at LDS address 0)
-  float (*s_amax)[WAVES] = (float (*)[WAVES])(smem + 4 * kStageBytes);
+  // MODE 2: highest scores (relative to the rows' reference points) of a tile over the rows of each wave, for two tiles in turn,
+  // behind the tile rings
+  constexpr uint32_t kTopOff = 4 * kStageBytes;
 
   // ---- schedule: blockIdx -> (pair = (b, kvh), item = (q block descending, head in group))
   int pair, item;
@@ -872,6 +844,17 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     pend_t = -1;
   };
 
+  // MODE 2: this wave's share of a tile's highest score, and the share of the other wave of its 64 rows (slot: tile's parity)
+  const uint32_t top_addr = smem_addr + kTopOff + 4 * (uint32_t)wave;
+  auto post_top = [&](int slot, float top) __attribute__((always_inline)) {
+    if (lane == 0) asm volatile("ds_write_b32 %0, %1" ::"v"(top_addr + 4 * WAVES * slot), "v"(top) : "memory");
+  };
+  auto read_top = [&](int slot) __attribute__((always_inline)) {
+    float r;
+    asm volatile("ds_read_b32 %0, %1" : "=v"(r) : "v"((WAVES > 1 ? top_addr ^ 4u : top_addr) + 4 * WAVES * slot));
+    return r;
+  };
+
   // softmax update + P.V for the tile whose scores are in S.  Once the running maximum of this tile is settled,
   // the Q.K^T MFMAs of the following tile (K in knext, result in Snext) are issued in the same straight-line
   // block as the exponentials, conversions and P.V MFMAs, so that the matrix pipe and the vector ALU of this
@@ -928,12 +911,15 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
       tmax = xor32_max(tmax);
       slow = first || __any(tmax > kMove);
     }
+    float my_top = 0.f;
+    float row_top = tmax;   // MODE 2: the row's highest score relative to its reference point
     if (slow) {
       // some row's maximum moved by d (on the first tile: from the arbitrary reference 0 to the row maximum):
       // shift the scores, rescale the accumulators, re-centre the accumulator initialiser
       asm volatile("; new row maximum" ::: "memory");
       const float d = first ? (tmax - kC) : ((tmax > kMove) ? tmax - kC : 0.f);
       const float alpha = first ? 0.f : __builtin_amdgcn_exp2f(-d);
+      row_top = tmax - d;
       m_run += d;
       l_run *= alpha;
 #pragma unroll
@@ -1189,7 +1175,23 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
       __builtin_amdgcn_s_setprio(3);
       return;
     }
-    if constexpr (MODE == 0 || MODE == 1 || MODE == 3) {
+    if constexpr (MODE == 0 || MODE == 1 || MODE == 2 || MODE == 3) {
+      if constexpr (MODE == 2) {
+        // The largest probability of the 64-row block (this wave's rows and those of wave ^ 1) is 2^(its highest score): the
+        // row maxima are there already, so the block's scale is known before the first exponential.  This wave's share goes to
+        // LDS now, the other's is read behind a barrier in the Q.K^T slots.  A score of +inf leaves NaN behind, which drops out.
+        // (Bound by vector work, 1.05 x MODE 1's.  With the maximum taken over the exponentiated probabilities and the step left to
+        // the compiler's schedule: 32768 tokens, 28 / 4 heads 9.61 -> 7.55 ms, a tile of an 8-wave workgroup 2.6 -> 2.05 us,
+        // 777 tokens 39.0 -> 30.6 us.  Barrier two slots earlier, or vector work in front of the MFMA: the same within 0.5 %.)
+        float top = (row_w0 + c32 < a.Nq) ? row_top : -INFINITY;   // rows past the end are clamped copies, not part of the block
+        top = fmaxf(top, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(top), 0x121, 0xf, 0xf, false)));
+        top = fmaxf(top, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(top), 0x122, 0xf, 0xf, false)));
+        top = fmaxf(top, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(top), 0x124, 0xf, 0xf, false)));
+        top = fmaxf(top, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(top), 0x128, 0xf, 0xf, false)));
+        const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(top), __float_as_uint(top), false, false);
+        my_top = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+        post_top(R & 1, my_top);
+      }
       // Hand-scheduled tile step, fp16 P.V: 16 slots of {Q.K^T MFMA of the next tile, one LDS prefetch, two
       // exponentials, and every other slot the conversion of four finished probabilities}, then 16 slots of
       // {P.V MFMA, one LDS prefetch, two additions of the row sum, later two steps of the next tile's row maximum}.
@@ -1202,6 +1204,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
       const uint32_t vlane = smem_addr + 4 * kKTileBytes + (it & 3) * kVTileBytes + c32 * kVStride + ((g ^ vsw) << 4);
       u32x4_t vf[16];
       uint32_t Pw[4][4];
+      float p_sc = 448.f, p_inv = 1.0f / 448.0f, other_top = 0.f;
       auto vread = [&](auto I) {
         constexpr int sl = decltype(I)::value;
         if constexpr (kStaticRing) vf[sl] = lds_read128<R * kVTileBytes + (sl & 3) * 32 * kVStride>(vxr[sl >> 2]);
@@ -1211,12 +1214,15 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
         constexpr int u = decltype(U)::value;
         const f32x16_t& sv = S[u >> 2];
         constexpr int o = 4 * (u & 3);
-        quant_pack4<MODE>(sv[o], sv[o + 1], sv[o + 2], sv[o + 3], Pw[u >> 1][2 * (u & 1)], Pw[u >> 1][2 * (u & 1) + 1]);
+        quant_pack4<MODE>(sv[o], sv[o + 1], sv[o + 2], sv[o + 3], Pw[u >> 1][2 * (u & 1)], Pw[u >> 1][2 * (u & 1) + 1], p_sc, p_inv);
       };
       static_for<0, 16>([&](auto I) {
         constexpr int i = decltype(I)::value;
         constexpr int bn = i & 1, kk = i >> 1;
-        lds_wait<kDepth - 1>(kf[i]);
+        // (MODE 2's read of the other wave's share is one more request between slots 6 and 7: the waits there are one request
+        // stricter than they need to be, and the one of slot 8 covers it)
+        if constexpr (MODE == 2 && i == 8) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(kf[i]), "+v"(other_top) : "n"(kDepth - 1));
+        else lds_wait<kDepth - 1>(kf[i]);
         __builtin_amdgcn_sched_barrier(0);
         const uint4 ka = make_uint4(kf[i][0], kf[i][1], kf[i][2], kf[i][3]);
         if constexpr (kk == 0) Snext[bn] = mfma_qk32<BF16>(ka, qf[0], Cinit);
@@ -1225,10 +1231,32 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
         if constexpr (i + kDepth < 16) kread(std::integral_constant<int, i + kDepth>{});
         else vread(std::integral_constant<int, i + kDepth - 16>{});
         __builtin_amdgcn_sched_barrier(0);
-        constexpr int sb = i >> 3, e = 2 * (i & 7);
-        S[sb][e] = __builtin_amdgcn_exp2f(S[sb][e]);
-        S[sb][e + 1] = __builtin_amdgcn_exp2f(S[sb][e + 1]);
-        if constexpr (i >= 2 && (i & 1) == 0) pack_unit(std::integral_constant<int, (i - 2) / 2>{});
+        if constexpr (MODE == 2) {
+          if constexpr (i == 6) {
+            // the write of this wave's share is older than the K fragments this wave has already waited for
+            asm volatile("s_barrier" ::: "memory");
+            other_top = read_top(R & 1);
+          }
+          if constexpr (i < 8) {   // all exponentials in the first eight slots, the conversions in the others
+            constexpr int sb = i >> 2, e = 4 * (i & 3);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) S[sb][e + j] = __builtin_amdgcn_exp2f(S[sb][e + j]);
+          } else {
+            if constexpr (i == 8) {
+              // 448 / largest probability and its inverse; both 0 or finite where the block's probabilities all vanish
+              const float amax = __builtin_amdgcn_exp2f(fmaxf(my_top, other_top));
+              p_sc = fminf(448.f * __builtin_amdgcn_rcpf(amax), 3e38f);
+              p_inv = amax * (1.0f / 448.0f);
+            } else {
+              pack_unit(std::integral_constant<int, i - 9>{});
+            }
+          }
+        } else {
+          constexpr int sb = i >> 3, e = 2 * (i & 7);
+          S[sb][e] = __builtin_amdgcn_exp2f(S[sb][e]);
+          S[sb][e + 1] = __builtin_amdgcn_exp2f(S[sb][e + 1]);
+          if constexpr (i >= 2 && (i & 1) == 0) pack_unit(std::integral_constant<int, (i - 2) / 2>{});
+        }
         __builtin_amdgcn_sched_barrier(0);
       });
       float ps[2] = {0.f, 0.f}, cm[4], tm = 0.f;
@@ -1278,26 +1306,11 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
       }
     l_run += psum;
 
-    float sc = 448.f, inv = 1.0f / 448.0f;
-    if constexpr (MODE == 2) {  // block absmax over the 64-row group: this wave and its neighbour (wave ^ 1)
-      float amax = fmaxf(S[0][0], S[1][0]);
-#pragma unroll
-      for (int i = 1; i < 16; ++i) amax = fmaxf(amax, fmaxf(S[0][i], S[1][i]));
-      if (row_w0 + c32 >= a.Nq) amax = 0.f;   // rows past the end are clamped copies, not part of the block
-#pragma unroll
-      for (int sh = 1; sh < 32; sh <<= 1) amax = wave_xor_max(amax, sh);
-      amax = xor32_max(amax);
-      if (lane == 0) s_amax[it & 1][wave] = amax;
-      __syncthreads();  // see the matching barrier for waves that skip this tile
-      if constexpr (WAVES > 1) amax = fmaxf(amax, s_amax[it & 1][wave ^ 1]);
-      sc = 448.f / amax;   // amax > 0: every visited tile has an unmasked key in every row
-      inv = amax / 448.f;
-    }
     uint4 P[2][2];  // [bn][t]
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) P[bn][t] = quant_pack8<(kPV8 ? 3 : (kQK8 ? 0 : MODE))>(S[bn], t, sc, inv);
+      for (int t = 0; t < 2; ++t) P[bn][t] = pack8(S[bn], t);
     // O^T[d, row] += V^T[d, key] . P^T[key, row]
 #pragma unroll
     for (int bd = 0; bd < 4; ++bd)
@@ -1547,8 +1560,8 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
         }
       }
       if constexpr (MODE == 2) {
-        if (lane == 0) s_amax[t & 1][wave] = 0.f;  // a wave that skips the tile contributes nothing to the block maximum
-        __syncthreads();                            // every wave passes one such barrier per tile
+        post_top(t & 1, -INFINITY);   // a wave that skips the tile contributes nothing to the block maximum,
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // and every wave passes one such barrier per tile
       }
     }
     if (t & 1) {          // end of a pair

@@ -40,8 +40,8 @@ inline int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, in
 //  * Split key ranges: several workgroups per query block, each with a contiguous share of the block's steps, and a second
 //    kernel that merges their accumulators.  The e4m3 modes with a static or absmax grid (1 .. 4), whose P depends on the
 //    row's running maximum, first run a pass that only forms the parts' row maxima (MODE 7), so that every part starts from
-//    the reference point it would have had.  4096 tokens, 4 / 1 heads: mode 0 88 -> 42 us, mode 1 132 -> 66, mode 2 186 ->
-//    69; a chunk of 512 rows behind 16384 tokens at 28 / 4 heads 325 -> 132 us in mode 0.  Mode 5 stays whole: where its reference
+//    the reference point it would have had.  4096 tokens, 4 / 1 heads: mode 0 88 -> 42 us, mode 1 132 -> 66, mode 2 141 ->
+//    62; a chunk of 512 rows behind 16384 tokens at 28 / 4 heads 325 -> 132 us in mode 0.  Mode 5 stays whole: where its reference
 //    point stands depends on every tile sum before (a jump of 2^100 puts it on that tile's maximum), not on a maximum.
 //  * Workgroups of 128 rows (4 waves): one wave per SIMD walks a tile in 0.7 to 0.82 of the time two take for theirs.  Short
 //    prompts, where a merge costs more than it saves: 777 tokens, 28 / 4 heads, mode 0 30.5 -> 24.1 us (split: 34), mode 1
@@ -52,12 +52,13 @@ inline int tiles_of_block(const sq_prefill_params* p, int64_t r0, int64_t r1, in
 //    tiles 69.8 / 65.8 (2049 tiles 1560 / 1376); int8 Q.K^T: 1 tile 13.3 / 15.0, 17 tiles 33.8 / 33.7, 65 tiles 95.6 / 90.7.
 // A tile of an 8-wave workgroup takes kStepUs on an otherwise idle chip and about 30 % more on a full one, which lowers its
 // clock: 8192 rows behind 24576 tokens, 3.5 workgroups per CU, take 2685 us split evenly or not.
+// Mode 2 (26 sizes, every form forced): the plan within 8 % of the best form everywhere, 1.5 % in the mean.
 inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_t Hq, int64_t Nq, LaunchPlan& plan, bool int8qk = false) {
   const int mode = int8qk ? 6 : p->p_quant;
   constexpr int kCUs = kPlanCUs, kMaxRounds = kPlanMaxRounds, kMinTiles = 4;
-  static const float kStepUs[7] = {1.35f, 1.75f, 2.6f, 1.4f, 1.15f, 1.15f, 1.35f};   // by P mode; 6: int8 Q.K^T
+  static const float kStepUs[7] = {1.35f, 1.75f, 2.05f, 1.4f, 1.15f, 1.15f, 1.35f};   // by P mode; 6: int8 Q.K^T
   constexpr float kFixUs = 8.f;      // a workgroup's launch, first loads and epilogue
-  static const float kFourWaves[7] = {0.76f, 0.7f, 0.82f, 1.f, 1.f, 0.76f, 0.76f};
+  static const float kFourWaves[7] = {0.76f, 0.7f, 0.73f, 1.f, 1.f, 0.76f, 0.76f};
   static const int kFewRowsTiles[7] = {2, 2, 5, 0, 0, 16, 11};
   constexpr float kFullChip = 0.3f;
   constexpr float kMergeUs = 6.f, kPartUs = 0.07f;   // the merge; a part's 130 KB written and read again
