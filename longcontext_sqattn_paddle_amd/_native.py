@@ -172,6 +172,30 @@ def probe_lib() -> ctypes.CDLL:
     return _probe_lib
 
 
+HOST_CALLS_PATH = os.path.join(_PKG_DIR, "_host_calls.so")
+# the library functions that csrc/host_calls.cpp calls, in its order
+_HOST_CALLS_USE = ("sq_decode_num_splits", "sq_decode_workspace_bytes", "sq_decode_fwd", "sq_decode_selected_fwd",
+                   "sq_kmeans_workspace_bytes", "sq_topk_select", "sq_prefill_workspace_bytes_split", "sq_prefill_fwd")
+_host_calls = None
+
+
+def host_calls():
+    """The native short way of the calls whose kernels are shorter than a call's Python side (csrc/host_calls.cpp), bound to the
+    loaded library.  Its functions return None, having done nothing, for arguments they leave to the general way."""
+    global _host_calls
+    if _host_calls is None:
+        if not os.path.exists(HOST_CALLS_PATH):
+            raise RuntimeError(f"{HOST_CALLS_PATH} is missing: build it with `python -m longcontext_sqattn_paddle_amd.build`")
+        import importlib.util
+
+        spec = importlib.util.spec_from_file_location("_host_calls", HOST_CALLS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _HOST_CALLS_USE))
+        _host_calls = module
+    return _host_calls
+
+
 _capsule_ptr = ctypes.pythonapi.PyCapsule_GetPointer
 _capsule_ptr.restype = ctypes.c_void_p
 _capsule_ptr.argtypes = [ctypes.py_object, ctypes.c_char_p]
@@ -205,8 +229,7 @@ def borrow(*tensors: Optional[torch.Tensor]):
     """(addresses, capsules) of several tensors for one library call, None for None.  The second list has to outlive the call:
     it holds the capsules the addresses point into.
 
-    For the calls whose kernels are shorter than their host side: a `dl` / `ptr` pair with a typed pointer took 1.8 us per
-    tensor, this takes 0.6 us (decode over 1531 tokens 22.0 -> 15.4 us a call, selection + decode over it 38.7 -> 26.3 us)."""
+    For calls of many tensors: a `dl` / `ptr` pair with a typed pointer takes 1.8 us per tensor, this 0.3 to 0.6."""
     capsules = [None if t is None else _to_dlpack(t) for t in tensors]
     return [None if c is None else _capsule_ptr(c, b"dltensor") for c in capsules], capsules
 
@@ -221,6 +244,13 @@ def check(code: int, library: Optional[ctypes.CDLL] = None) -> None:
     if code == SQ_ESHAPE:
         raise AssertionError(msg)
     raise RuntimeError(f"libsqattn_hip error {code}: {msg}")
+
+
+def result(res):
+    """What a function of `host_calls` returned: the output, or the exception of its error code."""
+    if isinstance(res, int):
+        check(res)
+    return res
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # missing in torch builds without a GPU runtime

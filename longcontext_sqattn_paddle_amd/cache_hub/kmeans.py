@@ -122,6 +122,9 @@ def topk_select(query, centroids, clusters, cluster_size, k: int, num_kv_groups:
     `out` (int32 [G,k], contiguous) and `workspace` (`_workspace(G, 1, C, device)`) may be passed by a caller that
     selects every step."""
     _require(query, "query")
+    res = N.host_calls().topk_select(query, centroids, clusters, cluster_size, k, num_kv_groups, out, workspace, N.current_stream(query.device))
+    if res is not None:
+        return N.result(res)
     G, C, _ = centroids.shape
     if out is None:
         out = torch.empty((G, k), dtype=torch.int32, device=query.device)

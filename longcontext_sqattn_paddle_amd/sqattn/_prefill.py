@@ -29,6 +29,10 @@ def run_prefill(q, k, v, *, tensor_layout="HND", output_dtype=torch.float16, ret
     if tensor_layout not in N.LAYOUT:
         raise ValueError(f"tensor_layout {tensor_layout} not supported")
     require_gpu(q, k, v, q4, k4, v_tiles)
+    if window is None and q_quant == 0 and v is not None and q4 is None and k4 is None and k_scale is None and v_tiles is None:
+        res = N.host_calls().prefill(q, k, v, N.LAYOUT[tensor_layout], output_dtype, return_lse, p_quant, q_offset, workspace, out, N.current_stream(q.device))
+        if res is not None:
+            return N.result(res)
     head_dim_og = q.size(-1)
     if k_scale is not None:
         if head_dim_og != 128 or q4 is not None or k4 is not None or p_quant != N.P_NONE or q_quant:

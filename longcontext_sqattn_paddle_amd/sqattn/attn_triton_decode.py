@@ -28,6 +28,11 @@ def attn_decode(q, k, v, tensor_layout="HND", output_dtype=torch.float16, return
     if tensor_layout not in N.LAYOUT:
         raise ValueError(f"tensor_layout {tensor_layout} not supported")
     require_gpu(q, k, v)
+    p_mode = N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE
+    res = N.host_calls().decode(q, k, v, None, seqlens, N.LAYOUT[tensor_layout], output_dtype, return_lse, p_mode, num_splits, workspace, out,
+                                N.current_stream(q.device))
+    if res is not None:
+        return N.result(res)
     head_dim_og = q.size(-1)
     q, k, v = pad_head_dim((q, k, v), head_dim_og)
     assert q.stride(-1) == 1 and k.stride(-1) == 1 and v.stride(-1) == 1
@@ -40,7 +45,7 @@ def attn_decode(q, k, v, tensor_layout="HND", output_dtype=torch.float16, return
         workspace = torch.empty(need // 4, dtype=torch.float32, device=q.device)
     o = out if out is not None else torch.empty(q.shape, dtype=output_dtype, device=q.device)
     lse = torch.empty([B, Hq, 1], dtype=torch.float32, device=q.device) if return_lse else None
-    params = N.DecodeParams(N.LAYOUT[tensor_layout], N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE, max(num_splits, 0), head_dim_og)
+    params = N.DecodeParams(N.LAYOUT[tensor_layout], p_mode, max(num_splits, 0), head_dim_og)
     ptrs, held = N.borrow(q, k, v, seqlens, o, lse, workspace)
     N.check(lib.sq_decode_fwd(*ptrs, params, N.current_stream(q.device)))
     if head_dim_og != KERNEL_HEAD_DIM:
@@ -74,6 +79,12 @@ def attn_decode_selected(q, k, v, token_ids, tensor_layout="NHD", output_dtype=t
     if tensor_layout not in N.LAYOUT:
         raise ValueError(f"tensor_layout {tensor_layout} not supported")
     require_gpu(q, k, v)
+    p_mode = N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE
+    if token_ids is not None:
+        res = N.host_calls().decode(q, k, v, token_ids, seqlens, N.LAYOUT[tensor_layout], output_dtype, return_lse, p_mode, num_splits, workspace, out,
+                                    N.current_stream(q.device))
+        if res is not None:
+            return N.result(res)
     head_dim_og = q.size(-1)
     q, k, v = pad_head_dim((q, k, v), head_dim_og)
     hdim = 1 if tensor_layout == "HND" else 2
@@ -85,7 +96,7 @@ def attn_decode_selected(q, k, v, token_ids, tensor_layout="NHD", output_dtype=t
         workspace = torch.empty(need // 4, dtype=torch.float32, device=q.device)
     o = out if out is not None else torch.empty(q.shape, dtype=output_dtype, device=q.device)
     lse = torch.empty([B, Hq, 1], dtype=torch.float32, device=q.device) if return_lse else None
-    params = N.DecodeParams(N.LAYOUT[tensor_layout], N.P_E4M3_STATIC if is_P_fp8_quant else N.P_NONE, max(num_splits, 0), head_dim_og)
+    params = N.DecodeParams(N.LAYOUT[tensor_layout], p_mode, max(num_splits, 0), head_dim_og)
     ptrs, held = N.borrow(q, k, v, token_ids, seqlens, o, lse, workspace)
     N.check(lib.sq_decode_selected_fwd(*ptrs, params, N.current_stream(q.device)))
     if head_dim_og != KERNEL_HEAD_DIM:

@@ -213,3 +213,19 @@ def test_window_sizes_in_any_number_type():
     assert once_each([np.array(0.5), np.array(0.25)], lambda r: 4 * float(r)) == [2.0, 1.0]
     with pytest.raises(TypeError):
         once_each([None], float)
+
+
+def test_native_calls_leave_host_tensors_and_other_arguments_alone():
+    """Nothing but plain GPU tensors is taken: the functions return None before they touch anything."""
+    from longcontext_sqattn_paddle_amd import _native as N
+
+    m = N.host_calls()
+    q, k = torch.zeros(1, 1, 4, 128, dtype=torch.bfloat16), torch.zeros(1, 9, 2, 128, dtype=torch.bfloat16)
+    args = [q, k, k, None, None, 1, torch.bfloat16, False, 0, 0, None, None, 0]
+    assert m.decode(*args) is None and m.decode() is None and m.decode(*args[:-1], "x") is None
+    for i in range(len(args)):
+        assert m.decode(*args[:i], object(), *args[i + 1:]) is None, i
+    assert m.prefill(q, k, k, 1, torch.bfloat16, False, 0, 0, None, None, 0) is None
+    assert m.topk_select(q, k, k, k, 1, 1, None, None, 0) is None
+    with pytest.raises(TypeError):
+        m.bind(1)
