@@ -42,6 +42,16 @@ constexpr int kKTileBytes = kBN * kKStride;
 constexpr int kVTileBytes = kD * kVStride;
 constexpr int kStageBytes = kKTileBytes + kVTileBytes;
 constexpr int kMaxHeads = 128;
+struct PrepArgs {
+  const void* v;
+  _Float16* vt;
+  uint8_t* vt8;          // e4m3 tiles (MODE 4)
+  uint32_t* vmax_bits;   // [B, Hkv, 128] running |v| maximum as fp32 bit patterns (MODE 4)
+  float* v_inv_scale;    // [B, Hkv, 128]
+  int64_t v_sb, v_sh, v_sn;
+  int32_t Nk, nT, Hkv, is_bf16;
+};
+
 struct PrefillArgs {
   const void* q;
   const void* k;
@@ -68,23 +78,14 @@ struct PrefillArgs {
   float sm;
   int32_t w8[kMaxHeads];
   int32_t w4[kMaxHeads];
+  PrepArgs prep;   // MODE 7: the V^T tiles to form beside the pass (prep.v null: none)
   SplitWork work[kMaxSplitWork];
 };
 
-struct PrepArgs {
-  const void* v;
-  _Float16* vt;
-  uint8_t* vt8;          // e4m3 tiles (MODE 4)
-  uint32_t* vmax_bits;   // [B, Hkv, 128] running |v| maximum as fp32 bit patterns (MODE 4)
-  float* v_inv_scale;    // [B, Hkv, 128]
-  int64_t v_sb, v_sh, v_sn;
-  int32_t Nk, nT, Hkv, is_bf16;
-};
-
-__global__ __launch_bounds__(256) void prefill_prep_v_kernel(PrepArgs a) {
-  const int j = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-  const int o = threadIdx.x & 15;    // channel octet
-  const int tq = threadIdx.x >> 4;   // key quad
+// One fp16 V^T tile by 256 threads (`t` of them)
+__device__ __forceinline__ void prep_v_tile(const PrepArgs& a, int b, int kvh, int j, int t) {
+  const int o = t & 15;    // channel octet
+  const int tq = t >> 4;   // key quad
   const uint16_t* vb = (const uint16_t*)a.v + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_sh;
   _Float16 h[4][8];
 #pragma unroll
@@ -107,6 +108,8 @@ __global__ __launch_bounds__(256) void prefill_prep_v_kernel(PrepArgs a) {
     *(f16x4_t*)(tile + (8 * o + e) * kBN + pos) = val;
   }
 }
+
+__global__ __launch_bounds__(256) void prefill_prep_v_kernel(PrepArgs a) { prep_v_tile(a, blockIdx.z, blockIdx.y, blockIdx.x, threadIdx.x); }
 
 // ---- fp8 P.V path (MODE 4): V is quantised to e4m3 with one scale per (batch, kv head, channel).
 // (1) per-channel |v| maximum over all keys: every workgroup reduces one 64-key tile and merges with an integer
@@ -491,7 +494,16 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   if constexpr (SPLIT) {
     t_off = nTot * sw.part / sw.parts;
     nTot = nTot * (sw.part + 1) / sw.parts - t_off;
-    if (kRefPass && sw.part + 1 == sw.parts) return;   // nobody comes after the last part
+    if (kRefPass && sw.part + 1 == sw.parts) {   // nobody comes after the last part
+      // The pass reads no values, so these workgroups, one per query block, form the V^T tiles of the launch behind it: a launch
+      // less in the chain where they are done before the pass is (prep_beside_pass).
+      if (a.prep.v) {
+        const int per = a.nT * a.Hkv, tiles = per * a.B, nb = (a.Nq + WAVES * ROWS - 1) / (WAVES * ROWS);
+        for (int i = 2 * ((b * a.Hq + head) * nb + qb) + (tid >> 8); i < tiles; i += 2 * a.B * a.Hq * nb)
+          prep_v_tile(a.prep, i / per, i % per / a.nT, i % a.nT, tid & 255);
+      }
+      return;
+    }
   }
   // ---- Q~ fragments (B operand of S^T = K.Q~^T): lane (column = query row c32, k-group g)
   uint4 qf[8];
@@ -1870,10 +1882,8 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
     hipLaunchKernelGGL(prefill_fill_u32_kernel, dim3(1), dim3(256), 0, st, pa.vmax_bits, (int)(B * Hkv * kD));
     hipLaunchKernelGGL(prefill_vabsmax_kernel, pgrid, dim3(256), 0, st, pa);
     hipLaunchKernelGGL(prefill_prep_v8_kernel, pgrid, dim3(256), 0, st, pa);
-  } else {
-    hipLaunchKernelGGL(prefill_prep_v_kernel, pgrid, dim3(256), 0, st, pa);
   }
-  SQ_HIP(hipGetLastError());
+  // (fp16 tiles: below, where it is known whether a row-maximum pass can form them)
 
   // passed to the kernel by value: 1.3 KB with the per-head windows and 3 KB of a split launch's work list (handing the list to
   // split launches only measured the same: 172 small calls, 0.2 % in the mean, within the spread)
@@ -1964,6 +1974,11 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
     local.sched_xpp = 1;
     blocks = (unsigned)pairs * (unsigned)items;
   }
+  const bool ref_pass = split && p->p_quant >= SQ_P_E4M3_STATIC && p->p_quant <= SQ_P_E4M3_FP8_PV;   // as in plan_launch
+  if (!pv8 && !v_tiles) {
+    if (ref_pass && prep_beside_pass(plan.share, B * Hkv * nT, B * Hq * ((Nq + 255) / 256))) local.prep = pa;
+    else hipLaunchKernelGGL(prefill_prep_v_kernel, pgrid, dim3(256), 0, st, pa);
+  }
   const size_t smem = 4 * (size_t)kStageBytes + 64;   // rings of 4 K tiles and 4 V^T tiles, MODE 2's block maxima
   const bool bf = dt == DType::BF16;
 #define SQ_LAUNCH_PREFILL(BF, W, M)                                                                              \
@@ -2032,7 +2047,6 @@ int prefill_impl(const DLTensor* q, const DLTensor* k, const DLTensor* v, const 
       default: SQ_LAUNCH_PREFILL(BF, W, 3); break;               \
     }                                                           \
   } while (0)
-  const bool ref_pass = p->p_quant >= SQ_P_E4M3_STATIC && p->p_quant <= SQ_P_E4M3_FP8_PV;   // as in plan_launch
   if (split) {
     if (bf) SQ_LAUNCH_SPLITS(true); else SQ_LAUNCH_SPLITS(false);
   } else if (waves == 8 && q4) {

@@ -23,6 +23,7 @@ struct SplitWork {
 struct LaunchPlan {
   int waves = 8;                 // per workgroup, where the launch is not split (a split one has 8)
   int n_work = 0, n_slots = 0;   // n_work == 0: not to be split
+  int share = 0;                 // tiles of the longest part
   SplitWork work[kMaxSplitWork];
 };
 
@@ -146,6 +147,7 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
     }
   }
   if (cap == 0) return;
+  plan.share = cap;
   for (int64_t qb = nQB - 1; qb >= 0; --qb) {
     const int parts = std::min((len[qb] + cap - 1) / cap, 255);
     for (int i = 0; i < parts; ++i) plan.work[plan.n_work++] = SplitWork{(uint16_t)qb, (uint16_t)plan.n_slots, (uint8_t)i, (uint8_t)parts};
@@ -154,5 +156,12 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
   // longest shares first
   std::stable_sort(plan.work, plan.work + plan.n_work, [&](const SplitWork& x, const SplitWork& y) { return (int64_t)len[x.qb] * y.parts > (int64_t)len[y.qb] * x.parts; });
 }
+
+// Whether the row-maximum pass of a split launch also forms the V^T tiles, two at a time in each of its workgroups that have no
+// part to look at (one per query block): where they are done with it before the parts are, at 1.3 us a round against
+// 0.6 us a tile.  4096 tokens, 4 / 1 heads, mode 2 (1 round, shares of 16) 64.4 -> 59.3 us; 512 rows behind 16384 tokens, 28 / 4
+// heads, mode 1 (10 rounds, shares of 66) 224 -> 214.  Beyond it the pass would wait for them: 64 rows behind 16384 tokens (19 rounds, shares of
+// 29) keep the launch of their own.
+inline bool prep_beside_pass(int share, int64_t v_tiles, int64_t idle) { return 1.3f * (float)((v_tiles + 2 * idle - 1) / (2 * idle)) <= 0.6f * share + 1.f; }
 
 }  // namespace sq
