@@ -35,6 +35,7 @@
  *   sq_rope                   model_hub/utils.py:21-106 (apply_rope_with_cos_sin_cache_inplace; caller qwen.py:352-367)
  *   sq_linear_rows            the matmuls of a decode step: model_hub/qwen.py:293-300 (lm), :302-312 (wqkv), :314-317 (wo),
  *                             :319-326 (mlp), called from model_hub/LLM.py:88-116 (layer_decode)
+ *   sq_linear                 the same matmuls of a prompt: model_hub/qwen.py:302-326, called from model_hub/LLM.py:40-86 (layer_prefill)
  *   sq_linear_rows_silu_and_mul  model_hub/qwen.py:320-324 (gate_up_proj and silu_and_mul of mlp) on a decode step
  *   sq_linear_rows_rope       model_hub/qwen.py:302-312 (wqkv) + :352-379 (rotary embedding of q and k) on a decode step
  *   sq_rmsnorm_linear_rows, sq_rmsnorm_linear_rows_silu_and_mul, sq_rmsnorm_linear_rows_rope
@@ -381,6 +382,18 @@ int sq_silu_and_mul(const DLTensor* x, DLTensor* out, void* stream);
  */
 int sq_linear_rows(const DLTensor* x, const DLTensor* weight, const DLTensor* bias, const DLTensor* residual,
                    DLTensor* out, void* stream);
+
+/*
+ * out = x . weight^T (+ bias) for the rows of a prompt, with the sum over K split over workgroups where the output alone does not
+ * fill the GPU (model_hub/qwen.py:302-326 on a prompt's activation).  x [M, K], weight [N, K], bias [N] or NULL, out [M, N]; bf16 or
+ * fp16, all of one dtype; K a multiple of 64, N of 4; last dimensions contiguous, rows of x and weight on 16-byte, of out
+ * on 8-byte boundaries, operands below 4 GiB.  fp32 accumulation, the sum plus the bias is rounded once.  workspace:
+ * sq_linear_workspace_bytes(M, N, K) bytes (0: may be NULL).  sq_linear_preferred: 1 where this is faster than the BLAS
+ * library's product, 0 otherwise.
+ */
+int32_t sq_linear_preferred(int64_t M, int64_t N, int64_t K);
+size_t sq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int sq_linear(const DLTensor* x, const DLTensor* weight, const DLTensor* bias, DLTensor* out, DLTensor* workspace, void* stream);
 
 /*
  * out = silu_and_mul(x . weight^T (+ bias)) for 1 to 8 rows of x: the first projection of the MLP and the activation

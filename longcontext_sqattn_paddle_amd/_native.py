@@ -111,6 +111,9 @@ SYMBOLS = {
     "sq_rmsnorm": (ctypes.c_int, [_P, _P, _P, ctypes.c_float, ctypes.c_void_p]),
     "sq_silu_and_mul": (ctypes.c_int, [_P, _P, ctypes.c_void_p]),
     "sq_rope": (ctypes.c_int, [_P] * 6 + [ctypes.c_int32, ctypes.c_void_p]),
+    "sq_linear_preferred": (ctypes.c_int32, [ctypes.c_int64] * 3),
+    "sq_linear_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 3),
+    "sq_linear": (ctypes.c_int, [_P] * 5 + [ctypes.c_void_p]),
     "sq_linear_rows": (ctypes.c_int, [_P] * 5 + [ctypes.c_void_p]),
     "sq_linear_rows_silu_and_mul": (ctypes.c_int, [_P] * 4 + [ctypes.c_void_p]),
     "sq_linear_rows_rope": (ctypes.c_int, [_P] * 5 + [ctypes.c_int32, ctypes.c_int32] + [_P] * 5 + [ctypes.c_void_p]),
@@ -175,7 +178,8 @@ def probe_lib() -> ctypes.CDLL:
 HOST_CALLS_PATH = os.path.join(_PKG_DIR, "_host_calls.so")
 # the library functions that csrc/host_calls.cpp calls, in its order
 _HOST_CALLS_USE = ("sq_decode_num_splits", "sq_decode_workspace_bytes", "sq_decode_fwd", "sq_decode_selected_fwd",
-                   "sq_kmeans_workspace_bytes", "sq_topk_select", "sq_prefill_workspace_bytes_split", "sq_prefill_fwd")
+                   "sq_kmeans_workspace_bytes", "sq_topk_select", "sq_prefill_workspace_bytes_split", "sq_prefill_fwd",
+                   "sq_linear_preferred", "sq_linear_workspace_bytes", "sq_linear")
 _host_calls = None
 
 

@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libsqattn_hip.so")
 PROBE_LIB_PATH = os.path.join(PKG_DIR, "libsqattn_probe.so")
 HOST_CALLS_PATH = os.path.join(PKG_DIR, "_host_calls.so")   # host code on torch's tensors, no GPU code in it
 HOST_CALLS_SOURCE = "host_calls.cpp"
-SOURCES = ["capi.hip", "decode_gfx950.hip", "prefill_gfx950.hip", "kmeans_gfx950.hip", "prepass_gfx950.hip", "kvcache_gfx950.hip", "layer_gfx950.hip", "linear_gfx950.hip", "calib_gfx950.hip"]
+SOURCES = ["capi.hip", "decode_gfx950.hip", "prefill_gfx950.hip", "kmeans_gfx950.hip", "prepass_gfx950.hip", "kvcache_gfx950.hip", "layer_gfx950.hip", "linear_gfx950.hip", "gemm_gfx950.hip", "calib_gfx950.hip"]
 PROBE_SOURCES = ["capi.hip", "probe_gfx950.hip"]   # its own copy of the error string and the tensor checks
 
 HIPCC_FLAGS = [
@@ -27,7 +27,8 @@ HIPCC_FLAGS = [
 # Per-source flags.  The k-means assign kernel reads its MFMA results with the vector ALU right away (arg-max): the MFMAs
 # are kept in their VGPR form there, otherwise every score passes through a v_accvgpr_read first.
 # The 4-wave prefill workgroups may use 512 registers per lane; in the other form their score accumulators move to AGPRs and back.
-SOURCE_FLAGS = {"kmeans_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "prefill_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+SOURCE_FLAGS = {"kmeans_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "prefill_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                "gemm_gfx950.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def host_calls_command() -> list:

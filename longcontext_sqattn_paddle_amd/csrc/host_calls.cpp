@@ -17,6 +17,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <vector>
+
 #include "sqattn.h"
 
 namespace {
@@ -31,6 +33,9 @@ struct Library {
   decltype(&sq_topk_select) topk_select;
   decltype(&sq_prefill_workspace_bytes_split) prefill_workspace_bytes_split;
   decltype(&sq_prefill_fwd) prefill_fwd;
+  decltype(&sq_linear_preferred) linear_preferred;
+  decltype(&sq_linear_workspace_bytes) linear_workspace_bytes;
+  decltype(&sq_linear) linear;
 } lib;
 
 struct Arg : DLTensor {
@@ -207,11 +212,55 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// linear(x, weight, bias, stream): None also where the BLAS library's product is the faster one, or the operands do not lie as
+// sq_linear takes them
+PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 4 || !plain_context() || !plain(a[0]) || !plain(a[1]) || !plain_or_none(a[2]) || !is_int(a[3])) Py_RETURN_NONE;
+  const at::Tensor &x = THPVariable_Unpack(a[0]), &w = THPVariable_Unpack(a[1]);
+  if (x.dim() < 1 || w.dim() != 2 || !x.is_contiguous() || !w.is_contiguous() || x.numel() == 0 || w.numel() == 0) Py_RETURN_NONE;
+  const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
+  const auto aligned = [](const at::Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; };
+  if (w.size(1) != K || !lib.linear_preferred(M, N, K) || !aligned(x) || !aligned(w) || x.device() != w.device() || x.scalar_type() != w.scalar_type() ||
+      (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf) || x.numel() >= (int64_t)1 << 31 || w.numel() >= (int64_t)1 << 31)
+    Py_RETURN_NONE;
+  const bool biased = a[2] != Py_None;
+  if (biased) {
+    const at::Tensor& b = THPVariable_Unpack(a[2]);
+    if (b.dim() != 1 || b.size(0) != N || !b.is_contiguous() || !aligned(b) || b.scalar_type() != x.scalar_type() || b.device() != x.device()) Py_RETURN_NONE;
+  }
+  void* const stream = PyLong_AsVoidPtr(a[3]);
+  at::Tensor o;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = N;
+    o = at::empty(shape, x.options());
+    const size_t bytes = lib.linear_workspace_bytes(M, N, K);
+    at::Tensor ws = bytes ? scratch(bytes, at::kByte, x) : at::Tensor();
+    Arg dx(x), dw(w), dout(o);
+    int64_t x_shape[2] = {M, K}, x_strides[2] = {K, 1}, o_shape[2] = {M, N}, o_strides[2] = {N, 1};
+    dx.ndim = dout.ndim = 2;
+    dx.shape = x_shape;
+    dx.strides = x_strides;
+    dout.shape = o_shape;
+    dout.strides = o_strides;
+    c10::optional<Arg> db, dws;
+    if (biased) db.emplace(THPVariable_Unpack(a[2]));
+    if (bytes) dws.emplace(ws);
+    rc = lib.linear(&dx, &dw, db ? &*db : nullptr, &dout, dws ? &*dws : nullptr, stream);
+  }
+  if (rc != SQ_OK) return PyLong_FromLong(rc);
+  return THPVariable_Wrap(o);
+  END_HANDLE_TH_ERRORS
+}
+
 // bind(addresses): the library's functions, in the order of `Library`
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  static_assert(sizeof(Library) == 8 * sizeof(void*), "one address per function");
-  if (n != 8) {
-    PyErr_SetString(PyExc_TypeError, "bind takes 8 addresses");
+  constexpr Py_ssize_t kFunctions = sizeof(Library) / sizeof(void*);
+  if (n != kFunctions) {
+    PyErr_SetString(PyExc_TypeError, "bind takes one address per function");
     return nullptr;
   }
   for (Py_ssize_t i = 0; i < n; ++i) {
@@ -229,6 +278,7 @@ PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
     {"decode", (PyCFunction)(void (*)(void))decode, METH_FASTCALL, nullptr},
     {"topk_select", (PyCFunction)(void (*)(void))topk_select, METH_FASTCALL, nullptr},
+    {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"prefill", (PyCFunction)(void (*)(void))prefill, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

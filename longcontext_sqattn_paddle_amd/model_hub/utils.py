@@ -50,12 +50,19 @@ def _norm_fits(norm, rows: int, K: int, fuse_rows: int = 1) -> bool:
     return rows <= fuse_rows and K <= cap and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.shape == (K,)
 
 
+def _product(x, weight, bias):
+    """x @ weight.T (+ bias) of more rows than a decode step has: `sq_linear` where splitting the sum over K fills the chip (down_proj of
+    512 rows 197 -> 86 us), the BLAS library otherwise, and for everything that is not a plain tensor or wants a gradient."""
+    y = N.host_calls().linear(x, weight, bias, N.current_stream(x.device))
+    return torch.nn.functional.linear(x, weight, bias) if y is None else N.result(y)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, residual: Optional[torch.Tensor] = None,
            max_rows: int = 4, norm=None, fuse_norm_rows: int = 1) -> torch.Tensor:
     """`x @ weight.T (+ bias) (+ residual)` over the last dimension of x, weight [N, K] (the matmuls of
     model_hub/qwen.py:293-326).  Up to `max_rows` rows of x (a decode step) go through the weight-streaming HIP
-    kernel; longer activations (a prompt) are a GEMM and go to the BLAS library.  The kernel takes up to
-    LINEAR_ROWS_MAX rows; from five rows on the library's GEMM is as fast, hence the default.
+    kernel; longer activations (a prompt) are a GEMM (`_product`).  The kernel takes up to
+    LINEAR_ROWS_MAX rows; from five rows on a GEMM is as fast, hence the default.
 
     `norm` = (weight, epsilon): the product is taken of `rmsnorm(x, weight, epsilon)`; with up to `fuse_norm_rows` rows
     on the kernel's route the norm is part of the same pass (same values as the two calls)."""
@@ -66,7 +73,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     if norm is not None and not (on_kernel and _norm_fits(norm, rows, K, fuse_norm_rows)):
         x, norm = rmsnorm(x, norm[0], norm[1]), None
     if not on_kernel:
-        y = torch.nn.functional.linear(x, weight, bias)
+        y = _product(x, weight, bias)
         return y if residual is None else residual + y
     x2 = x.reshape(rows, K)
     if x2.stride(-1) != 1 or (rows > 1 and x2.stride(0) % 8) or x2.data_ptr() % 16:

@@ -172,6 +172,73 @@ def test_linear_rows_matches_oracle(dtype, M, N, K, bias, residual):
     _check_linear(out, x, w, b, r)
 
 
+def _sq_linear(x, w, b, out):
+    from longcontext_sqattn_paddle_amd import _native as NV
+
+    lib = NV.lib()
+    ws = torch.empty(lib.sq_linear_workspace_bytes(x.shape[0], w.shape[0], x.shape[1]), dtype=torch.uint8, device=DEV)
+    ptrs, held = NV.borrow(x, w, b, out, ws if ws.numel() else None)
+    NV.check(lib.sq_linear(*ptrs, NV.current_stream(torch.device(DEV))))
+    return ws.numel()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,bias,split", [
+    (1, 4, 64, True, False), (63, 132, 128, False, False), (64, 128, 192, True, False), (65, 260, 256, False, False),   # 64-row tiles, short K
+    (5, 132, 1024, True, True), (64, 3584, 3584, False, True), (300, 100, 3584, True, True),                             # 64-row tiles, parts
+    (65, 1000, 18944, True, True), (257, 8192, 128, False, False),                                                       # 128-row tiles
+    (150, 3584, 18944, True, True), (513, 8192, 64, True, False)])                                                       # 256-row tiles
+def test_linear_of_a_prompt_matches_oracle(dtype, M, N, K, bias, split):
+    """`sq_linear` at the edges of its tiles and parts; rows of x and out further apart than they are long, NaN around them."""
+    print(f"case prompt linear {dtype} M={M} N={N} K={K} bias={bias}", flush=True)
+    x, w, b, _ = _linear_case(M, N, K, dtype, 3 * M + N + K, bias, False)
+    wide = torch.full((M, K + 8), float("nan"), dtype=dtype, device=DEV)
+    wide[:, :K] = x.to(DEV)
+    room = torch.full((M + 1, N + 4), float("nan"), dtype=dtype, device=DEV)
+    parts = _sq_linear(wide[:, :K], w.to(DEV), b.to(DEV) if bias else None, room[:M, :N])
+    torch.cuda.synchronize()
+    assert (parts > 0) is split
+    _check_linear(room[:M, :N], x, w, b, None)
+    assert bool(room[M].isnan().all()) and bool(room[:, N:].isnan().all())
+
+
+def test_linear_of_a_prompt_special_values_and_refusals():
+    """A NaN in a row of x stays in that row, one in a row of the weight in its feature; what the kernel does not take is refused."""
+    from longcontext_sqattn_paddle_amd import _native as NV
+
+    x, w = torch.randn(70, 3584, device=DEV).bfloat16(), torch.randn(260, 3584, device=DEV).bfloat16()
+    x[3, 17] = float("nan")
+    w[259, 5] = float("inf")
+    out = torch.empty(70, 260, dtype=torch.bfloat16, device=DEV)
+    _sq_linear(x, w, None, out)
+    want = x.float() @ w.float().T
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    for bad in (lambda: _sq_linear(x[:, :40], w[:, :40], None, out), lambda: _sq_linear(x, w[:258], None, out[:, :258]),
+                lambda: _sq_linear(x.half(), w, None, out), lambda: _sq_linear(x, w, x[0], out), lambda: _sq_linear(x, w[:, :64], None, out)):
+        with pytest.raises((ValueError, AssertionError)):
+            bad()
+    lib = NV.lib()
+    ptrs, held = NV.borrow(x, w, None, out, None)
+    with pytest.raises(RuntimeError):   # parts without a workspace
+        NV.check(lib.sq_linear(*ptrs, 0))
+
+
+def test_linear_of_a_prompt_is_chosen_by_size_and_leaves_gradients_to_torch():
+    from longcontext_sqattn_paddle_amd import _native as NV
+    from longcontext_sqattn_paddle_amd.model_hub.utils import linear
+
+    x, w, b = torch.randn(2, 20, 512, device=DEV).bfloat16(), torch.randn(256, 512, device=DEV).bfloat16(), torch.randn(256, device=DEV).bfloat16()
+    st = NV.current_stream(torch.device(DEV))
+    own = NV.host_calls().linear(x, w, b, st)
+    got = linear(x, w, b)
+    assert own.shape == (2, 20, 256) and torch.equal(own, got)
+    _check_linear(got.reshape(40, 256), x.reshape(40, 512).cpu(), w.cpu(), b.cpu(), None)
+    for args in ((x.requires_grad_(), w, b), (x.detach()[..., ::2], w[:, ::2], b), (x.detach()[..., :500], w[:, :500].contiguous(), b), (x.detach().float(), w.float(), None)):
+        assert NV.host_calls().linear(*args, st) is None
+    linear(x, w, b).float().sum().backward()
+    assert torch.allclose(x.grad[0, 0].float(), w.float().sum(0), rtol=2e-2, atol=0.5)
+
+
 def test_linear_rows_views_batch_shapes_and_the_gemm_hand_over():
     from longcontext_sqattn_paddle_amd import _native as NV
     from longcontext_sqattn_paddle_amd.model_hub.utils import linear
