@@ -235,7 +235,8 @@ def test_linear_of_a_prompt_is_chosen_by_size_and_leaves_gradients_to_torch():
     _check_linear(got.reshape(40, 256), x.reshape(40, 512).cpu(), w.cpu(), b.cpu(), None)
     for args in ((x.requires_grad_(), w, b), (x.detach()[..., ::2], w[:, ::2], b), (x.detach()[..., :500], w[:, :500].contiguous(), b), (x.detach().float(), w.float(), None)):
         assert NV.host_calls().linear(*args, st) is None
-    linear(x, w, b).float().sum().backward()
+    with torch.enable_grad():   # wherever another test left the mode
+        linear(x, w, b).float().sum().backward()
     assert torch.allclose(x.grad[0, 0].float(), w.float().sum(0), rtol=2e-2, atol=0.5)
 
 
