@@ -72,17 +72,14 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs a) {
     const uint32_t chunk = (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u;
     off[c] = is_x ? (uint32_t)min(m0 + r, a.M - 1) * (uint32_t)a.x_row + chunk : (uint32_t)min(n0 + r, a.N - 1) * (uint32_t)a.w_row + chunk;
   }
-  auto stage = [&](int s, int buf) __attribute__((always_inline)) {
-    const int64_t k = (int64_t)(s0 + s) * kRowBytes;
-#pragma unroll
-    for (int c = 0; c < PER; ++c) {
-      const int q = PER * wave + c;
-      const char* base = (q < BM / 8 ? a.x : a.w) + k;
-      uint32_t o = off[c];
-      asm volatile("" : "+v"(o));   // a 32-bit per-lane offset next to the uniform 64-bit base
-      __builtin_amdgcn_global_load_lds((const void*)(base + o), (lds_ptr_t)(smem + buf * kBuf + q * 1024), 16, 0, 0);
-    }
+  auto copy = [&](int s, int buf, int c) __attribute__((always_inline)) {
+    const int q = PER * wave + c;
+    const char* base = (q < BM / 8 ? a.x : a.w) + (int64_t)(s0 + s) * kRowBytes;
+    uint32_t o = off[c];
+    asm volatile("" : "+v"(o));   // a 32-bit per-lane offset next to the uniform 64-bit base
+    __builtin_amdgcn_global_load_lds((const void*)(base + o), (lds_ptr_t)(smem + buf * kBuf + q * 1024), 16, 0, 0);
   };
+  auto stage = [&](int s, int buf) __attribute__((always_inline)) { static_for<0, PER>([&](auto C) { copy(s, buf, decltype(C)::value); }); };
   const int c32 = lane & 31, g = lane >> 5, wm = wave / WN, wn = wave % WN;
   const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   uint32_t xa[4], wa[4];   // k-step j of 16: the lane's chunk 2 j + g
@@ -100,36 +97,84 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-#pragma unroll
-  for (int s = 0; s < NB - 1; ++s)
-    if (s < n_steps) stage(s, s);
+  constexpr int kReads = MA + MB, kMfmas = MA * MB;
+  u32x4_t fx[2][MA], fw[2][MB];
   int buf = 0;
-  for (int s = 0; s < n_steps; ++s) {
-    // the copies of this step have landed: at most those of the NB - 2 steps behind it are still on their way
-    if (n_steps - 1 - s >= NB - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * PER) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");   // ... everybody's; and everybody is done with the buffer that is refilled now
-    if (s + NB - 1 < n_steps) stage(s + NB - 1, buf == 0 ? NB - 1 : buf - 1);
-    const uint32_t base = (uint32_t)(buf * kBuf);
-    u32x4_t fx[2][MA], fw[2][MB];
-    auto read = [&](auto J) __attribute__((always_inline)) {
-      constexpr int j = decltype(J)::value;
-      static_for<0, MA>([&](auto I) { fx[j & 1][decltype(I)::value] = lds_read128<decltype(I)::value * 32 * kRowBytes>(xa[j] + base); });
-      static_for<0, MB>([&](auto I) { fw[j & 1][decltype(I)::value] = lds_read128<decltype(I)::value * 32 * kRowBytes>(wa[j] + base); });
+  auto read = [&](auto J, auto R) __attribute__((always_inline)) {
+    constexpr int j = decltype(J)::value, r = decltype(R)::value;
+    if constexpr (r < MA) fx[j & 1][r] = lds_read128<r * 32 * kRowBytes>(xa[j] + (uint32_t)(buf * kBuf));
+    else fw[j & 1][r - MA] = lds_read128<(r - MA) * 32 * kRowBytes>(wa[j] + (uint32_t)(buf * kBuf));
+  };
+  auto arrived = [&](auto J, auto Behind) __attribute__((always_inline)) {   // with Behind reads requested after them
+    constexpr int j = decltype(J)::value, n = decltype(Behind)::value;
+    static_for<0, MA>([&](auto I) { lds_wait<n>(fx[j & 1][decltype(I)::value]); });
+    static_for<0, MB>([&](auto I) { lds_wait<n>(fw[j & 1][decltype(I)::value]); });
+  };
+  using std::integral_constant;
+  using zero = integral_constant<int, 0>;
+  if constexpr (kMfmas > 2) {
+    // The barrier stands in front of a step's last k-step: the next step's copies have landed there (everybody's, once it is passed), so that
+    // its first fragments are read between this step's last MFMAs; and this step's buffer, read out by then, is refilled.  The matrix pipe
+    // does not stand for the reads between two steps: a step of the 256 x 128 tile 0.74 us, in the order below 0.82.
+    constexpr auto reads_before = [](int i) { return 2 * i >= kMfmas ? kReads : 2 * i * kReads / kMfmas; };   // with the first half of the MFMAs
+    auto multiply = [&](auto J, auto Copies, int s, int refill) __attribute__((always_inline)) {
+      constexpr int j = decltype(J)::value, next = (j + 1) & 3;
+      static_for<0, kMfmas>([&](auto I) {
+        constexpr int i = decltype(I)::value, p = i / MB, q = i % MB;
+        static_for<reads_before(i), reads_before(i + 1)>([&](auto R) { read(integral_constant<int, next>{}, R); });
+        if constexpr (decltype(Copies)::value) static_for<i * PER / kMfmas, (i + 1) * PER / kMfmas>([&](auto C) { copy(s + NB, refill, decltype(C)::value); });
+        acc[p][q] = mfma32<BF16>(fx[j & 1][p], fw[j & 1][q], acc[p][q]);
+        __builtin_amdgcn_sched_barrier(0);   // left alone, the scheduler moves MFMAs behind the next k-step's waits
+      });
+      arrived(integral_constant<int, next>{}, zero{});
     };
-    read(std::integral_constant<int, 0>{});
-    static_for<0, 4>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      if constexpr (j < 3) read(std::integral_constant<int, j + 1>{});
-      constexpr int behind = j < 3 ? MA + MB : 0;
-      static_for<0, MA>([&](auto I) { lds_wait<behind>(fx[j & 1][decltype(I)::value]); });
-      static_for<0, MB>([&](auto I) { lds_wait<behind>(fw[j & 1][decltype(I)::value]); });
+    auto step = [&](int s, auto Copies) __attribute__((always_inline)) {
+      static_for<0, 3>([&](auto J) { multiply(J, std::false_type{}, 0, 0); });
+      const int refill = buf;
+      if (decltype(Copies)::value || s + 1 < n_steps) {
+        // copies of the NB - 2 steps behind the next one may still be on their way
+        if (decltype(Copies)::value || n_steps - 1 - s >= NB - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * PER) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");
+        buf = buf == NB - 1 ? 0 : buf + 1;
+      }
+      multiply(integral_constant<int, 3>{}, Copies, s, refill);   // the last step reads its own buffer once more, for nobody
+    };
 #pragma unroll
-      for (int p = 0; p < MA; ++p)
+    for (int s = 0; s < NB; ++s)
+      if (s < n_steps) stage(s, s);
+    if (n_steps >= NB) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 1) * PER) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    static_for<0, kReads>([&](auto R) { read(zero{}, R); });
+    arrived(zero{}, zero{});
+    int s = 0;
+    for (; s + NB < n_steps; ++s) step(s, std::true_type{});
+    for (; s < n_steps; ++s) step(s, std::false_type{});
+  } else {
+    // One or two MFMAs a k-step: memory bounds these tiles.  The order above is no faster here and its deeper queue of copies costs launches
+    // of few steps 2 to 4 us (4096 x 4096 of 200 rows 22.7 against 25.9, 1024 x 8192 of 512 rows 22.7 against 29.5).
 #pragma unroll
-        for (int q = 0; q < MB; ++q) acc[p][q] = mfma32<BF16>(fx[j & 1][p], fw[j & 1][q], acc[p][q]);
-    });
-    buf = buf == NB - 1 ? 0 : buf + 1;
+    for (int s = 0; s < NB - 1; ++s)
+      if (s < n_steps) stage(s, s);
+    for (int s = 0; s < n_steps; ++s) {
+      // the copies of this step have landed: at most those of the NB - 2 steps behind it are still on their way
+      if (n_steps - 1 - s >= NB - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * PER) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_barrier" ::: "memory");   // ... everybody's; and everybody is done with the buffer that is refilled now
+      if (s + NB - 1 < n_steps) stage(s + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+      static_for<0, kReads>([&](auto R) { read(zero{}, R); });
+      static_for<0, 4>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        if constexpr (j < 3) static_for<0, kReads>([&](auto R) { read(integral_constant<int, j + 1>{}, R); });
+        arrived(J, integral_constant<int, (j < 3 ? kReads : 0)>{});
+#pragma unroll
+        for (int p = 0; p < MA; ++p)
+#pragma unroll
+          for (int q = 0; q < MB; ++q) acc[p][q] = mfma32<BF16>(fx[j & 1][p], fw[j & 1][q], acc[p][q]);
+      });
+      buf = buf == NB - 1 ? 0 : buf + 1;
+    }
   }
 #pragma unroll
   for (int q = 0; q < MB; ++q) {
@@ -182,8 +227,9 @@ struct GemmPlan {
   float us = 0.f;
 };
 
-// Tile and number of parts by an estimate of the time; constants measured (us).  3584 features, K = 18944, tile / parts: 64 rows 64 / 1 133,
-// 64 / 4 45, 64 / 8 31, 64 / 16 (two rounds) 37; 512 rows 256 / 1 244, 256 / 4 87, 256 / 8 98, 128 / 2 93, 64 / 1 130.
+// Tile and number of parts by an estimate of the time; constants fitted (us) over 11 shapes of 64 to 1024 rows.  3584 features, K = 18944,
+// tile / parts: 64 rows 64 / 1 133, 64 / 4 45, 64 / 8 31, 64 / 16 (two rounds) 37; 512 rows 256 / 1 225, 256 / 4 80, 256 / 8 97, 128 / 2 93,
+// 64 / 1 130.
 GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
   constexpr int kCUs = 256, kBN = 128;
   const int steps = (int)(K / kBK);
@@ -213,9 +259,9 @@ using namespace sq;
 //  * up to 256 rows and 8192 features the library's tiles fill less than a quarter of the chip: 4608 x 3584 of 64 rows 19.5 / 14.9,
 //    256 rows 35.6 / 22.8; 3584 x 3584 of 128 rows 22.5 / 16.0; 4096 x 4096 of 256 rows 24.3 / 22.3; 2048 x 8192 of 5 rows 19.2 /
 //    13.4; 6144 x 4096 of 200 rows 26.2 / 28.9 is the worst.  More features fill it: 14336 x 4096 of 64 rows 29.6 / 34.1;
-//  * beyond 256 rows where K is at least twice N: 3584 x 18944 of 512 rows 196.7 / 86.3, 1024 rows 187.5 / 150.2; 4096 x 14336 of 512
-//    rows 88.4 / 69.8; 1024 x 8192 of 1024 rows 34.2 / 29.3.  Not 4608 x 3584 (512 rows 32.5 / 36.2) or 4096 x 4096 (30.8 / 30.6);
-//  * beyond 1024 rows only where K is five times N: 3584 x 18944 of 2048 rows 355.7 / 281.8, but 2048 x 8192 of 1500 56.0 / 66.2.
+//  * beyond 256 rows where K is at least twice N: 3584 x 18944 of 512 rows 197.9 / 82, 1024 rows 191.2 / 140; 4096 x 14336 of 512
+//    rows 94.9 / 70.4; 1024 x 8192 of 1024 rows 34.2 / 29.3.  Not 4608 x 3584 (512 rows 32.5 / 36.2) or 4096 x 4096 (30.8 / 30.6);
+//  * beyond 1024 rows only where K is five times N: 3584 x 18944 of 2048 rows 355.7 / 259, but 2048 x 8192 of 1500 56.0 / 66.2.
 extern "C" int32_t sq_linear_preferred(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K < kBK || K % kBK || N % 4) return 0;
   if (M <= 256) return N <= 8192;
