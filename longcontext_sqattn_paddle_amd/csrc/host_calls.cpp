@@ -2,8 +2,8 @@
 // output and the scratch and calls the library, in place of a dozen Python and ctypes steps.  Host side per call: decode over 1531 tokens
 // 14.5 -> 8.2 us (of which two launches are 5), selection of 4096 tokens 10.7 -> 6.5, 777-token prefill 16.0 -> 9.3.
 //
-// Only plain arguments are taken (`plain`): torch tensors on a GPU, strided, not subclassed, wrapped, traced or waiting for
-// a gradient, integers that are Python integers.  For anything else a function returns None before it has done
+// Only plain arguments are taken (`plain`): torch tensors on a GPU, strided, not subclassed, wrapped, waiting for a gradient or
+// carrying a forward-mode tangent, integers that are Python integers.  For anything else a function returns None before it has done
 // anything, and the caller goes the general way through DLPack capsules, which accepts or refuses it as it always has.
 // Returns the output (or a tuple), or the library's error code as an int.
 #include <Python.h>
@@ -67,6 +67,8 @@ bool plain(PyObject* o) {
                                             c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                             c10::DispatchKey::Negative, c10::DispatchKey::Conjugate, c10::DispatchKey::ZeroTensor});
   if (t.key_set().has_any(wrapped)) return false;
+  // a dual tensor shows neither in its type nor in its keys; without autograd metadata there is no tangent to ask for
+  if (t.unsafeGetTensorImpl()->autograd_meta() && t._fw_grad(0).defined()) return false;
   switch (t.scalar_type()) {
     case at::kBFloat16: case at::kHalf: case at::kFloat: case at::kInt: case at::kByte: case at::kChar: return true;
     default: return false;

@@ -186,3 +186,24 @@ def test_modes_and_transforms_see_what_they_saw(monkeypatch):
     a, b, taken = _both(monkeypatch, lambda: torch.vmap(lambda x: attn_decode(x, k, v, "NHD", torch.bfloat16))(torch.stack([q, q])))
     assert taken in ([], [False])
     _same(a, b)
+
+
+def _linear_case():
+    g = torch.Generator(device=DEV).manual_seed(5)
+    mk = lambda *s: torch.randn(s, device=DEV, generator=g).bfloat16()
+    return mk(2, 20, 512), mk(256, 512), mk(256)
+
+
+@pytest.mark.parametrize("which", ["x", "weight", "bias"])
+def test_linear_of_a_prompt_keeps_forward_mode_tangents(which):
+    """A dual tensor is an ordinary GPU tensor without gradient; its tangent goes through the product."""
+    import torch.autograd.forward_ad as fwd
+
+    from longcontext_sqattn_paddle_amd.model_hub.utils import linear
+
+    args = dict(zip(("x", "weight", "bias"), _linear_case()))
+    tangent = torch.ones_like(args[which])
+    with fwd.dual_level():
+        args[which] = fwd.make_dual(args[which], tangent)
+        got, want = fwd.unpack_dual(linear(**args)), fwd.unpack_dual(torch.nn.functional.linear(args["x"], args["weight"], args["bias"]))
+    assert got.tangent is not None and torch.equal(got.tangent, want.tangent) and torch.equal(got.primal, want.primal)
