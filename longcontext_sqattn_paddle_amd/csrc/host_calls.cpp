@@ -3,8 +3,9 @@
 // 14.5 -> 8.2 us (of which two launches are 5), selection of 4096 tokens 10.7 -> 6.5, 777-token prefill 16.0 -> 9.3.
 //
 // Only plain arguments are taken (`plain`): torch tensors on a GPU, strided, not subclassed, wrapped, waiting for a gradient or
-// carrying a forward-mode tangent, integers that are Python integers.  For anything else a function returns None before it has done
-// anything, and the caller goes the general way through DLPack capsules, which accepts or refuses it as it always has.
+// carrying a forward-mode tangent, outside modes, transforms and traces, integers that are Python integers.  For anything else a
+// function returns None before it has done anything, and the caller goes the general way (DLPack capsules, for `linear` torch's own),
+// which accepts or refuses it as it always has.
 // Returns the output (or a tuple), or the library's error code as an int.
 #include <Python.h>
 
@@ -76,11 +77,11 @@ bool plain(PyObject* o) {
 }
 bool plain_or_none(PyObject* o) { return o == Py_None || plain(o); }
 
-// no mode that would want to see the allocations and the call
+// no mode and no recording trace that would want to see the allocations and the call
 bool plain_context() {
   return !c10::impl::dispatch_mode_enabled() && !at::impl::torch_function_mode_enabled() &&
          !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
-         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize);
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize) && !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
 bool is_int(PyObject* o) { return PyLong_CheckExact(o); }

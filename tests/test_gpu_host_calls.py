@@ -207,3 +207,13 @@ def test_linear_of_a_prompt_keeps_forward_mode_tangents(which):
         args[which] = fwd.make_dual(args[which], tangent)
         got, want = fwd.unpack_dual(linear(**args)), fwd.unpack_dual(torch.nn.functional.linear(args["x"], args["weight"], args["bias"]))
     assert got.tangent is not None and torch.equal(got.tangent, want.tangent) and torch.equal(got.primal, want.primal)
+
+
+def test_linear_of_a_prompt_is_seen_by_a_trace():
+    from longcontext_sqattn_paddle_amd.model_hub.utils import linear
+
+    x, w, b = _linear_case()
+    traced = torch.jit.trace(lambda t: linear(t, w, b), (x,), check_trace=False)
+    assert "linear" in str(traced.graph)
+    other = x.flip(0) * 2
+    assert torch.equal(traced(other), torch.nn.functional.linear(other, w, b))
