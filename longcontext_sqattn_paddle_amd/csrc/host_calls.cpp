@@ -10,6 +10,7 @@
 #include <Python.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -227,6 +228,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (w.size(1) != K || !lib.linear_preferred(M, N, K) || !aligned(x) || !aligned(w) || x.device() != w.device() || x.scalar_type() != w.scalar_type() ||
       (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf) || x.numel() >= (int64_t)1 << 31 || w.numel() >= (int64_t)1 << 31)
     Py_RETURN_NONE;
+  // torch's linear computes in the type autocast names
+  if (at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()) Py_RETURN_NONE;
   const bool biased = a[2] != Py_None;
   if (biased) {
     const at::Tensor& b = THPVariable_Unpack(a[2]);

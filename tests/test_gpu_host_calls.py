@@ -217,3 +217,15 @@ def test_linear_of_a_prompt_is_seen_by_a_trace():
     assert "linear" in str(traced.graph)
     other = x.flip(0) * 2
     assert torch.equal(traced(other), torch.nn.functional.linear(other, w, b))
+
+
+def test_linear_of_a_prompt_takes_the_type_autocast_names():
+    from longcontext_sqattn_paddle_amd.model_hub.utils import linear
+
+    x, w, b = _linear_case()
+    with torch.autocast("cuda", dtype=torch.float16):
+        got, want = linear(x, w, b), torch.nn.functional.linear(x, w, b)
+    assert got.dtype == torch.float16 and torch.equal(got, want)
+    with torch.autocast("cuda", dtype=torch.bfloat16):   # the type the operands have: nothing to convert
+        got = linear(x, w, b)
+    assert got.dtype == torch.bfloat16 and torch.equal(got, linear(x, w, b))
