@@ -229,3 +229,14 @@ def test_native_calls_leave_host_tensors_and_other_arguments_alone():
     assert m.topk_select(q, k, k, k, 1, 1, None, None, 0) is None
     with pytest.raises(TypeError):
         m.bind(1)
+
+
+def test_products_of_a_prompt_stay_traceable_for_the_compiler(monkeypatch):
+    """`linear` of many rows inside a compiled region without graph breaks: the compiler cannot look into the native calls."""
+    from longcontext_sqattn_paddle_amd.model_hub import utils
+
+    monkeypatch.setattr(utils, "_need_gpu", lambda *ts: None)   # the trace needs no GPU
+    x, w, b = torch.randn(20, 64), torch.randn(32, 64), torch.randn(32)
+    torch._dynamo.reset()
+    compiled = torch.compile(lambda t: utils.linear(t, w, b), backend="eager", fullgraph=True)
+    assert torch.equal(compiled(x), torch.nn.functional.linear(x, w, b))
