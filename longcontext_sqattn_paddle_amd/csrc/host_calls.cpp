@@ -257,6 +257,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (bytes) dws.emplace(ws);
     rc = lib.linear(&dx, &dw, db ? &*db : nullptr, &dout, dws ? &*dws : nullptr, stream);
   }
+  if (rc == SQ_EDEVICE) Py_RETURN_NONE;   // the operands' GPU is not the current one: refused before any launch, torch's linear changes over to it
   if (rc != SQ_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(o);
   END_HANDLE_TH_ERRORS

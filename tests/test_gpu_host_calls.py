@@ -229,3 +229,25 @@ def test_linear_of_a_prompt_takes_the_type_autocast_names():
     with torch.autocast("cuda", dtype=torch.bfloat16):   # the type the operands have: nothing to convert
         got = linear(x, w, b)
     assert got.dtype == torch.bfloat16 and torch.equal(got, linear(x, w, b))
+
+
+def test_linear_of_a_prompt_on_a_gpu_that_is_not_current():
+    """`sq_linear` refuses tensors of another GPU than the current one, torch's linear does not.  One GPU is enough to see it: the
+    library's product is replaced by one that returns that refusal."""
+    import ctypes
+
+    from longcontext_sqattn_paddle_amd.model_hub.utils import linear
+
+    x, w, b = _linear_case()
+    m = N.host_calls()
+    addresses = [ctypes.cast(getattr(N.lib(), name), ctypes.c_void_p).value for name in N._HOST_CALLS_USE]
+    refuse = ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_void_p] * 6)(lambda *a: N.SQ_EDEVICE)
+    other = list(addresses)
+    other[N._HOST_CALLS_USE.index("sq_linear")] = ctypes.cast(refuse, ctypes.c_void_p).value
+    try:
+        m.bind(*other)
+        assert m.linear(x, w, b, N.current_stream(x.device)) is None
+        assert torch.equal(linear(x, w, b), torch.nn.functional.linear(x, w, b))
+    finally:
+        m.bind(*addresses)
+    assert m.linear(x, w, b, N.current_stream(x.device)) is not None
