@@ -108,7 +108,7 @@ def linear_silu_and_mul(x: torch.Tensor, weight: torch.Tensor, bias: Optional[to
     if norm is not None and not (on_kernel and _norm_fits(norm, rows, K, fuse_norm_rows)):
         x, norm = rmsnorm(x, norm[0], norm[1]), None
     if not on_kernel:
-        return silu_and_mul(torch.nn.functional.linear(x, weight, bias))
+        return silu_and_mul(_product(x, weight, bias))
     x2 = x.reshape(rows, K)
     if x2.stride(-1) != 1 or (rows > 1 and x2.stride(0) % 8) or x2.data_ptr() % 16:
         x2 = x2.contiguous()
@@ -148,7 +148,7 @@ def linear_rope(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     if norm is not None and not (on_kernel and _norm_fits(norm, rows, K, fuse_norm_rows)):
         x, norm = rmsnorm(x, norm[0], norm[1]), None
     if not on_kernel:
-        y = torch.nn.functional.linear(x, weight, bias)
+        y = _product(x, weight, bias)
         if rope_features > 0:   # the rotation works head by head: any split of the rotated part into two groups of heads will do
             flat = y.view(rows, n)
             cut = max(rope_features - head_dim, head_dim) if rope_features > head_dim else rope_features

@@ -263,7 +263,7 @@ def test_linear_rows_views_batch_shapes_and_the_gemm_hand_over():
     NV.check(NV.lib().sq_linear_rows(NV.ptr(b[0]), NV.ptr(b[1]), None, NV.ptr(b[2]), NV.ptr(b[2]), NV.current_stream(rd.device)))
     torch.cuda.synchronize()
     _check_linear(rd.view(4, 768), x.view(4, 512), w, None, r.view(4, 768))
-    # nine rows and more are a GEMM: the wrapper hands them to the BLAS library, the entry point refuses them
+    # nine rows and more are a GEMM (`sq_linear` or the BLAS library): the entry point refuses them
     x9 = torch.randn(9, 512, generator=g).bfloat16()
     out9 = linear(x9.to(DEV), w.to(DEV))
     assert float((out9.float().cpu() - OL.linear(x9, w).float()).abs().max()) <= 2.0 ** -6
@@ -319,10 +319,10 @@ def test_gated_projection_equals_projection_then_silu_and_mul(dtype, M, I, K, bi
         bb = [NV.dl(x), NV.dl(w[:2 * I - 1]), NV.dl(torch.empty(M, I, dtype=dtype, device=DEV))]
         with pytest.raises(AssertionError):
             NV.check(NV.lib().sq_linear_rows_silu_and_mul(NV.ptr(bb[0]), NV.ptr(bb[1]), None, NV.ptr(bb[2]), NV.current_stream(o.device)))
-    # more rows than the kernel takes: the wrapper runs the two passes
+    # more rows than the kernel takes: the wrapper runs the two passes, the product by the route `linear` takes
     if I % 8 == 0:
         x9 = torch.randn(9, K, generator=g).to(dtype).to(DEV)
-        assert torch.equal(linear_silu_and_mul(x9, w, b), silu_and_mul(torch.nn.functional.linear(x9, w, b)))
+        assert torch.equal(linear_silu_and_mul(x9, w, b), silu_and_mul(linear(x9, w, b)))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -355,11 +355,11 @@ def test_rotary_projection_equals_projection_then_rope(dtype, M, Hq, Hkv, D, K, 
     f32 = linear_rope(x, w, b, pos.to(torch.int32), D, (Hq + Hkv) * D, table, max_rows=8)
     assert torch.equal(f32, fused)
     assert torch.equal(linear_rope(x, w, b, pos, D, 0, table, max_rows=8).view(M, n), plain)
-    # more rows than the kernel takes: the two passes
+    # more rows than the kernel takes: the two passes, the product by the route `linear` takes
     x9 = torch.randn(9, 1, K, generator=g).to(dtype).to(DEV)
     p9 = torch.randint(0, 5000, (9, 1), generator=g).to(DEV)
     got = linear_rope(x9, w, b, p9, D, (Hq + Hkv) * D, table).view(9, n)
-    base = torch.nn.functional.linear(x9, w, b).view(9, n)
+    base = linear(x9, w, b).view(9, n)
     q9, k9 = apply_rope_with_cos_sin_cache_inplace(p9, base[:, :Hq * D], base[:, Hq * D:(Hq + Hkv) * D], D, table)
     assert torch.equal(got[:, :Hq * D], q9.reshape(9, -1)) and torch.equal(got[:, Hq * D:(Hq + Hkv) * D], k9.reshape(9, -1))
     assert torch.equal(got[:, (Hq + Hkv) * D:], base[:, (Hq + Hkv) * D:])
