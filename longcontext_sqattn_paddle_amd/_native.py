@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from typing import Optional
 
 import torch
@@ -183,19 +184,37 @@ _HOST_CALLS_USE = ("sq_decode_num_splits", "sq_decode_workspace_bytes", "sq_deco
 _host_calls = None
 
 
+class _NoHostCalls:
+    """Leaves every call to the general way."""
+
+    @staticmethod
+    def _leave(*args):
+        return None
+
+    decode = prefill = topk_select = linear = _leave
+
+
 def host_calls():
     """The native short way of the calls whose kernels are shorter than a call's Python side (csrc/host_calls.cpp), bound to the
-    loaded library.  Its functions return None, having done nothing, for arguments they leave to the general way."""
+    loaded library.  Its functions return None, having done nothing, for arguments they leave to the general way.  That serves
+    every call where the module is missing or was built for another torch."""
     global _host_calls
     if _host_calls is None:
-        if not os.path.exists(HOST_CALLS_PATH):
-            raise RuntimeError(f"{HOST_CALLS_PATH} is missing: build it with `python -m longcontext_sqattn_paddle_amd.build`")
         import importlib.util
 
-        spec = importlib.util.spec_from_file_location("_host_calls", HOST_CALLS_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        module.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _HOST_CALLS_USE))
+        addresses = [ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value for name in _HOST_CALLS_USE]
+        try:
+            spec = importlib.util.spec_from_file_location("_host_calls", HOST_CALLS_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            built = getattr(module, "torch_version", "of an unknown version")
+            if built != str(torch.__version__):
+                raise ImportError(f"built against torch {built}, this is {torch.__version__}")
+            module.bind(*addresses)
+        except ImportError as e:
+            warnings.warn(f"native host calls not available ({e}): short calls take about 6 us longer on the host, and products of a prompt go to the BLAS "
+                          "library; build with `python -m longcontext_sqattn_paddle_amd.build`", RuntimeWarning, stacklevel=3)
+            module = _NoHostCalls()
         _host_calls = module
     return _host_calls
 

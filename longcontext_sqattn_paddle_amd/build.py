@@ -39,7 +39,7 @@ def host_calls_command() -> list:
 
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", sysconfig.get_paths()["include"], "-I", INCLUDE,
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DSQ_TORCH_VERSION="{torch.__version__}"', "-I", sysconfig.get_paths()["include"], "-I", INCLUDE,
             *(x for p in include_paths() for x in ("-isystem", p)), os.path.join(CSRC, HOST_CALLS_SOURCE),
             "-L", torch_lib, "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-o", HOST_CALLS_PATH]
 

@@ -293,4 +293,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_calls(void) { return PyModule_Create(&module); }
+// torch_version: of the headers this was compiled against; the layout of a tensor is that version's
+PyMODINIT_FUNC PyInit__host_calls(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", SQ_TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

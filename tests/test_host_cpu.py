@@ -240,3 +240,24 @@ def test_products_of_a_prompt_stay_traceable_for_the_compiler(monkeypatch):
     torch._dynamo.reset()
     compiled = torch.compile(lambda t: utils.linear(t, w, b), backend="eager", fullgraph=True)
     assert torch.equal(compiled(x), torch.nn.functional.linear(x, w, b))
+
+
+@pytest.mark.parametrize("broken", ["missing", "not a library", "another torch"])
+def test_calls_take_the_general_way_without_the_native_host_calls(monkeypatch, tmp_path, broken):
+    """The native host calls are a short way beside the DLPack one: where they cannot be loaded, or were built against another torch,
+    every call is left to the general way, with one warning."""
+    from longcontext_sqattn_paddle_amd import _native as N
+
+    if broken == "another torch":
+        monkeypatch.setattr(torch, "__version__", "2.0.0")
+    else:
+        path = tmp_path / "_host_calls.so"
+        if broken == "not a library":
+            path.write_bytes(b"nothing")
+        monkeypatch.setattr(N, "HOST_CALLS_PATH", str(path))
+    monkeypatch.setattr(N, "_host_calls", None)
+    with pytest.warns(RuntimeWarning, match="host calls"):
+        m = N.host_calls()
+    for f in (m.decode, m.prefill, m.topk_select, m.linear):
+        assert f(1, 2, 3) is None
+    assert N.host_calls() is m
