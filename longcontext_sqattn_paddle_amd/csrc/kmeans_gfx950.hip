@@ -933,7 +933,8 @@ __global__ __launch_bounds__(1024) void topk_select_kernel(TopkArgs a) {
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk)
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, qf[kk]), __builtin_bit_cast(bf16x8_t, cf[blk][kk]), acc, 0, 0, 0);
-      const float v = max_of_rows(fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])));
+      // from -inf, so that a score that is NaN for every head ranks as in the two-kernel route and not by the sign of the NaN
+      const float v = max_of_rows(fmaxf(fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])), -INFINITY));
       if (q4 == 0) {
         if (parts == 1) sc[c] = v;
         else if (c < a.C) __hip_atomic_store(word + c, ((unsigned long long)a.tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -962,7 +963,7 @@ __global__ __launch_bounds__(1024) void topk_select_kernel(TopkArgs a) {
   const uint32_t key32 = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);   // ordered like the scores
   // ---- 2. histogram between the extremes of the scores (of clusters that hold tokens), weighted by size
   {
-    const bool in = sz > 0 && s == s;
+    const bool in = sz > 0;
     const float hi = max_of_rows(row_max16(in ? s : -INFINITY)), lo = max_of_rows(row_max16(in ? -s : -INFINITY));
     if (lane == 0) {
       s_ext[0][t >> 6] = hi;
@@ -972,12 +973,12 @@ __global__ __launch_bounds__(1024) void topk_select_kernel(TopkArgs a) {
   __syncthreads();
   const float top = row_max16(s_ext[0][lane & 15]), bottom = -row_max16(s_ext[1][lane & 15]);
   // Equal steps of the score.  Where the range is not a positive finite number (equal scores, infinities, nothing to
-  // select) every cluster is in bin 0, i.e. a candidate.  A NaN goes where its key is: above everything, or below.
+  // select) every cluster is in bin 0, i.e. a candidate.
   const float range = top - bottom;
   int bin = 0;
   if (range > 0.f && range < INFINITY) {
     const float x = (top - s) * ((float)(kSelBins - 1) / range);   // a range too small for the quotient: infinite or NaN, bin 0 or the last
-    bin = s == s ? (int)fminf(x, (float)(kSelBins - 1)) : (key32 >> 31 ? 0 : kSelBins - 1);
+    bin = (int)fminf(x, (float)(kSelBins - 1));
   }
   if (sz > 0) atomicAdd(&hw[bin], sz);
   __syncthreads();

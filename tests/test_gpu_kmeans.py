@@ -256,6 +256,36 @@ def test_topk_select_score_patterns(pattern, C):
         assert torch.equal(got.cpu(), KM.topk_select(q, cent, clusters, size, k, groups)), k
 
 
+@pytest.mark.parametrize("C", [64, 1000, 1024, 1100])
+@pytest.mark.parametrize("groups", [1, 3, 16])
+def test_topk_select_scores_that_are_not_numbers_come_last(C, groups):
+    """A NaN score never wins a maximum: a cluster whose centroid holds one ranks with -inf, behind every number (ties by index), a
+    query head that holds one is out of the maximum.  By every route: one workgroup, a shared score phase, two kernels."""
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import topk_select
+
+    print(f"case topk NaN C={C} groups={groups}", flush=True)
+    g = torch.Generator().manual_seed(C + groups)
+    Hkv = 2
+    cent, q = torch.zeros(Hkv, C, 128), torch.zeros(1, Hkv * groups, 128)
+    cent[..., 0] = torch.randn(Hkv, C, generator=g)
+    q[..., 0] = 1.0
+    size = torch.randint(0, 9, (Hkv, C), generator=g, dtype=torch.int32)
+    clusters = torch.randint(0, 100000, (Hkv, C, 9), generator=g, dtype=torch.int32)
+    want_cent = cent.clone()
+    cent[:, ::5, 0], want_cent[:, ::5, 0] = float("nan"), float("-inf")
+    cent[:, 3, 0], want_cent[:, 3, 0] = float("-inf"), float("-inf")
+    want_q = q.clone()
+    if groups > 1:
+        q[0, 1] = float("nan")
+        want_q[0, 1] = q[0, 0]
+    cent, q, want_cent, want_q = (t.bfloat16() for t in (cent, q, want_cent, want_q))
+    cent.view(torch.int16)[:, ::10, 0] ^= -32768   # NaNs of either sign
+    total = int(size.sum(dim=1).max())
+    for k in (7, total // 3, total + 5):
+        got = topk_select(q.to(DEV), cent.to(DEV), clusters.to(DEV), size.to(DEV), k, groups)
+        assert torch.equal(got.cpu(), KM.topk_select(want_q, want_cent, clusters, size, k, groups)), k
+
+
 @pytest.mark.parametrize("B", [1, 16, 25, 80])
 def test_topk_select_replayed_from_a_graph(B):
     """4 B heads share the score phase two, four, eight or sixteen waves a workgroup.  One captured call, replayed over another
