@@ -388,8 +388,8 @@ int sq_linear_rows(const DLTensor* x, const DLTensor* weight, const DLTensor* bi
  * fill the GPU (model_hub/qwen.py:302-326 on a prompt's activation).  x [M, K], weight [N, K], bias [N] or NULL, out [M, N]; bf16 or
  * fp16, all of one dtype; K a multiple of 64, N of 4; last dimensions contiguous, rows of x and weight on 16-byte, of out
  * on 8-byte boundaries, operands below 4 GiB.  fp32 accumulation, the sum plus the bias is rounded once.  workspace:
- * sq_linear_workspace_bytes(M, N, K) bytes (0: may be NULL).  sq_linear_preferred: 1 where this is faster than the BLAS
- * library's product, 0 otherwise.
+ * sq_linear_workspace_bytes(M, N, K) bytes (0: may be NULL).  sq_linear_preferred: 1 for the
+ * sizes where this is mostly faster than the BLAS library's product (a rule on M, N and K, measured), 0 otherwise.
  */
 int32_t sq_linear_preferred(int64_t M, int64_t N, int64_t K);
 size_t sq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);

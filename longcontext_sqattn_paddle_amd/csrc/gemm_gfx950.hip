@@ -227,8 +227,10 @@ struct GemmPlan {
   float us = 0.f;
 };
 
-// Tile and number of parts by an estimate of the time; constants fitted (us) over 11 shapes of 64 to 1024 rows.  3584 features, K = 18944,
-// tile / parts: 64 rows 64 / 1 133, 64 / 4 45, 64 / 8 31, 64 / 16 (two rounds) 37; 512 rows 256 / 1 225, 256 / 4 80, 256 / 8 97, 128 / 2 93,
+// Tile and number of parts by an estimate of the time; constants fitted (us) over 11 shapes of 64 to 1024 rows.  The 256-row tile is charged
+// the 0.82 us a step it took before its fragments were read across the barrier (0.74): with 0.74 another tile is chosen for 235 of
+// 7114 shapes, which then take 2.5 % longer in the mean (152 of them longer).  3584 features, K = 18944,
+// tile / parts: 64 rows 64 / 1 133, 64 / 4 45, 64 / 8 31, 64 / 16 (two rounds) 37; 512 rows 256 / 1 225, 256 / 4 80 (now 78), 256 / 8 97, 128 / 2 93,
 // 64 / 1 130.
 GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
   constexpr int kCUs = 256, kBN = 128;
@@ -255,17 +257,32 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
 
 using namespace sq;
 
-// Where the split product is the faster one.  us, library / here (K, N and M as below; every shape 5 to 2048 rows):
+// Where the split product is mostly the faster one: the BLAS library's time goes by its own tile and split choices for the exact
+// sizes, so no rule on sizes meets every one.  7865 shapes measured (N 64 to 8192, K 64 to 20352 in steps of 64, 5 to 2048 rows; weights
+// cold where they are large), library / here in us:
 //  * up to 256 rows and 8192 features the library's tiles fill less than a quarter of the chip: 4608 x 3584 of 64 rows 19.5 / 14.9,
-//    256 rows 35.6 / 22.8; 3584 x 3584 of 128 rows 22.5 / 16.0; 4096 x 4096 of 256 rows 24.3 / 22.3; 2048 x 8192 of 5 rows 19.2 /
-//    13.4; 6144 x 4096 of 200 rows 26.2 / 28.9 is the worst.  More features fill it: 14336 x 4096 of 64 rows 29.6 / 34.1;
-//  * beyond 256 rows where K is at least twice N: 3584 x 18944 of 512 rows 197.9 / 82, 1024 rows 191.2 / 140; 4096 x 14336 of 512
-//    rows 94.9 / 70.4; 1024 x 8192 of 1024 rows 34.2 / 29.3.  Not 4608 x 3584 (512 rows 32.5 / 36.2) or 4096 x 4096 (30.8 / 30.6);
-//  * beyond 1024 rows only where K is five times N: 3584 x 18944 of 2048 rows 355.7 / 259, but 2048 x 8192 of 1500 56.0 / 66.2.
+//    256 rows 35.6 / 22.8; 3584 x 3584 of 128 rows 22.5 / 16.0; 2048 x 8192 of 5 rows 19.2 / 13.4.  More features fill it: 14336 x 4096
+//    of 64 rows 29.6 / 34.1.  Small products are about as long on either side (K below 2048: 0.85 to 1.2), but a call of the library's
+//    takes 14 us on the host, one of these 5 to 7;
+//  * not few rows of a weight of 64 MB and more whose rows are multiples of 8 KB, which fall on few memory channels here: 8192 x 8192 of 16
+//    rows 31.1 / 43.6, of 64 rows 34.3 / 43.5; 4096 x 16384 of 24 rows 33.8 / 45.7 (58 shapes: 0.87 in the mean);
+//  * not 161 to 255 rows that leave half a 32-row block empty, of 6144 features and more at K of 2048 to 4096: 6144 x 4096 of
+//    200 rows 26.5 / 30.2, 8192 x 3584 of 176 rows 24.5 / 29.5 (54 shapes: 0.95; the whole blocks: 36 shapes, 1.20);
+//  * beyond 256 rows where K is at least twice N: 3584 x 18944 of 512 rows 197 / 78, 1024 rows 190 / 135; 4096 x 14336 of 512
+//    rows 94.9 / 70.4; 1024 x 8192 of 1024 rows 34.2 / 29.3.  Not 4608 x 3584 (512 rows 32.5 / 36.2) or 4096 x 4096 (30.8 / 30.6).
+//    Beyond 640 rows the output itself fills much of the chip where K is short: 1024 x 4096 of 1024 rows 17.8 / 21.8 (37 shapes: 0.85),
+//    3584 x 8192 of 777 rows 54.3 / 63.5 (19 shapes: 0.99);
+//  * beyond 1024 rows only where K is five times N: 3584 x 18944 of 2048 rows 361 / 254, but 2048 x 8192 of 1500 56.0 / 66.2.
+// Of the 7697 shapes taken 46 are more than 2 % slower as calls, by up to 16 % (3072 x 16384 of 2048 rows 180 / 210); in the mean 1.28 times
+// faster on the GPU, 1.8 times as calls.
 extern "C" int32_t sq_linear_preferred(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K < kBK || K % kBK || N % 4) return 0;
-  if (M <= 256) return N <= 8192;
-  if (M <= 1024) return K >= 2 * N;
+  if (M <= 256) {
+    if (N > 8192) return 0;
+    if (K % 4096 == 0 && N * K >= 1 << 25 && M <= (N > 6144 || K >= 4 * N ? 64 : 16)) return 0;
+    return !(M > 160 && M % 32 && N >= 6144 && K >= 2048 && K <= 4096);
+  }
+  if (M <= 1024) return K >= 2 * N && !(M > 640 && ((N >= 1024 && K <= 4096) || (N >= 3072 && K <= 8192)));
   return M <= 2048 && K >= 5 * N;
 }
 

@@ -52,7 +52,7 @@ def _norm_fits(norm, rows: int, K: int, fuse_rows: int = 1) -> bool:
 
 def _product(x, weight, bias):
     """x @ weight.T (+ bias) of more rows than a decode step has: `sq_linear` where splitting the sum over K fills the chip (down_proj of
-    512 rows 197 -> 86 us), the BLAS library otherwise, and for everything that is not a plain tensor or wants a gradient."""
+    512 rows 197 -> 78 us), the BLAS library otherwise, and for everything that is not a plain tensor or wants a gradient."""
     if torch.compiler.is_compiling():   # the compiler cannot look into a native call
         return torch.nn.functional.linear(x, weight, bias)
     y = N.host_calls().linear(x, weight, bias, N.current_stream(x.device))

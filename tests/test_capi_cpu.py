@@ -103,6 +103,16 @@ def test_prefill_rejects_cpu_tensors_and_bad_arguments():
     assert lib.sq_prefill_fwd(None, None, None, None, None, None, None, None, None, None) == N.SQ_EINVAL
 
 
+@pytest.mark.parametrize("M,N_,K,taken", [
+    (5, 3584, 3584, 1), (64, 4608, 3584, 1), (256, 8192, 3584, 1), (2048, 3584, 18944, 1), (1024, 4096, 14336, 1), (640, 1024, 4096, 1),   # faster here
+    (16, 8192, 8192, 0), (24, 4096, 16384, 0), (8, 6144, 8192, 0), (200, 6144, 4096, 0), (176, 8192, 3584, 0),                            # few rows; half-empty blocks
+    (1024, 1024, 4096, 0), (777, 3584, 8192, 0), (1024, 3072, 6144, 0), (64, 14336, 4096, 0), (512, 4096, 4096, 0), (1500, 2048, 8192, 0),
+    (65, 8192, 8192, 1), (17, 6144, 8192, 1), (192, 6144, 4096, 1), (224, 8192, 3584, 1), (256, 6144, 4096, 1),                           # the edges
+    (0, 256, 512, 0), (16, 255, 512, 0), (16, 256, 100, 0), (2049, 3584, 18944, 0)])
+def test_prompt_products_go_to_the_faster_side(M, N_, K, taken):
+    assert N.lib().sq_linear_preferred(M, N_, K) == taken
+
+
 def test_error_mapping():
     with pytest.raises(ValueError):
         _ = N.check(N.SQ_EINVAL)
