@@ -173,3 +173,32 @@ def test_split_blocks_see_all_of_the_first_tile(plan):
     calls = _calls()
     for c, (_, _, work, _) in zip(calls, plan(calls)):
         assert all(c["offset"] + 256 * qb >= 64 for qb, _, _, parts in work if parts > 1), c
+
+
+def test_value_tiles_beside_the_row_maximum_pass(tmp_path):
+    """The calls of the GPU test of that path take it, in one, two and ten rounds; short chunks behind long contexts keep the launch of
+    their own."""
+    src, exe = tmp_path / "beside.cpp", tmp_path / "beside"
+    src.write_text(r"""
+#include <stdio.h>
+#include "prefill_plan.hpp"
+int main() {
+  long long B, Hq, Hkv, Nq, off;
+  int pq;
+  while (scanf("%d %lld %lld %lld %lld %lld", &pq, &B, &Hq, &Hkv, &Nq, &off) == 6) {
+    sq_prefill_params p = {};
+    p.p_quant = pq; p.q_offset = off; p.block_m = 128;
+    sq::LaunchPlan plan;
+    sq::plan_launch(&p, false, B, Hq, Nq, plan);
+    const long long tiles = B * Hkv * ((off + Nq + 63) / 64), idle = B * Hq * ((Nq + 255) / 256);
+    printf("%d %lld\n", plan.n_work > 0 ? 1 + sq::prep_beside_pass(plan.share, tiles, idle) : 0, (tiles + 2 * idle - 1) / (2 * idle));
+  }
+}
+""")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "longcontext_sqattn_paddle_amd", "csrc"),
+                    str(src), "-o", str(exe)], check=True)
+    calls = {(2, 2, 4, 2, 2048, 0): (2, 1), (3, 2, 4, 2, 2048, 0): (2, 1), (2, 1, 8, 8, 2048, 0): (2, 2), (2, 2, 4, 4, 2000, 0): (2, 2), (3, 2, 4, 4, 2000, 0): (2, 2),
+             (2, 1, 14, 2, 300, 2048): (2, 2), (1, 1, 28, 4, 512, 16384): (2, 10), (1, 1, 28, 4, 64, 16384): (1, 19), (2, 1, 3, 1, 200, 3072): (1, 9)}
+    text = "".join(" ".join(map(str, c)) + "\n" for c in calls)
+    out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [tuple(map(int, out[i:i + 2])) for i in range(0, len(out), 2)] == list(calls.values())
