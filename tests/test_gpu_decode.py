@@ -83,7 +83,7 @@ def test_decode_workgroups_dealt_by_length(lens):
 @pytest.mark.parametrize("splits", [0, 1, 2, 31, 32, 33, 63, 64, 65])
 def test_decode_combine_of_few_and_of_many_splits(B, lens, splits):
     """Both combine kernels at the edges of their rounds (32 chains, 64 weights) and of the choice between them (64 splits): closed
-    form, and for a named count the bits of a sequence do not depend on its batch mates, whichever kernel the batch takes."""
+    form, and for a named count the bits of a sequence do not depend on its batch mates (which do not change the kernel then)."""
     print(f"case decode combine B={B} splits={splits} lens={lens}", flush=True)
     q, kc, vc, _ = inputs.decode_inputs(B, 28, 4, 2600, 128, seed=91)
     qh, kh, vh = _to_hnd(q, kc, vc)
@@ -99,6 +99,20 @@ def test_decode_combine_of_few_and_of_many_splits(B, lens, splits):
     if splits:
         alone = _run(q[:1], kc[:1], vc[:1], lens[:1], "NHD", output_dtype=torch.float32, num_splits=splits).cpu()
         assert torch.equal(alone[0], out[0])
+
+
+@pytest.mark.parametrize("L,lens", [(272, [272] * 4), (272, [272, 1, 1, 1]), (512, [512, 300, 7, 0]), (512, [1, 512, 2, 3]), (1024, [1024] * 4),
+                                    (1024, [1, 1, 1024, 1]), (1024, [1024, 1000, 64, 16]), (65536, [65536, 1, 30000, 5]), (65536, [3, 65536, 0, 1])])
+def test_both_decode_combines_give_the_same_bits(L, lens):
+    """Where workgroups go by length, four sequences of 28 query heads (112 rows) take the wide combine and of 32 (128 rows) the
+    four-wave one, over the same splits: 1 to 253 of them per sequence.  Seven of the eight heads of a kv head are the same query."""
+    print(f"case decode combines L={L} lens={lens}", flush=True)
+    q, kc, vc, _ = inputs.decode_inputs(4, 32, 4, L, 128, seed=92)   # [B, 1, Hq, D]
+    seven = q.view(4, 1, 4, 8, 128)[:, :, :, :7].reshape(4, 1, 28, 128).contiguous()
+    few, lse_few = _run(q, kc, vc, lens, "NHD", output_dtype=torch.float32, return_lse=True)
+    wide, lse_wide = _run(seven, kc, vc, lens, "NHD", output_dtype=torch.float32, return_lse=True)
+    assert torch.equal(few.view(4, 4, 8, 128)[:, :, :7], wide.view(4, 4, 7, 128))
+    assert torch.equal(lse_few.view(4, 4, 8)[:, :, :7], lse_wide.view(4, 4, 7))
 
 
 def test_decode_by_length_replayed_from_a_graph_with_changing_lengths():
