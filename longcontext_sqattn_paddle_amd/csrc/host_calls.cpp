@@ -238,13 +238,19 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* const stream = PyLong_AsVoidPtr(a[3]);
   at::Tensor o;
   int rc;
+  bool room = true;
   {
     pybind11::gil_scoped_release no_gil;
     std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = N;
     o = at::empty(shape, x.options());
     const size_t bytes = lib.linear_workspace_bytes(M, N, K);
-    at::Tensor ws = bytes ? scratch(bytes, at::kByte, x) : at::Tensor();
+    at::Tensor ws;
+    try {
+      if (bytes) ws = scratch(bytes, at::kByte, x);
+    } catch (const c10::OutOfMemoryError&) {
+      room = false;   // for the parts, which torch's linear does without
+    }
     Arg dx(x), dw(w), dout(o);
     int64_t x_shape[2] = {M, K}, x_strides[2] = {K, 1}, o_shape[2] = {M, N}, o_strides[2] = {N, 1};
     dx.ndim = dout.ndim = 2;
@@ -254,9 +260,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     dout.strides = o_strides;
     c10::optional<Arg> db, dws;
     if (biased) db.emplace(THPVariable_Unpack(a[2]));
-    if (bytes) dws.emplace(ws);
-    rc = lib.linear(&dx, &dw, db ? &*db : nullptr, &dout, dws ? &*dws : nullptr, stream);
+    if (ws.defined()) dws.emplace(ws);
+    rc = room ? lib.linear(&dx, &dw, db ? &*db : nullptr, &dout, dws ? &*dws : nullptr, stream) : SQ_OK;
   }
+  if (!room) Py_RETURN_NONE;
   if (rc == SQ_EDEVICE) Py_RETURN_NONE;   // the operands' GPU is not the current one: refused before any launch, torch's linear changes over to it
   if (rc != SQ_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(o);

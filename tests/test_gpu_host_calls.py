@@ -251,3 +251,25 @@ def test_linear_of_a_prompt_on_a_gpu_that_is_not_current():
     finally:
         m.bind(*addresses)
     assert m.linear(x, w, b, N.current_stream(x.device)) is not None
+
+
+def test_linear_of_a_prompt_without_memory_for_the_parts():
+    """The split product wants scratch that torch's linear does not (4 x 512 x 3584 fp32 here, 29 MB): where there is no room for it, the
+    product is torch's."""
+    from longcontext_sqattn_paddle_amd.model_hub.utils import linear
+
+    x, w = torch.randn(512, 18944, device=DEV).bfloat16(), torch.randn(3584, 18944, device=DEV).bfloat16()
+    want = torch.nn.functional.linear(x, w)   # and the BLAS library's own scratch is there
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (48 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+    taken = []
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                taken.append(torch.empty(12 << 20, dtype=torch.uint8, device=DEV))
+        taken.pop()
+        got = linear(x, w)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want)
+    assert N.host_calls().linear(x, w, None, N.current_stream(x.device)) is not None
