@@ -261,8 +261,9 @@ int sq_index_add(const DLTensor* value, const DLTensor* idx, DLTensor* out, DLTe
  * max_{h in group} <query[b,h], centroids[g,c]> (ties -> lower c); whole clusters taken in rank order
  * until k tokens are emitted; missing tail = -1.  query bf16 [B,Hq,D]; out int32 [G,k], rows contiguous and at least
  * k apart (it may be the leading columns of a wider list that sq_decode_selected_fwd reads).
- * With 1024 clusters the workgroups of a group share its score phase and hand over through one arrival word per
- * group in the workspace.  The workspace needs no initialisation (any contents are fine) and may be shared with the
+ * From 129 to 1024 clusters the workgroups of a group (several, where few groups fill the GPU) share its score phase and hand over through score words in the workspace
+ * that carry a 32-bit tag of the call.  The workspace needs no initialisation: what it holds is taken for a score only where a word's
+ * upper half happens to be this call's tag, a chance of 2^-32 per stale word.  It may be shared with the
  * other k-means entry points; calls that overlap in time must use different workspaces, as for every entry point
  * that takes one.
  */

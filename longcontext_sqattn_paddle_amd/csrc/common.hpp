@@ -75,8 +75,9 @@ inline bool is_compact(const DLTensor* t) {
 }
 
 // A number of its own for every call that hands results from workgroup to workgroup inside one launch: a word in the
-// workspace that carries it was written by this call, whatever the memory held before.  Never 0, spread over 32 bits
-// (a workspace full of one small number is not mistaken for it), repeats after 2^32 calls.  Defined in capi.hip.
+// workspace that carries it was written by this call, but for a chance of 2^-32 per word that holds something else from before
+// (least covered where a single word is waited for: 129 clusters).  Never 0, spread over 32 bits (a workspace full of one small
+// number is not mistaken for it), repeats after 2^32 calls.  Defined in capi.hip.
 uint32_t call_tag();
 
 // Common checks of one tensor argument: non-null, on a GPU, expected rank, last dim contiguous,

@@ -372,8 +372,9 @@ __device__ __forceinline__ uint4 pack8(const f32x16_t& s, int t) {
 //   MODE 2  fp16(e4m3(p*sc)*inv)    block absmax scale a: sc = 448/a, inv = a/448
 //   MODE 3  fp16(e4m3(p448))        p448 = 448*p, the factor folded into the exponent; the 1/448 cancels in
 //                                   acc/l because l is accumulated from p448 as well
-// MODE 2's largest product rounds to 448 (the block's maximum times 448 / maximum is within two units in the last place of it), so
-// nothing has to be clamped.
+// MODE 2's factors come from an approximate reciprocal (1 unit in the last place) and a multiplication by 1/448 where the formula divides: sc and
+// inv are within two units in the last place of fp32 of it (outputs move by 2.5e-5, relative, under a grid of 2^-4).  Its largest
+// product still rounds to 448, so nothing has to be clamped.
 template <int MODE>
 __device__ __forceinline__ void quant_pack4(float p0, float p1, float p2, float p3, uint32_t& w0, uint32_t& w1, float sc = 448.f, float inv = 1.0f / 448.0f) {
   if constexpr (MODE == 0) {
@@ -1281,7 +1282,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
             for (int j = 0; j < 4; ++j) S[sb][e + j] = __builtin_amdgcn_exp2f(S[sb][e + j]);
           } else {
             if constexpr (i == 8) {
-              // 448 / largest probability and its inverse; both 0 or finite where the block's probabilities all vanish
+              // 448 / largest probability (approximate reciprocal) and its inverse; both 0 or finite where the block's probabilities all vanish
               const float amax = __builtin_amdgcn_exp2f(fmaxf(my_top, other_top));
               p_sc = fminf(448.f * __builtin_amdgcn_rcpf(amax), 3e38f);
               p_inv = amax * (1.0f / 448.0f);

@@ -159,8 +159,8 @@ inline void plan_launch(const sq_prefill_params* p, bool own4, int64_t B, int64_
 
 // Whether the row-maximum pass of a split launch also forms the V^T tiles, two at a time in each of its workgroups that have no
 // part to look at (one per query block): where they are done with it before the parts are, at 1.3 us a round against
-// 0.6 us a tile.  4096 tokens, 4 / 1 heads, mode 2 (1 round, shares of 16) 64.4 -> 59.3 us; 512 rows behind 16384 tokens, 28 / 4
-// heads, mode 1 (10 rounds, shares of 66) 224 -> 214.  Beyond it the pass would wait for them: 64 rows behind 16384 tokens (19 rounds, shares of
+// 0.6 us a tile.  4096 tokens, 4 / 1 heads, mode 2 (1 round, shares of 10) 64.4 -> 59.3 us; 512 rows behind 16384 tokens, 28 / 4
+// heads, mode 1 (10 rounds, shares of 65) 224 -> 214.  Beyond it the pass would wait for them: 64 rows behind 16384 tokens (19 rounds, shares of
 // 29) keep the launch of their own.
 inline bool prep_beside_pass(int share, int64_t v_tiles, int64_t idle) { return 1.3f * (float)((v_tiles + 2 * idle - 1) / (2 * idle)) <= 0.6f * share + 1.f; }
 

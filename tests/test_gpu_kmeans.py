@@ -191,9 +191,9 @@ def _shared_phase_case(seed):
 
 
 @pytest.mark.parametrize("fill", ["ones", "random", "finished", "other_shape"])
-def test_topk_select_arrival_words_need_no_initialisation(fill):
-    """The arrival words of the shared score phase live in the caller's workspace and are never cleared by the host.
-    Whatever the memory holds -- all bits set, random words, the word a finished call leaves, or the words of a call
+def test_topk_select_tagged_words_need_no_initialisation(fill):
+    """The tagged score words of the shared score phase live in the caller's workspace and are never cleared by the host.
+    Whatever the memory holds -- all bits set, random words, the words a finished call leaves, or those of a call
     with another number of heads -- the first call over it must select what the oracle selects."""
     from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _workspace, topk_select
 
