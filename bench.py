@@ -53,7 +53,7 @@ def log(*a):
 
 
 def prefill_inputs(torch, N):
-    """BASELINE config 2's seeded inputs (CPU generator), uploaded once: q [1,28,N,128], k/v [1,4,N,128]."""
+    """The prefill's seeded inputs (CPU generator), uploaded once: q [1,28,N,128], k/v [1,4,N,128]."""
     from longcontext_sqattn_paddle_amd import workloads
 
     dev = torch.device("cuda:0")
@@ -676,7 +676,7 @@ def time_calibration(torch, N, iters=3):
 
 
 def time_kmeans(torch, iters=10):
-    """BASELINE config 4 at its shape (4 kv heads x 131072 tokens x 128, 1024 centroids): one Lloyd iteration (assign +
+    """K-means of a layer's keys (4 kv heads x 131072 tokens x 128, 1024 centroids): one Lloyd iteration (assign +
     counting sort + exact cluster sums + centroid update), the whole `segment_k_means` of 10 iterations with its value sums
     and reverse index, and the top-k selection behind it.  Two key sets alternate, so that a 134 MB key tensor does not
     simply stay in the 256 MB Infinity Cache between iterations."""
@@ -892,7 +892,7 @@ def main():
         for mode, name, note in ((0, "no_P_quant_fp16_PV", "attn_triton.py:83, is_P_fp8_quant=False (the reference's default)"),
                                  (1, "e4m3_P_reference_rounding_fp16_PV", "attn_triton.py:81-82 op for op: fp16(fp16(e4m3(448 p)) / 448)"),
                                  (3, "e4m3_P_folded_scale_fp16_PV", "the same e4m3 grid, 448 folded into the exponent (build-defined)"),
-                                 (2, "e4m3_P_block_absmax_fp16_PV", "per 64x64 block absmax scale on P (build-defined, BASELINE config 1)"),
+                                 (2, "e4m3_P_block_absmax_fp16_PV", "per 64x64 block absmax scale on P (build-defined)"),
                                  (4, "e4m3_P_static_scale_fp8_PV", "e4m3 V and fp8 MFMA P.V with the static scale 448 (build-defined)")):
             vms, _ = time_prefill(torch, qkv, 3, 1, mode)
             vpeak = PEAK_MFMA_BLEND_TFLOPS if mode >= 4 else PEAK_MFMA_BF16_TFLOPS
@@ -1036,7 +1036,7 @@ def main():
             torch.cuda.empty_cache()
         log(f"[bench] config 5 end to end: {result['e2e']}")
     if not args.no_cpu_baseline:
-        from oracle import cpu_baseline as CB   # the checker's CPU path, timed as the baseline only
+        from oracle import cpu_baseline as CB   # the CPU path, timed as the baseline only
 
         cpu_tflops, threads, dt, n = CB.time_cpu_baseline(budget_s=6.0)
         one_tflops, _, one_dt, one_n = CB.time_cpu_baseline(budget_s=4.0, threads=1)

@@ -136,7 +136,7 @@ def test_store_runs_on_the_callers_stream_and_sync_joins_another_one():
 
 
 def test_full_size_store_128k():
-    """BASELINE's 128K prompt with 4 kv heads: 268 MB into the cache, checked on the device."""
+    """A prompt of 131072 tokens with 4 kv heads: 268 MB into the cache, checked on the device."""
     print("case kv-cache store 128K", flush=True)
     T, H, D = 131072, 4, 128
     g = torch.Generator(device=DEV).manual_seed(9)
