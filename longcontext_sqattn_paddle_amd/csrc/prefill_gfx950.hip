@@ -396,22 +396,26 @@ __device__ __forceinline__ void quant_pack4(float p0, float p1, float p2, float 
   }
 }
 
-// Four neighbouring channels of an output row, `ch` their index in the per-channel scale table, `off` in the output
+// Four neighbouring channels of an output row, `ch` their index in the per-channel scale table
 template <bool PV8>
-__device__ __forceinline__ void store_out4(const PrefillArgs& a, int64_t ch, int64_t off, float v0, float v1, float v2, float v3) {
+__device__ __forceinline__ float4 scaled_out4(const PrefillArgs& a, int64_t ch, float v0, float v1, float v2, float v3) {
   if constexpr (PV8) {  // undo the per-channel V scale
     const float4 isc = *(const float4*)(a.v_inv_scale + ch);
-    v0 *= isc.x;
-    v1 *= isc.y;
-    v2 *= isc.z;
-    v3 *= isc.w;
+    return make_float4(v0 * isc.x, v1 * isc.y, v2 * isc.z, v3 * isc.w);
   }
+  return make_float4(v0, v1, v2, v3);
+}
+
+// ... stored in the output type, `off` their index there
+template <bool PV8>
+__device__ __forceinline__ void store_out4(const PrefillArgs& a, int64_t ch, int64_t off, float v0, float v1, float v2, float v3) {
+  const float4 v = scaled_out4<PV8>(a, ch, v0, v1, v2, v3);
   if (a.out_dtype == 0) {
-    *(uint2*)((uint16_t*)a.out + off) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+    *(uint2*)((uint16_t*)a.out + off) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
   } else if (a.out_dtype == 1) {
-    *(uint2*)((uint16_t*)a.out + off) = make_uint2(pack_f16(v0, v1), pack_f16(v2, v3));
+    *(uint2*)((uint16_t*)a.out + off) = make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
   } else {
-    *(float4*)((float*)a.out + off) = make_float4(v0, v1, v2, v3);
+    *(float4*)((float*)a.out + off) = v;
   }
 }
 
@@ -1644,17 +1648,44 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
     a.part_lm[wslot * 64 + lane] = make_float2(l, m_run);
     return;
   }
-  if (row >= a.Nq) return;
-  const int64_t obase = (int64_t)b * a.o_sb + (int64_t)head * a.o_sh + (int64_t)row * a.o_sn;
   const float inv_l = 1.0f / l;   // one division per row instead of 64 per lane: within 1 ulp of acc / l, before the rounding to the output type
+  const int64_t hbase = (int64_t)b * a.o_sb + (int64_t)head * a.o_sh;
+  const int64_t ch0 = ((int64_t)b * a.Hkv + kvh) * kD;
+  if (a.out_dtype == 2) {
+    if (row < a.Nq) {
+      float* const orow = (float*)a.out + hbase + (int64_t)row * a.o_sn;
 #pragma unroll
-  for (int bd = 0; bd < 4; ++bd)
+      for (int bd = 0; bd < 4; ++bd)
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int d = 32 * bd + 8 * i4 + 4 * g;
-      store_out4<kPV8>(a, ((int64_t)b * a.Hkv + kvh) * kD + d, obase + d, O[bd][4 * i4] * inv_l, O[bd][4 * i4 + 1] * inv_l, O[bd][4 * i4 + 2] * inv_l,
-                       O[bd][4 * i4 + 3] * inv_l);
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int d = 32 * bd + 8 * i4 + 4 * g;
+          *(float4*)(orow + d) = scaled_out4<kPV8>(a, ch0 + d, O[bd][4 * i4] * inv_l, O[bd][4 * i4 + 1] * inv_l, O[bd][4 * i4 + 2] * inv_l, O[bd][4 * i4 + 3] * inv_l);
+        }
     }
+  } else {
+    // A lane holds four channels here and four there of one row: stored as they are, an instruction touches 32 rows, and the
+    // eight waves' 128 such stores took 3.0 us of a workgroup.  Through LDS (8 KB a wave in the K ring, which nobody reads behind
+    // the loop's last barrier; chunk c of row r in slot c ^ (r & 15)) an instruction stores four whole rows: 2.0 us, and
+    // 1.7 us less until the stores have drained and the next workgroup runs (30011 tokens, 28 / 4 heads, relative windows 1295 -> 1259 us;
+    // 8192, absolute windows 422 -> 410; 777 causal 24.0 -> 23.1; 131072 causal, 1.3 ms a workgroup, the same).
+    char* const rows = smem + wave * 8192;
+#pragma unroll
+    for (int bd = 0; bd < 4; ++bd)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int c = 4 * bd + i4;
+        const float4 v = scaled_out4<kPV8>(a, ch0 + 8 * c + 4 * g, O[bd][4 * i4] * inv_l, O[bd][4 * i4 + 1] * inv_l, O[bd][4 * i4 + 2] * inv_l, O[bd][4 * i4 + 3] * inv_l);
+        *(uint2*)(rows + 256 * c32 + ((c ^ ksw) << 4) + 8 * g) =
+            a.out_dtype == 0 ? make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)) : make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
+      }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4), c = lane & 15;
+      if (row_w0 + r < a.Nq)
+        *(uint4*)((uint16_t*)a.out + hbase + (int64_t)(row_w0 + r) * a.o_sn + 8 * c) = *(const uint4*)(rows + 256 * r + ((c ^ (r & 15)) << 4));
+    }
+  }
+  if (row >= a.Nq) return;
   if (a.lse && g == 0) {
     const float lt = (MODE >= 3 && MODE <= 5) ? l * (1.0f / 448.0f) : l;
     a.lse[((int64_t)b * a.Hq + head) * a.Nq + row] = log2f(lt) + m_run;

@@ -229,6 +229,27 @@ def test_nhd_layout_bf16_out_and_gqa_7():
     assert float((o - ref).abs().max()) <= 2 ** -7 * float(ref.abs().max()) + 0.25 * float(ref.pow(2).mean().sqrt())
 
 
+@pytest.mark.parametrize("mode", [0, 2, 5])
+@pytest.mark.parametrize("N,heads", [(1, 2), (31, 2), (257, 2), (290, 128)])
+def test_16_bit_outputs_are_the_rounded_fp32_ones_and_stay_in_their_rows(mode, N, heads):
+    """16-bit outputs leave through LDS, fp32 ones from the accumulators: the same values, rounded once.  (290 rows of 128 heads:
+    workgroups of 256 rows, the others of 128.)  The output is a view with other rows and channels around it."""
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import run_prefill
+
+    print(f"case 16-bit outputs mode={mode} N={N} heads={heads}", flush=True)
+    q, k, v = (t.to(DEV).transpose(1, 2).contiguous() for t in _rand(1, heads, 2, N, 128, 40 + N))
+    for dt in (torch.bfloat16, torch.float16):
+        qd, kd, vd = q.to(dt), k.to(dt), v.to(dt)
+        ref = run_prefill(qd, kd, vd, tensor_layout="NHD", output_dtype=torch.float32, p_quant=mode)
+        around = torch.full((1, N + 40, heads + 1, 136), -7.0, dtype=dt, device=DEV)
+        view = around[:, :N, :heads, :128]
+        run_prefill(qd, kd, vd, tensor_layout="NHD", output_dtype=dt, p_quant=mode, out=view)
+        torch.cuda.synchronize()
+        assert torch.equal(view, ref.to(dt))
+        view.fill_(-7.0)
+        assert bool((around == -7.0).all())
+
+
 def test_fp16_inputs_and_head_dim_64():
     from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
 
