@@ -22,6 +22,7 @@
  *   sq_decode_selected_fwd    no reference counterpart: the same decode over the tokens sq_topk_select picked
  *   sq_kmeans_train           cache_hub/kmeans.py:127-196 (assign launch :147-173, update launch :175-193)
  *   sq_kmeans_train_stateful  the same step inside the iteration loop of segment_k_means (cache_hub/kmeans.py:356-368)
+ *   sq_kmeans_train_bounded   the same once more, for runs of several steps
  *   sq_reverse_index          cache_hub/kmeans.py:233-262
  *   sq_index_add              cache_hub/kmeans.py:307-329
  *   sq_topk_select            no reference counterpart (defined by this build's benchmark configuration)
@@ -248,6 +249,17 @@ int sq_kmeans_train(const DLTensor* data, DLTensor* centroids, DLTensor* idx, DL
 enum { SQ_KMEANS_STATELESS = 0, SQ_KMEANS_KEEP_SUMS = 1, SQ_KMEANS_APPLY_CHANGES = 2 };
 int sq_kmeans_train_stateful(const DLTensor* data, DLTensor* centroids, DLTensor* idx, DLTensor* cnt,
                              DLTensor* workspace, int32_t normalize, int32_t state, void* stream);
+
+/*
+ * sq_kmeans_train_stateful for runs with several APPLY_CHANGES steps behind the KEEP_SUMS one: KEEP_SUMS also prepares, and
+ * APPLY_CHANGES uses, bounds by which the assignment leaves out centroids that cannot win (triangle inequality; the same
+ * idx, centroids and cnt, bit for bit).  Where the data's clusters overlap nothing can be left out, and the steps then walk all
+ * centroids as the other entry does, a few us longer.  Up to 2048 centroids; the workspace (sq_kmeans_workspace_bytes_bounded, 256-byte
+ * aligned) holds the other entry's in front, so sq_reverse_index and sq_index_add take it too.  A run keeps to one of the two entries.
+ */
+size_t sq_kmeans_workspace_bytes_bounded(int64_t groups, int64_t num_tokens, int64_t num_centroids, int64_t dim);
+int sq_kmeans_train_bounded(const DLTensor* data, DLTensor* centroids, DLTensor* idx, DLTensor* cnt,
+                            DLTensor* workspace, int32_t normalize, int32_t state, void* stream);
 
 /* clusters[g,c,0:cnt] = token ids with idx == c in ascending order (rest 0); cluster_size = counts. */
 int sq_reverse_index(const DLTensor* idx, DLTensor* clusters, DLTensor* cluster_size, DLTensor* workspace,

@@ -100,6 +100,8 @@ SYMBOLS = {
     "sq_decode_selected_fwd": (ctypes.c_int, [_P] * 8 + [ctypes.POINTER(DecodeParams), ctypes.c_void_p]),
     "sq_kmeans_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 4),
     "sq_kmeans_train": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int32, ctypes.c_void_p]),
+    "sq_kmeans_workspace_bytes_bounded": (ctypes.c_size_t, [ctypes.c_int64] * 4),
+    "sq_kmeans_train_bounded": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]),
     "sq_kmeans_train_stateful": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]),
     "sq_reverse_index": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_void_p]),
     "sq_index_add": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_void_p]),

@@ -19,18 +19,21 @@ def _require(t, what):
         raise RuntimeError(f"{what} must live on the MI355X (got {t.device}); there is no CPU path")
 
 
-def _workspace(G: int, num_tokens: int, num_centroids: int, device) -> torch.Tensor:
-    need = N.lib().sq_kmeans_workspace_bytes(G, num_tokens, num_centroids, 128)
+def _workspace(G: int, num_tokens: int, num_centroids: int, device, bounded: bool = False) -> torch.Tensor:
+    size = N.lib().sq_kmeans_workspace_bytes_bounded if bounded else N.lib().sq_kmeans_workspace_bytes
+    need = size(G, num_tokens, num_centroids, 128)
     return torch.empty(need, dtype=torch.uint8, device=device)
 
 
 def _triton_k_means_train(data, centroids, max_idx=None, normalize_centroids=True, return_indices=False,
-                          workspace: Optional[torch.Tensor] = None, state: int = N.KMEANS_STATELESS):
+                          workspace: Optional[torch.Tensor] = None, state: int = N.KMEANS_STATELESS, bounded: bool = False):
     """One Lloyd step, centroids updated in place (kmeans.py:127-196).  With `return_indices` also returns
     the assignment and the largest cluster size (a host sync, like the reference's `.item()`, :195).
     `state` (extension, for a run of steps over the same data with the same `max_idx` and `workspace`):
     `N.KMEANS_KEEP_SUMS` leaves the clusters' exact sums in the workspace, `N.KMEANS_APPLY_CHANGES` forms the new
-    centroids from those sums and the tokens that changed cluster instead of re-summing every row (same bits)."""
+    centroids from those sums and the tokens that changed cluster instead of re-summing every row (same bits).
+    `bounded` (for a whole run, with the workspace of `_workspace(..., bounded=True)`): centroids that cannot win are left out of
+    the assignment (`sq_kmeans_train_bounded`, same bits)."""
     _require(data, "data")
     batch_size, num_tokens, dim = data.shape
     num_centroids = centroids.shape[1]
@@ -39,10 +42,10 @@ def _triton_k_means_train(data, centroids, max_idx=None, normalize_centroids=Tru
         max_idx = torch.empty((batch_size, num_tokens), dtype=torch.int32, device=data.device)
     data_cnt = torch.empty((batch_size, num_centroids), dtype=torch.int32, device=data.device)
     if workspace is None:
-        workspace = _workspace(batch_size, num_tokens, num_centroids, data.device)
+        workspace = _workspace(batch_size, num_tokens, num_centroids, data.device, bounded)
     b = [N.dl(t) for t in (data, centroids, max_idx, data_cnt, workspace)]
-    N.check(N.lib().sq_kmeans_train_stateful(*[N.ptr(x) for x in b], 1 if normalize_centroids else 0, int(state),
-                                             N.current_stream(data.device)))
+    train = N.lib().sq_kmeans_train_bounded if bounded else N.lib().sq_kmeans_train_stateful
+    N.check(train(*[N.ptr(x) for x in b], 1 if normalize_centroids else 0, int(state), N.current_stream(data.device)))
     if return_indices:
         return centroids, max_idx, int(data_cnt.max().item())
     return centroids
@@ -76,6 +79,15 @@ def triton_index_add(value, max_idx, num_centroids: int, workspace: Optional[tor
 FULL_RESUM_STEPS = 3   # Lloyd steps that re-sum every row before the sums are carried (most tokens still move in them)
 
 
+def _bounded(num_tokens: int, num_centroids: int, carried_steps: int) -> bool:
+    """Whether a run's carried steps leave out centroids that cannot win.  Preparing that takes 30 us and a pass over the rows, bounds 12 us
+    a step, and a step without most of its centroids is bound by its rows: 512 centroids gain little over it.  1024 centroids around
+    512 centres, us with / without: ten steps (seven carried) 4 x 131072 tokens 1102 / 1410, 4 x 70000 828 / 926, 8 x 33000 989 / 1052,
+    4 x 40000 643 / 647; five steps (two carried) 8 x 131072 1540 / 1704, 8 x 60000 830 / 822, 4 x 70000 591 / 572; 512 centroids, ten
+    steps, 4 x 131072 863 / 926, 8 x 20000 511 / 468."""
+    return 1024 <= num_centroids <= 2048 and carried_steps * num_tokens >= 1_750_000
+
+
 def segment_k_means(key, value, num_centroids: int, num_iters: int = 10, num_segments: int = 1):
     """kmeans.py:332-375: strided initial centroids, `num_iters-1` normalised steps on the segmented data,
     one un-normalised step on the whole data, then value sums and the reverse index.
@@ -95,17 +107,19 @@ def segment_k_means(key, value, num_centroids: int, num_iters: int = 10, num_seg
     data = key[:, : num_tokens_per_segment * num_segments].reshape((-1, num_tokens_per_segment, head_dim))
     centroids = centroids.reshape((-1, num_centroids_per_segment, head_dim)).contiguous()
     max_idx = torch.empty((data.shape[0], data.shape[1]), dtype=torch.int32, device=data.device)
-    ws = _workspace(data.shape[0], data.shape[1], num_centroids_per_segment, key.device)
+    one_run = num_segments == 1 and data.shape[1] == num_tokens   # the last step continues on the same tensors
+    bounded = _bounded(data.shape[0] * data.shape[1], num_centroids_per_segment, num_iters - FULL_RESUM_STEPS - (0 if one_run else 1))
+    ws = _workspace(data.shape[0], data.shape[1], num_centroids_per_segment, key.device, bounded)
     carried = False
     for it in range(num_iters - 1):
         state = N.KMEANS_STATELESS if it < FULL_RESUM_STEPS - 1 else (N.KMEANS_APPLY_CHANGES if carried else N.KMEANS_KEEP_SUMS)
         centroids = _triton_k_means_train(data, centroids, max_idx=max_idx, normalize_centroids=True,
-                                          return_indices=False, workspace=ws, state=state)
+                                          return_indices=False, workspace=ws, state=state, bounded=bounded)
         carried = state != N.KMEANS_STATELESS
-    if num_segments == 1 and carried and data.shape[1] == num_tokens:
+    if one_run and carried:
         # the same tensors, the same workspace: the last (un-normalised) step continues from the carried sums
         centroids, max_idx, max_cluster_size = _triton_k_means_train(data, centroids, max_idx=max_idx, normalize_centroids=False,
-                                                                      return_indices=True, workspace=ws, state=N.KMEANS_APPLY_CHANGES)
+                                                                      return_indices=True, workspace=ws, state=N.KMEANS_APPLY_CHANGES, bounded=bounded)
     else:
         data = key.reshape((-1, num_tokens, head_dim))
         centroids = centroids.reshape((-1, num_centroids, head_dim))

@@ -551,3 +551,74 @@ def test_split_centroids_with_special_values(G, N, C, parts):
         got.append(idx[:G].cpu())
     assert int(got[1].min()) >= 0 and int(got[1].max()) < C
     assert torch.equal(got[0], got[1])
+
+
+def _bounded_data(G, N, C, kind, seed):
+    """Rows around C / 2 centres, apart enough that the bounds leave most centroids out, and what they must not be misled by."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    mu = torch.randn(G, max(4, C // 2), 128, device=DEV, generator=g)
+    which = torch.randint(0, mu.shape[1], (G, N), device=DEV, generator=g)
+    sigma = {"overlap": 2.0, "half": 0.6}.get(kind, 0.3)
+    x = torch.gather(mu, 1, which[..., None].expand(G, N, 128)) + sigma * torch.randn(G, N, 128, device=DEV, generator=g)
+    if kind == "same":
+        x = x[:, :1].expand(G, N, 128)
+    if kind == "pairs":    # every row twice: ties wherever both copies are seeds
+        x = x[:, torch.arange(N, device=DEV) // 2]
+    if kind == "zero":
+        x[:, ::5] = 0.0
+    if kind == "nan":
+        x[0, N // 3, 7] = math.nan
+        x[-1, N // 2] = math.nan
+    if kind == "inf":
+        x[0, N // 3, 7] = math.inf
+        x[-1, N // 2, 3] = -math.inf
+    if kind in ("huge", "tiny"):
+        x = x * (1e18 if kind == "huge" else 1e-20)
+    if kind == "offset":
+        x = x + 40.0
+    if kind == "one_sided":   # scores of both signs
+        x[:, ::2] = -x[:, ::2]
+    return x.bfloat16().contiguous()
+
+
+BOUNDED_KINDS = ["apart", "half", "overlap", "same", "pairs", "zero", "nan", "inf", "huge", "tiny", "offset", "one_sided"]
+
+
+# (257 tokens for 2048 centroids: a NaN token seeds eight neighbouring centroids, and what a token without a comparable score gets then
+# already differs between the split and the unsplit assignment)
+@pytest.mark.parametrize("G,N,C,kind", [(G, N, C, kind) for G, N, C in [(2, 700, 64), (1, 257, 2048), (3, 5000, 1056), (2, 12289, 512), (1, 40, 32)]
+                                        for kind in BOUNDED_KINDS if not (C > N and kind in ("nan", "inf"))])
+def test_bounded_steps_have_the_bits_of_stateful_ones(G, N, C, kind):
+    """`sq_kmeans_train_bounded` against `sq_kmeans_train_stateful`: assignment, centroids and sizes after every step, sizes at the
+    edges of its tiles and lists.  One step starts from centroids that somebody else has changed in between."""
+    from longcontext_sqattn_paddle_amd import _native as NV
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _triton_k_means_train, _workspace
+
+    print(f"case bounded k-means G={G} N={N} C={C} {kind}", flush=True)
+    data = _bounded_data(G, N, C, kind, 7 * N + C)
+    seeds = (torch.arange(C, device=DEV) * N // C) % N
+    ca = data[:, seeds].contiguous()
+    cb = ca.clone()
+    ia, ib = (torch.zeros(G, N, dtype=torch.int32, device=DEV) for _ in range(2))
+    wa, wb = _workspace(G, N, C, DEV), _workspace(G, N, C, DEV, bounded=True)
+    wb.view(torch.uint8).fill_(0xA5)
+    for step in range(7):
+        state = NV.KMEANS_STATELESS if step == 0 else (NV.KMEANS_KEEP_SUMS if step == 1 else NV.KMEANS_APPLY_CHANGES)
+        if step == 4:
+            for c in (ca, cb):
+                c.copy_(c.roll(3, dims=1))
+        norm = step < 6
+        ra = _triton_k_means_train(data, ca, max_idx=ia, normalize_centroids=norm, return_indices=True, workspace=wa, state=state)
+        rb = _triton_k_means_train(data, cb, max_idx=ib, normalize_centroids=norm, return_indices=True, workspace=wb, state=state, bounded=True)
+        assert torch.equal(ia, ib), (step, int((ia != ib).sum()))
+        assert torch.equal(ca.view(torch.int16), cb.view(torch.int16)), step
+        assert ra[2] == rb[2]
+
+
+def test_bounded_steps_refuse_more_centroids_than_their_lists_hold():
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _triton_k_means_train
+
+    data = torch.zeros(1, 100, 128, dtype=torch.bfloat16, device=DEV)
+    cent = torch.zeros(1, 2080, 128, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(ValueError, match="more than 2048"):
+        _triton_k_means_train(data, cent, bounded=True)
