@@ -111,7 +111,7 @@ constexpr int kAssignWaves = 4;   // x 64 tokens; two workgroups per CU put two 
 // Tokens are taken in `order`, so a workgroup's 256 belong to a few clusters, and it walks the list of the centroids that can
 // win any of them.  Whatever is not a finite number has everything walked.
 // What it takes is a chain of dependent loads, some 9 us a workgroup, four rounds of them: ids, rows and old clusters, masks, the block of
-// centroids.  4 x 131072 tokens around 512 centres, 1024 centroids: 117 - 130 -> 47 us a step beside 12 us for the bounds, and of a
+// centroids.  4 x 131072 tokens around 512 centres, 1024 centroids: 117 - 130 -> 47 us a step beside 9 us for the bounds, and of a
 // run of ten steps, seven of which have bounds, 1410 -> 1102 us.  Three workgroups per CU (168 registers) spill: 35 us a workgroup.
 template <bool TRACK, int PARTS, bool NEAR = false>
 __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(AssignArgs a) {
@@ -544,9 +544,8 @@ struct BoundsArgs {
 constexpr int kBoundsWaves = 8, kPairSample = 8;
 __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(BoundsArgs a) {
   // rows of 256 bytes, chunk c of row r in slot c ^ (r & 15): centroids a, used centroids a, a block of centroids j per wave
+  // (80 KB and not a byte more: two workgroups on a CU, 9.1 us instead of 11.7; what is wanted in addition goes where a wave's block was)
   __shared__ __attribute__((aligned(16))) char smem[(2 + kBoundsWaves) * 32 * 256];
-  __shared__ __attribute__((aligned(16))) float s_norm2[kBoundsWaves][32];
-  __shared__ int32_t s_pairs[kBoundsWaves][32];
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   const int g_id = blockIdx.z;
   const int lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5;
@@ -587,7 +586,8 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
   uu += __shfl_xor(uu, 32);
   uc += __shfl_xor(uc, 32);
   jj += __shfl_xor(jj, 32);
-  if (g == 0) s_norm2[wave][c32] = jj;   // (read by this wave alone)
+  float* const norm2 = (float*)(smem + (2 + wave) * 8192);   // (the wave has read its block, and reads these alone)
+  if (g == 0) norm2[c32] = jj;
   if (jb == 0 && g == 0) {
     a.near.norm2[gc + cl] = cc;
     if (!(cc < INFINITY)) a.near.odd[g_id] = 1;
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
   uint32_t bits = 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const float4 n4 = *(const float4*)&s_norm2[wave][8 * q + 4 * g];
+    const float4 n4 = *(const float4*)&norm2[8 * q + 4 * g];
     const float n[4] = {n4.x, n4.y, n4.z, n4.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -612,14 +612,14 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
   if (jb >= words) bits = 0;   // (a wave without a block of its own: the last rows over again)
   if (g == 0) {
     if (jb < words) a.near.mask[(gc + cl) * words + jb] = bits;
-    s_pairs[wave][c32] = __popc(bits);
+    ((int32_t*)norm2)[32 + c32] = __popc(bits);
   }
   if (blockIdx.x % kPairSample != 0) return;   // (one word to add to, for all of them 5 us)
   __syncthreads();
   if (threadIdx.x < 64) {   // (lane: cluster c32 again)
     unsigned long long sum = 0;
     if (g == 0)
-      for (int w = 0; w < kBoundsWaves; ++w) sum += s_pairs[w][c32];
+      for (int w = 0; w < kBoundsWaves; ++w) sum += ((const int32_t*)(smem + (2 + w) * 8192))[32 + c32];
     sum *= (unsigned long long)size;
 #pragma unroll
     for (int d = 1; d < 32; d <<= 1) sum += __shfl_xor(sum, d);
