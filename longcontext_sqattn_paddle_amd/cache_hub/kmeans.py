@@ -25,15 +25,8 @@ def _workspace(G: int, num_tokens: int, num_centroids: int, device, bounded: boo
     return torch.empty(need, dtype=torch.uint8, device=device)
 
 
-def _triton_k_means_train(data, centroids, max_idx=None, normalize_centroids=True, return_indices=False,
-                          workspace: Optional[torch.Tensor] = None, state: int = N.KMEANS_STATELESS, bounded: bool = False):
-    """One Lloyd step, centroids updated in place (kmeans.py:127-196).  With `return_indices` also returns
-    the assignment and the largest cluster size (a host sync, like the reference's `.item()`, :195).
-    `state` (extension, for a run of steps over the same data with the same `max_idx` and `workspace`):
-    `N.KMEANS_KEEP_SUMS` leaves the clusters' exact sums in the workspace, `N.KMEANS_APPLY_CHANGES` forms the new
-    centroids from those sums and the tokens that changed cluster instead of re-summing every row (same bits).
-    `bounded` (for a whole run, with the workspace of `_workspace(..., bounded=True)`): centroids that cannot win are left out of
-    the assignment (`sq_kmeans_train_bounded`, same bits)."""
+def _step(data, centroids, max_idx, normalize_centroids, workspace, state, bounded):
+    """One Lloyd step, centroids updated in place; (assignment, cluster sizes)."""
     _require(data, "data")
     batch_size, num_tokens, dim = data.shape
     num_centroids = centroids.shape[1]
@@ -46,6 +39,19 @@ def _triton_k_means_train(data, centroids, max_idx=None, normalize_centroids=Tru
     b = [N.dl(t) for t in (data, centroids, max_idx, data_cnt, workspace)]
     train = N.lib().sq_kmeans_train_bounded if bounded else N.lib().sq_kmeans_train_stateful
     N.check(train(*[N.ptr(x) for x in b], 1 if normalize_centroids else 0, int(state), N.current_stream(data.device)))
+    return max_idx, data_cnt
+
+
+def _triton_k_means_train(data, centroids, max_idx=None, normalize_centroids=True, return_indices=False,
+                          workspace: Optional[torch.Tensor] = None, state: int = N.KMEANS_STATELESS, bounded: bool = False):
+    """One Lloyd step, centroids updated in place (kmeans.py:127-196).  With `return_indices` also returns
+    the assignment and the largest cluster size (a host sync, like the reference's `.item()`, :195).
+    `state` (extension, for a run of steps over the same data with the same `max_idx` and `workspace`):
+    `N.KMEANS_KEEP_SUMS` leaves the clusters' exact sums in the workspace, `N.KMEANS_APPLY_CHANGES` forms the new
+    centroids from those sums and the tokens that changed cluster instead of re-summing every row (same bits).
+    `bounded` (for a whole run, with the workspace of `_workspace(..., bounded=True)`): centroids that cannot win are left out of
+    the assignment (`sq_kmeans_train_bounded`, same bits)."""
+    max_idx, data_cnt = _step(data, centroids, max_idx, normalize_centroids, workspace, state, bounded)
     if return_indices:
         return centroids, max_idx, int(data_cnt.max().item())
     return centroids
@@ -118,16 +124,22 @@ def segment_k_means(key, value, num_centroids: int, num_iters: int = 10, num_seg
         carried = state != N.KMEANS_STATELESS
     if one_run and carried:
         # the same tensors, the same workspace: the last (un-normalised) step continues from the carried sums
-        centroids, max_idx, max_cluster_size = _triton_k_means_train(data, centroids, max_idx=max_idx, normalize_centroids=False,
-                                                                      return_indices=True, workspace=ws, state=N.KMEANS_APPLY_CHANGES, bounded=bounded)
+        state = N.KMEANS_APPLY_CHANGES
     else:
         data = key.reshape((-1, num_tokens, head_dim))
         centroids = centroids.reshape((-1, num_centroids, head_dim))
         ws = _workspace(num_groups, num_tokens, num_centroids, key.device)
-        centroids, max_idx, max_cluster_size = _triton_k_means_train(data, centroids, normalize_centroids=False,
-                                                                      return_indices=True, workspace=ws)
+        max_idx, state, bounded = None, N.KMEANS_STATELESS, False
+    max_idx, data_cnt = _step(data, centroids, max_idx, False, ws, state, bounded)
+    # The host has to know the largest cluster before it can lay out the token table.  The number travels while the value sums run, and
+    # the table's launches are there when these end; asked for in front of the sums the GPU waited for the host (4 x 131072 tokens, 1024
+    # centroids 1103 -> 1093 us a run, 4 x 70000 800 -> 791, 8 x 33000 944 -> 938).
+    largest = torch.empty((), dtype=torch.int32, device="cpu", pin_memory=True).copy_(data_cnt.max(), non_blocking=True)
+    known = torch.cuda.Event()
+    known.record(torch.cuda.current_stream(key.device))
     value_sum = triton_index_add(value.reshape((-1, num_tokens, head_dim)), max_idx, num_centroids, workspace=ws)
-    clusters, cluster_size = triton_reverse_index(max_idx, num_centroids, max_cluster_size, workspace=ws)
+    known.synchronize()
+    clusters, cluster_size = triton_reverse_index(max_idx, num_centroids, int(largest), workspace=ws)
     return centroids, value_sum, clusters, cluster_size
 
 
