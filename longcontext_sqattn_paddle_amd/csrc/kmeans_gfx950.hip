@@ -83,6 +83,17 @@ __device__ __forceinline__ float sum16(float v) {
 
 constexpr int kNearMaxC = 2048;
 constexpr uint32_t kInfBits = 0x7f800000u, kNanBits = 0x7fc00000u;
+// Squared lengths the bounds need of a token and of a centroid: 32-bit products of two of them are still good to 1e-7.  Below, they
+// know nothing, and everything is walked.
+constexpr float kFaint = 1e-18f;
+
+// Squared distance of a token x from the line along a centroid c, xx = |x|^2 and on_line = <x, c>^2 / |c|^2.  The fp32 sums are within
+// 3e-5 of the terms, 1e-3 of them covers that.  Not a number: unknown.
+__device__ __forceinline__ float far_squared(float xx, float on_line) {
+  const float d2 = xx - on_line + 1e-3f * (xx + on_line);
+  return xx >= kFaint && d2 >= 0.f ? d2 : __uint_as_float(kNanBits);
+}
+
 constexpr int kAssignWaves = 4;   // x 64 tokens; two workgroups per CU put two waves on every SIMD
 
 // Workgroup = 256 tokens of one group, 64 per wave (two 32-token operand sets in registers): every centroid fragment
@@ -430,14 +441,12 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
       bidx2[tb] = centroid_at(place[tb]);
     }
     if (!dense) {
-      // squared distance from the line along c: |x|^2 - s^2 / |c|^2; the fp32 sums are within 3e-5 of the terms, 1e-3 of them covers that
 #pragma unroll
       for (int tb = 0; tb < 2; ++tb) {
-        const float on_line = bv2[tb] * bv2[tb] / s_norm2[place[tb]];   // (written before the walk's barriers)
-        const float d2 = xx[tb] - on_line + 1e-3f * (xx[tb] + on_line);
+        const float d2 = far_squared(xx[tb], bv2[tb] * bv2[tb] / s_norm2[place[tb]]);   // (written before the walk's barriers)
         if (g == 0 && tok0 + 32 * tb + c32 < a.N) {
           atomicMin(&s_low[place[tb]], bv2[tb] > 0.f ? __float_as_uint(bv2[tb]) : 0u);
-          atomicMax(&s_far2[place[tb]], d2 >= 0.f ? __float_as_uint(d2) : kNanBits);   // not a number: above everything
+          atomicMax(&s_far2[place[tb]], __float_as_uint(d2));   // (not a number: above everything)
         }
       }
       __syncthreads();
@@ -593,8 +602,9 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
     if (!(cc < INFINITY)) a.near.odd[g_id] = 1;
   }
   // Left out where scale <c', c_a - c_j> - slack > R |c_j - c_a|, without the root of the right side.  |x| <= 32 R by the margin in
-  // R, so the slack covers the errors of two scores (2e-5 |x| times the centroids' lengths) and of the products here.
-  const float scale = low / uu, far2 = far * far, len_c = __builtin_amdgcn_sqrtf(cc);
+  // R, so the slack covers the errors of two scores (2e-5 |x| times the centroids' lengths) and of the products here.  Of a faint
+  // centroid nothing is known: scale is no number then, and nothing left out; a lead whose square is hardly above the smallest 32-bit numbers is none.
+  const float scale = fminf(uu, cc) >= kFaint ? low / uu : __uint_as_float(kNanBits), far2 = far * far, len_c = __builtin_amdgcn_sqrtf(cc);
   uint32_t bits = 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -605,7 +615,7 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
       const int i = 4 * q + e;
       const float dist2 = n[e] + cc - 2.f * vc[i] + 1e-3f * (n[e] + cc);
       const float lead = scale * (uc - vu[i]) - 4e-3f * far * (len_c + __builtin_amdgcn_sqrtf(n[e]));
-      if (!(lead > 0.f && lead * lead > far2 * dist2)) bits |= 1u << (8 * q + 4 * g + e);
+      if (!(lead > 1e-18f && lead * lead > far2 * dist2)) bits |= 1u << (8 * q + 4 * g + e);
     }
   }
   bits |= (uint32_t)__shfl_xor((int)bits, 32);
@@ -755,8 +765,7 @@ __global__ __launch_bounds__(256) void near_reach_kernel(ReachArgs a) {
     for (int u = 0; u < kRows; ++u) x[u] = *(const uint4*)(db + (int64_t)ids[SAMPLE ? 0 : min(i0 + 16 * u, m - 1)] * a.d_sn);
 #pragma unroll
     for (int u = 0; u < kRows; ++u) {
-      const float score = sum16(dot8_bf16(x[u], cen, 0.f)), xx = sum16(dot8_bf16(x[u], x[u], 0.f)), on_line = score * score * inv_n;
-      const float d2 = xx - on_line + 1e-3f * (xx + on_line);
+      const float score = sum16(dot8_bf16(x[u], cen, 0.f)), xx = sum16(dot8_bf16(x[u], x[u], 0.f)), d2 = far_squared(xx, score * score * inv_n);
       low = fminf(low, score);
       far2 = far2 != far2 || far2 >= d2 ? far2 : d2;   // keeps what is not a number
     }

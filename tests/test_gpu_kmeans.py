@@ -572,8 +572,12 @@ def _bounded_data(G, N, C, kind, seed):
     if kind == "inf":
         x[0, N // 3, 7] = math.inf
         x[-1, N // 2, 3] = -math.inf
-    if kind in ("huge", "tiny"):
-        x = x * (1e18 if kind == "huge" else 1e-20)
+    if kind in ("huge", "small", "tiny"):
+        x = x * {"huge": 1e18, "small": 1e-7, "tiny": 1e-20}[kind]
+    if kind in ("faint", "faint_means"):   # squares at and below the smallest 32-bit numbers
+        x = x * 1e-23
+    if kind == "signs":
+        x = 2.5e-23 * x.sign()
     if kind == "offset":
         x = x + 40.0
     if kind == "one_sided":   # scores of both signs
@@ -581,12 +585,13 @@ def _bounded_data(G, N, C, kind, seed):
     return x.bfloat16().contiguous()
 
 
-BOUNDED_KINDS = ["apart", "half", "overlap", "same", "pairs", "zero", "nan", "inf", "huge", "tiny", "offset", "one_sided"]
+BOUNDED_KINDS = ["apart", "half", "overlap", "same", "pairs", "zero", "nan", "inf", "huge", "small", "tiny", "faint", "faint_means", "signs",
+                 "offset", "one_sided"]
 
 
 # (257 tokens for 2048 centroids: a NaN token seeds eight neighbouring centroids, and what a token without a comparable score gets then
 # already differs between the split and the unsplit assignment)
-@pytest.mark.parametrize("G,N,C,kind", [(G, N, C, kind) for G, N, C in [(2, 700, 64), (1, 257, 2048), (3, 5000, 1056), (2, 12289, 512), (1, 40, 32)]
+@pytest.mark.parametrize("G,N,C,kind", [(G, N, C, kind) for G, N, C in [(2, 700, 64), (1, 257, 2048), (3, 5000, 1056), (2, 12289, 512), (1, 40, 32), (3, 40000, 512)]
                                         for kind in BOUNDED_KINDS if not (C > N and kind in ("nan", "inf"))])
 def test_bounded_steps_have_the_bits_of_stateful_ones(G, N, C, kind):
     """`sq_kmeans_train_bounded` against `sq_kmeans_train_stateful`: assignment, centroids and sizes after every step, sizes at the
@@ -607,7 +612,7 @@ def test_bounded_steps_have_the_bits_of_stateful_ones(G, N, C, kind):
         if step == 4:
             for c in (ca, cb):
                 c.copy_(c.roll(3, dims=1))
-        norm = step < 6
+        norm = step < 6 and kind != "faint_means"
         ra = _triton_k_means_train(data, ca, max_idx=ia, normalize_centroids=norm, return_indices=True, workspace=wa, state=state)
         rb = _triton_k_means_train(data, cb, max_idx=ib, normalize_centroids=norm, return_indices=True, workspace=wb, state=state, bounded=True)
         assert torch.equal(ia, ib), (step, int((ia != ib).sum()))
