@@ -253,8 +253,10 @@ int sq_kmeans_train_stateful(const DLTensor* data, DLTensor* centroids, DLTensor
 /*
  * sq_kmeans_train_stateful for runs with several APPLY_CHANGES steps behind the KEEP_SUMS one: KEEP_SUMS also prepares, and
  * APPLY_CHANGES uses, bounds by which the assignment leaves out centroids that cannot win (triangle inequality; the same
- * idx, centroids and cnt, bit for bit).  Where the data's clusters overlap nothing can be left out, and the steps then walk all
- * centroids as the other entry does, a few us longer.  Up to 2048 centroids; the workspace (sq_kmeans_workspace_bytes_bounded, 256-byte
+ * idx, centroids and cnt, bit for bit).  Where the data's clusters overlap, or are so small that 256 tokens lie in many of them, hardly
+ * anything can be left out; a run notices, and its steps then walk all centroids as the other entry does, behind a launch that ends
+ * at once.  Where the other entry splits the centroids over the waves of a workgroup (up to about 32768 tokens of all groups together), this
+ * one does the same without bounds.  Up to 2048 centroids; the workspace (sq_kmeans_workspace_bytes_bounded, 256-byte
  * aligned) holds the other entry's in front, so sq_reverse_index and sq_index_add take it too.  A run keeps to one of the two entries.
  */
 size_t sq_kmeans_workspace_bytes_bounded(int64_t groups, int64_t num_tokens, int64_t num_centroids, int64_t dim);

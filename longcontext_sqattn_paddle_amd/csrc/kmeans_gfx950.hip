@@ -42,7 +42,8 @@ struct NearState {
   uint32_t* mask;      // [G,C,C/32] bit j of row a: centroid j can win a token of cluster a
   unsigned long long* pairs;   // pairs of a token and a centroid the masks leave to be looked at, by every eighth block of clusters
   unsigned long long limit;    // more than these: everything is walked, from then on
-  int32_t* dense;      // not 0: that has happened
+  unsigned long long* excess;  // centroids walked by every kWalkSample-th workgroup of the assignment, kWalkShare times, less all; above 0 (signed): the same
+  int32_t* dense;      // not 0: one of the two has happened
   int32_t* odd;        // [G] not 0: a centroid that is no finite number
   int32_t G;
 };
@@ -82,6 +83,7 @@ __device__ __forceinline__ float sum16(float v) {
 }
 
 constexpr int kNearMaxC = 2048;
+constexpr int kWalkSample = 4, kWalkShare = 5;
 constexpr uint32_t kInfBits = 0x7f800000u, kNanBits = 0x7fc00000u;
 // Squared lengths the bounds need of a token and of a centroid: 32-bit products of two of them are still good to 1e-7.  Below, they
 // know nothing, and everything is walked.
@@ -422,6 +424,7 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
       n_list = a.C;
       whole = true;
     }
+    if (!dense && tid == 0 && (tile + g_id) % kWalkSample == 0) atomicAdd(a.near.excess, (unsigned long long)((long long)kWalkShare * n_list - a.C));
     auto centroid_at = [&](int at) { return whole ? at : (int)s_list[at]; };
     if (!dense)
       for (int i = tid; i < n_list; i += kAssignWaves * 64) {
@@ -540,7 +543,10 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
 
 // Which centroids can win a token of which cluster (NEAR).  With data whose clusters overlap nothing can be left out, and the gather
 // and the lists only cost: where more than an eighth of all (token, centroid) pairs remain, everything is walked in the tokens' own
-// order, from that step on (the same run around centres that are 0.6 to 5 standard deviations wide: 0 to 3 % longer than without bounds).
+// order, from that step on.  A cluster's mask does not say what a workgroup walks, which is all that any of its clusters wants: where clusters
+// are small, 256 tokens of many clusters have long lists out of short masks.  So what is walked is counted too, and more than a fifth
+// ends it the same way (ten steps of 16 x 16384 tokens, 1024 centroids around 512 centres of width 0.5: 1.20 times the run without bounds
+// -> 1.08; 64 x 4096, width 0.3: 1.54 -> 1.16; a third, a fifth and an eighth are alike within 1 % at 4 x 131072 and 4 x 70000).
 // A wave takes 32 clusters a (columns) against 32 centroids j (rows), so that a lane has one cluster.
 struct BoundsArgs {
   const uint16_t* cent;   // [G,C,128] bf16
@@ -656,6 +662,7 @@ __global__ __launch_bounds__(1024) void order_start_kernel(OrderArgs a) {
   if (g == 0) {
     if (t == 0) {
       *a.near.pairs = 0;
+      *a.near.excess = 0;
       *a.near.dense = 0;
     }
     for (int i = t; i < a.near.G; i += 1024) a.near.odd[i] = 0;
@@ -1142,8 +1149,9 @@ __global__ __launch_bounds__(kD) void kmeans_update_kernel(UpdateArgs a) {
   uint16_t* row = a.dst + (int64_t)g * a.d_sg + (int64_t)c * a.d_sc;
   if (a.near.order) {
     if (gc == 0 && t == 0) {
-      if (*a.near.pairs > a.near.limit) *a.near.dense = 1;
+      if (*a.near.pairs > a.near.limit || (long long)*a.near.excess > 0) *a.near.dense = 1;
       *a.near.pairs = 0;
+      *a.near.excess = 0;
     }
     a.near.used[gc * kD + t] = row[t];
     if (t == 0) {
@@ -1615,7 +1623,8 @@ struct WsLayout {
     n.far2 = (uint32_t*)take(table_bytes);
     n.norm2 = (float*)take(table_bytes);
     n.pairs = (unsigned long long*)take(ctl_bytes);
-    n.dense = (int32_t*)(n.pairs + 1);
+    n.excess = n.pairs + 1;
+    n.dense = (int32_t*)(n.pairs + 2);
     n.odd = n.dense + 2;
     n.limit = (unsigned long long)G * N * C / 8;
     n.G = (int)G;
@@ -1642,7 +1651,7 @@ WsLayout ws_layout(int64_t G, int64_t N, int64_t C, bool bounded = false) {
     w.used_bytes = up((size_t)G * C * kD * 2);
     w.mask_bytes = up((size_t)G * C * (C / 32) * 4);
     w.table_bytes = up((size_t)G * C * 4);
-    w.ctl_bytes = up((size_t)(4 + G) * 4);
+    w.ctl_bytes = up((size_t)(6 + G) * 4);
   }
   return w;
 }
@@ -1776,17 +1785,23 @@ namespace {
 //  * from 32 groups on, where every group has centroids of its own and a full chip reads them all at once, a launch over half
 //    the CUs, unless its chain is long: 32 groups x 500 tokens, 256 workgroups of four parts against 64 whole ones, 256
 //    centroids 12.1 us whole, 14.1 split, 1024: 27.4 / 26.2; 1000 tokens in two parts 320 centroids 14.3 / 15.7.
+int assign_parts(int64_t G, int64_t N, int64_t C) {
+  constexpr int64_t kCUs = 256;
+  const int64_t blocks = (C + kCB - 1) / kCB;
+  if (!(blocks > 3 || (blocks > 1 && N > 128))) return 1;
+  if (G * ((N + 63) / 64) <= (G < 32 || blocks >= 16 ? kCUs : kCUs / 2)) return 4;
+  return G * ((N + 127) / 128) <= (G < 32 || blocks >= 8 ? kCUs : kCUs / 2) ? 2 : 1;
+}
+
 template <bool TRACK>
 void launch_assign(const AssignArgs& a, int64_t G, hipStream_t st) {
-  constexpr int64_t kCUs = 256;
   const int64_t N = a.N;
   auto grid = [&](int tokens) { return dim3((unsigned)((N + tokens - 1) / tokens), (unsigned)G); };
   const dim3 block(kAssignWaves * 64);
-  const int blocks = (a.C + kCB - 1) / kCB;
-  const bool splits = blocks > 3 || (blocks > 1 && N > 128);
-  if (splits && G * ((N + 63) / 64) <= (G < 32 || blocks >= 16 ? kCUs : kCUs / 2))
+  const int parts = assign_parts(G, N, a.C);
+  if (parts == 4)
     hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 4>), grid(kTileTok / 4), block, 0, st, a);
-  else if (splits && G * ((N + 127) / 128) <= (G < 32 || blocks >= 8 ? kCUs : kCUs / 2))
+  else if (parts == 2)
     hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 2>), grid(kTileTok / 2), block, 0, st, a);
   else
     hipLaunchKernelGGL((kmeans_assign_kernel<TRACK, 1>), grid(kTileTok), block, 0, st, a);
@@ -1809,6 +1824,7 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
   SQ_REQUIRE(C <= kMaxC, SQ_EUNSUPPORTED, "%s: more than %d centroids", who, kMaxC);
   SQ_REQUIRE(N < (1ll << 31) - 65536, SQ_EUNSUPPORTED, "%s: too many tokens", who);
   SQ_REQUIRE(!bounded || C <= kNearMaxC, SQ_EUNSUPPORTED, "%s: more than %d centroids", who, kNearMaxC);
+  const bool near = bounded && assign_parts(G, N, C) == 1;
   const WsLayout w = ws_layout(G, N, C, bounded);
   if ((rc = check_ws(workspace, w.all(), dev, who)) || (rc = check_current_device(dev, who))) return rc;
   hipStream_t st = (hipStream_t)stream;
@@ -1828,7 +1844,7 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
   a.keep_sum = (double*)(wsp + w.sum_offset());
   a.keep_cnt = (int32_t*)(wsp + w.cnt_offset());
   const int mode = normalize ? 2 : 1;
-  a.near = w.near(wsp, G, N);
+  a.near = near ? w.near(wsp, G, N) : NearState{};
   auto launch_bounds = [&]() {
     BoundsArgs ba;
     ba.cent = a.cent;
@@ -1841,7 +1857,7 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
     hipLaunchKernelGGL(kmeans_bounds_kernel, dim3(rows, (rows + kBoundsWaves - 1) / kBoundsWaves, (unsigned)G), dim3(kBoundsWaves * 64), 0, st, ba);
   };
   if (state == SQ_KMEANS_APPLY_CHANGES) {
-    if (bounded) {
+    if (near) {
       const unsigned tiles = (unsigned)((N + kTileTok - 1) / kTileTok);
       launch_bounds();
       hipLaunchKernelGGL((kmeans_assign_kernel<true, 1, true>), dim3(tiles * (unsigned)G), dim3(kAssignWaves * 64), 0, st, a);
@@ -1866,7 +1882,7 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
   SQ_HIP(hipGetLastError());
   if ((rc = run_group(idx, data, wsp, w, st))) return rc;
   if ((rc = run_cluster_sum(data, wsp, w, centroids, (int32_t*)data_of(cnt), mode, st, state == SQ_KMEANS_KEEP_SUMS))) return rc;   // cnt = cluster sizes
-  if (state == SQ_KMEANS_KEEP_SUMS && bounded) {
+  if (state == SQ_KMEANS_KEEP_SUMS && near) {
     OrderArgs o;
     o.idx = a.idx;
     o.cnt = a.keep_cnt;

@@ -591,7 +591,8 @@ BOUNDED_KINDS = ["apart", "half", "overlap", "same", "pairs", "zero", "nan", "in
 
 # (257 tokens for 2048 centroids: a NaN token seeds eight neighbouring centroids, and what a token without a comparable score gets then
 # already differs between the split and the unsplit assignment)
-@pytest.mark.parametrize("G,N,C,kind", [(G, N, C, kind) for G, N, C in [(2, 700, 64), (1, 257, 2048), (3, 5000, 1056), (2, 12289, 512), (1, 40, 32), (3, 40000, 512)]
+@pytest.mark.parametrize("G,N,C,kind", [(G, N, C, kind) for G, N, C in [(2, 700, 64), (1, 257, 2048), (3, 5000, 1056), (2, 12289, 512), (1, 40, 32), (3, 40000, 512),
+                                                             (3, 12001, 1056), (1, 33000, 2048), (64, 1000, 96)]
                                         for kind in BOUNDED_KINDS if not (C > N and kind in ("nan", "inf"))])
 def test_bounded_steps_have_the_bits_of_stateful_ones(G, N, C, kind):
     """`sq_kmeans_train_bounded` against `sq_kmeans_train_stateful`: assignment, centroids and sizes after every step, sizes at the
@@ -618,6 +619,45 @@ def test_bounded_steps_have_the_bits_of_stateful_ones(G, N, C, kind):
         assert torch.equal(ia, ib), (step, int((ia != ib).sum()))
         assert torch.equal(ca.view(torch.int16), cb.view(torch.int16)), step
         assert ra[2] == rb[2]
+
+
+def _walks_everything(workspace, G):
+    """The bounded form's own answer, out of the end of its workspace: nothing is left out any more."""
+    return int(workspace[-((6 + G) * 4) // 256 * 256:].view(torch.int32)[4]) != 0
+
+
+def _run_bounded(data, C, steps=8):
+    from longcontext_sqattn_paddle_amd import _native as NV
+    from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _triton_k_means_train, _workspace
+
+    G, N, _ = data.shape
+    cent = data[:, (torch.arange(C, device=DEV) * N // C) % N].contiguous()
+    idx = torch.zeros(G, N, dtype=torch.int32, device=DEV)
+    ws = _workspace(G, N, C, DEV, bounded=True)
+    ws.fill_(0xA5)
+    for step in range(steps):
+        state = NV.KMEANS_STATELESS if step < 2 else (NV.KMEANS_KEEP_SUMS if step == 2 else NV.KMEANS_APPLY_CHANGES)
+        _triton_k_means_train(data, cent, max_idx=idx, workspace=ws, state=state, bounded=True)
+    torch.cuda.synchronize()
+    return ws
+
+
+# (64 groups of 4 tokens a cluster: short masks, but a workgroup's tokens are in 64 clusters)
+@pytest.mark.parametrize("G,N,C,kind,all_walked", [(3, 12001, 1056, "overlap", True), (3, 12001, 1056, "apart", False), (1, 33000, 2048, "apart", False),
+                                                   (3, 40000, 512, "apart", False), (64, 4096, 1024, "apart", True)])
+def test_bounded_steps_leave_centroids_out_where_that_is_less_work(G, N, C, kind, all_walked):
+    print(f"case bounded k-means, what is walked G={G} N={N} C={C} {kind}", flush=True)
+    assert _walks_everything(_run_bounded(_bounded_data(G, N, C, kind, 7 * N + C), C), G) == all_walked
+
+
+@pytest.mark.parametrize("G,N,C", [(1, 4096, 1024), (3, 5000, 1056), (2, 12289, 512)])
+def test_bounded_steps_are_the_stateful_ones_where_these_split_the_centroids(G, N, C):
+    """Up to about 32768 tokens: the workspace behind the stateful entry's stays as it was."""
+    from longcontext_sqattn_paddle_amd import _native as NV
+
+    print(f"case bounded k-means of few tokens G={G} N={N} C={C}", flush=True)
+    ws = _run_bounded(_bounded_data(G, N, C, "apart", 3), C)
+    assert bool((ws[NV.lib().sq_kmeans_workspace_bytes(G, N, C, 128):] == 0xA5).all())
 
 
 def test_bounded_steps_refuse_more_centroids_than_their_lists_hold():
