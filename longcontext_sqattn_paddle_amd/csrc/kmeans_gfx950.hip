@@ -40,8 +40,8 @@ struct NearState {
   uint32_t* far2;      // [G,C]
   float* norm2;        // [G,C] |c|^2 of the present centroids
   uint32_t* mask;      // [G,C,C/32] bit j of row a: centroid j can win a token of cluster a
-  unsigned long long* pairs;   // pairs of a token and a centroid the masks leave to be looked at, by every eighth block of clusters
-  unsigned long long limit;    // more than these: everything is walked, from then on
+  unsigned long long* pairs;   // pairs of a token and a centroid the masks leave to be looked at, by every kPairSample-th block of clusters
+  unsigned long long limit;    // more than these: everything is walked, from then on (an eighth of all pairs of such blocks)
   unsigned long long* excess;  // centroids walked by every kWalkSample-th workgroup of the assignment, kWalkShare times, less all; above 0 (signed): the same
   int32_t* dense;      // not 0: one of the two has happened
   int32_t* odd;        // [G] not 0: a centroid that is no finite number
@@ -83,7 +83,7 @@ __device__ __forceinline__ float sum16(float v) {
 }
 
 constexpr int kNearMaxC = 2048;
-constexpr int kWalkSample = 4, kWalkShare = 5;
+constexpr int kPairSample = 8, kWalkSample = 4, kWalkShare = 5;
 constexpr uint32_t kInfBits = 0x7f800000u, kNanBits = 0x7fc00000u;
 // Squared lengths the bounds need of a token and of a centroid: 32-bit products of two of them are still good to 1e-7.  Below, they
 // know nothing, and everything is walked.
@@ -554,9 +554,10 @@ struct BoundsArgs {
   const int32_t* cnt;     // [G,C]
   int64_t c_sg, c_sc;
   int32_t C;
+  int32_t every;          // blocks of clusters: every so many-th
 };
 
-constexpr int kBoundsWaves = 8, kPairSample = 8;
+constexpr int kBoundsWaves = 8;
 __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(BoundsArgs a) {
   // rows of 256 bytes, chunk c of row r in slot c ^ (r & 15): centroids a, used centroids a, a block of centroids j per wave
   // (80 KB and not a byte more: two workgroups on a CU, 9.1 us instead of 11.7; what is wanted in addition goes where a wave's block was)
@@ -565,26 +566,25 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
   const int g_id = blockIdx.z;
   const int lane = threadIdx.x & 63, c32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int cl = 32 * blockIdx.x + c32, words = a.C / 32, jb = kBoundsWaves * blockIdx.y + wave;
+  const int block = blockIdx.x * a.every, cl = 32 * block + c32, words = a.C / 32, jb = kBoundsWaves * blockIdx.y + wave;
   const uint16_t* cb = a.cent + (int64_t)g_id * a.c_sg;
   const uint16_t* ub = a.near.used + (int64_t)g_id * a.C * kD;
-  auto copy = [&](const uint16_t* base, int64_t stride, int row0, int block, int q) {   // rows 4 q .. 4 q + 3 of a block of 32
+  auto copy = [&](const uint16_t* base, int64_t stride, int row0, int part, int q) {   // rows 4 q .. 4 q + 3 of a block of 32
     const int r = 4 * q + (lane >> 4);
     __builtin_amdgcn_global_load_lds((const void*)(base + (int64_t)min(row0 + r, a.C - 1) * stride + 8 * ((lane & 15) ^ (r & 15))),
-                                     (lds_ptr_t)(smem + block * 8192 + q * 1024), 16, 0, 0);
+                                     (lds_ptr_t)(smem + part * 8192 + q * 1024), 16, 0, 0);
   };
-  copy(cb, a.c_sc, 32 * blockIdx.x, 0, wave);
-  copy(ub, kD, 32 * blockIdx.x, 1, wave);
+  if (*a.near.dense != 0) return;   // (asked before the rows are fetched: 16 groups of 1024 centroids 8.5 -> 4.6 us, 64 groups 29 -> 5)
+  copy(cb, a.c_sc, 32 * block, 0, wave);
+  copy(ub, kD, 32 * block, 1, wave);
 #pragma unroll
   for (int q = 0; q < 8; ++q) copy(cb, a.c_sc, 32 * jb, 2 + wave, q);
   const int64_t gc = (int64_t)g_id * a.C;
   const float far = a.near.used_far[gc + cl], low = a.near.used_low[gc + cl];
   const int size = a.cnt[gc + cl];
-  const bool dense = *a.near.dense != 0;
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (dense) return;
-  auto frag = [&](int block, int kk) { return *(const uint4*)(smem + block * 8192 + c32 * 256 + (((2 * kk + g) ^ (c32 & 15)) << 4)); };
+  auto frag = [&](int part, int kk) { return *(const uint4*)(smem + part * 8192 + c32 * 256 + (((2 * kk + g) ^ (c32 & 15)) << 4)); };
   float cc = 0.f, uu = 0.f, uc = 0.f, jj = 0.f;
   f32x16_t vu = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, vc = vu;
 #pragma unroll
@@ -630,7 +630,7 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
     if (jb < words) a.near.mask[(gc + cl) * words + jb] = bits;
     ((int32_t*)norm2)[32 + c32] = __popc(bits);
   }
-  if (blockIdx.x % kPairSample != 0) return;   // (one word to add to, for all of them 5 us)
+  if (block % kPairSample != 0) return;   // (one word to add to, for all of them 5 us)
   __syncthreads();
   if (threadIdx.x < 64) {   // (lane: cluster c32 again)
     unsigned long long sum = 0;
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
     sum *= (unsigned long long)size;
 #pragma unroll
     for (int d = 1; d < 32; d <<= 1) sum += __shfl_xor(sum, d);
-    if (lane == 0) atomicAdd(a.near.pairs, sum * kPairSample);
+    if (lane == 0) atomicAdd(a.near.pairs, sum);
   }
 }
 
@@ -723,10 +723,11 @@ __global__ __launch_bounds__(1024) void order_fill_kernel(OrderArgs a) {
 
 // What the bounds want to know of a cluster's tokens, before an assignment has collected it: against the centroid the sums have just
 // given (the one the tokens were assigned by can still be far from their mean: 121 us for the step to come, 62 us from here).
-// SAMPLE: one token from each of up to 16 tiles, out of the grouping of the sums.  Their distances are at most the cluster's, so
-// where the bounds leave too much in by these they do by all, and the order and the pass over all rows can be spared.  Otherwise
-// all tokens, bound by the rows it gathers: 30 us for 134 MB.  Not for clusters of 8 times the mean size and more, which would hold up
-// the launch.
+// SAMPLE: a trial with the clusters whose pairs are counted (every kPairSample-th block of 32), and of each a token from each of up to 16
+// tiles, out of the grouping of the sums.  Their distances are at most the cluster's, so where the bounds leave too much in by these
+// they do by all, and the order and the pass over all rows can be spared (this pass and its bounds, 8 x 33000 tokens, 1024 centroids:
+// 28 us with all clusters, 12 us with these).  Otherwise all tokens, bound by the rows it gathers: 30 us for 134 MB.  Not for clusters of
+// 8 times the mean size and more, which would hold up the launch.
 struct ReachArgs {
   const uint16_t* data;   // [G,N,128] bf16
   const uint16_t* cent;   // [G,C,128] bf16
@@ -742,7 +743,8 @@ template <bool SAMPLE>
 __global__ __launch_bounds__(256) void near_reach_kernel(ReachArgs a) {
   constexpr int kRows = SAMPLE ? 1 : 4;   // in flight per thread
   __shared__ float s_low[16], s_far2[16];
-  const int c = blockIdx.x, g = blockIdx.y, o = threadIdx.x & 15, r = threadIdx.x >> 4;
+  const int c = SAMPLE ? (int)(blockIdx.x / 32 * kPairSample * 32 + blockIdx.x % 32) : (int)blockIdx.x;
+  const int g = blockIdx.y, o = threadIdx.x & 15, r = threadIdx.x >> 4;
   const int64_t gc = (int64_t)g * a.C + c;
   int m = a.cnt[gc];
   if (!SAMPLE) {
@@ -750,7 +752,7 @@ __global__ __launch_bounds__(256) void near_reach_kernel(ReachArgs a) {
     if (*a.near.dense != 0) return;
   }
   const uint4 cen = *(const uint4*)(a.cent + (int64_t)g * a.c_sg + (int64_t)c * a.c_sc + 8 * o);
-  if (SAMPLE && threadIdx.x < 16) *(uint4*)(a.near.used + gc * kD + 8 * o) = cen;
+  if (threadIdx.x < 16) *(uint4*)(a.near.used + gc * kD + 8 * o) = cen;
   if (!SAMPLE && (int64_t)m * a.C >= 8 * (int64_t)a.N) {
     if (threadIdx.x == 0) a.near.used_far[gc] = __uint_as_float(kNanBits);
     return;
@@ -1147,7 +1149,7 @@ __global__ __launch_bounds__(kD) void kmeans_update_kernel(UpdateArgs a) {
   const int cnt = a.cnt[(int64_t)g * a.C + c];
   const int64_t gc = (int64_t)g * a.C + c;
   uint16_t* row = a.dst + (int64_t)g * a.d_sg + (int64_t)c * a.d_sc;
-  if (a.near.order) {
+  if (a.near.order && *a.near.dense == 0) {
     if (gc == 0 && t == 0) {
       if (*a.near.pairs > a.near.limit || (long long)*a.near.excess > 0) *a.near.dense = 1;
       *a.near.pairs = 0;
@@ -1626,7 +1628,8 @@ struct WsLayout {
     n.excess = n.pairs + 1;
     n.dense = (int32_t*)(n.pairs + 2);
     n.odd = n.dense + 2;
-    n.limit = (unsigned long long)G * N * C / 8;
+    const unsigned long long blocks = C / 32, looked_at = (blocks + kPairSample - 1) / kPairSample;
+    n.limit = (unsigned long long)G * N * C / 8 * looked_at / blocks;
     n.G = (int)G;
     return n;
   }
@@ -1845,7 +1848,8 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
   a.keep_cnt = (int32_t*)(wsp + w.cnt_offset());
   const int mode = normalize ? 2 : 1;
   a.near = near ? w.near(wsp, G, N) : NearState{};
-  auto launch_bounds = [&]() {
+  const unsigned blocks = (unsigned)C / 32, looked_at = (blocks + kPairSample - 1) / kPairSample;
+  auto launch_bounds = [&](bool trial) {
     BoundsArgs ba;
     ba.cent = a.cent;
     ba.near = a.near;
@@ -1853,13 +1857,13 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
     ba.c_sg = a.c_sg;
     ba.c_sc = a.c_sc;
     ba.C = (int)C;
-    const unsigned rows = (unsigned)C / 32;
-    hipLaunchKernelGGL(kmeans_bounds_kernel, dim3(rows, (rows + kBoundsWaves - 1) / kBoundsWaves, (unsigned)G), dim3(kBoundsWaves * 64), 0, st, ba);
+    ba.every = trial ? kPairSample : 1;
+    hipLaunchKernelGGL(kmeans_bounds_kernel, dim3(trial ? looked_at : blocks, (blocks + kBoundsWaves - 1) / kBoundsWaves, (unsigned)G), dim3(kBoundsWaves * 64), 0, st, ba);
   };
   if (state == SQ_KMEANS_APPLY_CHANGES) {
     if (near) {
       const unsigned tiles = (unsigned)((N + kTileTok - 1) / kTileTok);
-      launch_bounds();
+      launch_bounds(false);
       hipLaunchKernelGGL((kmeans_assign_kernel<true, 1, true>), dim3(tiles * (unsigned)G), dim3(kAssignWaves * 64), 0, st, a);
     } else {
       launch_assign<true>(a, G, st);
@@ -1905,8 +1909,8 @@ int kmeans_train_impl(const DLTensor* data, DLTensor* centroids, DLTensor* idx, 
     ra.nT = (int)((N + kBigTile - 1) / kBigTile);
     ra.tile_start = (const int32_t*)(wsp + w.off_bytes);
     ra.tile_order = (const int32_t*)(wsp + w.off_bytes + w.hist_bytes);
-    hipLaunchKernelGGL((near_reach_kernel<true>), dim3((unsigned)C, (unsigned)G), dim3(256), 0, st, ra);
-    launch_bounds();
+    hipLaunchKernelGGL((near_reach_kernel<true>), dim3(looked_at * 32, (unsigned)G), dim3(256), 0, st, ra);
+    launch_bounds(true);
     hipLaunchKernelGGL(order_fill_kernel, dim3((unsigned)((N + kOrderTile - 1) / kOrderTile), (unsigned)G), dim3(1024), 0, st, o);
     hipLaunchKernelGGL((near_reach_kernel<false>), dim3((unsigned)C, (unsigned)G), dim3(256), 0, st, ra);
     SQ_HIP(hipGetLastError());

@@ -644,7 +644,7 @@ def _run_bounded(data, C, steps=8):
 
 # (64 groups of 4 tokens a cluster: short masks, but a workgroup's tokens are in 64 clusters)
 @pytest.mark.parametrize("G,N,C,kind,all_walked", [(3, 12001, 1056, "overlap", True), (3, 12001, 1056, "apart", False), (1, 33000, 2048, "apart", False),
-                                                   (3, 40000, 512, "apart", False), (64, 4096, 1024, "apart", True)])
+                                                   (3, 40000, 512, "apart", False), (2, 9001, 64, "apart", False), (64, 4096, 1024, "apart", True)])
 def test_bounded_steps_leave_centroids_out_where_that_is_less_work(G, N, C, kind, all_walked):
     print(f"case bounded k-means, what is walked G={G} N={N} C={C} {kind}", flush=True)
     assert _walks_everything(_run_bounded(_bounded_data(G, N, C, kind, 7 * N + C), C), G) == all_walked
