@@ -85,13 +85,19 @@ def triton_index_add(value, max_idx, num_centroids: int, workspace: Optional[tor
 FULL_RESUM_STEPS = 3   # Lloyd steps that re-sum every row before the sums are carried (most tokens still move in them)
 
 
-def _bounded(num_tokens: int, num_centroids: int, carried_steps: int) -> bool:
-    """Whether a run's carried steps leave out centroids that cannot win.  Preparing that takes 30 us and a pass over the rows, bounds 12 us
-    a step, and a step without most of its centroids is bound by its rows: 512 centroids gain little over it.  1024 centroids around
-    512 centres, us with / without: ten steps (seven carried) 4 x 131072 tokens 1102 / 1410, 4 x 70000 828 / 926, 8 x 33000 989 / 1052,
-    4 x 40000 643 / 647; five steps (two carried) 8 x 131072 1540 / 1704, 8 x 60000 830 / 822, 4 x 70000 591 / 572; 512 centroids, ten
-    steps, 4 x 131072 863 / 926, 8 x 20000 511 / 468."""
-    return 1024 <= num_centroids <= 2048 and carried_steps * num_tokens >= 1_750_000
+def _bounded(groups: int, tokens: int, num_centroids: int, carried_steps: int) -> bool:
+    """Whether a run's carried steps leave out centroids that cannot win, `tokens` those of one group.  In us: what a step saves on keys
+    around C / 2 centres goes with the products left out, less the rows it gathers; its bounds go with the squares of the
+    centroids and its launch is there in any case.  Preparing takes some 50 us once, and a run that finds nothing to leave out has lost
+    20 us and 2 a step, so that much has to be won.  Ten steps (seven carried), us without / with around 512 centres of width 0.3, and
+    with bounds around centres that overlap (width 0.8, without them): 1024 centroids 4 x 131072 tokens 1474 / 1204 (1468, 1437), 4 x 70000 966 /
+    846 (970, 938), 16 x 33000 1683 / 1525 (1725, 1676), 2 x 131072 882 / 846 (877, 849); outside 8 x 33000 992 / 991 (1019, 980), 1 x 131072
+    610 / 649, 16 x 20000 1156 / 1241; 2048 centroids 4 x 65536 1407 / 1230, outside 4 x 33000 1066 / 1072; 512 centroids 8 x 131072
+    1713 / 1612, outside 4 x 131072 985 / 961 (982, 947).  Five steps: 4 x 131072 889 / 848, outside 8 x 70000 979 / 956 (972, 945).
+    Fifty: 4 x 131072 tokens, 512 centroids 3694 / 3284, outside 4 x 20000, 1024 centroids 1727 / 2246."""
+    rows, c = groups * tokens / 131072, num_centroids / 1024
+    saved = (16 * c - 3.5) * rows - 1.75 * groups * c * c - 6
+    return 512 <= num_centroids <= 2048 and carried_steps * saved >= 72
 
 
 def segment_k_means(key, value, num_centroids: int, num_iters: int = 10, num_segments: int = 1):
@@ -114,7 +120,7 @@ def segment_k_means(key, value, num_centroids: int, num_iters: int = 10, num_seg
     centroids = centroids.reshape((-1, num_centroids_per_segment, head_dim)).contiguous()
     max_idx = torch.empty((data.shape[0], data.shape[1]), dtype=torch.int32, device=data.device)
     one_run = num_segments == 1 and data.shape[1] == num_tokens   # the last step continues on the same tensors
-    bounded = _bounded(data.shape[0] * data.shape[1], num_centroids_per_segment, num_iters - FULL_RESUM_STEPS - (0 if one_run else 1))
+    bounded = _bounded(data.shape[0], data.shape[1], num_centroids_per_segment, num_iters - FULL_RESUM_STEPS - (0 if one_run else 1))
     ws = _workspace(data.shape[0], data.shape[1], num_centroids_per_segment, key.device, bounded)
     carried = False
     for it in range(num_iters - 1):

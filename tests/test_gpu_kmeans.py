@@ -667,3 +667,23 @@ def test_bounded_steps_refuse_more_centroids_than_their_lists_hold():
     cent = torch.zeros(1, 2080, 128, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(ValueError, match="more than 2048"):
         _triton_k_means_train(data, cent, bounded=True)
+
+
+# (two segments of an odd number of tokens: the last step starts over, on all tokens and a workspace of its own)
+@pytest.mark.parametrize("G,N,C,iters,segments", [(3, 40000, 1024, 8, 1), (2, 80001, 2048, 9, 2), (2, 80000, 2048, 10, 4), (1, 4096, 1024, 8, 1)])
+@pytest.mark.parametrize("kind", ["apart", "overlap"])
+def test_segment_k_means_is_the_same_with_and_without_bounds(monkeypatch, G, N, C, iters, segments, kind):
+    from longcontext_sqattn_paddle_amd.cache_hub import kmeans as HK
+
+    print(f"case segment_k_means with and without bounds G={G} N={N} C={C} iters={iters} segments={segments} {kind}", flush=True)
+    key = _bounded_data(G, N, C, kind, N + C)
+    value = torch.randn(key.shape, device=DEV, generator=torch.Generator(device=DEV).manual_seed(N)).bfloat16()
+    step, steps = HK._step, []
+    monkeypatch.setattr(HK, "_step", lambda *a: (steps.append(a[-1]), step(*a))[1])
+    got = {}
+    for bounded in (False, True):
+        monkeypatch.setattr(HK, "_bounded", lambda *a: bounded)
+        got[bounded] = HK.segment_k_means(key, value, C, iters, segments)
+    assert steps == [False] * iters + [True] * (iters - (segments > 1)) + [False] * (segments > 1)
+    for a, b in zip(got[False], got[True]):
+        assert torch.equal(a, b)
