@@ -1651,7 +1651,7 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
   const float inv_l = 1.0f / l;   // one division per row instead of 64 per lane: within 1 ulp of acc / l, before the rounding to the output type
   const int64_t hbase = (int64_t)b * a.o_sb + (int64_t)head * a.o_sh;
   const int64_t ch0 = ((int64_t)b * a.Hkv + kvh) * kD;
-  if constexpr (SPLIT) {   // (few workgroups of such a launch end here; with the other form 4096 tokens of 4 / 1 heads, mode 2, 57.4 -> 58.0 us)
+  if (SPLIT || a.out_dtype == 2) {   // (few workgroups of a split launch end here; with the other form 4096 tokens of 4 / 1 heads, mode 2, 57.4 -> 58.0 us)
     if (row < a.Nq)
 #pragma unroll
       for (int bd = 0; bd < 4; ++bd)
@@ -1661,23 +1661,12 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
           store_out4<kPV8>(a, ch0 + d, hbase + (int64_t)row * a.o_sn + d, O[bd][4 * i4] * inv_l, O[bd][4 * i4 + 1] * inv_l, O[bd][4 * i4 + 2] * inv_l,
                            O[bd][4 * i4 + 3] * inv_l);
         }
-  } else if (a.out_dtype == 2) {
-    if (row < a.Nq) {
-      float* const orow = (float*)a.out + hbase + (int64_t)row * a.o_sn;
-#pragma unroll
-      for (int bd = 0; bd < 4; ++bd)
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          const int d = 32 * bd + 8 * i4 + 4 * g;
-          *(float4*)(orow + d) = scaled_out4<kPV8>(a, ch0 + d, O[bd][4 * i4] * inv_l, O[bd][4 * i4 + 1] * inv_l, O[bd][4 * i4 + 2] * inv_l, O[bd][4 * i4 + 3] * inv_l);
-        }
-    }
   } else {
     // A lane holds four channels here and four there of one row: stored as they are, an instruction touches 32 rows, and the
     // eight waves' 128 such stores took 3.0 us of a workgroup.  Through LDS (8 KB a wave in the K ring, which nobody reads behind
     // the loop's last barrier; chunk c of row r in slot c ^ (r & 15)) an instruction stores four whole rows: 2.0 us, and
-    // 1.7 us less until the stores have drained and the next workgroup runs (30011 tokens, 28 / 4 heads, relative windows 1295 -> 1259 us;
-    // 8192, absolute windows 422 -> 410; 777 causal 24.0 -> 23.1; 131072 causal, 1.3 ms a workgroup, the same).
+    // 1.7 us less until the stores have drained and the next workgroup runs (30011 tokens, 28 / 4 heads, relative windows 1264 -> 1243 us;
+    // 8192, absolute windows 416 -> 407; 777 causal 23.9 -> 23.5; 131072 causal, 1.3 ms a workgroup, the same).
     char* const rows = smem + wave * 8192;
 #pragma unroll
     for (int bd = 0; bd < 4; ++bd)
@@ -1688,6 +1677,10 @@ __global__ __launch_bounds__(WAVES * 64) void prefill_kernel(PrefillArgs a) {
         *(uint2*)(rows + 256 * c32 + ((c ^ ksw) << 4) + 8 * g) =
             a.out_dtype == 0 ? make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)) : make_uint2(pack_f16(v.x, v.y), pack_f16(v.z, v.w));
       }
+    // other lanes of this wave read what a lane has written: LDS keeps a wave's order, the compiler has to
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r = 4 * i + (lane >> 4), c = lane & 15;

@@ -250,6 +250,32 @@ def test_16_bit_outputs_are_the_rounded_fp32_ones_and_stay_in_their_rows(mode, N
         assert bool((around == -7.0).all())
 
 
+# 256-row workgroups with windows, those of two query blocks (separate 4-bit operands, 128-row blocks), and 64-row workgroups
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("N", [513, 770])
+@pytest.mark.parametrize("block_m,own4", [(64, False), (128, True), (64, True)])
+def test_16_bit_outputs_of_windowed_launches(mode, N, block_m, own4):
+    from longcontext_sqattn_paddle_amd.sqattn._prefill import prefill_workspace, run_prefill
+
+    heads = 64
+    print(f"case 16-bit outputs mode={mode} N={N} block_m={block_m} own4={own4}", flush=True)
+    q, k, v = (t.to(DEV).transpose(1, 2).contiguous() for t in _rand(1, heads, 2, N, 128, 60 + N))
+    for dt in (torch.bfloat16, torch.float16):
+        qd, kd, vd = q.to(dt), k.to(dt), v.to(dt)
+        kw = dict(tensor_layout="NHD", p_quant=mode, workspace=prefill_workspace(1, 2, N, qd.device),
+                  window=dict(block_m=block_m, sink=64, w8=[128] * heads, w4=[256] * heads))
+        if own4:
+            kw.update(q4=(qd * 0.9).contiguous(), k4=(kd * 1.1).contiguous())
+        ref = run_prefill(qd, kd, vd, output_dtype=torch.float32, **kw)
+        around = torch.full((1, N + 40, heads + 1, 136), -7.0, dtype=dt, device=DEV)
+        view = around[:, :N, :heads, :128]
+        run_prefill(qd, kd, vd, output_dtype=dt, out=view, **kw)
+        torch.cuda.synchronize()
+        assert torch.equal(view, ref.to(dt))
+        view.fill_(-7.0)
+        assert bool((around == -7.0).all())
+
+
 def test_fp16_inputs_and_head_dim_64():
     from longcontext_sqattn_paddle_amd.sqattn.attn_triton import attn_causal
 
