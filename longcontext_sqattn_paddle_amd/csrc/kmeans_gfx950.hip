@@ -42,8 +42,8 @@ struct NearState {
   uint32_t* mask;      // [G,C,C/32] bit j of row a: centroid j can win a token of cluster a
   unsigned long long* pairs;   // pairs of a token and a centroid the masks leave to be looked at, by every kPairSample-th block of clusters
   unsigned long long limit;    // more than these: everything is walked, from then on (an eighth of all pairs of such blocks)
-  unsigned long long* excess;  // centroids walked by every kWalkSample-th workgroup of the assignment, kWalkShare times, less all; above 0 (signed): the same
-  int32_t* dense;      // not 0: one of the two has happened
+  unsigned long long* excess;  // centroids walked by every kWalkSample-th workgroup of the first such assignment, kWalkShare times, less all; above 0 (signed): the same
+  int32_t* dense;      // 1: one of the two has happened; 0: what is walked has not been counted yet
   int32_t* odd;        // [G] not 0: a centroid that is no finite number
   int32_t G;
 };
@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
   // token fragments (B operand of S^T = Cent . Data^T): lane (column = token 32 tb + c32, k-group g)
   const uint16_t* db = a.data + (int64_t)g_id * a.d_sg;
   uint4 tf[2][8];
-  const bool dense = NEAR && (*a.near.dense != 0 || *a.near.pairs > a.near.limit);
+  const int form = NEAR ? *a.near.dense : 0;
+  const bool dense = NEAR && (form == 1 || *a.near.pairs > a.near.limit);
   int tok[2];
 #pragma unroll
   for (int tb = 0; tb < 2; ++tb) {
@@ -424,7 +425,6 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
       n_list = a.C;
       whole = true;
     }
-    if (!dense && tid == 0 && (tile + g_id) % kWalkSample == 0) atomicAdd(a.near.excess, (unsigned long long)((long long)kWalkShare * n_list - a.C));
     auto centroid_at = [&](int at) { return whole ? at : (int)s_list[at]; };
     if (!dense)
       for (int i = tid; i < n_list; i += kAssignWaves * 64) {
@@ -458,6 +458,9 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
           atomicMin(a.near.low + (int64_t)g_id * a.C + centroid_at(i), s_low[i]);
           atomicMax(a.near.far2 + (int64_t)g_id * a.C + centroid_at(i), s_far2[i]);
         }
+      // (a run's first carried step has the longest lists; counted in each, in front of the walk, it was 0.3 - 2 us of a step)
+      if (form == 0 && tid == kAssignWaves * 64 - 1 && (tile + g_id) % kWalkSample == 0)
+        atomicAdd(a.near.excess, (unsigned long long)((long long)kWalkShare * n_list - a.C));
     }
   }
   if constexpr (PARTS > 1) {
@@ -544,9 +547,10 @@ __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(Ass
 // Which centroids can win a token of which cluster (NEAR).  With data whose clusters overlap nothing can be left out, and the gather
 // and the lists only cost: where more than an eighth of all (token, centroid) pairs remain, everything is walked in the tokens' own
 // order, from that step on.  A cluster's mask does not say what a workgroup walks, which is all that any of its clusters wants: where clusters
-// are small, 256 tokens of many clusters have long lists out of short masks.  So what is walked is counted too, and more than a fifth
-// ends it the same way (ten steps of 16 x 16384 tokens, 1024 centroids around 512 centres of width 0.5: 1.20 times the run without bounds
-// -> 1.08; 64 x 4096, width 0.3: 1.54 -> 1.16; a third, a fifth and an eighth are alike within 1 % at 4 x 131072 and 4 x 70000).
+// are small, 256 tokens of many clusters have long lists out of short masks.  So what is walked is counted too, in the first carried step,
+// and more than a fifth ends it the same way (ten steps of 16 x 16384 tokens, 1024 centroids around 512 centres of width 0.5: 1.28 times
+// the run without bounds -> 1.10, and of 64 x 4096, width 0.3: 1.97 -> 1.16, both with the trial's and the bounds' savings below; a
+// third, a fifth and an eighth are alike within 1 % at 4 x 131072 and 4 x 70000).
 // A wave takes 32 clusters a (columns) against 32 centroids j (rows), so that a lane has one cluster.
 struct BoundsArgs {
   const uint16_t* cent;   // [G,C,128] bf16
@@ -574,7 +578,7 @@ __global__ __launch_bounds__(kBoundsWaves * 64) void kmeans_bounds_kernel(Bounds
     __builtin_amdgcn_global_load_lds((const void*)(base + (int64_t)min(row0 + r, a.C - 1) * stride + 8 * ((lane & 15) ^ (r & 15))),
                                      (lds_ptr_t)(smem + part * 8192 + q * 1024), 16, 0, 0);
   };
-  if (*a.near.dense != 0) return;   // (asked before the rows are fetched: 16 groups of 1024 centroids 8.5 -> 4.6 us, 64 groups 29 -> 5)
+  if (*a.near.dense == 1) return;   // (asked before the rows are fetched: 16 groups of 1024 centroids 8.5 -> 4.6 us, 64 groups 29 -> 5)
   copy(cb, a.c_sc, 32 * block, 0, wave);
   copy(ub, kD, 32 * block, 1, wave);
 #pragma unroll
@@ -749,7 +753,7 @@ __global__ __launch_bounds__(256) void near_reach_kernel(ReachArgs a) {
   int m = a.cnt[gc];
   if (!SAMPLE) {
     if (g == 0 && c == 0 && threadIdx.x == 0) *a.near.pairs = 0;
-    if (*a.near.dense != 0) return;
+    if (*a.near.dense == 1) return;
   }
   const uint4 cen = *(const uint4*)(a.cent + (int64_t)g * a.c_sg + (int64_t)c * a.c_sc + 8 * o);
   if (threadIdx.x < 16) *(uint4*)(a.near.used + gc * kD + 8 * o) = cen;
@@ -1149,9 +1153,9 @@ __global__ __launch_bounds__(kD) void kmeans_update_kernel(UpdateArgs a) {
   const int cnt = a.cnt[(int64_t)g * a.C + c];
   const int64_t gc = (int64_t)g * a.C + c;
   uint16_t* row = a.dst + (int64_t)g * a.d_sg + (int64_t)c * a.d_sc;
-  if (a.near.order && *a.near.dense == 0) {
+  if (a.near.order && *a.near.dense != 1) {
     if (gc == 0 && t == 0) {
-      if (*a.near.pairs > a.near.limit || (long long)*a.near.excess > 0) *a.near.dense = 1;
+      *a.near.dense = *a.near.pairs > a.near.limit || (long long)*a.near.excess > 0 ? 1 : 2;
       *a.near.pairs = 0;
       *a.near.excess = 0;
     }

@@ -623,7 +623,7 @@ def test_bounded_steps_have_the_bits_of_stateful_ones(G, N, C, kind):
 
 def _walks_everything(workspace, G):
     """The bounded form's own answer, out of the end of its workspace: nothing is left out any more."""
-    return int(workspace[-((6 + G) * 4) // 256 * 256:].view(torch.int32)[4]) != 0
+    return int(workspace[-((6 + G) * 4) // 256 * 256:].view(torch.int32)[4]) == 1
 
 
 def _run_bounded(data, C, steps=8):
