@@ -705,8 +705,9 @@ def time_kmeans(torch, iters=10):
     us = e0.elapsed_time(e1) / iters * 1e3
     flops = 2.0 * N * C * D * G
     nbytes = G * (N * D * 2 + N * 4 + C * D * 2 * 2 + C * 4)   # keys read once, assignment written, centroids read and written, counts
-    # the iteration loop as segment_k_means runs it: three steps that re-sum every row, the third leaving the exact sums
-    # in the workspace, then steps that only apply the tokens that changed cluster (sq_kmeans_train_stateful).  Each key
+    # an iteration loop: three steps that re-sum every row, the third leaving the exact sums in the workspace, then steps that only
+    # apply the tokens that changed cluster (sq_kmeans_train_stateful).  segment_k_means, timed as a whole below, runs the same and, at this
+    # size, leaves out centroids that cannot win besides (sq_kmeans_train_bounded).  Each key
     # set has its own assignment and workspace (the carried state), and the two alternate as above.
     from longcontext_sqattn_paddle_amd import _native as NV
 
@@ -1018,11 +1019,11 @@ def main():
                             "us_per_iteration_carried_sums": round(us_carried, 1),
                             "frac_of_bound_carried_sums": round(max(t_mfma, t_hbm) / us_carried, 4),
                             "us_per_iteration_mean_of_the_10_iteration_run": round(us_run10, 1),
-                            "carried_sums_note": "the loop of segment_k_means: iterations 1-3 re-sum every row, 4-10 apply only the tokens that changed "
+                            "carried_sums_note": "sq_kmeans_train_stateful: iterations 1-3 re-sum every row, 4-10 apply only the tokens that changed "
                                                  "cluster to the exact sums kept in the workspace (same centroids bit for bit); iterations 4-10 alone, "
                                                  "and the mean over all ten",
                             "segment_k_means_10_iterations_ms": round(full_ms, 3),
-                            "segment_k_means_note": "10 iterations + value sums + reverse index, host wall clock including its one host "
+                            "segment_k_means_note": "10 iterations, 4-10 with bounds (sq_kmeans_train_bounded), + value sums + reverse index, host wall clock including its one host "
                                                     "synchronisation (the reference's Cnt.max().item(), cache_hub/kmeans.py:195)",
                             "topk_select_us": round(topk_us, 1),
                             "topk_shape": "4096 tokens per kv head for one 28-head query, 1024 clusters per kv head"}

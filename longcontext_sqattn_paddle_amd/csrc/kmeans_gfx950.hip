@@ -122,9 +122,9 @@ constexpr int kAssignWaves = 4;   // x 64 tokens; two workgroups per CU put two 
 // distance R from the line along c'.  For all of them <x, c_j - c_a> <= s / |c'|^2 <c', c_j - c_a> + R |c_j - c_a| where the first product
 // is negative, and that takes products of centroids only (kmeans_bounds_kernel).  A centroid for which it is clearly negative cannot win.
 // Tokens are taken in `order`, so a workgroup's 256 belong to a few clusters, and it walks the list of the centroids that can
-// win any of them.  Whatever is not a finite number has everything walked.
+// win any of them.  Whatever is not a finite number, or smaller than kFaint, has everything walked.
 // What it takes is a chain of dependent loads, some 9 us a workgroup, four rounds of them: ids, rows and old clusters, masks, the block of
-// centroids.  4 x 131072 tokens around 512 centres, 1024 centroids: 117 - 130 -> 47 us a step beside 9 us for the bounds, and of a
+// centroids.  4 x 131072 tokens around 512 centres, 1024 centroids: 117 - 130 -> 46 to 59 us a step, by the keys, beside 9 us for the bounds, and of a
 // run of ten steps, seven of which have bounds, 1410 -> 1102 us.  Three workgroups per CU (168 registers) spill: 35 us a workgroup.
 template <bool TRACK, int PARTS, bool NEAR = false>
 __global__ __launch_bounds__(kAssignWaves * 64, 1) void kmeans_assign_kernel(AssignArgs a) {
