@@ -89,15 +89,17 @@ def _bounded(groups: int, tokens: int, num_centroids: int, carried_steps: int) -
     """Whether a run's carried steps leave out centroids that cannot win, `tokens` those of one group.  In us: what a step saves on keys
     around C / 2 centres goes with the products left out, less the rows it gathers; its bounds go with the squares of the
     centroids and its launch is there in any case.  Preparing takes some 50 us once, and a run that finds nothing to leave out has lost
-    20 us and 2 a step, so that much has to be won.  Ten steps (seven carried), us without / with around 512 centres of width 0.3, and
-    with bounds around centres that overlap (width 0.8, without them): 1024 centroids 4 x 131072 tokens 1474 / 1204 (1468, 1437), 4 x 70000 966 /
-    846 (970, 938), 16 x 33000 1683 / 1525 (1725, 1676), 2 x 131072 882 / 846 (877, 849); outside 8 x 33000 992 / 991 (1019, 980), 1 x 131072
-    610 / 649, 16 x 20000 1156 / 1241; 2048 centroids 4 x 65536 1407 / 1230, outside 4 x 33000 1066 / 1072; 512 centroids 8 x 131072
-    1713 / 1612, outside 4 x 131072 985 / 961 (982, 947).  Five steps: 4 x 131072 889 / 848, outside 8 x 70000 979 / 956 (972, 945).
-    Fifty: 4 x 131072 tokens, 512 centroids 3694 / 3284, outside 4 x 20000, 1024 centroids 1727 / 2246."""
+    20 us and 2 a step, so that much has to be won.  Not where a step saves next to nothing, however many there are, nor with less than two
+    workgroups a CU, whose length is the chain of loads.  Ten steps (seven carried), us without / with around 512 centres of width 0.3, and
+    around centres that overlap (width 0.8): 1024 centroids 4 x 131072 tokens 1474 / 1204 (1437 / 1468), 4 x 62000 807 / 745
+    (785 / 817), 8 x 34000 970 / 930 (956 / 991), 16 x 28000 1397 / 1345 (1391 / 1432), 2 x 104000 769 / 743 (731 / 763); outside 8 x 33000
+    992 / 991 (980 / 1019), 1 x 131072 610 / 649, 16 x 24000 1256 / 1272.  2048 centroids 4 x 65536 1407 / 1230, outside 4 x 33000 1066 / 1072; 512
+    centroids 8 x 90000 1199 / 1139, outside 4 x 131072 985 / 961 (947 / 982).  Five steps, 1024 centroids: 4 x 122000 814 / 775 (791 / 813), outside
+    4 x 70000 599 / 605.  Forty or fifty: 4 x 131072 tokens, 512 centroids 3694 / 3284, 1024 centroids 8 x 34000 3223 / 2821, 4 x 45000 2109 /
+    1997, outside 1 x 131072 1634 / 1778, 4 x 20000 1727 / 2246."""
     rows, c = groups * tokens / 131072, num_centroids / 1024
-    saved = (16 * c - 3.5) * rows - 1.75 * groups * c * c - 6
-    return 512 <= num_centroids <= 2048 and carried_steps * saved >= 72
+    saved = (17.5 * c - 5) * rows - 1.4 * groups * c * c - 4
+    return 512 <= num_centroids <= 2048 and rows >= 1 and saved >= 7.5 and carried_steps * saved >= 72
 
 
 def segment_k_means(key, value, num_centroids: int, num_iters: int = 10, num_segments: int = 1):

@@ -265,11 +265,12 @@ def test_calls_take_the_general_way_without_the_native_host_calls(monkeypatch, t
 
 @pytest.mark.parametrize("groups,tokens,centroids,carried,bounded", [
     (4, 131072, 1024, 7, True), (4, 70000, 1024, 7, True), (8, 45000, 1024, 7, True), (16, 33000, 1024, 7, True), (4, 131072, 1024, 2, True),
-    (4, 65536, 2048, 7, True), (8, 131072, 512, 7, True), (4, 131072, 512, 47, True),
+    (4, 65536, 2048, 7, True), (8, 131072, 512, 7, True), (4, 131072, 512, 47, True), (8, 34000, 1024, 7, True), (2, 104000, 1024, 7, True),
+    (8, 34000, 1024, 37, True), (4, 45000, 1024, 37, True),
     # many groups of few tokens, and long runs over few tokens, where the bounds cost more than the products
     (64, 4096, 1024, 7, False), (16, 20000, 1024, 7, False), (1, 4096, 1024, 437, False), (1, 16384, 1024, 117, False), (1, 40000, 1024, 47, False),
     (8, 16384, 1024, 47, False), (16, 8192, 1024, 47, False), (8, 33000, 512, 47, False),
-    (1, 131072, 1024, 7, False), (4, 70000, 1024, 2, False), (8, 131072, 256, 7, False), (4, 131072, 4096, 7, False), (4, 131072, 1024, -2, False)])
+    (1, 131072, 1024, 7, False), (1, 131072, 1024, 37, False), (1, 100000, 2048, 7, False), (16, 24000, 1024, 7, False), (4, 70000, 1024, 2, False), (8, 131072, 256, 7, False), (4, 131072, 4096, 7, False), (4, 131072, 1024, -2, False)])
 def test_k_means_takes_bounds_where_they_measured_faster(groups, tokens, centroids, carried, bounded):
     from longcontext_sqattn_paddle_amd.cache_hub.kmeans import _bounded
 
